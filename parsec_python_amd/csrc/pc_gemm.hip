@@ -20,6 +20,7 @@
 // fixed order (deterministic).
 #include "pc_common.h"
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -44,22 +45,11 @@ template <> struct Acc<float> {
 };
 
 // Load 4 consecutive points [p, p+4) of column col; zero beyond n.
-template <typename T, bool VEC>
+template <typename T>
 __device__ __forceinline__ void load4(const T* __restrict__ base, long long ld, int col, int ncol, long long p,
                                       long long n, T out[4]) {
   if (col < ncol) {
     const T* src = base + (long long)col * ld + p;
-    if (VEC && p + 4 <= n) {
-      if constexpr (sizeof(T) == 4) {
-        const float4 t = *reinterpret_cast<const float4*>(src);
-        out[0] = t.x; out[1] = t.y; out[2] = t.z; out[3] = t.w;
-      } else {
-        const double2 t0 = *reinterpret_cast<const double2*>(src);
-        const double2 t1 = *reinterpret_cast<const double2*>(src + 2);
-        out[0] = t0.x; out[1] = t0.y; out[2] = t1.x; out[3] = t1.y;
-      }
-      return;
-    }
 #pragma unroll
     for (int s = 0; s < 4; ++s) out[s] = (p + s < n) ? src[s] : T(0);
     return;
@@ -86,8 +76,8 @@ __device__ __forceinline__ void tile_coords(int t, int ti_n, int tj_n, int sym, 
   tj = i + t;
 }
 
-// Workgroup = 4 waves, output tile 64x64 (each wave 32x32 = 2x2 MFMA tiles).
-template <typename T, bool VEC>
+// Any alignment: workgroup = 4 waves, output tile 64x64 (each wave 32x32 = 2x2 MFMA tiles).
+template <typename T>
 __global__ __launch_bounds__(256) void gram_kernel(const T* __restrict__ X, long long ldx, const T* __restrict__ Y,
                                                    long long ldy, long long n, int kx, int ky, int ti_n, int tj_n,
                                                    int ntile, int sym, int nchunk, long long chunk,
@@ -122,8 +112,8 @@ __global__ __launch_bounds__(256) void gram_kernel(const T* __restrict__ X, long
     const long long pl = p + 4 * lk;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      load4<T, VEC>(X, ldx, i0 + 16 * t + lm, kx, pl, pend, a[t]);
-      load4<T, VEC>(Y, ldy, j0 + 16 * t + lm, ky, pl, pend, bb[t]);
+      load4<T>(X, ldx, i0 + 16 * t + lm, kx, pl, pend, a[t]);
+      load4<T>(Y, ldy, j0 + 16 * t + lm, ky, pl, pend, bb[t]);
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s)
@@ -156,152 +146,201 @@ __global__ __launch_bounds__(256) void gram_kernel(const T* __restrict__ X, long
       }
 }
 
-// FP32 form with the operand tiles staged in LDS: per stage of 32 points the
-// workgroup loads its 64 X columns and 64 Y columns once (two float4 per thread
-// per operand) into one of two LDS buffers, and each wave reads its 32-column
-// halves from there, so every operand value comes from L2 once per workgroup
-// instead of once per wave.  The next stage's global loads are in flight while
-// the MFMAs run; one barrier per stage.  Same MFMA inputs and the same FP64
-// flush every 16 points as gram_kernel<float, true>, so the results match it.
-// Requires 16-byte aligned columns (ld % 4 == 0) and chunk % 32 == 0.
-__global__ __launch_bounds__(256) void gram_lds_f32(const float* __restrict__ X, long long ldx,
-                                                    const float* __restrict__ Y, long long ldy, long long n, int kx,
-                                                    int ky, int ti_n, int tj_n, int ntile, int sym, int nchunk,
-                                                    long long chunk, double* __restrict__ part) {
-  constexpr int SP = 32;        // points per stage
-  constexpr int LS = SP + 4;    // LDS row stride (floats)
-  __shared__ float xs[2][64 * LS], ys[2][64 * LS];
-  const int b0 = blockIdx.x;
-  const int tile = b0 % ntile;
-  const int ch = b0 / ntile;
+// Aligned operands: output tile 32 NT x 32 NT per workgroup (2 x 2 waves of
+// NT x NT MFMA tiles).  Per stage of 128 bytes of points (32 FP32, 16 FP64)
+// the workgroup loads its X and Y columns once, 16 bytes per lane and 128
+// contiguous bytes per column, into one of two LDS buffers; the next stage's
+// loads are in flight while the MFMAs run, one barrier per stage.  Columns past
+// the edge are loaded from the last column (their products only reach outputs
+// that gram_reduce skips), so the stage loop has no branches; only the last
+// chunk's last stage checks its points.  A symmetric tile on the diagonal of
+// X^T X reads one operand.  FP32: 16 points accumulate in the MFMA from zero
+// and are added to the FP64 accumulators while the next 16 run.
+// Bound by the MFMA rate once the operand strips stay on chip: consecutive
+// workgroups of one XCD take the tiles of one chunk, so its L2 serves the
+// columns to all of them (with the tiles dealt over the XCDs every L2 fetched
+// every column), and 96-wide tiles read each column a third less often than
+// 64-wide ones and pad 275 columns to 288, not 320.  FP32 MFMA and VALU do not
+// overlap on this chip (measured: 9 MFMAs and 16 FP64 additions take the sum of
+// their times), so the FP64 flush costs a fifth.  605,808 x 275, symmetric and
+// full: FP32 668 and 1027 us (803 and 1338 us with 64-wide tiles, every column
+// staged once per tile), FP64 1134 and 1701 us = 64 TF/s on the padded product
+// (2081 and 3987 us with operands loaded by each wave).
+constexpr int kGramStage = 128;   // bytes of one column per stage
+
+template <typename T, int NT>
+__global__ __launch_bounds__(256, 2) void gram_tile(const T* __restrict__ X, long long ldx, const T* __restrict__ Y,
+                                                    long long ldy, long long n, int kx, int ky, int ti_n, int tj_n,
+                                                    int ntile, int sym, int nblocks, int nb8, long long chunk,
+                                                    double* __restrict__ part) {
+  typedef typename Acc<T>::type AT;
+  constexpr int W = 32 * NT;
+  constexpr int SP = kGramStage / (int)sizeof(T);   // points per stage
+  constexpr int E = 16 / (int)sizeof(T);            // values per 16-byte load
+  constexpr int LS = SP + E;                        // LDS row stride (16 bytes of skew)
+  constexpr int G = SP / 16;                        // 16-point groups per stage
+  typedef T VT __attribute__((ext_vector_type(E)));
+  __shared__ __align__(16) T xs[2][W * LS], ys[2][W * LS];
+  const int L = (blockIdx.x & 7) * nb8 + (blockIdx.x >> 3);
+  if (L >= nblocks) return;
+  const int ch = L / ntile;
   int ti, tj;
-  tile_coords(tile, ti_n, tj_n, sym, ti, tj);
+  tile_coords(L - ch * ntile, ti_n, tj_n, sym, ti, tj);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int wi = w >> 1, wj = w & 1;
   const int lm = lane & 15, lk = lane >> 4;
-  const int ib = ti * 64, jb = tj * 64;
-  // loader: thread -> column lc of the tile, 8-point segment ls of the stage
-  const int lc = threadIdx.x >> 2, ls = (threadIdx.x & 3) * 8;
-  const bool xin = ib + lc < kx, yin = jb + lc < ky;
-  const float* __restrict__ xcol = X + (long long)(xin ? ib + lc : 0) * ldx;
-  const float* __restrict__ ycol = Y + (long long)(yin ? jb + lc : 0) * ldy;
-  const long long pbeg = (long long)ch * chunk;
-  const long long pend = min(n, pbeg + chunk);
-  float gx[8], gy[8];
-  auto gload = [&](long long p) {
-    const long long q = p + ls;
-    if (q + 8 <= pend) {
-      if (xin) {
-        const float4 t0 = *reinterpret_cast<const float4*>(xcol + q);
-        const float4 t1 = *reinterpret_cast<const float4*>(xcol + q + 4);
-        gx[0] = t0.x; gx[1] = t0.y; gx[2] = t0.z; gx[3] = t0.w; gx[4] = t1.x; gx[5] = t1.y; gx[6] = t1.z; gx[7] = t1.w;
-      } else {
+  const int seg = E * (threadIdx.x & 7);
+  double* out = part + (long long)L * (W * W);
+  // points [pbeg, pend): whole stages, or (EDGE) one stage with some points missing
+  auto body = [&](auto edge, long long pbeg, long long pend) {
+    constexpr bool EDGE = decltype(edge)::value;
+    const T *xp[NT], *yp[NT];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) gx[e] = 0.0f;
-      }
-      if (yin) {
-        const float4 t0 = *reinterpret_cast<const float4*>(ycol + q);
-        const float4 t1 = *reinterpret_cast<const float4*>(ycol + q + 4);
-        gy[0] = t0.x; gy[1] = t0.y; gy[2] = t0.z; gy[3] = t0.w; gy[4] = t1.x; gy[5] = t1.y; gy[6] = t1.z; gy[7] = t1.w;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) gy[e] = 0.0f;
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        gx[e] = (xin && q + e < pend) ? xcol[q + e] : 0.0f;
-        gy[e] = (yin && q + e < pend) ? ycol[q + e] : 0.0f;
-      }
+    for (int t = 0; t < NT; ++t) {
+      const int c = (threadIdx.x >> 3) + 32 * t;
+      xp[t] = X + (long long)min(ti * W + c, kx - 1) * ldx + seg;
+      yp[t] = Y + (long long)min(tj * W + c, ky - 1) * ldy + seg;
     }
-  };
-  auto sstore = [&](int bf) {
-    float* xd = &xs[bf][lc * LS + ls];
-    float* yd = &ys[bf][lc * LS + ls];
-    *reinterpret_cast<float4*>(xd) = make_float4(gx[0], gx[1], gx[2], gx[3]);
-    *reinterpret_cast<float4*>(xd + 4) = make_float4(gx[4], gx[5], gx[6], gx[7]);
-    *reinterpret_cast<float4*>(yd) = make_float4(gy[0], gy[1], gy[2], gy[3]);
-    *reinterpret_cast<float4*>(yd + 4) = make_float4(gy[4], gy[5], gy[6], gy[7]);
-  };
-  v4f acc[2][2];
-  double acc64[2][2][4];
+    VT gx[NT], gy[NT];
+    auto gload = [&](long long p) {
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+      for (int t = 0; t < NT; ++t) {
+        if constexpr (EDGE) {
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      acc[a][c] = v4f{0, 0, 0, 0};
+          for (int e = 0; e < E; ++e) {
+            const bool in = p + seg + e < pend;
+            gx[t][e] = in ? xp[t][p + e] : T(0);
+            gy[t][e] = in ? yp[t][p + e] : T(0);
+          }
+        } else {
+          gx[t] = *reinterpret_cast<const VT*>(xp[t] + p);
+          gy[t] = *reinterpret_cast<const VT*>(yp[t] + p);
+        }
+      }
+    };
+    auto sstore = [&](int bf) {
+      const int o = (threadIdx.x >> 3) * LS + seg;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc64[a][c][r] = 0.0;
-    }
-  if (pbeg < pend) {
+      for (int t = 0; t < NT; ++t) {
+        *reinterpret_cast<VT*>(&xs[bf][o + 32 * t * LS]) = gx[t];
+        *reinterpret_cast<VT*>(&ys[bf][o + 32 * t * LS]) = gy[t];
+      }
+    };
+    AT acc[NT][NT];
+    double acc64[NT][NT][4];
+#pragma unroll
+    for (int a = 0; a < NT; ++a)
+#pragma unroll
+      for (int c = 0; c < NT; ++c) {
+        acc[a][c] = AT{0, 0, 0, 0};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc64[a][c][r] = 0.0;
+      }
+    auto flush = [&]() {
+      if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int a = 0; a < NT; ++a)
+#pragma unroll
+          for (int c = 0; c < NT; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc64[a][c][r] += (double)acc[a][c][r];
+      }
+    };
     gload(pbeg);
     sstore(0);
-  }
-  __syncthreads();
-  int bf = 0;
-  for (long long p = pbeg; p < pend; p += SP) {
-    const bool more = p + SP < pend;
-    if (more) gload(p + SP);
-#pragma unroll
-    for (int g = 0; g < SP / 16; ++g) {
-      float a[2][4], bb[2][4];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const float4 av = *reinterpret_cast<const float4*>(&xs[bf][(wi * 32 + 16 * t + lm) * LS + 16 * g + 4 * lk]);
-        const float4 bv = *reinterpret_cast<const float4*>(&ys[bf][(wj * 32 + 16 * t + lm) * LS + 16 * g + 4 * lk]);
-        a[t][0] = av.x; a[t][1] = av.y; a[t][2] = av.z; a[t][3] = av.w;
-        bb[t][0] = bv.x; bb[t][1] = bv.y; bb[t][2] = bv.z; bb[t][3] = bv.w;
-      }
-#pragma unroll
-      for (int s2 = 0; s2 < 4; ++s2)
-#pragma unroll
-        for (int ta = 0; ta < 2; ++ta)
-#pragma unroll
-          for (int tb = 0; tb < 2; ++tb) acc[ta][tb] = Acc<float>::mfma(a[ta][s2], bb[tb][s2], acc[ta][tb]);
-#pragma unroll
-      for (int ta = 0; ta < 2; ++ta)
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc64[ta][tb][r] += (double)acc[ta][tb][r];
-          acc[ta][tb] = v4f{0, 0, 0, 0};
-        }
-    }
-    if (more) sstore(bf ^ 1);
     __syncthreads();
-    bf ^= 1;
-  }
-  double* out = part + ((long long)ch * ntile + tile) * 4096;
+    int bf = 0;
+    for (long long p = pbeg; p < pend; p += SP) {
+      if constexpr (!EDGE) gload(min(p + SP, pend - SP));   // (the last stage re-reads itself)
+      __builtin_amdgcn_sched_barrier(0);   // or the loads are sunk to their uses
+      const T* xb = &xs[bf][(wi * 16 * NT + lm) * LS + 4 * lk];
+      const T* yb = &ys[bf][(wj * 16 * NT + lm) * LS + 4 * lk];
 #pragma unroll
-  for (int ta = 0; ta < 2; ++ta)
+      for (int g = 0; g < G; ++g) {
+        T a[NT][4], b[NT][4];
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb)
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int ii = wi * 32 + 16 * ta + Acc<float>::row(lk, r);
-        const int jj = wj * 32 + 16 * tb + lm;
-        out[jj * 64 + ii] = acc64[ta][tb][r];
+          for (int h = 0; h < 4 / E; ++h) {
+            const VT av = *reinterpret_cast<const VT*>(xb + 16 * t * LS + 16 * g + E * h);
+            const VT bv = *reinterpret_cast<const VT*>(yb + 16 * t * LS + 16 * g + E * h);
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+              a[t][E * h + e] = av[e];
+              b[t][E * h + e] = bv[e];
+            }
+          }
+        flush();   // the previous 16 points
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int ta = 0; ta < NT; ++ta)
+#pragma unroll
+            for (int tb = 0; tb < NT; ++tb) {
+              const AT c0 = (sizeof(T) == 4 && s == 0) ? AT{0, 0, 0, 0} : acc[ta][tb];
+              acc[ta][tb] = Acc<T>::mfma(a[ta][s], b[tb][s], c0);
+            }
       }
+      bf ^= 1;
+      if constexpr (!EDGE) sstore(bf);
+      __syncthreads();
+    }
+    flush();
+#pragma unroll
+    for (int ta = 0; ta < NT; ++ta)
+#pragma unroll
+      for (int tb = 0; tb < NT; ++tb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int ii = (wi * NT + ta) * 16 + Acc<T>::row(lk, r);
+          const int jj = (wj * NT + tb) * 16 + lm;
+          out[jj * W + ii] = (sizeof(T) == 4) ? acc64[ta][tb][r] : (double)acc[ta][tb][r];
+        }
+  };
+  // chunk 0 is the last n % SP points when there are any, the others are whole stages
+  const long long nw = n / SP * SP;
+  if (nw < n && ch == 0) {
+    body(std::true_type{}, nw, n);
+  } else {
+    const long long pbeg = (long long)(ch - (nw < n ? 1 : 0)) * chunk;
+    body(std::false_type{}, pbeg, min(nw, pbeg + chunk));
+  }
 }
 
-// 16 workgroups per 64x64 tile, one element per thread; chunks summed in
-// order (deterministic)
-__global__ void gram_reduce(const double* __restrict__ part, int ntile, int nchunk, int ti_n, int tj_n, int kx,
-                            int ky, double* __restrict__ S, long long lds, int sym) {
-  const int tile = blockIdx.x >> 4;
+// Sum of the chunk partials of a W x W tile (W a multiple of 32): a workgroup
+// takes 32 consecutive elements, 8 threads each; thread g of an element adds
+// the chunks g, g + 8, ... in order and the 8 sums are added in order
+// (deterministic).  With one thread per element the chunks of a single-tile
+// Gram matrix were one serial chain (23 us at 385 chunks).
+__global__ __launch_bounds__(256) void gram_reduce(const double* __restrict__ part, int W, int ntile, int nchunk,
+                                                   int ti_n, int tj_n, int kx, int ky, double* __restrict__ S,
+                                                   long long lds, int sym) {
+  __shared__ double red[8][32];
+  const int per = W * W / 32;
+  const int tile = blockIdx.x / per;
   int ti, tj;
   tile_coords(tile, ti_n, tj_n, sym, ti, tj);
-  {
-    const int e = (blockIdx.x & 15) * 256 + threadIdx.x;
-    const int ii = e & 63, jj = e >> 6;
-    const int i = ti * 64 + ii, j = tj * 64 + jj;
-    if (i >= kx || j >= ky) return;
-    double s = 0.0;
-    // unrolled so that 16 loads per thread are in flight (the sum keeps its order)
-#pragma unroll 16
-    for (int c = 0; c < nchunk; ++c) s += part[((long long)c * ntile + tile) * 4096 + e];
-    S[(long long)j * lds + i] = s;
-    if (sym && ti != tj) S[(long long)i * lds + j] = s;
+  const int el = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const int e = (blockIdx.x - tile * per) * 32 + el;
+  const int jj = e / W, ii = e - jj * W;
+  const int i = ti * W + ii, j = tj * W + jj;
+  const bool in = i < kx && j < ky;
+  double s = 0.0;
+  if (in) {
+    const double* p = part + (long long)tile * W * W + e;
+    const long long st = (long long)ntile * W * W;
+#pragma unroll 8
+    for (int c = g; c < nchunk; c += 8) s += p[c * st];
+  }
+  red[g][el] = s;
+  __syncthreads();
+  if (g == 0 && in) {
+    double t = red[0][el];
+#pragma unroll
+    for (int q = 1; q < 8; ++q) t += red[q][el];
+    S[(long long)j * lds + i] = t;
+    if (sym && ti != tj) S[(long long)i * lds + j] = t;
   }
 }
 
@@ -357,117 +396,147 @@ __global__ __launch_bounds__(256) void rotate_kernel(const T* __restrict__ X, lo
       }
 }
 
-// FP32 form with every output column in one workgroup, so X is read from
-// memory once: waves (pw, cw) = (point half, column half) of 128 points x
-// 32*NCH columns; a wave accumulates 64 points x NCH column tiles.  Its 64
-// points form 4 interleaved tiles (tile j = points 4 n + j), so each lane loads
-// the 4 consecutive points it feeds to the 4 tiles with one float4 per
-// 4-vector step and stores them back with one float4 per output row.  Q^T
-// comes through LDS in 16-vector slabs (double-buffered; the next slab is
-// fetched into registers while the MFMAs run).  Requires ky <= 32*NCH,
-// 16-byte aligned X/Z columns (ld % 4 == 0).
-template <int NCH>
-__global__ __launch_bounds__(256, 2) void rotate_wide_f32(const float* __restrict__ X, long long ldx,
-                                                       const float* __restrict__ Qt, float* __restrict__ Z,
-                                                       long long ldz, long long n, int kx, int ky, int nblocks,
-                                                       int nb8) {
-  constexpr int KS = 16;             // vectors per Q slab
-  constexpr int NC = 32 * NCH;       // columns per workgroup
-  constexpr int QPT = KS * NC / 256; // slab values per thread
-  __shared__ float qs[2][KS * NC];
+// Aligned operands: up to 288 output columns in one workgroup, so X is read
+// from memory once.  Waves (pw, cw) = (point half, column half) of 32 E points x
+// 32 NCH columns, E = 16 / sizeof(T) points per lane: a wave's points form E
+// interleaved tiles (tile j = points E n + j), so each lane loads the E
+// consecutive points it feeds to the E tiles with one 16-byte load per vector
+// and stores them back with one per output row.  Q^T comes through LDS in slabs
+// of KS vectors (two buffers; the next slab's Q and X are in flight while the
+// MFMAs run).  Only the last slab and the last workgroup check their edges, so
+// the slab loop has no branches.  The k order is that of rotate_kernel, so the
+// results are the same bits.  Bound by the MFMA rate and the stores at a
+// workgroup's end (without them 80 us less); 605,808 x 275: FP32 818 us = 112
+// TF/s (1067 us with Q guarded per value, 115 instead of 31 vector instructions
+// beside a slab's 144 MFMAs), FP64 1669 us (2987 us with 64 columns per
+// workgroup and Q from memory).
+template <typename T, int NCH>
+__global__ __launch_bounds__(256, 2) void rotate_wide(const T* __restrict__ X, long long ldx,
+                                                      const T* __restrict__ Qt, T* __restrict__ Z, long long ldz,
+                                                      long long n, int kx, int ky, int ncb, int nblocks, int nb8) {
+  typedef typename Acc<T>::type AT;
+  constexpr int E = 16 / (int)sizeof(T);
+  constexpr int KS = 16;                         // vectors per slab
+  constexpr int ST = KS / 4;                     // MFMA steps per slab
+  constexpr int NC = 32 * NCH;                   // columns per workgroup
+  constexpr int LQ = NC + 64 / (int)sizeof(T);   // LDS row stride
+  constexpr int TR = 256 / KS;                   // threads per Q row
+  constexpr int QPT = NC / TR;                   // Q values per thread
+  typedef T VT __attribute__((ext_vector_type(E)));
+  __shared__ T qs[2][KS * LQ];
   const int L = (blockIdx.x & 7) * nb8 + (blockIdx.x >> 3);
   if (L >= nblocks) return;
+  const int cb = L % ncb;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int pw = w >> 1, cw = w & 1;
   const int lm = lane & 15, lk = lane >> 4;
-  const long long pl = (long long)L * 128 + pw * 64 + 4 * lm;   // this lane's 4 points
-  const int c0 = cw * 16 * NCH;
-  v4f acc[NCH][4];
+  const long long p0 = (long long)(L / ncb) * (32 * E);
+  const long long pl = p0 + pw * 16 * E + E * lm;   // this lane's E points
+  // blocks of NC columns, the last one moved back to end at ky (the columns it
+  // shares with its neighbour are the same bits)
+  const int c0 = min(cb * NC, max(ky - NC, 0));
+  const int qk = threadIdx.x / TR, qc = threadIdx.x % TR;
+  // the whole product for one kind of workgroup (EDGE: some points past n)
+  auto body = [&](auto edge) {
+    constexpr bool EDGE = decltype(edge)::value;
+    AT acc[NCH][E];
 #pragma unroll
-  for (int c = 0; c < NCH; ++c)
+    for (int c = 0; c < NCH; ++c)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[c][j] = v4f{0, 0, 0, 0};
-  float qr[QPT];
-  auto qfetch = [&](int kb) {
+      for (int j = 0; j < E; ++j) acc[c][j] = AT{0, 0, 0, 0};
+    // vectors past kx (last slab) are read from the last one and replaced by
+    // zero before use; only the last 32 columns of a block can lie past ky:
+    // they are read from column ky - 1 and their products are not stored
+    T qr[QPT], x[ST][E];
+    auto qfetch = [&](int kb) {
+      const T* src = Qt + (long long)kb * ky + c0 + (unsigned)(min(qk, kx - 1 - kb) * ky);
 #pragma unroll
-    for (int t = 0; t < QPT; ++t) {
-      const int e = threadIdx.x + 256 * t;
-      const int kk = e / NC, col = e - kk * NC;
-      qr[t] = (kb + kk < kx && col < ky) ? Qt[(long long)(kb + kk) * ky + col] : 0.0f;
-    }
-  };
-  auto qstore = [&](int bf) {
-#pragma unroll
-    for (int t = 0; t < QPT; ++t) qs[bf][threadIdx.x + 256 * t] = qr[t];
-  };
-  const bool full = pl + 3 < n;
-  // X of one slab (4 steps x 4 points per lane), fetched one slab ahead
-  float xc[KS / 4][4], xn[KS / 4][4];
-  auto xfetch = [&](int kb, float (&xo)[KS / 4][4]) {
-#pragma unroll
-    for (int st = 0; st < KS / 4; ++st) {
-      const int kk = kb + 4 * st + lk;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) xo[st][j] = 0.0f;
-      if (kk < kx) {
-        const float* xr = X + (long long)kk * ldx + pl;
-        if (full) {
-          const float4 t = *reinterpret_cast<const float4*>(xr);
-          xo[st][0] = t.x; xo[st][1] = t.y; xo[st][2] = t.z; xo[st][3] = t.w;
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) xo[st][j] = pl + j < n ? xr[j] : 0.0f;
-        }
+      for (int t = 0; t < QPT; ++t) {
+        const int col = qc + TR * t;
+        qr[t] = src[t < QPT - 32 / TR ? col : min(col, ky - 1 - c0)];
       }
-    }
-  };
-  qfetch(0);
-  xfetch(0, xc);
-  qstore(0);
-  __syncthreads();
-  int bf = 0;
-  for (int kb = 0; kb < kx; kb += KS) {
-    const bool more = kb + KS < kx;
-    if (more) {
-      qfetch(kb + KS);
-      xfetch(kb + KS, xn);
-    }
+    };
+    auto qstore = [&](int bf) {
 #pragma unroll
-    for (int st = 0; st < KS / 4; ++st) {
-      const float* qrow = &qs[bf][(4 * st + lk) * NC + c0 + lm];
+      for (int t = 0; t < QPT; ++t) qs[bf][qk * LQ + qc + TR * t] = qr[t];
+    };
+    // X of step st of the slab at kb (32-bit offsets from the slab's first vector)
+    auto xfetch = [&](int kb, int st) {
+      const char* base = reinterpret_cast<const char*>(X + (long long)kb * ldx);
+      const unsigned off = ((unsigned)min(4 * st + lk, kx - 1 - kb) * (unsigned)ldx + (unsigned)pl) * (unsigned)sizeof(T);
+      if constexpr (EDGE) {
+#pragma unroll
+        for (int j = 0; j < E; ++j) x[st][j] = pl + j < n ? *reinterpret_cast<const T*>(base + off + sizeof(T) * j) : T(0);
+      } else {
+        const VT t = *reinterpret_cast<const VT*>(base + off);
+#pragma unroll
+        for (int j = 0; j < E; ++j) x[st][j] = t[j];
+      }
+    };
+    auto step = [&](int bf, int st) {
+      const T* qrow = &qs[bf][(4 * st + lk) * LQ + cw * 16 * NCH + lm];
 #pragma unroll
       for (int c = 0; c < NCH; ++c) {
-        const float qa = qrow[16 * c];
+        const T qa = qrow[16 * c];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[c][j] = Acc<float>::mfma(qa, xc[st][j], acc[c][j]);
+        for (int j = 0; j < E; ++j) acc[c][j] = Acc<T>::mfma(qa, x[st][j], acc[c][j]);
       }
-    }
-    if (more) {
-      qstore(bf ^ 1);
+    };
+    const int klast = (kx - 1) / KS * KS;   // the last slab, whole or not
+    qfetch(0);
 #pragma unroll
-      for (int st = 0; st < KS / 4; ++st)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) xc[st][j] = xn[st][j];
-    }
+    for (int st = 0; st < ST; ++st) xfetch(0, st);
+    qstore(0);
     __syncthreads();
-    bf ^= 1;
-  }
-  // lane (lm, lk) register r of tile (c, j): column c0 + 16c + 4lk + r, point pl + j
+    int bf = 0;
+    for (int kb = 0; kb < klast; kb += KS) {
+      qfetch(kb + KS);
+      __builtin_amdgcn_sched_barrier(0);   // or the loads are sunk to their uses
 #pragma unroll
-  for (int c = 0; c < NCH; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int col = c0 + 16 * c + Acc<float>::row(lk, r);
-      if (col >= ky) continue;
-      float* zr = Z + (long long)col * ldz + pl;
-      if (full) {
-        *reinterpret_cast<float4*>(zr) = make_float4(acc[c][0][r], acc[c][1][r], acc[c][2][r], acc[c][3][r]);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (pl + j < n) zr[j] = acc[c][j][r];
+      for (int st = 0; st < ST; ++st) {
+        step(bf, st);
+        xfetch(kb + KS, st);   // into the registers the step has read
+        __builtin_amdgcn_sched_barrier(0);
       }
+      bf ^= 1;
+      qstore(bf);
+      __syncthreads();
     }
+    if (klast + KS > kx) {
+      if (klast + qk >= kx) {
+#pragma unroll
+        for (int t = 0; t < QPT; ++t) qs[bf][qk * LQ + qc + TR * t] = T(0);
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int st = 0; st < ST; ++st) {
+#pragma unroll
+      for (int j = 0; j < E; ++j) x[st][j] = klast + 4 * st + lk < kx ? x[st][j] : T(0);
+      if (klast + 4 * st < kx) step(bf, st);
+    }
+    // register r of tile (c, j): column c0 + 16 c + row(lk, r), point pl + j
+#pragma unroll
+    for (int c = 0; c < NCH; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int col = c0 + (cw * NCH + c) * 16 + Acc<T>::row(lk, r);
+        if (col >= ky) continue;
+        T* zr = Z + (long long)col * ldz + pl;
+        if constexpr (EDGE) {
+#pragma unroll
+          for (int j = 0; j < E; ++j)
+            if (pl + j < n) zr[j] = acc[c][j][r];
+        } else {
+          VT t;
+#pragma unroll
+          for (int j = 0; j < E; ++j) t[j] = acc[c][j][r];
+          *reinterpret_cast<VT*>(zr) = t;
+        }
+      }
+  };
+  if (p0 + 32 * E <= n) body(std::false_type{});
+  else body(std::true_type{});
 }
 
 // FP32 rotation on bf16 MFMA with three-way splits: every FP32 operand value
@@ -653,27 +722,55 @@ __global__ void convert_q_f64(const double* __restrict__ Q, int ldq, int kx, int
 }
 
 struct GramPlan {
+  int nt;                    // MFMA tiles per wave and side (tile of 32 nt columns)
   int ti_n, tj_n, ntile, nchunk;
   long long chunk;
+  long long tile_size() const { return 1024LL * nt * nt; }
 };
 
-GramPlan plan_gram(long long n, int kx, int ky, int sym) {
-  GramPlan p;
-  p.ti_n = (kx + 63) / 64;
-  p.tj_n = (ky + 63) / 64;
-  p.ntile = sym ? p.ti_n * (p.ti_n + 1) / 2 : p.ti_n * p.tj_n;
-  long long target = std::max<long long>(1, 2048 / p.ntile);
-  long long maxch = std::max<long long>(1, (n + 1023) / 1024);
+// Tile width: the one whose padded tiles cost least, a 64-wide tile's product
+// counted at 1.1 and a 32-wide one's at 1.4 of a 96-wide one's (they read each
+// column 1.5 and 3 times as often); so 33..64 and 193..256 columns take 64-wide
+// tiles, 65..96 and 257..288 columns 96-wide ones.  Chunks: about as many workgroups as the
+// chip holds at once, all with the same work (one round, no short last one),
+// and at least 256 points each; sp = points per stage.
+GramPlan plan_gram(long long n, int kx, int ky, int sym, int sp) {
+  GramPlan p{};
+  double best = 0.0;
+  for (int nt = 3; nt >= 1; --nt) {
+    const int w = 32 * nt, ti = (kx + w - 1) / w, tj = (ky + w - 1) / w;
+    const int ntile = sym ? ti * (ti + 1) / 2 : ti * tj;
+    const double cost = (double)ntile * w * w * (nt == 3 ? 1.0 : nt == 2 ? 1.1 : 1.4);
+    if (p.nt == 0 || cost < best) {
+      best = cost;
+      p.nt = nt; p.ti_n = ti; p.tj_n = tj; p.ntile = ntile;
+    }
+  }
+  const int resident = p.nt == 3 ? 512 : p.nt == 2 ? 1024 : 2048;
+  const int rest = n % sp != 0;   // the points past the last whole stage are a chunk of their own
+  const long long target = std::max<long long>(1, resident / p.ntile - rest);
+  const long long maxch = std::max<long long>(1, (n + 255) / 256);
+  const long long nw = n - n % sp;
   p.nchunk = (int)std::min(target, maxch);
-  long long chunk = (n + p.nchunk - 1) / p.nchunk;
-  chunk = (chunk + 31) / 32 * 32;   // whole 32-point stages of gram_lds_f32
-  p.chunk = chunk;
-  p.nchunk = (int)((n + chunk - 1) / chunk);
-  if (p.nchunk < 1) p.nchunk = 1;
+  p.chunk = std::max<long long>(32, ((nw + p.nchunk - 1) / p.nchunk + 31) / 32 * 32);
+  p.nchunk = (int)((nw + p.chunk - 1) / p.chunk) + rest;
   return p;
 }
 
-size_t gram_work_bytes(const GramPlan& p) { return (size_t)p.nchunk * p.ntile * 4096 * sizeof(double); }
+// The form for unaligned columns keeps 64-wide tiles.
+GramPlan plan_gram_unaligned(long long n, int kx, int ky, int sym) {
+  GramPlan p{};
+  p.nt = 2;
+  p.ti_n = (kx + 63) / 64;
+  p.tj_n = (ky + 63) / 64;
+  p.ntile = sym ? p.ti_n * (p.ti_n + 1) / 2 : p.ti_n * p.tj_n;
+  p.nchunk = (int)std::min(std::max<long long>(1, 2048 / p.ntile), std::max<long long>(1, (n + 1023) / 1024));
+  p.chunk = ((n + p.nchunk - 1) / p.nchunk + 31) / 32 * 32;
+  p.nchunk = (int)((n + p.chunk - 1) / p.chunk);
+  return p;
+}
+
+size_t gram_work_bytes(const GramPlan& p) { return (size_t)p.nchunk * p.ntile * p.tile_size() * sizeof(double); }
 
 template <typename T>
 int gram_impl(const T* X, long long ldx, const T* Y, long long ldy, long long n, int kx, int ky, double* S,
@@ -682,34 +779,30 @@ int gram_impl(const T* X, long long ldx, const T* Y, long long ldy, long long n,
   PC_CHECK_ARG(n >= 1 && kx >= 1 && ky >= 1, "empty operand");
   PC_CHECK_ARG(ldx >= n && ldy >= n && lds >= kx, "leading dimension too small");
   PC_CHECK_ARG(!sym || (kx == ky), "sym requires kx == ky");
-  GramPlan p = plan_gram(n, kx, ky, sym);
+  constexpr int E = 16 / (int)sizeof(T);
+  const bool vec = (ldx % E == 0) && (ldy % E == 0) && (reinterpret_cast<uintptr_t>(X) % 16 == 0) &&
+                   (reinterpret_cast<uintptr_t>(Y) % 16 == 0);
+  const GramPlan p = vec ? plan_gram(n, kx, ky, sym, kGramStage / (int)sizeof(T)) : plan_gram_unaligned(n, kx, ky, sym);
   PC_CHECK_ARG(work_bytes >= gram_work_bytes(p), "workspace too small");
   hipStream_t st = static_cast<hipStream_t>(stream);
   double* part = static_cast<double*>(work);
-  const bool vec = (ldx % 4 == 0) && (ldy % 4 == 0) &&
-                   (reinterpret_cast<uintptr_t>(X) % (4 * sizeof(T)) == 0) &&
-                   (reinterpret_cast<uintptr_t>(Y) % (4 * sizeof(T)) == 0);
-  dim3 grid(p.ntile * p.nchunk);
-  if constexpr (sizeof(T) == 4) {
-    if (vec) {
-      hipLaunchKernelGGL(gram_lds_f32, grid, dim3(256), 0, st, X, ldx, Y, ldy, n, kx, ky, p.ti_n, p.tj_n, p.ntile,
-                         sym, p.nchunk, p.chunk, part);
-      PC_LAUNCH_CHECK();
-      hipLaunchKernelGGL(gram_reduce, dim3(16 * p.ntile), dim3(256), 0, st, part, p.ntile, p.nchunk, p.ti_n, p.tj_n,
-                         kx, ky, S, lds, sym);
-      PC_LAUNCH_CHECK();
-      return pc::PC_OK;
-    }
+  const int nb = p.ntile * p.nchunk, nb8 = (nb + 7) / 8;
+  if (vec) {
+#define PC_GRAM(NT)                                                                                              \
+  hipLaunchKernelGGL((gram_tile<T, NT>), dim3(8 * nb8), dim3(256), 0, st, X, ldx, Y, ldy, n, kx, ky, p.ti_n, p.tj_n, \
+                     p.ntile, sym, nb, nb8, p.chunk, part)
+    if (p.nt == 1) PC_GRAM(1);
+    else if (p.nt == 2) PC_GRAM(2);
+    else PC_GRAM(3);
+#undef PC_GRAM
+  } else {
+    hipLaunchKernelGGL((gram_kernel<T>), dim3(nb), dim3(256), 0, st, X, ldx, Y, ldy, n, kx, ky, p.ti_n, p.tj_n,
+                       p.ntile, sym, p.nchunk, p.chunk, part);
   }
-  if (vec)
-    hipLaunchKernelGGL((gram_kernel<T, true>), grid, dim3(256), 0, st, X, ldx, Y, ldy, n, kx, ky, p.ti_n, p.tj_n,
-                       p.ntile, sym, p.nchunk, p.chunk, part);
-  else
-    hipLaunchKernelGGL((gram_kernel<T, false>), grid, dim3(256), 0, st, X, ldx, Y, ldy, n, kx, ky, p.ti_n, p.tj_n,
-                       p.ntile, sym, p.nchunk, p.chunk, part);
   PC_LAUNCH_CHECK();
-  hipLaunchKernelGGL(gram_reduce, dim3(16 * p.ntile), dim3(256), 0, st, part, p.ntile, p.nchunk, p.ti_n, p.tj_n, kx,
-                     ky, S, lds, sym);
+  const int w = 32 * p.nt;
+  hipLaunchKernelGGL(gram_reduce, dim3(p.ntile * (w * w / 32)), dim3(256), 0, st, part, w, p.ntile, p.nchunk, p.ti_n,
+                     p.tj_n, kx, ky, S, lds, sym);
   PC_LAUNCH_CHECK();
   return pc::PC_OK;
 }
@@ -733,9 +826,11 @@ int rotate_impl(const T* X, long long ldx, const double* Q, int ldq, T* Z, long 
     PC_LAUNCH_CHECK();
     return pc::PC_OK;
   };
+  constexpr int E = 16 / (int)sizeof(T);
+  const bool vec = (ldx % E == 0) && (ldz % E == 0) && (reinterpret_cast<uintptr_t>(X) % 16 == 0) &&
+                   (reinterpret_cast<uintptr_t>(Z) % 16 == 0) &&
+                   ldx < (1LL << 24);   // 16 vectors in 32-bit byte offsets
   if constexpr (sizeof(T) == 4) {
-    const bool vec = (ldx % 4 == 0) && (ldz % 4 == 0) && (reinterpret_cast<uintptr_t>(X) % 16 == 0) &&
-                     (reinterpret_cast<uintptr_t>(Z) % 16 == 0);
     const int nch = (ky + 31) / 32;
     if (vec && nch <= 9 && g_rotate_bf3 && work_bytes >= bf3_work_bytes(kx, ky)) {
       unsigned short* qp = static_cast<unsigned short*>(work);
@@ -757,21 +852,27 @@ int rotate_impl(const T* X, long long ldx, const double* Q, int ldq, T* Z, long 
       PC_LAUNCH_CHECK();
       return pc::PC_OK;
     }
-    if (vec && nch <= 9) {
-      if (convert_q() != pc::PC_OK) return pc::PC_ERR_HIP;
-      const int nb = (int)((n + 127) / 128);
-      const int nb8 = (nb + 7) / 8;
-      switch (nch) {
-#define PC_ROT(N)                                                                                                 \
-  case N:                                                                                                         \
-    hipLaunchKernelGGL(rotate_wide_f32<N>, dim3(8 * nb8), dim3(256), 0, st, X, ldx, qt, Z, ldz, n, kx, ky, nb, nb8); \
+  }
+  if (vec) {
+    if (convert_q() != pc::PC_OK) return pc::PC_ERR_HIP;
+    // column blocks of at most 288, of equal width
+    const int ncb = (ky + 287) / 288;
+    const int nch = ((ky + ncb - 1) / ncb + 31) / 32;
+    const long long npt = (n + 32 * E - 1) / (32 * E);
+    PC_CHECK_ARG(npt * ncb < (1LL << 30), "too many workgroups");
+    const int nb = (int)(npt * ncb);
+    const int nb8 = (nb + 7) / 8;
+    switch (nch) {
+#define PC_ROT(N)                                                                                                   \
+  case N:                                                                                                           \
+    hipLaunchKernelGGL((rotate_wide<T, N>), dim3(8 * nb8), dim3(256), 0, st, X, ldx, qt, Z, ldz, n, kx, ky, ncb, nb, \
+                       nb8);                                                                                        \
     break;
-        PC_ROT(1) PC_ROT(2) PC_ROT(3) PC_ROT(4) PC_ROT(5) PC_ROT(6) PC_ROT(7) PC_ROT(8) PC_ROT(9)
+      PC_ROT(1) PC_ROT(2) PC_ROT(3) PC_ROT(4) PC_ROT(5) PC_ROT(6) PC_ROT(7) PC_ROT(8) PC_ROT(9)
 #undef PC_ROT
-      }
-      PC_LAUNCH_CHECK();
-      return pc::PC_OK;
     }
+    PC_LAUNCH_CHECK();
+    return pc::PC_OK;
   }
   if (convert_q() != pc::PC_OK) return pc::PC_ERR_HIP;
   const int npt = (int)((n + 127) / 128);
@@ -790,7 +891,8 @@ extern "C" {
 
 int pc_gram_workspace(long long n, int kx, int ky, int sym, size_t* out_bytes) {
   PC_CHECK_ARG(out_bytes, "null pointer");
-  *out_bytes = gram_work_bytes(plan_gram(n, kx, ky, sym));
+  *out_bytes = std::max({gram_work_bytes(plan_gram(n, kx, ky, sym, 16)), gram_work_bytes(plan_gram(n, kx, ky, sym, 32)),
+                         gram_work_bytes(plan_gram_unaligned(n, kx, ky, sym))});
   return pc::PC_OK;
 }
 
