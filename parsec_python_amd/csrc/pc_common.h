@@ -43,10 +43,39 @@ constexpr int kWave = 64;
 
 #define PC_LAUNCH_CHECK() PC_HIP(hipGetLastError())
 
+// Sum over the 64 lanes of a wavefront, in every lane: lane l and l ^ 32, then
+// ^ 16, 8, 4, 2, 1 (the order of a shuffle-down tree, whose lane 0 has the same
+// bits).  Lane swaps and row rotations instead of six LDS permutes, which a
+// short kernel's reduction waits for one after the other.
+__device__ __forceinline__ double pc_wave_sum(double v) {
+  auto bits = [](double x) { return __builtin_bit_cast(unsigned long long, x); };
+  auto make = [](unsigned lo, unsigned hi) {
+    return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+  };
+  {
+    const unsigned lo = (unsigned)bits(v), hi = (unsigned)(bits(v) >> 32);
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    v = make(l[0], h[0]) + make(l[1], h[1]);
+  }
+  {
+    const unsigned lo = (unsigned)bits(v), hi = (unsigned)(bits(v) >> 32);
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    v = make(l[0], h[0]) + make(l[1], h[1]);
+  }
+#define PC_ROW_ROR(N)                                                                                       \
+  v += make((unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)bits(v), 0x120 + N, 0xf, 0xf, true),          \
+            (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(bits(v) >> 32), 0x120 + N, 0xf, 0xf, true));
+  PC_ROW_ROR(8) PC_ROW_ROR(4) PC_ROW_ROR(2) PC_ROW_ROR(1)
+#undef PC_ROW_ROR
+  return v;
+}
+
 // Block-wide FP64 sum of one value per thread (blockDim.x multiple of 64,
 // <= 1024).  Result valid in thread 0.
 __device__ inline double pc_block_sum(double v, double* sh) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+  v = pc_wave_sum(v);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   __syncthreads();
   if (lane == 0) sh[wid] = v;
@@ -56,5 +85,38 @@ __device__ inline double pc_block_sum(double v, double* sh) {
     const int nw = (blockDim.x + 63) >> 6;
     for (int w = 0; w < nw; ++w) r += sh[w];
   }
+  return r;
+}
+
+// Sum of part[0 .. nb), nb <= 8 NT, in every thread: thread t < NT adds
+// part[t], part[t + NT], ... in order, then the wavefronts' sums are added in
+// order.  All loads are in flight together.  sh: blockDim.x / 64 doubles, not
+// used since the last barrier by anything else.
+template <int NT>
+__device__ __forceinline__ double pc_parts_load(const double* part, int nb) {
+  double v[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    v[k] = 0.0;
+    if (NT * k < nb) {   // the same in every thread
+      const int b = (int)threadIdx.x + NT * k;
+      const double t = part[b < nb ? b : 0];
+      v[k] = b < nb && threadIdx.x < NT ? t : 0.0;
+    }
+  }
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) s += v[k];
+  return s;
+}
+__device__ __forceinline__ void pc_parts_post(double s, double* sh) {
+  s = pc_wave_sum(s);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+}
+template <int NT>   // after a barrier
+__device__ __forceinline__ double pc_parts_get(const double* sh) {
+  double r = 0.0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) r += sh[w];
   return r;
 }

@@ -730,8 +730,8 @@ struct GramPlan {
 
 // Tile width: the one whose padded tiles cost least, a 64-wide tile's product
 // counted at 1.1 and a 32-wide one's at 1.4 of a 96-wide one's (they read each
-// column 1.5 and 3 times as often); so 33..64 and 193..256 columns take 64-wide
-// tiles, 65..96 and 257..288 columns 96-wide ones.  Chunks: about as many workgroups as the
+// column 1.5 and 3 times as often); so 275 columns take 96-wide
+// tiles, 256 take 64-wide ones and a symmetric product of up to 96 32-wide ones.  Chunks: about as many workgroups as the
 // chip holds at once, all with the same work (one round, no short last one),
 // and at least 256 points each; sp = points per stage.
 GramPlan plan_gram(long long n, int kx, int ky, int sym, int sp) {

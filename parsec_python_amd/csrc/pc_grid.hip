@@ -1273,40 +1273,56 @@ int launch_direct_r(const GridDev* gd, const T* Y, const T* X, T* Out, const T* 
   return pc::PC_OK;
 }
 
-// One FP64 vector (the Lanczos bounds): the z-march of the CG step over
-// z-chunks (pc_zmarch.h), so each point's neighbours come from registers and
-// LDS instead of dependent row-table loads.  Out may alias X.
+// One FP64 vector (the Lanczos bounds): the pass of the CG step (pc_zmarch.h),
+// so each point's neighbours come from registers and LDS instead of dependent
+// row-table loads.  Out may alias X.
+struct SinglePass {
+  struct Raw { double y; };
+  struct Ext { double v, x; };
+  static constexpr bool DOT = false, POST = false;
+  const double* __restrict__ Y;
+  const double* X;
+  double* Out;
+  const double* __restrict__ V;
+  double ca, cb, cc;
+  __device__ __forceinline__ Raw load(long long idx, bool, int, int, int) const { return {Y[idx]}; }
+  __device__ __forceinline__ Ext ext(long long idx) const { return {V[idx], X ? X[idx] : 0.0}; }
+  __device__ __forceinline__ bool pre() const { return true; }
+  __device__ __forceinline__ double comb(Raw r) const { return r.y; }
+  __device__ __forceinline__ void out(bool in, long long idx, Raw, Ext e, double qc, double acc, double&,
+                                      double&) const {
+    double o = acc + (ca * e.v + cb) * qc;
+    if (X) o += cc * e.x;
+    if (in) Out[idx] = o;
+  }
+};
+
 template <int R, int SX>
-__global__ __launch_bounds__(256) void stencil_single(pcz::ZMap zm, const double* __restrict__ Y, const double* X,
-                                                      double* Out, const double* __restrict__ V, double ca,
-                                                      double cb, double cc) {
+__global__ __launch_bounds__(pcz::threads(SX), SX == 2 ? 4 : 2) void stencil_single(pcz::ZMap zm, SinglePass p) {
   __shared__ double tile[pcz::Tile<R, SX>::SIZE];
   const int L = pcz::block_of(zm);
   if (L >= zm.nwg) return;
-  pcz::zmarch<R, SX>(
-      zm, L, tile, [&](long long idx, int, int, int) { return Y[idx]; },
-      [&](long long idx, int, int, int, double qc, double acc) {
-        double o = acc + (ca * V[idx] + cb) * qc;
-        if (X) o += cc * X[idx];
-        Out[idx] = o;
-      });
+  double s;
+  pcz::zpass<R, SX, pcz::kZW, false, false, false>(zm, L, tile, p, s);
 }
 
 template <int R>
 int launch_single_r(const pcz::ZMap& zm, const double* Y, const double* X, double* Out, const double* V, double ca,
                     double cb, double cc, hipStream_t st) {
-  const dim3 grid(8 * zm.nwg8), block(256);
+  const dim3 grid(8 * zm.nwg8), block(pcz::threads(zm.sx));
+  const SinglePass p{Y, X, Out, V, ca, cb, cc};
   switch (zm.sx) {
-    case 1: hipLaunchKernelGGL((stencil_single<R, 1>), grid, block, 0, st, zm, Y, X, Out, V, ca, cb, cc); break;
-    case 2: hipLaunchKernelGGL((stencil_single<R, 2>), grid, block, 0, st, zm, Y, X, Out, V, ca, cb, cc); break;
-    default: hipLaunchKernelGGL((stencil_single<R, 4>), grid, block, 0, st, zm, Y, X, Out, V, ca, cb, cc); break;
+    case 1: hipLaunchKernelGGL((stencil_single<R, 1>), grid, block, 0, st, zm, p); break;
+    case 2: hipLaunchKernelGGL((stencil_single<R, 2>), grid, block, 0, st, zm, p); break;
+    default: hipLaunchKernelGGL((stencil_single<R, 4>), grid, block, 0, st, zm, p); break;
   }
   PC_LAUNCH_CHECK();
   return pc::PC_OK;
 }
 
-// Measured on Si87H76 (605,808 points, radius 4): one FP64 vector 17 us, 46 us
-// with stencil_direct (same summation order, so the same bits).
+// Measured on the C10H8 sphere (394,264 points, radius 4): one FP64 vector 12.2
+// us (17.0 us marching with one plane of loads in flight; on Si87H76's 605,808
+// points that was 17 us, stencil_direct 46 us; the same bits).
 int single_dispatch(void* grid, const double* Y, const double* X, double* Out, const double* V, double scale,
                     double ca, double cb, double cc, hipStream_t st, bool* done) {
   *done = false;

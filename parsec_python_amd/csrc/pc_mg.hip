@@ -20,12 +20,18 @@
 // are one kernel, and the prolongation with the post-smooth is another.
 //
 // Launches per iteration:
-//   fine level   mg_res0 (z-march: t0 = r - c0 A r), mg_restrict0,
-//                mg_up0 (z-march: z = post-smooth(c0 r + P e_1), partials of r.z),
-//                mg_apply (z-march: p = z + beta p, A p, partials of p.Ap), mg_update;
+//   fine level   mg_res0 (b_1 = R (r - c0 A r); rows of more than 128 points:
+//                t0 = r - c0 A r and mg_restrict0),
+//                mg_up0 (z = post-smooth(c0 r + P e_1), partials of r.z),
+//                mg_apply (p = z + beta p, A p, partials of p.Ap), mg_update;
 //   cube levels  mg_down / mg_up per level above the tail;
 //   tail         mg_tail: the smallest levels and the coarsest Chebyshev in
 //                one workgroup with every level in LDS.
+// Every launch moves a few MB and is bound by latency.  Si87H76 sphere (605,808
+// points), per iteration: 81 us in 9 launches (120 us in 12, before the fine
+// passes had all their loads in flight and the small levels were merged):
+// res0 10.2, down 4.6 + 4.6, tail 9.2, up 5.0 + 5.3, up0 14.0, apply 15.4,
+// update 6.5.
 // Arrays of a cube level hold zero on inactive cells, so a neighbour read
 // needs no mask.  Every kernel returns at once when the iteration has
 // converged, so the host reads the state back only every check_every
@@ -48,7 +54,7 @@ constexpr int kNB = 512;          // workgroups of the point-wise launches (= r.
 constexpr int kMaxLev = 8;
 constexpr int kCheb = 8;          // Chebyshev steps on the coarsest cube
 constexpr int kCoarsest = 512;    // cells of the coarsest cube, at most
-constexpr int kTailCells = 512;   // cells of the levels held in LDS by mg_tail, at most (measured: one level beats more)
+constexpr int kTailCells = 4608;  // cells of the levels held in LDS by mg_tail, at most (16^3 + 8^3)
 constexpr int kTailThreads = 1024;
 // Damped Jacobi: the cycle stays SPD while omega < 2 / lambda_max(D^-1 A)
 // (lambda_max(D^-1 A) of the radius-R stencil: 2.28 at R = 4, 2.37 at R = 6,
@@ -79,21 +85,6 @@ struct Cube {
   double* e;
 };
 
-__device__ __forceinline__ double block_sum_bcast(double v, double* red) {
-  const double t = pc_block_sum(v, red);
-  __shared__ double bc;
-  if (threadIdx.x == 0) bc = t;
-  __syncthreads();
-  return bc;
-}
-
-// Sum of part[0..nb) in a fixed order; the same in every workgroup.
-__device__ __forceinline__ double sum_parts(const double* part, int nb, double* red) {
-  double s = 0.0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) s += part[b];
-  return block_sum_bcast(s, red);
-}
-
 __device__ __forceinline__ int chunk_of(int nb8) { return (blockIdx.x & 7) * nb8 + (blockIdx.x >> 3); }
 
 // value of a compact-domain array at cube coordinates (0 outside the domain)
@@ -105,6 +96,20 @@ __device__ __forceinline__ double dom_at(const Fine& g, const double* __restrict
 }
 
 // ---------------------------------------------------------------- fine level
+// Rows of at most 128 points: slabs of 8 rows, which read 3.3 values per output
+// and fill the chip once on a 106^3 box (4 rows: 4.3 values and two rounds; 32.6
+// instead of 15.4 us for mg_apply, whose registers then spilled); 4 rows for rows of one
+// x-chunk, where twice as many workgroups fill more of the chip.  Chunks of planes from
+// multiples of zc, so that every 2 x 2 x 2 cell lies in one workgroup and the
+// restriction needs no launch of its own.  Wider rows: the march.
+constexpr int mg_rows(int sx) { return sx == 2 ? 8 : pcz::kZW; }
+template <int R, int SX, int VALUES, class P>   // VALUES loaded per point
+__device__ __forceinline__ bool mg_pass(const ZMap& zm, int L, double* tile, P& p, double& s) {
+  // 128 registers per thread: two values per point of radius 4 do not fit beside the formed field
+  constexpr bool early = SX == 2 && VALUES * (2 * R + pcz::kZP) > 20;
+  return pcz::zpass<R, SX, mg_rows(SX), false, SX <= 2, early>(zm, L, tile, p, s);
+}
+
 // r = rhs - A x; partials of r.r (once per solve)
 template <int R>
 __global__ __launch_bounds__(kB) void mg_init(Fine g, const double* __restrict__ x, const double* __restrict__ rhs,
@@ -132,16 +137,58 @@ __global__ __launch_bounds__(kB) void mg_init(Fine g, const double* __restrict__
 }
 
 // t0 = r - c0 A r: the residual after one damped-Jacobi step from zero
+// (rows of more than 128 points), or restricted at once: b_1 = the average of
+// each cell's children.
+template <int SX>
+struct Res0Pass {
+  struct Raw { double r; };
+  typedef pcz::NoExt Ext;
+  static constexpr bool DOT = false, POST = SX <= 2;
+  double c0;
+  const double* __restrict__ r;
+  double* __restrict__ t0;
+  double* __restrict__ b1;
+  int cx, cy, cz;   // cells of level 1
+  const double* sc;
+  double* buf;      // [kZP / 2][rows / 2][32 SX]
+  __device__ __forceinline__ Raw load(long long idx, bool, int, int, int) const { return {r[idx]}; }
+  __device__ __forceinline__ Ext ext(long long) const { return {}; }
+  __device__ __forceinline__ bool pre() const { return sc[S_DONE] == 0.0; }
+  __device__ __forceinline__ double comb(Raw v) const { return v.r; }
+  __device__ __forceinline__ void out(bool in, long long idx, Raw, Ext, double qc, double acc, double& a,
+                                      double&) const {
+    if (POST) a = in ? qc - c0 * acc : 0.0;
+    else if (in) t0[idx] = qc - c0 * acc;
+  }
+  // the plane, x and y pairs of each cell: registers, neighbouring lanes, LDS
+  __device__ __forceinline__ void post(const double* t, int i, int j, int z, int zend, int row) const {
+    constexpr int W = 32 * SX, H = mg_rows(SX) / 2;
+    double c[pcz::kZP / 2];
+#pragma unroll
+    for (int q = 0; q < pcz::kZP / 2; ++q) {
+      c[q] = t[2 * q] + t[2 * q + 1];
+      c[q] += __shfl_xor(c[q], 1, 64);
+      if ((row & 1) && !(i & 1)) buf[(q * H + (row >> 1)) * W + (i >> 1)] = c[q];
+    }
+    __syncthreads();
+    const int I = i >> 1, J = j >> 1;
+    if ((row & 1) || (i & 1) || I >= cx || J >= cy) return;
+#pragma unroll
+    for (int q = 0; q < pcz::kZP / 2; ++q) {
+      const int K = (z >> 1) + q;
+      if (K < cz && 2 * K < zend) b1[((long long)K * cy + J) * cx + I] = 0.125 * (c[q] + buf[(q * H + (row >> 1)) * W + I]);
+    }
+  }
+};
 template <int R, int SX>
-__global__ __launch_bounds__(256) void mg_res0(ZMap zm, double c0, const double* __restrict__ r,
-                                               double* __restrict__ t0, const double* sc) {
-  __shared__ double tile[pcz::Tile<R, SX>::SIZE];
-  if (sc[S_DONE] != 0.0) return;
+__global__ __launch_bounds__(pcz::threads(SX, mg_rows(SX))) void mg_res0(ZMap zm, Res0Pass<SX> p) {
+  __shared__ double tile[pcz::Tile<R, SX, mg_rows(SX)>::SIZE];
+  __shared__ double buf[SX <= 2 ? pcz::kZP / 2 * (mg_rows(SX) / 2) * 32 * SX : 1];
   const int L = pcz::block_of(zm);
   if (L >= zm.nwg) return;
-  pcz::zmarch<R, SX>(
-      zm, L, tile, [&](long long idx, int, int, int) { return r[idx]; },
-      [&](long long idx, int, int, int, double qc, double acc) { t0[idx] = qc - c0 * acc; });
+  p.buf = buf;
+  double s;
+  mg_pass<R, SX, 1>(zm, L, tile, p, s);
 }
 
 // level-1 right-hand side: average of the domain children of each cell
@@ -157,27 +204,41 @@ __global__ __launch_bounds__(kB) void mg_restrict0(Fine g, const double* __restr
 }
 
 // z = post-smooth(c0 r + P e_1) with the domain's stencil; partials of r.z
+struct Up0Pass {
+  struct Raw { double r, e; };
+  typedef pcz::NoExt Ext;
+  static constexpr bool DOT = true, POST = false;
+  double c0;
+  const double* __restrict__ r;
+  const double* __restrict__ e1;
+  int enx, eny;
+  double* __restrict__ z;
+  const double* sc;
+  __device__ __forceinline__ Raw load(long long idx, bool in, int i, int j, int k) const {
+    const int e = in ? ((k >> 1) * eny + (j >> 1)) * enx + (i >> 1) : 0;
+    return {r[idx], e1[e]};
+  }
+  __device__ __forceinline__ Ext ext(long long) const { return {}; }
+  __device__ __forceinline__ bool pre() const { return sc[S_DONE] == 0.0; }
+  __device__ __forceinline__ double comb(Raw v) const { return c0 * v.r + v.e; }
+  __device__ __forceinline__ void out(bool in, long long idx, Raw v, Ext, double qc, double acc, double& a,
+                                      double& b) const {
+    if (in) {
+      const double zn = qc + c0 * (v.r - acc);
+      z[idx] = zn;
+      a = v.r;
+      b = zn;
+    }
+  }
+};
 template <int R, int SX>
-__global__ __launch_bounds__(256) void mg_up0(ZMap zm, double c0, const double* __restrict__ r, Cube c1,
-                                              double* __restrict__ z, double* __restrict__ prz, const double* sc) {
-  __shared__ double tile[pcz::Tile<R, SX>::SIZE];
-  __shared__ double red[pcz::kZW];
-  if (sc[S_DONE] != 0.0) return;
+__global__ __launch_bounds__(pcz::threads(SX, mg_rows(SX))) void mg_up0(ZMap zm, Up0Pass p, double* __restrict__ prz) {
+  __shared__ double tile[pcz::Tile<R, SX, mg_rows(SX)>::SIZE];
+  __shared__ double red[16];
   const int L = pcz::block_of(zm);
   if (L >= zm.nwg) return;
-  double s = 0.0;
-  const double* __restrict__ e1 = c1.e;
-  pcz::zmarch<R, SX>(
-      zm, L, tile,
-      [&](long long idx, int i, int j, int k) {
-        return c0 * r[idx] + e1[((long long)(k >> 1) * c1.ny + (j >> 1)) * c1.nx + (i >> 1)];
-      },
-      [&](long long idx, int, int, int, double qc, double acc) {
-        const double rv = r[idx];
-        const double zn = qc + c0 * (rv - acc);
-        z[idx] = zn;
-        s += rv * zn;
-      });
+  double s;
+  if (!mg_pass<R, SX, 2>(zm, L, tile, p, s)) return;
   const double t = pc_block_sum(s, red);
   if (threadIdx.x == 0) prz[L] = t;
 }
@@ -185,65 +246,115 @@ __global__ __launch_bounds__(256) void mg_up0(ZMap zm, double c0, const double* 
 // PCG step t: convergence from r_t.r_t, beta = rz_t / rz_{t-1}, p = z + beta p_old
 // (at t = 0 the caller passes p_old = z and beta is 0), A p, partials of p.Ap.
 // Workgroup 0 records the scalars.
+struct ApplyPass {
+  struct Raw { double z, p; };
+  typedef pcz::NoExt Ext;
+  static constexpr bool DOT = true, POST = false;
+  int t, maxit, nb_rr, nb_rz;
+  double tol;
+  const double* __restrict__ z;
+  const double* __restrict__ p_old;
+  double* __restrict__ p_new;
+  double* __restrict__ ap;
+  const double* __restrict__ prr;
+  const double* __restrict__ prz;
+  double* sc;
+  bool first;
+  double *red, *red2;
+  double beta;
+  __device__ __forceinline__ Raw load(long long idx, bool, int, int, int) const { return {z[idx], p_old[idx]}; }
+  __device__ __forceinline__ Ext ext(long long) const { return {}; }
+  __device__ __forceinline__ bool pre() {
+    const double done0 = t > 0 ? sc[S_DONE] : 0.0, tol0 = t > 0 ? sc[S_TOL1] : 0.0;
+    const double rz0 = t > 0 ? sc[S_RZ0 + ((t - 1) & 1)] : 1.0;
+    const double s1 = pc_parts_load<256>(prr, nb_rr), s2 = pc_parts_load<256>(prz, nb_rz);
+    pc_parts_post(s1, red);
+    pc_parts_post(s2, red2);
+    __syncthreads();
+    if (done0 != 0.0) return false;
+    const double rr = pc_parts_get<256>(red), rz = pc_parts_get<256>(red2);
+    const double tol1 = t == 0 ? tol * tol * rr : tol0;
+    const bool done = t >= maxit || !(rr > tol1);
+    beta = t > 0 ? rz / rz0 : 0.0;
+    if (first && threadIdx.x == 0) {
+      sc[S_RZ0 + (t & 1)] = rz;
+      if (t == 0) {
+        sc[S_TOL1] = tol1;
+        sc[S_RR0] = rr;
+      }
+      sc[S_ITS] = (double)t;
+      sc[S_RES] = rr;
+      sc[S_DONE] = done ? 1.0 : 0.0;
+    }
+    return !done;
+  }
+  __device__ __forceinline__ double comb(Raw v) const { return v.z + beta * v.p; }
+  __device__ __forceinline__ void out(bool in, long long idx, Raw, Ext, double qc, double acc, double& a,
+                                      double& b) const {
+    if (in) {
+      p_new[idx] = qc;
+      ap[idx] = acc;
+      a = qc;
+      b = acc;
+    }
+  }
+};
 template <int R, int SX>
-__global__ __launch_bounds__(256) void mg_apply(ZMap zm, int t, int maxit, double tol, int nb_rr,
-                                                const double* __restrict__ z, const double* __restrict__ p_old,
-                                                double* __restrict__ p_new, double* __restrict__ ap,
-                                                const double* __restrict__ prr, const double* __restrict__ prz,
-                                                double* __restrict__ ppq, double* sc) {
-  __shared__ double tile[pcz::Tile<R, SX>::SIZE];
-  __shared__ double red[pcz::kZW];
-  if (t > 0 && sc[S_DONE] != 0.0) return;
+__global__ __launch_bounds__(pcz::threads(SX, mg_rows(SX))) void mg_apply(ZMap zm, ApplyPass p, double* __restrict__ ppq) {
+  __shared__ double tile[pcz::Tile<R, SX, mg_rows(SX)>::SIZE];
+  __shared__ double red[16], red2[16], red3[16];
   const int L = pcz::block_of(zm);
   if (L >= zm.nwg) return;
-  const double rr = sum_parts(prr, nb_rr, red);
-  const double rz = sum_parts(prz, zm.nwg, red);
-  const double tol1 = t == 0 ? tol * tol * rr : sc[S_TOL1];
-  const bool done = t >= maxit || !(rr > tol1);
-  const double beta = t > 0 ? rz / sc[S_RZ0 + ((t - 1) & 1)] : 0.0;
-  if (L == 0 && threadIdx.x == 0) {
-    sc[S_RZ0 + (t & 1)] = rz;
-    if (t == 0) {
-      sc[S_TOL1] = tol1;
-      sc[S_RR0] = rr;
-    }
-    sc[S_ITS] = (double)t;
-    sc[S_RES] = rr;
-    sc[S_DONE] = done ? 1.0 : 0.0;
-  }
-  if (done) return;
-  double s = 0.0;
-  pcz::zmarch<R, SX>(
-      zm, L, tile, [&](long long idx, int, int, int) { return z[idx] + beta * p_old[idx]; },
-      [&](long long idx, int, int, int, double qc, double acc) {
-        p_new[idx] = qc;
-        ap[idx] = acc;
-        s += qc * acc;
-      });
-  const double tt = pc_block_sum(s, red);
+  p.first = L == 0;
+  p.red = red;
+  p.red2 = red2;
+  double s;
+  if (!mg_pass<R, SX, 2>(zm, L, tile, p, s)) return;
+  const double tt = pc_block_sum(s, red3);
   if (threadIdx.x == 0) ppq[L] = tt;
 }
 
-// alpha = rz_t / p.Ap; x += alpha p; r -= alpha Ap; partials of r_{t+1}.r_{t+1}
+// alpha = rz_t / p.Ap; x += alpha p; r -= alpha Ap; partials of
+// r_{t+1}.r_{t+1}.  The first points' values are loaded while the p.Ap partials
+// are summed.
 __global__ __launch_bounds__(kB) void mg_update(Fine g, int npq, int t, const double* sc, double* __restrict__ x,
                                                 double* __restrict__ r, const double* __restrict__ p,
                                                 const double* __restrict__ ap, const double* __restrict__ ppq,
                                                 double* __restrict__ prr) {
-  __shared__ double red[kB / 64];
-  if (sc[S_DONE] != 0.0) return;
+  constexpr int U = 5;   // points per thread in flight
+  __shared__ double red[kB / 64], red2[kB / 64];
   const int c = chunk_of(g.nb8);
   if (c >= g.nb) return;
-  const double pq = sum_parts(ppq, npq, red);
-  const double alpha = sc[S_RZ0 + (t & 1)] / pq;
+  const double done = sc[S_DONE], rz = sc[S_RZ0 + (t & 1)];
   const long long p0 = (long long)c * g.chunk, p1 = min(p0 + g.chunk, g.n);
+  double xv[U], rv[U], pv[U], av[U];
+  auto load = [&](long long i0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long long i = min(i0 + (long long)u * kB, p1 - 1);
+      xv[u] = x[i]; rv[u] = r[i]; pv[u] = p[i]; av[u] = ap[i];
+    }
+  };
+  load(p0 + threadIdx.x);
+  pc_parts_post(pc_parts_load<kB>(ppq, npq), red);
+  __syncthreads();
+  if (done != 0.0) return;
+  const double alpha = rz / pc_parts_get<kB>(red);
   double s = 0.0;
-  for (long long i = p0 + threadIdx.x; i < p1; i += kB) {
-    x[i] += alpha * p[i];
-    const double rv = r[i] - alpha * ap[i];
-    r[i] = rv;
-    s += rv * rv;
+  for (long long i0 = p0 + threadIdx.x; i0 < p1; i0 += U * kB) {
+    if (i0 != p0 + threadIdx.x) load(i0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long long i = i0 + (long long)u * kB;
+      if (i < p1) {
+        x[i] = xv[u] + alpha * pv[u];
+        const double v = rv[u] - alpha * av[u];
+        r[i] = v;
+        s += v * v;
+      }
+    }
   }
-  const double tt = pc_block_sum(s, red);
+  const double tt = pc_block_sum(s, red2);
   if (threadIdx.x == 0) prr[c] = tt;
 }
 
@@ -304,50 +415,90 @@ __global__ __launch_bounds__(kB) void mg_up(Cube f, Cube c, const double* sc) {
 // ---------------------------------------------------------------- tail
 // Levels T..L (T >= 1) in LDS, one workgroup: restriction down to L, the
 // Chebyshev iteration on L, prolongation and post-smoothing back up to T.
-// Input b_T, output e_T (global).
+// Input b_T, output e_T (global).  Bound by latency: the levels of at most 4608
+// cells together take one launch of 9.2 us instead of three of 3.2, 7.8 and
+// 4.6 us (106^3 box: 14^3 and 7^3 cells; 13.9 us with cell coordinates divided
+// out in the kernel instead of neighbour flags and parents from a table), and
+// the Chebyshev steps' scalars come from the host instead of two divisions per
+// step.
 struct TailLev {
   int nx, ny, nz, cells, off;   // off: first cell of the level in the LDS arrays
   double inv_h2;
-  const unsigned char* mask;
+  const unsigned char* flags;   // bits 0..5: the x-, x+, y-, y+, z-, z+ neighbour is in the box; bit 6: active
+  const unsigned short* par;    // cell of the next level over each cell
 };
 struct Tail {
   int nlev;                     // levels T..L = lev[0..nlev)
+  int ncell;                    // cells of all of them
   TailLev lev[kMaxLev];
   const double* bT;
   double* eT;
-  double lmin, lmax;
+  double d0;                    // first correction b / theta
+  double cd[kCheb], cr[kCheb];  // Chebyshev: d = cd d + cr r
 };
+inline size_t tail_lds(int ncell) { return (size_t)ncell * (2 * sizeof(double) + 3) + 2 * kCoarsest * sizeof(double) + 8; }
 
 __global__ __launch_bounds__(kTailThreads) void mg_tail(Tail tl, const double* sc) {
-  __shared__ double bl[kTailCells], el[kTailCells];
-  __shared__ unsigned char ml[kTailCells];
-  __shared__ double xs[2][kCoarsest];
-  if (sc[S_DONE] != 0.0) return;
+  extern __shared__ double lds[];
+  double* bl = lds;
+  double* el = bl + tl.ncell;
+  double* xs = el + tl.ncell;   // [2][kCoarsest]
+  unsigned short* pl = reinterpret_cast<unsigned short*>(xs + 2 * kCoarsest);
+  unsigned char* ml = reinterpret_cast<unsigned char*>(pl + tl.ncell);
+  constexpr int U = (kTailCells + kTailThreads - 1) / kTailThreads;
+  const double done = sc[S_DONE];
   const int tid = threadIdx.x;
-  const int ncell = tl.lev[tl.nlev - 1].off + tl.lev[tl.nlev - 1].cells;
-  for (int l = 0; l < tl.nlev; ++l)
-    for (int q = tid; q < tl.lev[l].cells; q += kTailThreads) ml[tl.lev[l].off + q] = tl.lev[l].mask[q];
-  for (int q = tid; q < tl.lev[0].cells; q += kTailThreads) bl[q] = tl.bT[q];
-  for (int q = tid; q < ncell; q += kTailThreads) el[q] = 0.0;
+  for (int l = 0; l < tl.nlev; ++l) {
+    const TailLev& f = tl.lev[l];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = tid + u * kTailThreads;
+      if (q < f.cells) {
+        ml[f.off + q] = f.flags[q];
+        pl[f.off + q] = f.par[q];
+        if (l == 0) bl[q] = tl.bT[q];
+      }
+    }
+  }
+  if (done != 0.0) return;
   __syncthreads();
-  auto at = [&](const double* a, const TailLev& v, int i, int j, int k) -> double {
-    const bool in = i >= 0 && j >= 0 && k >= 0 && i < v.nx && j < v.ny && k < v.nz;
-    return in ? a[v.off + (k * v.ny + j) * v.nx + i] : 0.0;
+  // the sum of a level array's six neighbours, cells outside the box zero
+  auto nb6 = [&](const double* a, int sy, int sz, int q, unsigned fl) -> double {
+    const double xm = a[fl & 1 ? q - 1 : q], xp = a[fl & 2 ? q + 1 : q], ym = a[fl & 4 ? q - sy : q];
+    const double yp = a[fl & 8 ? q + sy : q], zm = a[fl & 16 ? q - sz : q], zp = a[fl & 32 ? q + sz : q];
+    double s = fl & 1 ? xm : 0.0;
+    s += fl & 2 ? xp : 0.0;
+    s += fl & 4 ? ym : 0.0;
+    s += fl & 8 ? yp : 0.0;
+    s += fl & 16 ? zm : 0.0;
+    s += fl & 32 ? zp : 0.0;
+    return s;
   };
-  // down: b_{l+1} = R (b_l - A_l omega b_l / D_l)
+  // down: t = b - A omega b / D on the active cells (in the level's e array, free until the way up), b_{l+1} = R t
   for (int l = 0; l + 1 < tl.nlev; ++l) {
     const TailLev& f = tl.lev[l];
     const TailLev& c = tl.lev[l + 1];
+    const int sy = f.nx, sz = f.nx * f.ny;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = tid + u * kTailThreads;
+      if (q < f.cells) {
+        const unsigned fl = ml[f.off + q];
+        const double t = (1.0 - kOmegaC) * bl[f.off + q] + (kOmegaC / 6.0) * nb6(bl + f.off, sy, sz, q, fl);
+        el[f.off + q] = fl & 64 ? t : 0.0;
+      }
+    }
+    __syncthreads();
     for (int q = tid; q < c.cells; q += kTailThreads) {
       const int I = q % c.nx, J = (q / c.nx) % c.ny, K = q / (c.nx * c.ny);
+      const int fq = f.off + (2 * K * f.ny + 2 * J) * f.nx + 2 * I;
+      const bool x1 = 2 * I + 1 < f.nx, y1 = 2 * J + 1 < f.ny, z1 = 2 * K + 1 < f.nz;
       double s = 0.0;
+#pragma unroll
       for (int d = 0; d < 8; ++d) {
-        const int i = 2 * I + (d & 1), j = 2 * J + ((d >> 1) & 1), k = 2 * K + (d >> 2);
-        if (i >= f.nx || j >= f.ny || k >= f.nz) continue;
-        const int fq = f.off + (k * f.ny + j) * f.nx + i;
-        const double nb = at(bl, f, i - 1, j, k) + at(bl, f, i + 1, j, k) + at(bl, f, i, j - 1, k) +
-                          at(bl, f, i, j + 1, k) + at(bl, f, i, j, k - 1) + at(bl, f, i, j, k + 1);
-        s += ml[fq] ? (1.0 - kOmegaC) * bl[fq] + (kOmegaC / 6.0) * nb : 0.0;
+        const bool in = (!(d & 1) || x1) && (!(d & 2) || y1) && (!(d & 4) || z1);
+        const double t = el[in ? fq + (d & 1) + (d & 2 ? sy : 0) + (d & 4 ? sz : 0) : fq];
+        s += in ? t : 0.0;
       }
       bl[c.off + q] = 0.125 * s;
     }
@@ -357,57 +508,62 @@ __global__ __launch_bounds__(kTailThreads) void mg_tail(Tail tl, const double* s
   // barrier per step (x alternates between two LDS buffers)
   {
     const TailLev& c = tl.lev[tl.nlev - 1];
-    const bool act = tid < c.cells && ml[c.off + tid];
-    const int I = tid % c.nx, J = (tid / c.nx) % c.ny, K = tid / (c.nx * c.ny);
-    const double theta = 0.5 * (tl.lmax + tl.lmin), delta = 0.5 * (tl.lmax - tl.lmin);
-    const double sigma = theta / delta;
-    double rho = 1.0 / sigma;
+    const unsigned fl = tid < c.cells ? ml[c.off + tid] : 0;
+    const bool act = fl & 64;
+    const int sy = c.nx, sz = c.nx * c.ny;
     const double b = act ? bl[c.off + tid] : 0.0;
-    double x = 0.0, d = b / theta;
-    auto xat = [&](const double* a, int i, int j, int k) -> double {
-      const bool in = i >= 0 && j >= 0 && k >= 0 && i < c.nx && j < c.ny && k < c.nz;
-      return in ? a[(k * c.ny + j) * c.nx + i] : 0.0;
-    };
+    double x = 0.0, d = b * tl.d0;
+#pragma unroll
     for (int it = 0; it < kCheb; ++it) {
       x += d;
-      double* xb = xs[it & 1];
-      if (tid < c.cells) xb[tid] = act ? x : 0.0;
+      double* xb = xs + (it & 1) * kCoarsest;
+      if (tid < c.cells) xb[tid] = x;   // (d and x stay zero on inactive cells)
       __syncthreads();
-      double r = 0.0;
-      if (act)
-        r = b - c.inv_h2 * (6.0 * x - xat(xb, I - 1, J, K) - xat(xb, I + 1, J, K) - xat(xb, I, J - 1, K) -
-                            xat(xb, I, J + 1, K) - xat(xb, I, J, K - 1) - xat(xb, I, J, K + 1));
-      const double rho1 = 1.0 / (2.0 * sigma - rho);
-      d = act ? rho1 * rho * d + 2.0 * rho1 / delta * r : 0.0;
-      rho = rho1;
+      if (act) {
+        const double r = b - c.inv_h2 * (6.0 * x - nb6(xb, sy, sz, tid, fl));
+        d = tl.cd[it] * d + tl.cr[it] * r;
+      }
     }
-    if (tid < c.cells) el[c.off + tid] = act ? x + d : 0.0;
+    x += d;
+    if (tid < c.cells) {
+      el[c.off + tid] = x;
+      if (tl.nlev == 1) tl.eT[tid] = x;
+    }
     __syncthreads();
   }
-  // up: e_l = post-smooth(omega b_l / D_l + P e_{l+1})
+  // up: e_l = post-smooth(omega b_l / D_l + P e_{l+1}); the smoothed field first
+  // replaces b, which the post-smoothing needs only at its own cell
   for (int l = tl.nlev - 2; l >= 0; --l) {
     const TailLev& f = tl.lev[l];
     const TailLev& c = tl.lev[l + 1];
     const double s0 = kOmegaC / (6.0 * f.inv_h2);
-    auto ev = [&](int a, int b, int cc) -> double {
-      const bool in = a >= 0 && b >= 0 && cc >= 0 && a < f.nx && b < f.ny && cc < f.nz;
-      if (!in) return 0.0;
-      const int fq = f.off + (cc * f.ny + b) * f.nx + a;
-      return ml[fq] ? s0 * bl[fq] + el[c.off + ((cc >> 1) * c.ny + (b >> 1)) * c.nx + (a >> 1)] : 0.0;
-    };
-    for (int q = tid; q < f.cells; q += kTailThreads) {
-      const int i = q % f.nx, j = (q / f.nx) % f.ny, k = q / (f.nx * f.ny);
-      const double e0 = ev(i, j, k);
-      const double ae = f.inv_h2 * (6.0 * e0 - ev(i - 1, j, k) - ev(i + 1, j, k) - ev(i, j - 1, k) -
-                                    ev(i, j + 1, k) - ev(i, j, k - 1) - ev(i, j, k + 1));
-      const double e = ml[f.off + q] ? e0 + s0 * (bl[f.off + q] - ae) : 0.0;
-      if (l == 0) tl.eT[q] = e;
-      else el[f.off + q] = e;
+    const int sy = f.nx, sz = f.nx * f.ny;
+    double bq[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = tid + u * kTailThreads;
+      bq[u] = 0.0;
+      if (q < f.cells) {
+        bq[u] = bl[f.off + q];
+        const double e0 = s0 * bq[u] + el[c.off + pl[f.off + q]];
+        bl[f.off + q] = ml[f.off + q] & 64 ? e0 : 0.0;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = tid + u * kTailThreads;
+      if (q < f.cells) {
+        const unsigned fl = ml[f.off + q];
+        const double e0 = bl[f.off + q];
+        const double ae = f.inv_h2 * (6.0 * e0 - nb6(bl + f.off, sy, sz, q, fl));
+        const double e = fl & 64 ? e0 + s0 * (bq[u] - ae) : 0.0;
+        if (l == 0) tl.eT[q] = e;
+        else el[f.off + q] = e;
+      }
     }
     __syncthreads();
   }
-  if (tl.nlev == 1)
-    for (int q = tid; q < tl.lev[0].cells; q += kTailThreads) tl.eT[q] = el[q];
 }
 
 __global__ void mg_reset(double* sc) {
@@ -435,18 +591,26 @@ size_t work_bytes_for(long long n) {
 
 template <int R, int SX>
 struct FineLaunch {
+  static dim3 grid(const MGCtx* c) { return dim3(8 * c->zm.nwg8); }
+  static dim3 block() { return dim3(pcz::threads(SX, mg_rows(SX))); }
   static void res0(const MGCtx* c, hipStream_t st, const double* r, const double* sc) {
-    hipLaunchKernelGGL((mg_res0<R, SX>), dim3(8 * c->zm.nwg8), dim3(256), 0, st, c->zm, c->g.c0, r, c->t0, sc);
+    const Cube& c1 = c->lev[1];
+    const Res0Pass<SX> p{c->g.c0, r, c->t0, c1.b, c1.nx, c1.ny, c1.nz, sc, nullptr};
+    hipLaunchKernelGGL((mg_res0<R, SX>), grid(c), block(), 0, st, c->zm, p);
+    if (SX > 2)
+      hipLaunchKernelGGL(mg_restrict0, dim3((unsigned)((c1.cells + kB - 1) / kB)), dim3(kB), 0, st, c->g, c->t0, c1, sc);
   }
   static void up0(const MGCtx* c, hipStream_t st, const double* r, double* z, double* prz, const double* sc) {
-    hipLaunchKernelGGL((mg_up0<R, SX>), dim3(8 * c->zm.nwg8), dim3(256), 0, st, c->zm, c->g.c0, r, c->lev[1], z, prz,
-                       sc);
+    const Cube& c1 = c->lev[1];
+    const Up0Pass p{c->g.c0, r, c1.e, c1.nx, c1.ny, z, sc};
+    hipLaunchKernelGGL((mg_up0<R, SX>), grid(c), block(), 0, st, c->zm, p, prz);
   }
   static void apply(const MGCtx* c, hipStream_t st, int t, int maxit, double tol, const double* z,
                     const double* p_old, double* p_new, double* ap, const double* prr, const double* prz, double* ppq,
                     double* sc) {
-    hipLaunchKernelGGL((mg_apply<R, SX>), dim3(8 * c->zm.nwg8), dim3(256), 0, st, c->zm, t, maxit, tol, c->g.nb, z,
-                       p_old, p_new, ap, prr, prz, ppq, sc);
+    const ApplyPass p{t, maxit, c->g.nb, c->zm.nwg, tol, z, p_old, p_new, ap, prr, prz, sc,
+                      false, nullptr, nullptr, 0.0};
+    hipLaunchKernelGGL((mg_apply<R, SX>), grid(c), block(), 0, st, c->zm, p, ppq);
   }
   static void init(const MGCtx* c, hipStream_t st, const double* x, const double* rhs, double* r, double* prr) {
     hipLaunchKernelGGL((mg_init<R>), dim3(8 * c->g.nb8), dim3(kB), 0, st, c->g, x, rhs, r, prr);
@@ -512,7 +676,7 @@ int pc_mg_create(void* grid, double h, void** out_mg) {
   g.nb = (int)((g.n + g.chunk - 1) / g.chunk);
   g.nb8 = (g.nb + 7) / 8;
   int rz = 0;
-  if (pcz::zmap_init(grid, g.w, c->zm, &rz)) {
+  if (pcz::zmap_init(grid, g.w, c->zm, &rz, mg_rows(g.nx <= 64 ? 1 : (g.nx <= 128 ? 2 : 4)), 2)) {
     delete c;
     PC_CHECK_ARG(false, "nx > 256");
   }
@@ -571,19 +735,51 @@ int pc_mg_create(void* grid, double h, void** out_mg) {
   int off = 0;
   for (int l = 0; l < tl.nlev; ++l) {
     const Cube& L = c->lev[c->tail + l];
-    tl.lev[l] = {L.nx, L.ny, L.nz, (int)L.cells, off, L.inv_h2, L.mask};
+    std::vector<unsigned char> m((size_t)L.cells);
+    std::vector<unsigned short> par((size_t)L.cells);
+    PC_HIP(hipMemcpy(m.data(), L.mask, m.size(), hipMemcpyDeviceToHost));
+    const int px = (L.nx + 1) / 2, py = (L.ny + 1) / 2;
+    for (int q = 0; q < (int)L.cells; ++q) {
+      const int i = q % L.nx, j = (q / L.nx) % L.ny, k = q / (L.nx * L.ny);
+      m[q] = (unsigned char)((i > 0) | (i + 1 < L.nx) << 1 | (j > 0) << 2 | (j + 1 < L.ny) << 3 | (k > 0) << 4 |
+                             (k + 1 < L.nz) << 5 | (m[q] ? 64 : 0));
+      par[q] = (unsigned short)((k / 2 * py + j / 2) * px + i / 2);
+    }
+    unsigned char* fd = nullptr;
+    unsigned short* pd = nullptr;
+    PC_HIP(hipMalloc(&fd, m.size()));
+    c->allocs.push_back(fd);
+    PC_HIP(hipMalloc(&pd, par.size() * sizeof(unsigned short)));
+    c->allocs.push_back(pd);
+    PC_HIP(hipMemcpy(fd, m.data(), m.size(), hipMemcpyHostToDevice));
+    PC_HIP(hipMemcpy(pd, par.data(), par.size() * sizeof(unsigned short), hipMemcpyHostToDevice));
+    tl.lev[l] = {L.nx, L.ny, L.nz, (int)L.cells, off, L.inv_h2, fd, pd};
     off += (int)L.cells;
   }
+  tl.ncell = off;
   tl.bT = c->lev[c->tail].b;
   tl.eT = c->lev[c->tail].e;
   // Chebyshev interval of the coarsest 7-point operator: lambda_max <= 12/h^2
   // (Gershgorin); lambda_min >= that of the full box (Dirichlet on a subset)
   const Cube& C = c->lev[c->nlev];
   auto lam1 = [](int n) { return 2.0 * (1.0 - std::cos(M_PI / (n + 1))); };
-  tl.lmin = C.inv_h2 * (lam1(C.nx) + lam1(C.ny) + lam1(C.nz));
-  tl.lmax = 12.0 * C.inv_h2;
-  PC_HIP(hipMalloc(&c->t0, g.n * sizeof(double)));
-  c->allocs.push_back(c->t0);
+  const double lmin = C.inv_h2 * (lam1(C.nx) + lam1(C.ny) + lam1(C.nz)), lmax = 12.0 * C.inv_h2;
+  const double theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin), sigma = theta / delta;
+  tl.d0 = 1.0 / theta;
+  double rho = 1.0 / sigma;
+  for (int it = 0; it < kCheb; ++it) {
+    const double rho1 = 1.0 / (2.0 * sigma - rho);
+    tl.cd[it] = rho1 * rho;
+    tl.cr[it] = 2.0 * rho1 / delta;
+    rho = rho1;
+  }
+  PC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mg_tail), hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)tail_lds(kTailCells)));
+  c->t0 = nullptr;
+  if (c->zm.sx > 2) {
+    PC_HIP(hipMalloc(&c->t0, g.n * sizeof(double)));
+    c->allocs.push_back(c->t0);
+  }
   *out_mg = c;
   return pc::PC_OK;
 }
@@ -638,12 +834,10 @@ int pc_pcg_solve_mg(void* mg, const double* rhs, double* x, int maxit, double to
   const int T = c->tail;
   auto vcycle = [&](const double* rr, double* zz) {
     ops.res0(c, st, rr, sc);
-    hipLaunchKernelGGL(mg_restrict0, dim3((unsigned)((c->lev[1].cells + kB - 1) / kB)), dim3(kB), 0, st, c->g, c->t0,
-                       c->lev[1], sc);
     for (int l = 1; l < T; ++l)
       hipLaunchKernelGGL(mg_down, dim3((unsigned)((8 * c->lev[l + 1].cells + kB - 1) / kB)), dim3(kB), 0, st,
                          c->lev[l], c->lev[l + 1], sc);
-    hipLaunchKernelGGL(mg_tail, dim3(1), dim3(kTailThreads), 0, st, c->tl, sc);
+    hipLaunchKernelGGL(mg_tail, dim3(1), dim3(kTailThreads), tail_lds(c->tl.ncell), st, c->tl, sc);
     for (int l = T - 1; l >= 1; --l)
       hipLaunchKernelGGL(mg_up, dim3((unsigned)((c->lev[l].cells + kB - 1) / kB)), dim3(kB), 0, st, c->lev[l],
                          c->lev[l + 1], sc);

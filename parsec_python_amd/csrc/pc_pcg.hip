@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 long long pc_internal_grid_npts(void* grid);
 
@@ -50,17 +51,6 @@ struct PointMap {
 // ids are dealt round-robin over the 8 XCDs), so the z-neighbour planes a
 // chunk reads are mostly in that XCD's L2.
 __device__ __forceinline__ int chunk_of(int nb8) { return (blockIdx.x & 7) * nb8 + (blockIdx.x >> 3); }
-
-// Sum of part[0..nb) in a fixed order; the same in every workgroup.
-__device__ __forceinline__ double sum_parts(const double* part, int nb, double* red) {
-  double s = 0.0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) s += part[b];
-  double t = pc_block_sum(s, red);
-  __shared__ double bc;
-  if (threadIdx.x == 0) bc = t;
-  __syncthreads();
-  return bc;
-}
 
 template <int MODE>
 __device__ __forceinline__ double qv(const double* __restrict__ a, const double* __restrict__ b, double beta,
@@ -132,64 +122,119 @@ __global__ __launch_bounds__(kBlk) void cg_init(PointMap g, const double* __rest
 // one per workgroup.
 using pcz::ZMap;
 
+template <int MODE>
+struct ApplyPass {
+  struct Raw { double r, p; };
+  typedef pcz::NoExt Ext;
+  static constexpr bool DOT = true, POST = false;
+  int t, maxit, nb_rr;
+  double tol;
+  const double* __restrict__ r;
+  const double* __restrict__ p_old;
+  double* __restrict__ p_new;
+  double* __restrict__ ap;
+  const double* __restrict__ part_rr;
+  double* sc;
+  bool first;       // workgroup 0 records the scalars
+  double* red;
+  double beta;
+  __device__ __forceinline__ Raw load(long long idx, bool, int, int, int) const {
+    return {r[idx], MODE == M_NORMAL ? p_old[idx] : 0.0};
+  }
+  __device__ __forceinline__ Ext ext(long long) const { return {}; }
+  __device__ __forceinline__ bool pre() {
+    const double done0 = t > 0 ? sc[S_DONE] : 0.0, tol0 = t > 0 ? sc[S_TOL1] : 0.0;
+    const double rr0 = t > 0 ? sc[S_RO0 + ((t - 1) & 1)] : 1.0;
+    pc_parts_post(pc_parts_load<256>(part_rr, nb_rr), red);
+    __syncthreads();
+    if (done0 != 0.0) return false;
+    const double rr = pc_parts_get<256>(red);
+    const double tol1 = t == 0 ? tol * tol * rr : tol0;
+    const bool done = t >= maxit || !(rr > tol1);
+    beta = t > 0 ? rr / rr0 : 0.0;
+    if (first && threadIdx.x == 0) {
+      sc[S_RO0 + (t & 1)] = rr;
+      if (t == 0) sc[S_TOL1] = tol1;
+      sc[S_ITS] = (double)t;
+      sc[S_RES] = rr;
+      sc[S_DONE] = done ? 1.0 : 0.0;
+    }
+    return !done;
+  }
+  __device__ __forceinline__ double comb(Raw v) const {
+    if (MODE == M_FIRST) return v.r;
+    if (MODE == M_ALIAS) return v.r + beta * v.r;
+    return v.r + beta * v.p;
+  }
+  __device__ __forceinline__ void out(bool in, long long idx, Raw, Ext, double qc, double acc, double& a,
+                                      double& b) const {
+    if (in) {
+      p_new[idx] = qc;
+      ap[idx] = acc;
+      a = qc;
+      b = acc;
+    }
+  }
+};
+
 template <int R, int SX, int MODE>
-__global__ __launch_bounds__(256) void cg_apply_z(ZMap g, int t, int maxit, double tol, int nb_rr,
-                                                  const double* __restrict__ r, const double* __restrict__ p_old,
-                                                  double* __restrict__ p_new, double* __restrict__ ap,
-                                                  const double* __restrict__ part_rr, double* __restrict__ part_pq,
-                                                  double* sc) {
-  __shared__ double tile[pcz::Tile<R, SX>::SIZE];
-  __shared__ double red[pcz::kZW];
-  if (t > 0 && sc[S_DONE] != 0.0) return;
+__global__ __launch_bounds__(pcz::threads(SX), SX == 2 ? 4 : 2) void cg_apply_z(ZMap g, ApplyPass<MODE> p, double* __restrict__ part_pq) {
+  __shared__ double tile[pcz::Tile<R, SX, pcz::kZW, true>::SIZE];
+  __shared__ double red[8], red2[8];
   const int L = pcz::block_of(g);
   if (L >= g.nwg) return;
-  const double rr = sum_parts(part_rr, nb_rr, red);
-  const double tol1 = t == 0 ? tol * tol * rr : sc[S_TOL1];
-  const bool done = t >= maxit || !(rr > tol1);
-  const double beta = t > 0 ? rr / sc[S_RO0 + ((t - 1) & 1)] : 0.0;
-  if (L == 0 && threadIdx.x == 0) {
-    sc[S_RO0 + (t & 1)] = rr;
-    if (t == 0) sc[S_TOL1] = tol1;
-    sc[S_ITS] = (double)t;
-    sc[S_RES] = rr;
-    sc[S_DONE] = done ? 1.0 : 0.0;
-  }
-  if (done) return;
-  double sacc = 0.0;
-  pcz::zmarch<R, SX>(
-      g, L, tile, [&](long long idx, int, int, int) { return qv<MODE>(r, p_old, beta, idx); },
-      [&](long long idx, int, int, int, double qc, double acc) {
-        p_new[idx] = qc;
-        ap[idx] = acc;
-        sacc += qc * acc;
-      });
-  const double bs = pc_block_sum(sacc, red);
+  p.first = L == 0;
+  p.red = red;
+  double sacc;
+  if (!pcz::zpass<R, SX, pcz::kZW, true, false, SX == 2>(g, L, tile, p, sacc)) return;
+  const double bs = pc_block_sum(sacc, red2);
   if (threadIdx.x == 0) part_pq[L] = bs;
 }
 
-// alpha = r_t.r_t / p.Ap; x += alpha p; r -= alpha Ap; partials of r_{t+1}.r_{t+1}
+// alpha = r_t.r_t / p.Ap; x += alpha p; r -= alpha Ap; partials of
+// r_{t+1}.r_{t+1}.  The first points' values are loaded while the p.Ap partials
+// are summed.
+template <int U>   // points per thread in flight
 __global__ __launch_bounds__(kBlk) void cg_update(long long n, long long chunk, int nb, int nb8, int npq, int t,
                                                   const double* sc,
                                                   double* __restrict__ x, double* __restrict__ r,
                                                   const double* __restrict__ p, const double* __restrict__ ap,
                                                   const double* __restrict__ part_pq,
                                                   double* __restrict__ part_rr_next) {
-  __shared__ double red[kBlk / 64];
-  if (sc[S_DONE] != 0.0) return;
+  __shared__ double red[kBlk / 64], red2[kBlk / 64];
   const int c = chunk_of(nb8);
   if (c >= nb) return;
-  const double pq = sum_parts(part_pq, npq, red);
-  const double alpha = sc[S_RO0 + (t & 1)] / pq;
+  const double done = sc[S_DONE], rr = sc[S_RO0 + (t & 1)];
   const long long p0 = (long long)c * chunk;
   const long long p1 = min(p0 + chunk, n);
+  double xv[U], rv[U], pv[U], av[U];
+  auto load = [&](long long i0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long long i = min(i0 + (long long)u * kBlk, p1 - 1);
+      xv[u] = x[i]; rv[u] = r[i]; pv[u] = p[i]; av[u] = ap[i];
+    }
+  };
+  load(p0 + threadIdx.x);
+  pc_parts_post(pc_parts_load<kBlk>(part_pq, npq), red);
+  __syncthreads();
+  if (done != 0.0) return;
+  const double alpha = rr / pc_parts_get<kBlk>(red);
   double s = 0.0;
-  for (long long i = p0 + threadIdx.x; i < p1; i += kBlk) {
-    x[i] += alpha * p[i];
-    const double rv = r[i] - alpha * ap[i];
-    r[i] = rv;
-    s += rv * rv;
+  for (long long i0 = p0 + threadIdx.x; i0 < p1; i0 += U * kBlk) {
+    if (i0 != p0 + threadIdx.x) load(i0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long long i = i0 + (long long)u * kBlk;
+      if (i < p1) {
+        x[i] = xv[u] + alpha * pv[u];
+        const double v = rv[u] - alpha * av[u];
+        r[i] = v;
+        s += v * v;
+      }
+    }
   }
-  const double tt = pc_block_sum(s, red);
+  const double tt = pc_block_sum(s, red2);
   if (threadIdx.x == 0) part_rr_next[c] = tt;
 }
 
@@ -214,24 +259,16 @@ int launch_init(int nb, hipStream_t st, const PointMap& g, const double* x, cons
 
 template <int R, int SX>
 int launch_apply_z(int mode, hipStream_t st, const ZMap& z, int t, int maxit, double tol, int nb_rr, const Work& w) {
-  const double* p_old = w.p[t & 1];
-  double* p_new = w.p[(t + 1) & 1];
-  const double* prr = w.prr[t & 1];
-  const dim3 grid(8 * z.nwg8);
-  switch (mode) {
-    case M_FIRST:
-      hipLaunchKernelGGL((cg_apply_z<R, SX, M_FIRST>), grid, dim3(256), 0, st, z, t, maxit, tol, nb_rr, w.r, p_old,
-                         p_new, w.ap, prr, w.ppq, w.sc);
-      break;
-    case M_ALIAS:
-      hipLaunchKernelGGL((cg_apply_z<R, SX, M_ALIAS>), grid, dim3(256), 0, st, z, t, maxit, tol, nb_rr, w.r, p_old,
-                         p_new, w.ap, prr, w.ppq, w.sc);
-      break;
-    default:
-      hipLaunchKernelGGL((cg_apply_z<R, SX, M_NORMAL>), grid, dim3(256), 0, st, z, t, maxit, tol, nb_rr, w.r, p_old,
-                         p_new, w.ap, prr, w.ppq, w.sc);
-      break;
-  }
+  const dim3 grid(8 * z.nwg8), block(pcz::threads(SX));
+  auto launch = [&](auto m) {
+    constexpr int MODE = decltype(m)::value;
+    const ApplyPass<MODE> p{t, maxit, nb_rr, tol, w.r, w.p[t & 1], w.p[(t + 1) & 1], w.ap, w.prr[t & 1], w.sc,
+                            false, nullptr, 0.0};
+    hipLaunchKernelGGL((cg_apply_z<R, SX, MODE>), grid, block, 0, st, z, p, w.ppq);
+  };
+  if (mode == M_FIRST) launch(std::integral_constant<int, M_FIRST>{});
+  else if (mode == M_ALIAS) launch(std::integral_constant<int, M_ALIAS>{});
+  else launch(std::integral_constant<int, M_NORMAL>{});
   return hipGetLastError() == hipSuccess ? pc::PC_OK : pc::PC_ERR_HIP;
 }
 
@@ -308,8 +345,8 @@ int pcg_solve_impl(void* grid, double inv_h2, const double* rhs, double* x, int 
       const int mode = t == 0 ? M_FIRST : ((t == 1 && alias_first) ? M_ALIAS : M_NORMAL);
       status = L.apply(mode, st, zm, t, maxit, tol, nb_used, w);
       if (!status && t < maxit) {
-        hipLaunchKernelGGL(cg_update, dim3(nb_launch), dim3(kBlk), 0, st, n, g.chunk, g.nb, g.nb8, zm.nwg, t, w.sc, x,
-                           w.r,
+        auto update = g.chunk <= kBlk ? cg_update<1> : cg_update<3>;
+        hipLaunchKernelGGL(update, dim3(nb_launch), dim3(kBlk), 0, st, n, g.chunk, g.nb, g.nb8, zm.nwg, t, w.sc, x, w.r,
                            w.p[(t + 1) & 1], w.ap, w.ppq, w.prr[(t + 1) & 1]);
         if (hipGetLastError() != hipSuccess) status = pc::PC_ERR_HIP;
       }
