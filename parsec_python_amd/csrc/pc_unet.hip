@@ -7,15 +7,14 @@
 // Weights: W[co][t][ci] (tap t = (dz+1)*9 + (dy+1)*3 + (dx+1), ci fastest),
 // 3x3x3 taps, zero padding 1.
 //
-// conv3d (implicit GEMM, M = output channels, N = voxels, K = 27 * C_in):
-// each wavefront owns 16*MT output channels x 32 voxels and issues
-// v_mfma_f32_16x16x16_bf16 on fragments gathered straight from the
-// channel-last tensors (4 consecutive channels = one 8-byte load per lane).
-// The input gradient is the same kernel on the tap-flipped, channel-transposed
-// weights; the weight gradient is a GEMM over voxels per tap.
+// conv3d (implicit GEMM, M = output channels, N = voxels, K = 27 * C_in): a
+// workgroup owns a box of voxels, stages it with its halo in LDS and issues
+// v_mfma_f32_16x16x16_bf16 tap by tap.  The input gradient is the same kernel on the tap-flipped, channel-transposed
+// weights; the weight gradient is a GEMM over voxels, one wavefront per dz.
 #include "pc_common.h"
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace {
 
@@ -41,12 +40,63 @@ __device__ __forceinline__ void tap_offsets(int t, int& dz, int& dy, int& dx) {
   dx = t % 3 - 1;
 }
 
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+                                                 0);
+}
+
+// Boxes of a TX x TY x TZ tiling and the box of this workgroup (consecutive
+// boxes on one XCD, whose L2 then serves the halos).
+struct Boxes {
+  int nx, ny, nz;     // boxes per axis
+  int nblocks, nb8;   // boxes x channel blocks
+};
+
+// One result of lane (n, lk): channels co0 .. co0 + 3 of a voxel.
+// mode: 0 = FP32 output with bias, 1 = leaky ReLU -> BF16 output (with bias),
+//       2 = FP32 output, no bias
+__device__ __forceinline__ void conv_store(f32x4 acc, long long v, int co0, int cout, const float* __restrict__ bias,
+                                           int mode, float slope, void* Y, int ldy, bool vec) {
+  float o[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    o[r] = acc[r];
+    if (mode != 2) o[r] += bias[min(co0 + r, cout - 1)];
+    if (mode == 1) o[r] = o[r] > 0.f ? o[r] : slope * o[r];
+  }
+  if (mode == 1) {
+    unsigned short* y = static_cast<unsigned short*>(Y) + v * ldy + co0;
+    if (vec && co0 + 3 < cout) {
+      const u32x2 t = {f2bf(o[0]) | (unsigned)f2bf(o[1]) << 16, f2bf(o[2]) | (unsigned)f2bf(o[3]) << 16};
+      *reinterpret_cast<u32x2*>(y) = t;
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (co0 + r < cout) y[r] = f2bf(o[r]);
+    }
+  } else {
+    float* y = static_cast<float*>(Y) + v * ldy + co0;
+    if (vec && co0 + 3 < cout) {
+      *reinterpret_cast<f32x4*>(y) = f32x4{o[0], o[1], o[2], o[3]};
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (co0 + r < cout) y[r] = o[r];
+    }
+  }
+}
+
 constexpr int kNT = 2;   // 16-voxel tiles per wavefront
 constexpr int kWaves = 4;
 
-// mode: 0 = FP32 output with bias, 1 = leaky ReLU -> BF16 output (with bias),
-//       2 = FP32 output, no bias
-template <int MT, bool CIN1>
+// Any number of input channels (a multiple of 16): each wavefront owns 16*MT
+// output channels x 32 voxels, its operands gathered straight from the
+// channel-last tensors.
+template <int MT>
 __global__ __launch_bounds__(256) void conv_fwd(Vol vol, const unsigned short* __restrict__ X, int ldx, int cin,
                                                 const unsigned short* __restrict__ Wt, const float* __restrict__ bias,
                                                 int cout, int mode, float slope, void* Y, int ldy) {
@@ -74,7 +124,7 @@ __global__ __launch_bounds__(256) void conv_fwd(Vol vol, const unsigned short* _
 #pragma unroll
     for (int n = 0; n < kNT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  if constexpr (!CIN1) {
+  {
     const int ncb = cin >> 4;
     for (int t = 0; t < 27; ++t) {
       int dz, dy, dx;
@@ -104,36 +154,6 @@ __global__ __launch_bounds__(256) void conv_fwd(Vol vol, const unsigned short* _
         }
       }
     }
-  } else {
-    // one input channel: K = the 27 taps (two k-steps of 16, taps 27..31 zero)
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      bf16x4 b[kNT];
-      short av[MT][4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int t = ks * 16 + 4 * lk + j;
-        int dz = 0, dy = 0, dx = 0;
-        if (t < 27) tap_offsets(t, dz, dy, dx);
-#pragma unroll
-        for (int n = 0; n < kNT; ++n) {
-          const int z = vz[n] + dz, y = vy[n] + dy, x = vx[n] + dx;
-          const bool ok = t < 27 && vin[n] && z >= 0 && z < vol.D && y >= 0 && y < vol.H && x >= 0 && x < vol.W;
-          b[n][j] = ok ? (short)X[((long long)(z * vol.H + y) * vol.W + x) * ldx] : (short)0;
-        }
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          const int co = co_base + 16 * m + ln;
-          av[m][j] = (t < 27 && co < cout) ? (short)Wt[(long long)co * 27 + t] : (short)0;
-        }
-      }
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        const bf16x4 a = {av[m][0], av[m][1], av[m][2], av[m][3]};
-#pragma unroll
-        for (int n = 0; n < kNT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[n], acc[m][n], 0, 0, 0);
-      }
-    }
   }
 
   // epilogue: lane holds D[co = 16m + 4*lk + r][voxel = 16n + ln]
@@ -161,6 +181,155 @@ __global__ __launch_bounds__(256) void conv_fwd(Vol vol, const unsigned short* _
   }
 }
 
+// Workgroup: 4 wavefronts, a box of TX x TY x TZ voxels (NT tiles of 16 per
+// wavefront, in the box's flat order) x 16 output channels.  The box with its
+// halo goes to LDS once, all 16 NCB channels of a voxel together, 8 loads per
+// thread in flight; the products then run tap by tap and, inside a tap, 16
+// channels by 16 channels (the order of conv_fwd, so the same bits), each tile's
+// operand one 8-byte LDS read per lane, the next tap's weights loaded meanwhile.
+// Bound by the LDS reads (2 bytes per voxel, tap and channel) and the staging;
+// 64^3 volume: 48 -> 16 channels 39 us, 16 -> 48 31 us (115
+// and 91 us with every operand gathered from global memory per tap).
+template <int NCB, int TX, int TY, int TZ>
+__global__ __launch_bounds__(256, NCB == 1 ? 4 : 2) void conv_tile(Vol vol, Boxes bx,
+                                                                   const unsigned short* __restrict__ X, int ldx,
+                                                                   const unsigned short* __restrict__ Wt,
+                                                                   const float* __restrict__ bias, int cout, int mode,
+                                                                   float slope, void* Y, int ldy, bool yvec) {
+  constexpr int CIN = 16 * NCB;
+  constexpr int VS = CIN + 8;   // LDS voxel stride: an odd number of 16-byte pieces, so 16 voxels meet different banks
+  constexpr int NT = TX * TY * TZ / 64;
+  constexpr int HX = TX + 2, HY = TY + 2, HZ = TZ + 2, HV = HX * HY * HZ;
+  __shared__ __align__(16) unsigned short xs[HV * VS];
+  const int L = (blockIdx.x & 7) * bx.nb8 + (blockIdx.x >> 3);
+  if (L >= bx.nblocks) return;
+  const int nbox = bx.nx * bx.ny * bx.nz;
+  const int cb = L / nbox, box = L - cb * nbox;
+  const int x0 = box % bx.nx * TX, y0 = box / bx.nx % bx.ny * TY, z0 = box / (bx.nx * bx.ny) * TZ;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int ln = lane & 15, lk = lane >> 4;
+  // the box and its halo, zero outside the volume, 8 channels per step
+  constexpr int PV = 2 * NCB, UNITS = HV * PV, U = 8;
+  for (int e0 = threadIdx.x; e0 < UNITS; e0 += 256 * U) {
+    u32x4 t[U];
+    unsigned inside = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = e0 + 256 * u, q = e / PV, h = e % PV * 8;
+      const int x = x0 + q % HX - 1, y = y0 + q / HX % HY - 1, z = z0 + q / (HX * HY) - 1;
+      const bool in = e < UNITS && x >= 0 && x < vol.W && y >= 0 && y < vol.H && z >= 0 && z < vol.D;
+      inside |= (unsigned)in << u;
+      t[u] = *reinterpret_cast<const u32x4*>(X + (in ? ((long long)(z * vol.H + y) * vol.W + x) * ldx + h : 0));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = e0 + 256 * u;
+      if (e < UNITS) *reinterpret_cast<u32x4*>(&xs[e / PV * VS + e % PV * 8]) = inside >> u & 1 ? t[u] : u32x4{0, 0, 0, 0};
+    }
+  }
+  int base[NT];          // LDS position of this lane's voxel of each tile (its tap (0, 0, 0))
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const int q = (wv * NT + n) * 16 + ln;
+    base[n] = ((q / (TX * TY) * HY + q / TX % TY) * HX + q % TX) * VS + 4 * lk;
+  }
+  f32x4 acc[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bool win = cb * 16 + ln < cout;
+  const unsigned short* wp = Wt + (long long)min(cb * 16 + ln, cout - 1) * 27 * CIN + 4 * lk;
+  // the three taps of a row at a time; the next row's weights are in flight meanwhile
+  bf16x4 a[3][NCB], an[3][NCB];
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int c = 0; c < NCB; ++c) a[k][c] = *reinterpret_cast<const bf16x4*>(wp + k * CIN + 16 * c);
+  __syncthreads();
+  for (int r = 0; r < 9; ++r) {
+    const int rn = min(r + 1, 8);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int c = 0; c < NCB; ++c) an[k][c] = *reinterpret_cast<const bf16x4*>(wp + (3 * rn + k) * CIN + 16 * c);
+    __builtin_amdgcn_sched_barrier(0);   // or the loads are sunk to their uses
+    const int off = (r / 3 * HY + r % 3) * HX * VS;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int c = 0; c < NCB; ++c) {
+        const bf16x4 av = win ? a[k][c] : bf16x4{0, 0, 0, 0};
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          const bf16x4 b = *reinterpret_cast<const bf16x4*>(&xs[base[n] + off + k * VS + 16 * c]);
+          acc[n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b, acc[n], 0, 0, 0);
+        }
+      }
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int c = 0; c < NCB; ++c) a[k][c] = an[k][c];
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const int q = (wv * NT + n) * 16 + ln;
+    const int x = x0 + q % TX, y = y0 + q / TX % TY, z = z0 + q / (TX * TY);
+    if (x < vol.W && y < vol.H && z < vol.D && cb * 16 + 4 * lk < cout)
+      conv_store(acc[n], (long long)(z * vol.H + y) * vol.W + x, cb * 16 + 4 * lk, cout, bias, mode, slope, Y, ldy,
+                 yvec);
+  }
+}
+
+// One input channel: K = the 27 taps in two products of 16 (lane group lk holds
+// taps 16 ks + 4 lk .. + 3, those past 26 zero), the box with its halo in LDS.
+template <int TX, int TY, int TZ>
+__global__ __launch_bounds__(256) void conv_tile1(Vol vol, Boxes bx, const unsigned short* __restrict__ X, int ldx,
+                                                  const unsigned short* __restrict__ Wt,
+                                                  const float* __restrict__ bias, int cout, int mode, float slope,
+                                                  void* Y, int ldy, bool yvec) {
+  constexpr int NT = TX * TY * TZ / 64;
+  constexpr int HX = TX + 2, HY = TY + 2, HZ = TZ + 2, HV = HX * HY * HZ;
+  __shared__ unsigned short xs[HV];
+  const int L = (blockIdx.x & 7) * bx.nb8 + (blockIdx.x >> 3);
+  if (L >= bx.nblocks) return;
+  const int nbox = bx.nx * bx.ny * bx.nz;
+  const int cb = L / nbox, box = L - cb * nbox;
+  const int x0 = box % bx.nx * TX, y0 = box / bx.nx % bx.ny * TY, z0 = box / (bx.nx * bx.ny) * TZ;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int ln = lane & 15, lk = lane >> 4;
+  for (int q = threadIdx.x; q < HV; q += 256) {
+    const int x = x0 + q % HX - 1, y = y0 + q / HX % HY - 1, z = z0 + q / (HX * HY) - 1;
+    const bool in = x >= 0 && x < vol.W && y >= 0 && y < vol.H && z >= 0 && z < vol.D;
+    xs[q] = in ? X[((long long)(z * vol.H + y) * vol.W + x) * ldx] : (unsigned short)0;
+  }
+  const int co = cb * 16 + ln;
+  int off[8];
+  unsigned av[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int t = 16 * (e >> 2) + 4 * lk + (e & 3), tt = t < 27 ? t : 0;
+    off[e] = (tt / 9 * HY + tt / 3 % 3) * HX + tt % 3;
+    av[e] = (t < 27 && co < cout) ? Wt[(long long)co * 27 + t] : 0;
+  }
+  const u32x2 a0 = {av[0] | av[1] << 16, av[2] | av[3] << 16}, a1 = {av[4] | av[5] << 16, av[6] | av[7] << 16};
+  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const int q = (wv * NT + n) * 16 + ln;
+    const int p = (q / (TX * TY) * HY + q / TX % TY) * HX + q % TX;
+    u32x4 b;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b[e] = xs[p + off[2 * e]] | (unsigned)xs[p + off[2 * e + 1]] << 16;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(bf16x4, a0),
+                                                    __builtin_bit_cast(bf16x4, u32x2{b[0], b[1]}), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(bf16x4, a1),
+                                                    __builtin_bit_cast(bf16x4, u32x2{b[2], b[3]}), acc, 0, 0, 0);
+    const int x = x0 + q % TX, y = y0 + q / TX % TY, z = z0 + q / (TX * TY);
+    if (x < vol.W && y < vol.H && z < vol.D && cb * 16 + 4 * lk < cout)
+      conv_store(acc, (long long)(z * vol.H + y) * vol.W + x, cb * 16 + 4 * lk, cout, bias, mode, slope, Y, ldy, yvec);
+  }
+}
+
 // Wt[ci][t][co] = W[co][26 - t][ci]: the weights of the input-gradient conv
 __global__ void conv_wflip(const unsigned short* __restrict__ W, int cout, int cin, unsigned short* __restrict__ Wt) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -172,75 +341,163 @@ __global__ void conv_wflip(const unsigned short* __restrict__ W, int cout, int c
   Wt[((long long)ci * 27 + (26 - t)) * cout + co] = W[i];
 }
 
-// Weight gradient for one tap-block: workgroup (tap t, 16 output channels,
-// 16*NT input channels, voxel split s).  dW_part[s][co][t][ci].
-template <int NTC>
-__global__ __launch_bounds__(256) void conv_wgrad(Vol vol, const unsigned short* __restrict__ dZ, int ldz, int cout,
-                                                  const unsigned short* __restrict__ X, int ldx, int cin,
-                                                  long long vchunk, float* __restrict__ part) {
-  __shared__ float red[kWaves][16 * 16 * NTC];
-  const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  const int ln = lane & 15, lk = lane >> 4;
-  const int t = blockIdx.x % 27;
-  const int cob = blockIdx.x / 27;
-  const int cib = blockIdx.y;
+// Weight gradient: workgroup (16 output channels, 16 input channels, voxel split
+// s); it stages boxes of TX x TY x TZ voxels of dZ and, with the halo, of X into
+// LDS transposed (channel by channel, x fastest), so that a lane's 8 voxels of
+// one channel are two 8-byte reads.  Wavefronts (dz, k): the 9 taps of one dz on
+// every second group of 32 voxels; the x-shifted operands of a row's three taps
+// share their reads (funnel shifts).  dW_part[s][co][t][ci].  Bound by LDS reads
+// and the transposing staging; 64^3 volume, 48 x 16 channels: 47 us (611 us
+// with 2-byte gathers from global memory per tap).
+template <int TX, int TY, int TZ, bool ZVEC, bool XVEC>   // 16-byte aligned channels, a multiple of 16
+__global__ __launch_bounds__(384) void conv_wgrad(Vol vol, Boxes bx, const unsigned short* __restrict__ dZ, int ldz,
+                                                  int cout, const unsigned short* __restrict__ X, int ldx, int cin,
+                                                  int nsplit, float* __restrict__ part) {
+  constexpr int HY = TY + 2, HZ = TZ + 2;
+  constexpr int RS = TX + 8;                      // row stride: x = -4 .. TX + 3
+  // channel strides of 40 bytes beyond a multiple of 256, so that 16 channels' reads meet different banks
+  constexpr int CX = (HZ * HY * RS + 107) / 128 * 128 + 20;
+  constexpr int CZ = (TZ * TY * TX + 107) / 128 * 128 + 20;
+  constexpr int RPK = 32 / TX;                    // rows per group of 32 voxels
+  constexpr int NG = TX * TY * TZ / 32;           // groups per box
+  __shared__ __align__(16) unsigned short xs[16 * CX], zs[16 * CZ];
+  const int co0 = blockIdx.x * 16, ci0 = blockIdx.y * 16;
   const int s = blockIdx.z;
-  int dz, dy, dx;
-  tap_offsets(t, dz, dy, dx);
-  const int co = cob * 16 + ln;
-  const long long v0 = (long long)s * vchunk;
-  const long long v1 = min(v0 + vchunk, vol.V);
-  f32x4 acc[NTC];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int ln = lane & 15, lk = lane >> 4;
+  const int dz = wv % 3, kh = wv / 3;
+  f32x4 acc[9];
 #pragma unroll
-  for (int n = 0; n < NTC; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // each wavefront takes every 4th group of 16 voxels
-  for (long long vb = v0 + 16 * wv; vb < v1; vb += 16 * kWaves) {
-    bf16x4 a;
-    bf16x4 b[NTC];
+  for (int t = 0; t < 9; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // staging unit: 4 voxels x 8 channels of a row, transposed in registers on
+  // the way to LDS
+  constexpr int XG = RS / 4, ZG = TX / 4;         // 4-voxel groups per row
+  constexpr int XU = HZ * HY * XG * 2, ZU = TZ * TY * ZG * 2;
+  constexpr int NX = (XU + 383) / 384, NZ = (ZU + 383) / 384;
+  u32x4 tx[NX][4], tz[NZ][4];
+  unsigned mx[NX], mz[NZ];                        // which of a unit's voxels lie in the volume
+  auto fetch = [&](auto vec, const unsigned short* __restrict__ src, int ld, int nch, int c0, int e, int units,
+                   int groups, int ny, int xo, int bx0, int by0, int bz0, u32x4 (&t)[4], unsigned& m) {
+    const int h = (e & 1) * 8, g = (e >> 1) % groups, row = (e >> 1) / groups;
+    const int y = by0 + row % ny, z = bz0 + row / ny;
+    const bool rin = e < units && y >= 0 && y < vol.H && z >= 0 && z < vol.D;
+    m = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const long long v = vb + 4 * lk + j;
-      const bool vok = v < v1;
-      a[j] = (vok && co < cout) ? (short)dZ[v * ldz + co] : (short)0;
-      long long src = -1;
-      if (vok) {
-        const int x = (int)(v % vol.W) + dx;
-        const int y = (int)((v / vol.W) % vol.H) + dy;
-        const int z = (int)(v / ((long long)vol.W * vol.H)) + dz;
-        if (z >= 0 && z < vol.D && y >= 0 && y < vol.H && x >= 0 && x < vol.W)
-          src = ((long long)(z * vol.H + y) * vol.W + x) * ldx;
-      }
+    for (int k = 0; k < 4; ++k) {
+      const int x = bx0 + 4 * g + xo + k;
+      const bool in = rin && x >= 0 && x < vol.W;
+      m |= (unsigned)in << k;
+      const unsigned short* p = src + (in ? ((long long)(z * vol.H + y) * vol.W + x) * ld + c0 : 0);
+      if constexpr (decltype(vec)::value) {
+        t[k] = *reinterpret_cast<const u32x4*>(p + (in ? h : 0));
+      } else {
+        t[k] = u32x4{0, 0, 0, 0};
 #pragma unroll
-      for (int n = 0; n < NTC; ++n) {
-        const int ci = cib * 16 * NTC + 16 * n + ln;
-        b[n][j] = (src >= 0 && ci < cin) ? (short)X[src + ci] : (short)0;
+        for (int c = 0; c < 8; ++c)
+          if (in && c0 + h + c < nch) t[k][c >> 1] |= (unsigned)p[h + c] << (16 * (c & 1));
       }
     }
+  };
+  auto put = [&](u32x4 (&t)[4], unsigned m, unsigned short* dst, int cstride, int rs, int groups, int e) {
+    const int h = (e & 1) * 8, g = (e >> 1) % groups, row = (e >> 1) / groups;
 #pragma unroll
-    for (int n = 0; n < NTC; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[n], acc[n], 0, 0, 0);
+    for (int k = 0; k < 4; ++k) t[k] = m >> k & 1 ? t[k] : u32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const unsigned sel = c & 1 ? 0x07060302u : 0x05040100u;   // the high or the low halves of two words
+      const u32x2 w = {__builtin_amdgcn_perm(t[1][c >> 1], t[0][c >> 1], sel),
+                       __builtin_amdgcn_perm(t[3][c >> 1], t[2][c >> 1], sel)};
+      *reinterpret_cast<u32x2*>(&dst[(h + c) * cstride + row * rs + 4 * g]) = w;
+    }
+  };
+  const int nbox = bx.nx * bx.ny * bx.nz;
+  auto fetch_box = [&](int box) {
+    const int x0 = box % bx.nx * TX, y0 = box / bx.nx % bx.ny * TY, z0 = box / (bx.nx * bx.ny) * TZ;
+#pragma unroll
+    for (int u = 0; u < NX; ++u)
+      fetch(std::integral_constant<bool, XVEC>{}, X, ldx, cin, ci0, threadIdx.x + 384 * u, XU, XG, HY, -4, x0, y0 - 1,
+            z0 - 1, tx[u], mx[u]);
+#pragma unroll
+    for (int u = 0; u < NZ; ++u)
+      fetch(std::integral_constant<bool, ZVEC>{}, dZ, ldz, cout, co0, threadIdx.x + 384 * u, ZU, ZG, TY, 0, x0, y0, z0,
+            tz[u], mz[u]);
+  };
+  fetch_box(s);
+  for (int box = s; box < nbox; box += nsplit) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < NX; ++u)
+      if ((int)threadIdx.x + 384 * u < XU) put(tx[u], mx[u], xs, CX, RS, XG, threadIdx.x + 384 * u);
+#pragma unroll
+    for (int u = 0; u < NZ; ++u)
+      if ((int)threadIdx.x + 384 * u < ZU) put(tz[u], mz[u], zs, CZ, TX, ZG, threadIdx.x + 384 * u);
+    __syncthreads();
+    if (box + nsplit < nbox) fetch_box(box + nsplit);   // in flight during the products
+#pragma unroll 2
+    for (int g = kh; g < NG; g += 2) {
+      const int row = g * RPK + (TX == 16 ? lk >> 1 : lk);        // this lane's row of the box
+      const int xh = TX == 16 ? 8 * (lk & 1) : 0;
+      const int y = row % TY, z = row / TY;
+      const u32x2* za = reinterpret_cast<const u32x2*>(&zs[ln * CZ + row * TX + xh]);
+      const u32x2 z0v = za[0], z1v = za[1];
+      const u32x4 a = {z0v[0], z0v[1], z1v[0], z1v[1]};
+#pragma unroll
+      for (int dy = 0; dy < 3; ++dy) {
+        const unsigned short* xr = &xs[ln * CX + ((z + dz) * HY + y + dy) * RS + 4 + xh];
+        const unsigned wm = *reinterpret_cast<const unsigned*>(xr - 2), wp = *reinterpret_cast<const unsigned*>(xr + 8);
+        const u32x2 wa = *reinterpret_cast<const u32x2*>(xr), wb = *reinterpret_cast<const u32x2*>(xr + 4);
+        const unsigned s0 = __builtin_amdgcn_alignbit(wa[0], wm, 16), s1 = __builtin_amdgcn_alignbit(wa[1], wa[0], 16);
+        const unsigned s2 = __builtin_amdgcn_alignbit(wb[0], wa[1], 16), s3 = __builtin_amdgcn_alignbit(wb[1], wb[0], 16);
+        const unsigned s4 = __builtin_amdgcn_alignbit(wp, wb[1], 16);
+        acc[3 * dy] = mfma32(a, u32x4{s0, s1, s2, s3}, acc[3 * dy]);
+        acc[3 * dy + 1] = mfma32(a, u32x4{wa[0], wa[1], wb[0], wb[1]}, acc[3 * dy + 1]);
+        acc[3 * dy + 2] = mfma32(a, u32x4{s1, s2, s3, s4}, acc[3 * dy + 2]);
+      }
+    }
   }
-  // D[m = co row 4*lk + r][n = ci col ln]
-#pragma unroll
-  for (int n = 0; n < NTC; ++n)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) red[wv][(4 * lk + r) * (16 * NTC) + 16 * n + ln] = acc[n][r];
+  // add the two k-halves (lane (ln, lk) register r: channel 4 lk + r of dZ, channel ln of X)
   __syncthreads();
-  for (int e = threadIdx.x; e < 16 * 16 * NTC; e += 256) {
-    const float sum = red[0][e] + red[1][e] + red[2][e] + red[3][e];
-    const int m = e / (16 * NTC), c = e % (16 * NTC);
-    const int com = cob * 16 + m, cim = cib * 16 * NTC + c;
-    if (com < cout && cim < cin) part[(((long long)s * cout + com) * 27 + t) * cin + cim] = sum;
+  f32x4* red = reinterpret_cast<f32x4*>(xs);     // 3 * 9 * 64 of them
+  static_assert(sizeof(f32x4) * 3 * 9 * 64 <= sizeof(xs), "partial sums do not fit");
+  if (kh == 1) {
+#pragma unroll
+    for (int t = 0; t < 9; ++t) red[(dz * 9 + t) * 64 + lane] = acc[t];
+  }
+  __syncthreads();
+  if (kh == 0 && ci0 + ln < cin) {
+#pragma unroll
+    for (int t = 0; t < 9; ++t) {
+      const f32x4 o = red[(dz * 9 + t) * 64 + lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int co = co0 + 4 * lk + r;
+        if (co < cout) part[(((long long)s * cout + co) * 27 + dz * 9 + t) * cin + ci0 + ln] = acc[t][r] + o[r];
+      }
+    }
   }
 }
 
-// dW[i] = sum_s part[s][i] (fixed order)
-__global__ void reduce_splits(const float* __restrict__ part, int nsplit, long long n, float* __restrict__ out) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// dW[i] = sum_s part[s][i]: 32 elements per workgroup, 8 threads each taking
+// every 8th split in order, their sums added in order
+__global__ __launch_bounds__(256) void reduce_splits(const float* __restrict__ part, int nsplit, long long n,
+                                                     float* __restrict__ out) {
+  __shared__ float red[8][32];
+  const int el = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const long long i = (long long)blockIdx.x * 32 + el;
   float s = 0.f;
-  for (int k = 0; k < nsplit; ++k) s += part[(long long)k * n + i];
-  out[i] = s;
+  if (i < n) {
+#pragma unroll 8
+    for (int k = g; k < nsplit; k += 8) s += part[(long long)k * n + i];
+  }
+  red[g][el] = s;
+  __syncthreads();
+  if (g == 0 && i < n) {
+    float t = red[0][el];
+#pragma unroll
+    for (int q = 1; q < 8; ++q) t += red[q][el];
+    out[i] = t;
+  }
 }
 
 // dZ = dA * (a > 0 ? 1 : slope) (a == nullptr: identity), rounded to BF16;
@@ -272,6 +529,43 @@ __global__ __launch_bounds__(256) void act_bwd(const float* __restrict__ dA, int
     for (int k = 0; k < nslot; ++k) tot += red[k * C + threadIdx.x];
     dbpart[(long long)blockIdx.x * C + threadIdx.x] = tot;
   }
+}
+
+// The same for C = 4 C4 channels in 16- and 8-byte pieces: a thread takes 4
+// channels of every (256 / C4)-th voxel.
+__global__ __launch_bounds__(256) void act_bwd4(const float* __restrict__ dA, int lda,
+                                                const unsigned short* __restrict__ a, int lda_a, int C4, long long V,
+                                                float slope, unsigned short* __restrict__ dZ, int ldz,
+                                                long long vchunk, float* __restrict__ dbpart) {
+  __shared__ f32x4 red[256];
+  const int c = threadIdx.x % C4 * 4, slot = threadIdx.x / C4, nslot = 256 / C4;
+  const long long v0 = (long long)blockIdx.x * vchunk;
+  const long long v1 = slot < nslot ? min(v0 + vchunk, V) : v0;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (long long v = v0 + slot; v < v1; v += nslot) {
+    f32x4 g = *reinterpret_cast<const f32x4*>(dA + v * lda + c);
+    if (a) {
+      const u32x2 t = *reinterpret_cast<const u32x2*>(a + v * lda_a + c);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float av = __uint_as_float(r & 1 ? t[r >> 1] & 0xffff0000u : t[r >> 1] << 16);
+        g[r] = av > 0.f ? g[r] : slope * g[r];
+      }
+    }
+    const u32x2 o = {f2bf(g[0]) | (unsigned)f2bf(g[1]) << 16, f2bf(g[2]) | (unsigned)f2bf(g[3]) << 16};
+    *reinterpret_cast<u32x2*>(dZ + v * ldz + c) = o;
+    s += g;
+  }
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int n = nslot; n > 1;) {
+    const int h = (n + 1) / 2;
+    if (slot + h < n) red[threadIdx.x] += red[threadIdx.x + h * C4];
+    __syncthreads();
+    n = h;
+  }
+  if (slot == 0) *reinterpret_cast<f32x4*>(dbpart + (long long)blockIdx.x * 4 * C4 + c) = red[threadIdx.x];
 }
 
 __global__ void pool2_fwd(Vol out, const unsigned short* __restrict__ X, int ldx, int C,
@@ -369,12 +663,20 @@ __global__ __launch_bounds__(256) void mse(const float* __restrict__ y, const fl
   if (threadIdx.x == 0) part[blockIdx.x] = tot;
 }
 
-__global__ void sum_parts_f32(const float* __restrict__ part, int nblk, int C, float* __restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= C) return;
+// out[c] = sum over the blocks, one workgroup per channel
+__global__ __launch_bounds__(256) void sum_parts_f32(const float* __restrict__ part, int nblk, int C,
+                                                     float* __restrict__ out) {
+  __shared__ float red[256];
+  const int c = blockIdx.x;
   float s = 0.f;
-  for (int b = 0; b < nblk; ++b) s += part[(long long)b * C + c];
-  out[c] = s;
+  for (int b = threadIdx.x; b < nblk; b += 256) s += part[(long long)b * C + c];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int h = 128; h > 0; h >>= 1) {
+    if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) out[c] = red[0];
 }
 
 __global__ void sum_parts_f64(const double* __restrict__ part, int nblk, double* __restrict__ out) {
@@ -388,9 +690,25 @@ Vol make_vol(int D, int H, int W) { return Vol{D, H, W, (long long)D * H * W}; }
 
 inline int nblk(long long n, int b = 256) { return (int)((n + b - 1) / b); }
 
-constexpr int kWgradSplit = 64;
-constexpr int kActChunk = 2048;
+constexpr int kWgradSplit = 128;     // voxel splits of the weight gradient, at most
+constexpr int kWgradSplitMin = 64;   // splits whose workspace every caller has to bring
+constexpr int kActChunk = 512;       // voxels per workgroup of the activation backward, at least
+constexpr int kActChunkMax = 2048;   // (chunk whose workspace every caller has to bring)
 constexpr int kMseBlocks = 512;
+
+Boxes make_boxes(const Vol& v, int tx, int ty, int tz, int cblocks) {
+  Boxes b;
+  b.nx = (v.W + tx - 1) / tx;
+  b.ny = (v.H + ty - 1) / ty;
+  b.nz = (v.D + tz - 1) / tz;
+  b.nblocks = b.nx * b.ny * b.nz * cblocks;
+  b.nb8 = (b.nblocks + 7) / 8;
+  return b;
+}
+inline long long box_count(const Vol& v, int tx, int ty, int tz) {
+  return (long long)((v.W + tx - 1) / tx) * ((v.H + ty - 1) / ty) * ((v.D + tz - 1) / tz);
+}
+inline bool aligned(const void* p, size_t n) { return reinterpret_cast<uintptr_t>(p) % n == 0; }
 
 }  // namespace
 
@@ -408,26 +726,87 @@ int pc_unet_conv3d_fwd(const void* X, int ldx, int cin, const void* W, const flo
   PC_CHECK_ARG(mode == 2 || bias, "bias required");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const Vol vol = make_vol(D, H, Wd);
-  const long long vox_per_block = 16LL * kNT * kWaves;
-  dim3 grid((unsigned)((vol.V + vox_per_block - 1) / vox_per_block), (unsigned)((cout + 63) / 64));
-  const int mt = std::min(4, (cout + 15) / 16);
+  PC_CHECK_ARG(vol.V < (1LL << 31), "volume too large");
   auto X16 = static_cast<const unsigned short*>(X);
   auto W16 = static_cast<const unsigned short*>(W);
-#define PC_CONV_LAUNCH(MT, C1)                                                                                  \
-  hipLaunchKernelGGL((conv_fwd<MT, C1>), grid, dim3(256), 0, st, vol, X16, ldx, cin, W16, bias, cout, mode, slope, \
-                     Y, ldy)
+  const int ct = (cout + 15) / 16;
+  const bool yvec = ldy % 4 == 0 && aligned(Y, mode == 1 ? 8 : 16);
+  const bool xvec = ldx % 8 == 0 && aligned(X, 16);
+  // Boxes of 512 voxels for one group of 16 input channels, 256 for two or
+  // three and 128 for up to seven (LDS: two workgroups per CU), 16 or 8 wide
+  // (whichever pads the volume less); 128 also where larger ones would not give
+  // every CU a workgroup.  More input channels, or columns without 16-byte
+  // alignment: conv_fwd.
+  const int ncb = cin / 16;
+  auto padded = [&](int tx, int ty, int tz) { return box_count(vol, tx, ty, tz) * tx * ty * tz; };
+  const bool fill512 = padded(16, 8, 4) / 512 * ct >= 256, fill256 = padded(16, 4, 4) / 256 * ct >= 256;
+  const int size = cin == 1 || ncb == 1 ? (fill512 ? 512 : 128) : ncb <= 3 ? (fill256 ? 256 : 128) : 128;
+  const bool w8 = size == 512   ? padded(8, 8, 8) < padded(16, 8, 4)
+                  : size == 256 ? padded(8, 8, 4) < padded(16, 4, 4)
+                                : padded(8, 4, 4) < padded(16, 4, 2);
+#define PC_CONV(NCB, TX, TY, TZ)                                                                                     \
+  do {                                                                                                               \
+    const Boxes bx = make_boxes(vol, TX, TY, TZ, ct);                                                                \
+    hipLaunchKernelGGL((conv_tile<NCB, TX, TY, TZ>), dim3(8 * bx.nb8), dim3(256), 0, st, vol, bx, X16, ldx, W16, bias, \
+                       cout, mode, slope, Y, ldy, yvec);                                                             \
+  } while (0)
+#define PC_CONV1(TX, TY, TZ)                                                                                         \
+  do {                                                                                                               \
+    const Boxes bx = make_boxes(vol, TX, TY, TZ, ct);                                                                \
+    hipLaunchKernelGGL((conv_tile1<TX, TY, TZ>), dim3(8 * bx.nb8), dim3(256), 0, st, vol, bx, X16, ldx, W16, bias,   \
+                       cout, mode, slope, Y, ldy, yvec);                                                             \
+  } while (0)
+#define PC_CONV128(NCB)                \
+  do {                                 \
+    if (w8) PC_CONV(NCB, 8, 4, 4);     \
+    else PC_CONV(NCB, 16, 4, 2);       \
+  } while (0)
+#define PC_CONV256(NCB)                \
+  do {                                 \
+    if (w8) PC_CONV(NCB, 8, 8, 4);     \
+    else PC_CONV(NCB, 16, 4, 4);       \
+  } while (0)
   if (cin == 1) {
-    if (mt == 1) PC_CONV_LAUNCH(1, true);
-    else if (mt == 2) PC_CONV_LAUNCH(2, true);
-    else if (mt == 3) PC_CONV_LAUNCH(3, true);
-    else PC_CONV_LAUNCH(4, true);
+    if (size == 512) {
+      if (w8) PC_CONV1(8, 8, 8);
+      else PC_CONV1(16, 8, 4);
+    } else {
+      if (w8) PC_CONV1(8, 4, 4);
+      else PC_CONV1(16, 4, 2);
+    }
+  } else if (ncb > 7 || !xvec) {
+    const long long vox_per_block = 16LL * kNT * kWaves;
+    dim3 grid((unsigned)((vol.V + vox_per_block - 1) / vox_per_block), (unsigned)((cout + 63) / 64));
+    auto general = ct == 1 ? conv_fwd<1> : ct == 2 ? conv_fwd<2> : ct == 3 ? conv_fwd<3> : conv_fwd<4>;
+    hipLaunchKernelGGL(general, grid, dim3(256), 0, st, vol, X16, ldx, cin, W16, bias, cout, mode, slope, Y, ldy);
   } else {
-    if (mt == 1) PC_CONV_LAUNCH(1, false);
-    else if (mt == 2) PC_CONV_LAUNCH(2, false);
-    else if (mt == 3) PC_CONV_LAUNCH(3, false);
-    else PC_CONV_LAUNCH(4, false);
+    switch (ncb) {
+      case 1:
+        if (size == 512) {
+          if (w8) PC_CONV(1, 8, 8, 8);
+          else PC_CONV(1, 16, 8, 4);
+        } else {
+          PC_CONV128(1);
+        }
+        break;
+      case 2:
+        if (size == 256) PC_CONV256(2);
+        else PC_CONV128(2);
+        break;
+      case 3:
+        if (size == 256) PC_CONV256(3);
+        else PC_CONV128(3);
+        break;
+      case 4: PC_CONV128(4); break;
+      case 5: PC_CONV128(5); break;
+      case 6: PC_CONV128(6); break;
+      default: PC_CONV128(7); break;
+    }
   }
-#undef PC_CONV_LAUNCH
+#undef PC_CONV
+#undef PC_CONV1
+#undef PC_CONV128
+#undef PC_CONV256
   PC_LAUNCH_CHECK();
   return pc::PC_OK;
 }
@@ -454,25 +833,37 @@ int pc_unet_conv3d_wgrad(const void* dZ, int ldz, int cout, const void* X, int l
   PC_CHECK_ARG(dZ && X && dW && work, "null pointer");
   PC_CHECK_ARG(D > 0 && H > 0 && Wd > 0, "bad volume");
   PC_CHECK_ARG(ldz >= cout && ldx >= cin, "channel stride smaller than the channel count");
-  size_t need = 0;
-  pc_unet_wgrad_workspace(cout, cin, &need);
-  PC_CHECK_ARG(work_bytes >= need, "workspace too small");
+  const long long n = (long long)cout * 27 * cin;
+  PC_CHECK_ARG(work_bytes >= kWgradSplitMin * n * sizeof(float), "workspace too small");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const Vol vol = make_vol(D, H, Wd);
-  const int nsplit = (int)std::min<long long>(kWgradSplit, (vol.V + 255) / 256);
-  const long long vchunk = (vol.V + nsplit - 1) / nsplit;
-  const int ntc = cin >= 32 ? 2 : 1;
-  dim3 grid(27 * ((cout + 15) / 16), (cin + 16 * ntc - 1) / (16 * ntc), nsplit);
+  PC_CHECK_ARG(vol.V < (1LL << 31), "volume too large");
   auto dZ16 = static_cast<const unsigned short*>(dZ);
   auto X16 = static_cast<const unsigned short*>(X);
   float* part = static_cast<float*>(work);
-  if (ntc == 2)
-    hipLaunchKernelGGL((conv_wgrad<2>), grid, dim3(256), 0, st, vol, dZ16, ldz, cout, X16, ldx, cin, vchunk, part);
-  else
-    hipLaunchKernelGGL((conv_wgrad<1>), grid, dim3(256), 0, st, vol, dZ16, ldz, cout, X16, ldx, cin, vchunk, part);
+  const bool zvec = ldz % 8 == 0 && cout % 16 == 0 && aligned(dZ, 16);
+  const bool xvec = ldx % 8 == 0 && cin % 16 == 0 && aligned(X, 16);
+  const bool w8 = box_count(vol, 8, 8, 4) * 8 < box_count(vol, 16, 8, 4) * 16;   // padded rows
+  const Boxes bx = w8 ? make_boxes(vol, 8, 8, 4, 1) : make_boxes(vol, 16, 8, 4, 1);
+  const int room = (int)std::min<long long>(kWgradSplit, (long long)(work_bytes / sizeof(float)) / n);
+  const int nsplit = std::min(room, bx.nblocks);
+  dim3 grid((cout + 15) / 16, (cin + 15) / 16, nsplit);
+#define PC_WGRAD(TX, ZV, XV)                                                                                     \
+  hipLaunchKernelGGL((conv_wgrad<TX, 8, 4, ZV, XV>), grid, dim3(384), 0, st, vol, bx, dZ16, ldz, cout, X16, ldx, \
+                     cin, nsplit, part)
+#define PC_WGRAD_V(TX)                                 \
+  do {                                                 \
+    if (zvec && xvec) PC_WGRAD(TX, true, true);        \
+    else if (zvec) PC_WGRAD(TX, true, false);          \
+    else if (xvec) PC_WGRAD(TX, false, true);          \
+    else PC_WGRAD(TX, false, false);                   \
+  } while (0)
+  if (w8) PC_WGRAD_V(8);
+  else PC_WGRAD_V(16);
+#undef PC_WGRAD
+#undef PC_WGRAD_V
   PC_LAUNCH_CHECK();
-  const long long n = (long long)cout * 27 * cin;
-  hipLaunchKernelGGL(reduce_splits, dim3(nblk(n)), dim3(256), 0, st, part, nsplit, n, dW);
+  hipLaunchKernelGGL(reduce_splits, dim3(nblk(n, 32)), dim3(256), 0, st, part, nsplit, n, dW);
   PC_LAUNCH_CHECK();
   return pc::PC_OK;
 }
@@ -489,16 +880,24 @@ int pc_unet_act_bwd(const float* dA, int lda, const void* a, int lda_a, int C, i
   PC_CHECK_ARG(dA && dZ && db && work, "null pointer");
   PC_CHECK_ARG(C >= 1 && C <= 256, "C must be in [1, 256]");
   const long long V = (long long)D * H * Wd;
-  size_t need = 0;
-  pc_unet_act_bwd_workspace(C, V, &need);
-  PC_CHECK_ARG(work_bytes >= need, "workspace too small");
+  PC_CHECK_ARG(work_bytes >= (size_t)((V + kActChunkMax - 1) / kActChunkMax) * C * sizeof(float), "workspace too small");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int nb = (int)((V + kActChunk - 1) / kActChunk);
+  // the smallest chunk of at least kActChunk voxels whose partial sums fit
+  long long chunk = kActChunk;
+  while ((size_t)((V + chunk - 1) / chunk) * C * sizeof(float) > work_bytes) chunk *= 2;
+  const int nb = (int)((V + chunk - 1) / chunk);
   float* part = static_cast<float*>(work);
-  hipLaunchKernelGGL(act_bwd, dim3(nb), dim3(256), 0, st, dA, lda, static_cast<const unsigned short*>(a), lda_a, C, V,
-                     slope, static_cast<unsigned short*>(dZ), ldz, (long long)kActChunk, part);
+  auto a16 = static_cast<const unsigned short*>(a);
+  auto z16 = static_cast<unsigned short*>(dZ);
+  const int c4 = C / 4;
+  const bool vec = C % 4 == 0 && lda % 4 == 0 && aligned(dA, 16) && ldz % 4 == 0 &&
+                   aligned(dZ, 8) && (!a || (lda_a % 4 == 0 && aligned(a, 8))) && aligned(part, 16);
+  if (vec)
+    hipLaunchKernelGGL(act_bwd4, dim3(nb), dim3(256), 0, st, dA, lda, a16, lda_a, c4, V, slope, z16, ldz, chunk, part);
+  else
+    hipLaunchKernelGGL(act_bwd, dim3(nb), dim3(256), 0, st, dA, lda, a16, lda_a, C, V, slope, z16, ldz, chunk, part);
   PC_LAUNCH_CHECK();
-  hipLaunchKernelGGL(sum_parts_f32, dim3(nblk(C)), dim3(256), 0, st, part, nb, C, db);
+  hipLaunchKernelGGL(sum_parts_f32, dim3(C), dim3(256), 0, st, part, nb, C, db);
   PC_LAUNCH_CHECK();
   return pc::PC_OK;
 }
