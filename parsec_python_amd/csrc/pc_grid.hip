@@ -16,11 +16,11 @@
 // Chebyshev filters (src/Eigensolvers/ch_filter.py:66-80, first_filt.py:94-101).
 // x may alias out (each point reads x before writing out at the same place).
 //
-// Kernel shape (CDNA4): a workgroup owns one vector, a slab of TY y-rows and
-// all x, and marches along z.  Each thread keeps its points' 2R+1 z-values in
-// registers; the current plane of the slab plus R halo rows above/below sits
-// in LDS for the x/y differences.  Workgroup ids are remapped so the slabs of
-// one vector run on the same XCD (its L2 then serves the halo rows).
+// Kernel shape (CDNA4): a workgroup owns one vector, a slab of y-rows and a window
+// of up to 64 columns, and marches along z.  Each thread keeps its point's 2R+1
+// z-values in registers; the current plane of the slab plus R halo rows
+// above/below sits in LDS for the x/y differences.  Workgroup ids are remapped so
+// the windows of one vector run on the same XCD (its L2 then serves the halos).
 #include "pc_common.h"
 #include "pc_zmarch.h"
 #include <type_traits>
@@ -41,8 +41,10 @@ struct GridDev {
   int* prow;     // [npts]: row (j + ny*k) of each domain point
   int radius;
   double w[8];   // 1D -d2/dx2 weights, centre first (unscaled)
-  int* cc_tab;   // stencil_cc: per slab of 8 rows, the own and halo columns (tile row << 16 | x), -1 padded
-  int cc_wmax;   // its wavefronts per workgroup (0: not built)
+  int4* win;     // stencil_win: windows {first row, first column | columns << 16 | left halo lanes << 28, zb, ze}
+  int nwin;
+  int2* pmeta;   // its padded row table {offset, lo | length << 16}, nyp x nzp
+  int nyp, nzp;
 };
 
 struct StArgs {
@@ -58,7 +60,6 @@ struct StArgs {
   int nvec;
   int nblocks;   // real (unpadded) number of workgroups
   int nb8;       // ceil(nblocks/8)
-  int nzc, zc;   // z-chunks per slab and planes per chunk (lean and paired kernels)
   double w[8];   // scaled weights; w[0] already includes the factor 3
 };
 
@@ -339,20 +340,38 @@ __global__ __launch_bounds__(64 * NW) void stencil_zmarch(StArgs g, const T* __r
 }
 
 
-// ---- the lean z-march (one vector per workgroup, no partial sums) ------------
-// The same computation as stencil_zmarch<T,R,SX,1,1,2,HASX,false,1,NW>, written
-// to spend fewer vector instructions per plane:
-//   * the z-queue is a ring of QL registers per x-chunk, indexed by the plane's
+// ---- the windowed z-march (one vector per workgroup, no partial sums) ---------
+// A workgroup owns one vector and one window of a slab of win_ty(R) y-rows, one
+// wavefront of 64 columns per row.  A window is all the columns that the slab's
+// rows touch, where these are at most 64 (the columns beyond are zero); else a
+// part of them, with R columns of each neighbouring window among its 64 lanes.
+// The host lists the windows with the planes they touch.  The march along z:
+//   * the z-queue is a ring of QL registers per lane, indexed by the plane's
 //     phase; the plane loop is unrolled QL times so the ring turns by renaming
 //     instead of register moves (slot (z - zb + R) mod QL holds plane z);
-//   * every global access is a raw buffer access on a per-vector resource whose
-//     range is the vector's npts points: a lane outside its row's chord gets an
-//     out-of-range offset, so its load returns 0 and its store is dropped, with
-//     no branches around the memory instructions;
-//   * X and V are read at unmasked offsets (their values only reach stored
-//     lanes); X, V and the halo rows of plane z+2 go out before plane z is
-//     computed, and the queue front of plane z-R+QL right after plane z's last
-//     use of slot z-R (QL-2R-1 planes ahead of its use).
+//   * every global access is a raw buffer access on the row's own chord (base and
+//     size from scalar registers): a lane outside the chord, before or after it,
+//     has an out-of-range offset, so its load returns 0 and its store is dropped;
+//     one vector subtraction per access, no masks and no branches;
+//   * a row's {offset, extent} of 64 planes sits in a lane each and is read with
+//     v_readlane; the table is padded with empty rows, so nothing is clamped;
+//   * X, V and the halo rows of plane z+1 go out before plane z is computed, the
+//     queue front of plane z-R+QL right after plane z's last use of slot z-R.
+// What bounds it: per row and plane 37 vector, 38 scalar and 11 LDS instructions
+// at radius 4 against 5 loads and stores, with one barrier; on large blocks the
+// three passes over memory take 60 % of the time.  Occupancy is the registers':
+// two vectors per workgroup, three register sets or forced occupancy (spills)
+// were slower, and so were 4, 6 and 16 rows at radius 4 (the halo is 2R rows per
+// slab, the barrier is over all its wavefronts) and non-temporal X or stores.
+// One recurrence step; before: one slab and two 64-column chunks of a row in one
+// workgroup, masks and tables in vector registers, the windows full or half empty:
+//   605,808 points, radius 4 (Si87H76 sphere), 275 vectors:
+//                                   FP32 721 -> 700 us, FP64 1508 -> 1260 us
+//   C10H8 sphere, radius 4:         FP32 111 -> 98 us,  FP64 260 -> 186 us
+//   52^3 cube, radius 4, 23:        FP32 17.2 -> 16.8,  FP64 30.2 -> 24.8 us
+//   radius 6 (FD12), 103 columns:   256 vectors FP32 1310 -> 1212 us,
+//                                   64 vectors FP64 640 -> 587 us
+//   70^3 cube, 40 vectors:          radius 3 FP32 48.9 -> 47.6, radius 2 FP64 87.5 -> 81.5 us
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t pc_rsrc(const void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
@@ -379,411 +398,144 @@ __device__ __forceinline__ void pc_unroll_seq(std::integer_sequence<int, I...>, 
   (f(std::integral_constant<int, I>{}), ...);
 }
 
-#ifndef PC_LEAN_NS
-#define PC_LEAN_NS 3
-#endif
-#ifndef PC_LEAN_PF
-#define PC_LEAN_PF 3
-#endif
-#ifndef PC_LEAN_WAVES
-#define PC_LEAN_WAVES 0
-#endif
-// queue length: 2R+1 planes plus PC_LEAN_PF fronts in flight, rounded up to a
-// multiple of 2*NS (tile parity and register sets repeat within the block)
-constexpr int pc_lean_ql(int R) {
-  return (2 * R + 1 + PC_LEAN_PF + 2 * PC_LEAN_NS - 1) / (2 * PC_LEAN_NS) * (2 * PC_LEAN_NS);
-}
+// rows (wavefronts) per workgroup: one halo row per wavefront from radius 4 on
+constexpr int win_ty(int R) { return R <= 4 ? 8 : 2 * R; }
+constexpr int kWinNS = 2;    // register sets of X, V and halo values in flight
+// queue length: 2R+1 planes plus 3 fronts in flight, rounded up to a multiple of
+// 2 kWinNS (tile parity and register sets repeat within the block)
+constexpr int win_ql(int R) { return (2 * R + 1 + 3 + 2 * kWinNS - 1) / (2 * kWinNS) * (2 * kWinNS); }
+constexpr int kWinPadY = 24;  // empty rows around the padded row table (>= win_ty(R) + R) ...
+constexpr int kWinPadZ = 64;  // ... and planes above (>= 2 win_ql(R)); R planes below
 
-// Workgroup: TY y-rows of one vector; wave w owns row w % TY and the CPW
-// x-chunks of 64 points starting at chunk (w / TY) * CPW, so a workgroup has
-// TY * SX / CPW waves and each wave keeps only CPW chunks of queue registers.
-// ZC: the slab's z-range is split into chunks of g.zc planes (few vectors);
-// a separate instantiation, so the unchunked kernel keeps its registers.
-template <typename T, int R, int SX, int TY, int CPW, bool HASX, bool ZC>
-__global__ __launch_bounds__(64 * TY * SX / CPW)
-#if PC_LEAN_WAVES > 0
-__attribute__((amdgpu_waves_per_eu(PC_LEAN_WAVES, PC_LEAN_WAVES)))
-#endif
-void stencil_lean(StArgs g, const T* Y, const T* X, T* Out, const T* V, T ca, T cb, T cc) {
-  constexpr int NWV = TY * SX / CPW;          // waves per workgroup
-  constexpr int NXP = 64 * SX;
-  constexpr int LW = NXP + 2 * R;
+struct WinArgs {
+  const int4* win;     // {first row, first column | columns << 16 | halo lanes << 28, zb, ze}
+  const int2* meta;    // padded row table {offset, lo | length << 16}
+  int nyp, nzp;        // its rows and planes
+  long long ld;
+  int nwin, nzc, zc;   // windows, z-chunks per window and planes per chunk
+  int nblocks, nb8;
+  double w[8];         // scaled weights; w[0] already includes the factor 3
+};
+
+template <typename T, int R, bool HASX>
+__global__ __launch_bounds__(64 * win_ty(R)) void stencil_win(WinArgs g, const T* Y, const T* X, T* Out, const T* V, T ca,
+                                                          T cb, T cc) {
+  constexpr int TY = win_ty(R), NS = kWinNS, QL = win_ql(R);
   constexpr int LR = TY + 2 * R;
-  constexpr int NHI = 2 * R * (SX / CPW);     // halo items: (halo row, chunk group)
-  constexpr int HT = (NHI + NWV - 1) / NWV;   // halo items per wave
-  constexpr int NS = PC_LEAN_NS;
-  constexpr int QL = pc_lean_ql(R);
+  constexpr int HT = (2 * R + TY - 1) / TY;   // halo rows per wavefront
   constexpr int ES = (int)sizeof(T);
-  constexpr int OOB = 0x7ffffff0;     // beyond every range (npts * ES < 2^31 is checked on the host)
-  static_assert(SX % CPW == 0, "chunks per wave must divide the chunks per row");
-  __shared__ T tile[2][LR * LW];
-  // row metadata of the slab's LR rows for the planes the march touches (the
-  // launch sizes it for the grid's nz), read with uniform addresses every plane
-  extern __shared__ int2 mtab[];
-
-  const int bid = blockIdx.x;
-  const int L = (bid & 7) * g.nb8 + (bid >> 3);
+  constexpr int LW = 64 + 2 * R;         // R zero columns either side
+  // row LR takes what wavefronts without a halo row write
+  __shared__ T tile[2][(LR + 1) * LW];
+  const int L = (blockIdx.x & 7) * g.nb8 + (blockIdx.x >> 3);
   if (L >= g.nblocks) return;
-  // workgroup L: vector v, z-chunk zci, slab of TY rows (slab fastest)
-  const int nvz = ZC ? g.nslab * g.nzc : g.nslab;
-  const int v = L / nvz;
-  const int zci = ZC ? (L - v * nvz) / g.nslab : 0;
-  const int slab = L - v * nvz - zci * g.nslab;
-  const int j0 = slab * TY;
+  // workgroup L: vector v, z-chunk zci, window wi (fastest)
+  const int per = g.nwin * g.nzc;
+  const int v = L / per, zci = (L - v * per) / g.nwin, wi = L - v * per - zci * g.nwin;
+  const int4 win = g.win[wi];
+  const int zb = win.z + zci * g.zc, ze = min(win.w, zb + g.zc);
+  if (zb >= ze) return;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ny = g.ny, nz = g.nz;
-
-  int zb = nz, ze = 0;
-  for (int t = 0; t < TY; ++t) {
-    const int j = j0 + t;
-    if (j < ny) {
-      zb = min(zb, g.zrange[2 * j]);
-      ze = max(ze, g.zrange[2 * j + 1]);
-    }
-  }
-  // this workgroup's chunk of the slab's z-range; planes past its end are
-  // computed by the march's last block but not stored (the next chunk's
-  // workgroup stores them; see the store range below)
-  if constexpr (ZC) {
-    zb = max(zb, zci * g.zc);
-    ze = min(ze, (zci + 1) * g.zc);
-  }
-  if (zb >= ze) return;
-  const int zlo = zb - R;
-  // planes zb-R .. zb-R + QL*(ceil((ze-zb)/QL) + 1) - 1: the launch sizes the
-  // table for nz + 2 QL planes
-  const int zm = (ze - zb + QL - 1) / QL * QL + QL;
-
-  const unsigned nbytes = (unsigned)(g.npts * ES);
   const long long base = (long long)v * g.ld;
-  const __amdgpu_buffer_rsrc_t ry = pc_rsrc(Y + base, nbytes);
-  const __amdgpu_buffer_rsrc_t rx = pc_rsrc(HASX ? X + base : Y + base, nbytes);
-  // Points are stored plane by plane, so every point of planes >= ze lies at
-  // or past the first point of plane ze: a chunk's store range ends there and
-  // the planes its march computes past its end are dropped by the range check.
-  unsigned sbytes = nbytes;
-  if constexpr (ZC) sbytes = (unsigned)((ze < nz ? (long long)g.off[ny * ze] : g.npts) * ES);
-  const __amdgpu_buffer_rsrc_t ro = pc_rsrc(Out + base, sbytes);
-  const __amdgpu_buffer_rsrc_t rv = pc_rsrc(V, nbytes);
-
-  for (int t = threadIdx.x; t < 2 * LR * LW; t += 64 * NWV) (&tile[0][0])[t] = T(0);
-  for (int e = threadIdx.x; e < LR * zm; e += 64 * NWV) {
-    const int t = e / zm, z = zlo + (e - t * zm);
-    const int j = j0 - R + t;
-    mtab[e] = (j >= 0 && j < ny && z >= 0 && z < nz) ? g.meta[j + ny * z] : make_int2(0, 0);
+  const T* __restrict__ yv = Y + base;
+  const T* xv = HASX ? X + base : Y + base;
+  T* ov = Out + base;
+  // win.y: first column | columns << 16 | halo lanes << 28
+  const int halo = win.y >> 28, width = win.y >> 16 & 0xfff;
+  const int lx = ((win.y & 0xffff) - halo + lane) * ES;                         // loads of Y
+  const int lo_ = lane >= halo && lane < halo + width ? lx : 0x40000000;        // X, V and the store: the window's columns
+  for (int e = threadIdx.x; e < 2 * (LR + 1) * 2 * R; e += 64 * TY) {
+    const int row = e / (2 * R), c = e % (2 * R);
+    (&tile[0][0])[row * LW + (c < R ? c : 64 + c)] = T(0);
   }
-  __syncthreads();
 
-  // metadata of slab row t (0 .. LR-1, own rows at R .. R+TY-1) at plane z, as scalars
-  auto mrow = [&](int t, int z) -> int2 {
-    const int2 m = mtab[t * zm + (z - zlo)];
-    return make_int2(__builtin_amdgcn_readfirstlane(m.x), __builtin_amdgcn_readfirstlane(m.y));
-  };
-  // byte offset of x-chunk c in a row with metadata m: masked (out of range
-  // outside the chord) or plain (any in-range or out-of-range address)
-  auto off_masked = [&](int2 m, int c) -> int {
-    const int i = lane + 64 * c;
-    const int lo = m.y & 0xffff, len = (m.y >> 16) - lo;
-    return (unsigned)(i - lo) < (unsigned)len ? (m.x + i) * ES : OOB;
-  };
-  auto off_plain = [&](int2 m, int c) -> int { return (m.x + lane + 64 * c) * ES; };
-
-  const int town = R + wv % TY;               // own row in the tile
-  const int c0 = (wv / TY) * CPW;              // first own chunk
-  int th[HT], tc[HT];                          // halo items: tile row and first chunk
+  // row metadata: lane l holds plane wb + l
+  const int jo = win.x + wv + kWinPadY;
+  int jh[HT], th[HT];
 #pragma unroll
   for (int u = 0; u < HT; ++u) {
-    const int k = wv + NWV * u;
-    const int hr = k % (2 * R);
-    th[u] = hr < R ? hr : hr + TY;
-    tc[u] = (k / (2 * R)) * CPW;
+    const int k = wv + TY * u;
+    th[u] = k < 2 * R ? (k < R ? k : k + TY) : LR;
+    jh[u] = k < 2 * R ? win.x - R + th[u] + kWinPadY : 0;                  // (row 0 of the table is empty)
   }
-  auto has_halo = [&](int u) { return wv + NWV * u < NHI; };
+  int wb;
+  int2 wo, wh[HT];
+  auto windows = [&](int z) {
+    wb = z;
+    const int row = min(z + R + lane, g.nzp - 1) * g.nyp;
+    wo = g.meta[row + jo];
+#pragma unroll
+    for (int u = 0; u < HT; ++u) wh[u] = g.meta[row + jh[u]];
+  };
+  struct Row { int off, lo, len; };
+  auto row_of = [&](int2 m, int z) -> Row {
+    const int a = __builtin_amdgcn_readlane(m.x, z - wb), b = __builtin_amdgcn_readlane(m.y, z - wb);
+    return {a, b & 0xffff, b >> 16};
+  };
+  auto yload = [&](Row r) -> T { return pc_bload<T>(pc_rsrc(yv + r.off, (unsigned)(r.len * ES)), lx - r.lo * ES); };
 
-  T q[CPW][QL];
-  T xq[NS][CPW], vq[NS][CPW], hq[NS][HT][CPW];
-  int so[NS][CPW];
-  // prefill: planes zb-R .. zb-R+QL-1 into slots 0 .. QL-1 (slot of plane p: (p - zb + R) mod QL)
+  T q[QL];
+  T xq[NS], vq[NS], hq[NS][HT];
+  Row ro[NS];
+  windows(zb - R);
 #pragma unroll
-  for (int d = 0; d < QL; ++d) {
-    const int2 m = mrow(town, zb - R + d);
-#pragma unroll
-    for (int c = 0; c < CPW; ++c) q[c][d] = pc_bload<T>(ry, off_masked(m, c0 + c));
-  }
-  // X, V, halo rows and store offsets of plane z into set S
+  for (int d = 0; d < QL; ++d) q[d] = yload(row_of(wo, zb - R + d));
+  // X, V, halo rows of plane z into set S
   auto issue_plane = [&](auto set, int z) {
     constexpr int S = decltype(set)::value;
-    const int2 mo = mrow(town, z);
+    const Row r = row_of(wo, z);
+    ro[S] = r;
+    const int off = lo_ - r.lo * ES;
+    vq[S] = pc_bload<T>(pc_rsrc(V + r.off, (unsigned)(r.len * ES)), off);
+    if constexpr (HASX) xq[S] = pc_bload<T>(pc_rsrc(xv + r.off, (unsigned)(r.len * ES)), off);
 #pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-      const int po = off_plain(mo, c0 + c);
-      so[S][c] = off_masked(mo, c0 + c);
-      vq[S][c] = pc_bload<T>(rv, po);
-      if constexpr (HASX) xq[S][c] = pc_bload<T>(rx, po);
-    }
-#pragma unroll
-    for (int u = 0; u < HT; ++u) {
-      if (has_halo(u)) {
-        const int2 mh = mrow(th[u], z);
-#pragma unroll
-        for (int c = 0; c < CPW; ++c) hq[S][u][c] = pc_bload<T>(ry, off_masked(mh, tc[u] + c));
-      }
-    }
+    for (int u = 0; u < HT; ++u) hq[S][u] = yload(row_of(wh[u], z));
   };
   pc_unroll_seq(std::make_integer_sequence<int, NS - 1>{}, [&](auto k) {
     constexpr int K = decltype(k)::value;
     issue_plane(std::integral_constant<int, K>{}, zb + K);
   });
-
   const T w0 = T(g.w[0]);
   T wd[R + 1];
 #pragma unroll
   for (int d = 1; d <= R; ++d) wd[d] = T(g.w[d]);
 
   // Planes run in whole blocks of QL, past ze up to the next multiple of QL:
-  // there the slab's rows are empty, so those planes' stores are all out of
-  // range, and the loads they issue read zeros or stay inside the vectors.
-  // No branch separates a load from its use, which keeps the compiler from
-  // sinking the prefetches to their uses.
+  // those planes are not stored (their store size is 0; the next z-chunk's
+  // workgroup stores them) and what they load is empty or not used.
   auto plane = [&](auto phase, int z) {
     constexpr int P = decltype(phase)::value;
     constexpr int S = P % NS;      // (z - zb) mod NS: the register set of plane z
     constexpr int B = P & 1;       // LDS tile of this plane
     issue_plane(std::integral_constant<int, (P + NS - 1) % NS>{}, z + NS - 1);
     __builtin_amdgcn_sched_barrier(0);
-    T* tb = tile[B];
+    T* tb = &tile[B][R];
+    tb[(wv + R) * LW + lane] = q[(P + R) % QL];
 #pragma unroll
-    for (int c = 0; c < CPW; ++c) tb[town * LW + R + lane + 64 * (c0 + c)] = q[c][(P + R) % QL];
-#pragma unroll
-    for (int u = 0; u < HT; ++u) {
-      if (has_halo(u)) {
-#pragma unroll
-        for (int c = 0; c < CPW; ++c) tb[th[u] * LW + R + lane + 64 * (tc[u] + c)] = hq[S][u][c];
-      }
-    }
+    for (int u = 0; u < HT; ++u) tb[th[u] * LW + lane] = hq[S][u];
     lds_barrier();
-#pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-      const T* trow = tb + town * LW + R + lane + 64 * (c0 + c);
-      const T yc = q[c][(P + R) % QL];
-      T acc = w0 * yc;
-#pragma unroll
-      for (int d = 1; d <= R; ++d) {
-        const T nb = trow[-d] + trow[d] + trow[-d * LW] + trow[d * LW] + q[c][(P + R - d) % QL] +
-                     q[c][(P + R + d) % QL];
-        acc += wd[d] * nb;
-      }
-      T o = acc + (ca * vq[S][c] + cb) * yc;
-      if constexpr (HASX) o += cc * xq[S][c];
-      pc_bstore<T>(ro, so[S][c], o);
-    }
-    // slot P (plane z-R) is free: plane z-R+QL, the queue front of plane z-2R+QL
-    {
-      const int2 m = mrow(town, z - R + QL);
-#pragma unroll
-      for (int c = 0; c < CPW; ++c) q[c][P] = pc_bload<T>(ry, off_masked(m, c0 + c));
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  for (int z0 = zb; z0 < ze; z0 += QL) {
-    pc_unroll_seq(std::make_integer_sequence<int, QL>{}, [&](auto ph) {
-      constexpr int P = decltype(ph)::value;
-      plane(ph, z0 + P);
-    });
-  }
-}
-
-#ifndef PC_LEAN_TY
-#define PC_LEAN_TY 8
-#endif
-
-// z-chunks for the lean and paired kernels: with few vectors the slab x vector
-// workgroups do not fill the chip (256 CUs x 32 wavefronts), so each slab's
-// z-range is split until the wavefronts would fill it once, keeping at least 8
-// planes per chunk (a chunk re-reads 2R queue planes of its neighbour and runs
-// a variant with a few more registers).  Measured (FP32, radius 4): H2O sphere
-// (69,264 points, k 23, 8 waves per workgroup) 30 -> 20 us; C10H8 sphere
-// (k 49, 16 waves per workgroup: 9,408 wavefronts already) 134 us unchunked,
-// 159-164 us when chunked to 1024-2048 workgroups.
-#ifndef PC_LEAN_ZCHUNK_WAVES
-#define PC_LEAN_ZCHUNK_WAVES 8192
-#endif
-#ifndef PC_LEAN_FORCE_ZC
-#define PC_LEAN_FORCE_ZC 0
-#endif
-inline void pc_zchunks(StArgs& a, int nz, int waves_per_wg) {
-  constexpr long long kWaves = PC_LEAN_ZCHUNK_WAVES;
-  const long long base = (long long)a.nslab * a.nvec * waves_per_wg;
-  int nzc = 1;
-  if (base < kWaves) nzc = (int)std::min<long long>((kWaves + base - 1) / base, std::max(1, nz / 8));
-  a.zc = (nz + nzc - 1) / nzc;
-  if (PC_LEAN_FORCE_ZC > 0) a.zc = std::min(nz, PC_LEAN_FORCE_ZC);
-  a.nzc = (nz + a.zc - 1) / a.zc;
-}
-
-template <typename T, int R, int SX>
-int launch_lean(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, int nvec, long long ld, double scale,
-                double ca, double cb, double cc, hipStream_t st) {
-  constexpr int TY = PC_LEAN_TY;
-  constexpr int CPW = SX > 2 ? SX / 2 : 1;     // at most 16 waves (1024 threads) per workgroup
-  constexpr int QL = pc_lean_ql(R);
-  constexpr int WPG = TY * SX / CPW;
-  StArgs a;
-  a.nx = gd->nx; a.ny = gd->ny; a.nz = gd->nz; a.npts = gd->npts;
-  a.lo = gd->lo; a.hi = gd->hi; a.off = gd->off; a.zrange = gd->zrange; a.meta = gd->meta;
-  a.ld = ld;
-  a.nslab = (gd->ny + TY - 1) / TY;
-  a.nvec = nvec;
-  pc_zchunks(a, gd->nz, WPG);
-  a.nblocks = a.nslab * a.nzc * nvec;
-  a.nb8 = (a.nblocks + 7) / 8;
-  for (int d = 0; d < 8; ++d) a.w[d] = 0.0;
-  a.w[0] = 3.0 * gd->w[0] * scale;
-  for (int d = 1; d <= R; ++d) a.w[d] = gd->w[d] * scale;
-  const dim3 grid(8 * a.nb8), block(64 * TY * SX / CPW);
-  const size_t mbytes = sizeof(int2) * (size_t)(TY + 2 * R) * (size_t)(gd->nz + 2 * QL);
-  if (a.nzc > 1) {
-    if (X)
-      hipLaunchKernelGGL((stencil_lean<T, R, SX, TY, CPW, true, true>), grid, block, mbytes, st, a, Y, X, Out, V,
-                         T(ca), T(cb), T(cc));
-    else
-      hipLaunchKernelGGL((stencil_lean<T, R, SX, TY, CPW, false, true>), grid, block, mbytes, st, a, Y, X, Out, V,
-                         T(ca), T(cb), T(cc));
-  } else if (X) {
-    hipLaunchKernelGGL((stencil_lean<T, R, SX, TY, CPW, true, false>), grid, block, mbytes, st, a, Y, X, Out, V,
-                       T(ca), T(cb), T(cc));
-  } else {
-    hipLaunchKernelGGL((stencil_lean<T, R, SX, TY, CPW, false, false>), grid, block, mbytes, st, a, Y, X, Out, V,
-                       T(ca), T(cb), T(cc));
-  }
-  PC_LAUNCH_CHECK();
-  return pc::PC_OK;
-}
-
-// ---- the compacted-column z-march (one vector per workgroup) ----------------
-// stencil_lean gives each wavefront a fixed 64-point x-chunk of one row, so on a
-// sphere about half of its lanes hold no point.  Here the lanes of a workgroup
-// are dealt the slab's actual columns: the host lists, per slab of TY rows,
-// the columns (tile row, x) that any plane of the slab's march touches, row
-// after row (own rows first, then the 2R halo rows' columns for the halo
-// loads), and a workgroup has as many wavefronts as the larger list needs.
-// Each lane keeps the z-queue of its own column, loads one halo column per
-// plane, and reads its row metadata per plane from the LDS table (per lane:
-// the rows of one wavefront differ).  The arithmetic and its order are those
-// of stencil_lean, so the results are the same bits.
-constexpr int kCcTY = 8;
-
-template <typename T, int R, int NXP, bool HASX>
-__global__ __launch_bounds__(1024) void stencil_cc(StArgs g, const int* __restrict__ ctab, int wmax, const T* Y,
-                                                   const T* X, T* Out, const T* V, T ca, T cb, T cc) {
-  constexpr int TY = kCcTY;
-  constexpr int LW = NXP + 2 * R;
-  constexpr int LR = TY + 2 * R;
-  constexpr int NS = PC_LEAN_NS;
-  constexpr int QL = pc_lean_ql(R);
-  constexpr int ES = (int)sizeof(T);
-  constexpr int OOB = 0x7ffffff0;
-  __shared__ T tile[2][LR * LW];
-  extern __shared__ int2 mtab[];
-
-  const int bid = blockIdx.x;
-  const int L = (bid & 7) * g.nb8 + (bid >> 3);
-  if (L >= g.nblocks) return;
-  const int v = L / g.nslab;
-  const int slab = L - v * g.nslab;
-  const int j0 = slab * TY;
-  const int ny = g.ny, nz = g.nz;
-  int zb = nz, ze = 0;
-  for (int t = 0; t < TY; ++t) {
-    const int j = j0 + t;
-    if (j < ny) {
-      zb = min(zb, g.zrange[2 * j]);
-      ze = max(ze, g.zrange[2 * j + 1]);
-    }
-  }
-  if (zb >= ze) return;
-  const int zlo = zb - R;
-  const int zm = (ze - zb + QL - 1) / QL * QL + QL;
-
-  const unsigned nbytes = (unsigned)(g.npts * ES);
-  const long long base = (long long)v * g.ld;
-  const __amdgpu_buffer_rsrc_t ry = pc_rsrc(Y + base, nbytes);
-  const __amdgpu_buffer_rsrc_t rx = pc_rsrc(HASX ? X + base : Y + base, nbytes);
-  const __amdgpu_buffer_rsrc_t ro = pc_rsrc(Out + base, nbytes);
-  const __amdgpu_buffer_rsrc_t rv = pc_rsrc(V, nbytes);
-
-  // this lane's own column (tile row tr, x) and halo column (tile row th, x)
-  const int* cs = ctab + (long long)slab * 2 * wmax * 64;
-  const int co = cs[threadIdx.x], ch = cs[wmax * 64 + threadIdx.x];
-  const bool own = co >= 0, hal = ch >= 0;
-  const int tr = own ? (co >> 16) : R, xo = own ? (co & 0xffff) : 0;
-  const int th = hal ? (ch >> 16) : 0, xh = hal ? (ch & 0xffff) : 0;
-
-  for (int t = threadIdx.x; t < 2 * LR * LW; t += blockDim.x) (&tile[0][0])[t] = T(0);
-  for (int e = threadIdx.x; e < LR * zm; e += blockDim.x) {
-    const int t = e / zm, z = zlo + (e - t * zm);
-    const int j = j0 - R + t;
-    mtab[e] = (j >= 0 && j < ny && z >= 0 && z < nz) ? g.meta[j + ny * z] : make_int2(0, 0);
-  }
-  __syncthreads();
-
-  auto mrow = [&](int t, int z) -> int2 { return mtab[t * zm + (z - zlo)]; };
-  auto off_masked = [&](int2 m, int x, bool ok) -> int {
-    const int lo = m.y & 0xffff, len = (m.y >> 16) - lo;
-    return (ok && (unsigned)(x - lo) < (unsigned)len) ? (m.x + x) * ES : OOB;
-  };
-  auto off_plain = [&](int2 m, int x, bool ok) -> int { return ok ? (m.x + x) * ES : OOB; };
-
-  T q[QL];
-  T xq[NS], vq[NS], hq[NS];
-  int so[NS];
-#pragma unroll
-  for (int d = 0; d < QL; ++d) q[d] = pc_bload<T>(ry, off_masked(mrow(tr, zb - R + d), xo, own));
-  auto issue_plane = [&](auto set, int z) {
-    constexpr int S = decltype(set)::value;
-    const int2 mo = mrow(tr, z);
-    const int po = off_plain(mo, xo, own);
-    so[S] = off_masked(mo, xo, own);
-    vq[S] = pc_bload<T>(rv, po);
-    if constexpr (HASX) xq[S] = pc_bload<T>(rx, po);
-    hq[S] = pc_bload<T>(ry, off_masked(mrow(th, z), xh, hal));
-  };
-  pc_unroll_seq(std::make_integer_sequence<int, NS - 1>{}, [&](auto k) {
-    constexpr int K = decltype(k)::value;
-    issue_plane(std::integral_constant<int, K>{}, zb + K);
-  });
-
-  const T w0 = T(g.w[0]);
-  T wd[R + 1];
-#pragma unroll
-  for (int d = 1; d <= R; ++d) wd[d] = T(g.w[d]);
-
-  auto plane = [&](auto phase, int z) {
-    constexpr int P = decltype(phase)::value;
-    constexpr int S = P % NS;
-    constexpr int B = P & 1;
-    issue_plane(std::integral_constant<int, (P + NS - 1) % NS>{}, z + NS - 1);
-    __builtin_amdgcn_sched_barrier(0);
-    T* tb = tile[B];
-    if (own) tb[tr * LW + R + xo] = q[(P + R) % QL];
-    if (hal) tb[th * LW + R + xh] = hq[S];
-    lds_barrier();
-    const T* trow = tb + tr * LW + R + xo;
+    const T* trow = tb + (wv + R) * LW + lane;
     const T yc = q[(P + R) % QL];
     T acc = w0 * yc;
 #pragma unroll
     for (int d = 1; d <= R; ++d) {
       const T nb = trow[-d] + trow[d] + trow[-d * LW] + trow[d * LW] + q[(P + R - d) % QL] + q[(P + R + d) % QL];
       acc += wd[d] * nb;
+      // one distance's LDS reads at a time: all 24 at once cost radius 6 its
+      // second workgroup per CU (FP32 1598 -> 1209 us), radius 4 nothing
+      if (R > 4 && d < R) __builtin_amdgcn_sched_barrier(0);
     }
     T o = acc + (ca * vq[S] + cb) * yc;
     if constexpr (HASX) o += cc * xq[S];
-    pc_bstore<T>(ro, so[S], o);
-    q[P] = pc_bload<T>(ry, off_masked(mrow(tr, z - R + QL), xo, own));
+    const Row r = ro[S];
+    pc_bstore<T>(pc_rsrc(ov + r.off, z < ze ? (unsigned)(r.len * ES) : 0u), lo_ - r.lo * ES, o);
+    // slot P (plane z-R) is free: plane z-R+QL, the queue front of plane z-2R+QL
+    q[P] = yload(row_of(wo, z - R + QL));
     __builtin_amdgcn_sched_barrier(0);
   };
   for (int z0 = zb; z0 < ze; z0 += QL) {
+    if (z0 + 2 * QL > wb + 64) windows(z0);
     pc_unroll_seq(std::make_integer_sequence<int, QL>{}, [&](auto ph) {
       constexpr int P = decltype(ph)::value;
       plane(ph, z0 + P);
@@ -791,391 +543,79 @@ __global__ __launch_bounds__(1024) void stencil_cc(StArgs g, const int* __restri
   }
 }
 
-// pc_stencil_set_variant: 0 = stencil_lean, 1 = stencil_cc, 2 = stencil_cc for
-// FP32 launches of fewer than 128 vectors that stencil_lean would not split
-// into z-chunks (the default).  Measured (FP32 step, radius 4, same bits):
-// C10H8 sphere (nx 92, 49 vectors) 118 us against 133 us; Si87H76 sphere
-// (nx 106, 275 vectors) 824 against 787 us; H2O sphere (nx 52, 23 vectors,
-// z-chunked by stencil_lean) 30 against 18 us.
-int g_stencil_cc = 2;
+// z-chunks: with few vectors the windows x vectors do not fill the chip (256
+// CUs x 32 wavefronts), so each window's z-range is split until the wavefronts
+// would fill it once, keeping at least 8 planes per chunk (a chunk re-reads 2R
+// queue planes of its neighbour).
+constexpr long long kWinWaves = 8192;
+inline void win_zchunks(WinArgs& a, int nz, int nvec, int waves_per_wg) {
+  const long long base = (long long)a.nwin * nvec * waves_per_wg;
+  int nzc = 1;
+  if (base < kWinWaves) nzc = (int)std::min<long long>((kWinWaves + base - 1) / base, std::max(1, nz / 8));
+  a.zc = (nz + nzc - 1) / nzc;
+  a.nzc = (nz + a.zc - 1) / a.zc;
+}
 
 template <typename T, int R>
-int launch_cc(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, int nvec, long long ld, double scale,
-              double ca, double cb, double cc, hipStream_t st) {
-  constexpr int TY = kCcTY;
-  constexpr int QL = pc_lean_ql(R);
+int launch_win(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, int nvec, long long ld, double scale,
+               double ca, double cb, double cc, hipStream_t st) {
+  WinArgs a;
+  a.win = gd->win;
+  a.nwin = gd->nwin;
+  if (a.nwin == 0) return pc::PC_OK;   // no points
+  a.meta = gd->pmeta; a.nyp = gd->nyp; a.nzp = gd->nzp;
+  a.ld = ld;
+  win_zchunks(a, gd->nz, nvec, win_ty(R));
+  const long long nb = (long long)a.nwin * a.nzc * nvec;
+  PC_CHECK_ARG(nb < (1LL << 30), "too many workgroups");
+  a.nblocks = (int)nb;
+  a.nb8 = (a.nblocks + 7) / 8;
+  for (int d = 0; d < 8; ++d) a.w[d] = 0.0;
+  a.w[0] = 3.0 * gd->w[0] * scale;
+  for (int d = 1; d <= R; ++d) a.w[d] = gd->w[d] * scale;
+  const dim3 grid(8 * a.nb8), block(64 * win_ty(R));
+  if (X)
+    hipLaunchKernelGGL((stencil_win<T, R, true>), grid, block, 0, st, a, Y, X, Out, V, T(ca), T(cb), T(cc));
+  else
+    hipLaunchKernelGGL((stencil_win<T, R, false>), grid, block, 0, st, a, Y, X, Out, V, T(ca), T(cb), T(cc));
+  PC_LAUNCH_CHECK();
+  return pc::PC_OK;
+}
+
+// With per-vector partial sums: one vector and 4 rows (wavefronts) per workgroup.
+template <typename T, int R, int SX>
+int launch_dot(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, int nvec, long long ld, double scale,
+               double ca, double cb, double cc, double* dot_part, hipStream_t st) {
+  constexpr int NW = 4;
   StArgs a;
   a.nx = gd->nx; a.ny = gd->ny; a.nz = gd->nz; a.npts = gd->npts;
   a.lo = gd->lo; a.hi = gd->hi; a.off = gd->off; a.zrange = gd->zrange; a.meta = gd->meta;
   a.ld = ld;
-  a.nslab = (gd->ny + TY - 1) / TY;
+  a.nslab = (gd->ny + NW - 1) / NW;
   a.nvec = nvec;
-  a.nzc = 1; a.zc = gd->nz;
   a.nblocks = a.nslab * nvec;
   a.nb8 = (a.nblocks + 7) / 8;
   for (int d = 0; d < 8; ++d) a.w[d] = 0.0;
   a.w[0] = 3.0 * gd->w[0] * scale;
   for (int d = 1; d <= R; ++d) a.w[d] = gd->w[d] * scale;
-  const dim3 grid(8 * a.nb8), block(64 * gd->cc_wmax);
-  const size_t mbytes = sizeof(int2) * (size_t)(TY + 2 * R) * (size_t)(gd->nz + 2 * QL);
-  if (gd->nx <= 64) {
-    if (X) hipLaunchKernelGGL((stencil_cc<T, R, 64, true>), grid, block, mbytes, st, a, gd->cc_tab, gd->cc_wmax, Y, X, Out, V, T(ca), T(cb), T(cc));
-    else hipLaunchKernelGGL((stencil_cc<T, R, 64, false>), grid, block, mbytes, st, a, gd->cc_tab, gd->cc_wmax, Y, X, Out, V, T(ca), T(cb), T(cc));
-  } else {
-    if (X) hipLaunchKernelGGL((stencil_cc<T, R, 128, true>), grid, block, mbytes, st, a, gd->cc_tab, gd->cc_wmax, Y, X, Out, V, T(ca), T(cb), T(cc));
-    else hipLaunchKernelGGL((stencil_cc<T, R, 128, false>), grid, block, mbytes, st, a, gd->cc_tab, gd->cc_wmax, Y, X, Out, V, T(ca), T(cb), T(cc));
-  }
-  PC_LAUNCH_CHECK();
-  return pc::PC_OK;
-}
-
-// ---- the paired z-march (FP32, rows of 65..128 points) ---------------------
-// stencil_lean with two adjacent x points per lane: lane l holds x = 2l, 2l+1,
-// so one wavefront covers a whole row and every Y / X / V access and the store
-// move 8 bytes per lane (64-bit buffer accesses) instead of 4.  The row data
-// starts at any element, so a pair straddles the chord ends: a pair with at
-// least one point in the chord is loaded whole and its outside point is set to
-// zero at first use (queue entries: when the plane enters the stencil as z+R;
-// halo rows: before they go to LDS), and a store writes the pair when both
-// points are in the chord, else the one point that is (a 32-bit store).  The
-// two pairs that would straddle the ends of the array (flat start -1 or
-// npts-1) are loaded from 0 or npts-2 and shifted into place, so every 64-bit
-// access lies wholly inside the vector.
-typedef float pc_f2 __attribute__((ext_vector_type(2)));
-typedef unsigned pc_u2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ pc_f2 pc_bload2(__amdgpu_buffer_rsrc_t r, int off) {
-  return __builtin_bit_cast(pc_f2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
-}
-
-template <int R, int TY, bool HASX>
-__global__ __launch_bounds__(64 * TY)
-void stencil_pair(StArgs g, const float* Y, const float* X, float* Out, const float* V, float ca, float cb, float cc) {
-  using T = float;
-  constexpr int NWV = TY;                     // one wave per row
-  constexpr int LW = 128 + 2 * R;
-  constexpr int LR = TY + 2 * R;
-  constexpr int NHI = 2 * R;                  // halo rows
-  constexpr int HT = (NHI + NWV - 1) / NWV;
-  constexpr int NS = PC_LEAN_NS;
-  constexpr int QL = pc_lean_ql(R);
-  constexpr int ES = 4;
-  constexpr int OOB = 0x7ffffff0;
-  __shared__ __align__(16) T tile[2][LR * LW];
-  extern __shared__ int2 mtab[];
-
-  const int bid = blockIdx.x;
-  const int L = (bid & 7) * g.nb8 + (bid >> 3);
-  if (L >= g.nblocks) return;
-  // workgroup L: vector v, z-chunk zci, slab of TY rows (slab fastest)
-  const int nvz = g.nslab * g.nzc;
-  const int v = L / nvz;
-  const int zci = (L - v * nvz) / g.nslab;
-  const int slab = L - v * nvz - zci * g.nslab;
-  const int j0 = slab * TY;
-  const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ny = g.ny, nz = g.nz;
-
-  int zb = nz, ze = 0;
-  for (int t = 0; t < TY; ++t) {
-    const int j = j0 + t;
-    if (j < ny) {
-      zb = min(zb, g.zrange[2 * j]);
-      ze = max(ze, g.zrange[2 * j + 1]);
-    }
-  }
-  zb = max(zb, zci * g.zc);
-  ze = min(ze, (zci + 1) * g.zc);
-  if (zb >= ze) return;
-  const int zlo = zb - R;
-  const int zm = (ze - zb + QL - 1) / QL * QL + QL;
-
-  const unsigned nbytes = (unsigned)(g.npts * ES);
-  const long long base = (long long)v * g.ld;
-  const __amdgpu_buffer_rsrc_t ry = pc_rsrc(Y + base, nbytes);
-  const __amdgpu_buffer_rsrc_t rx = pc_rsrc(HASX ? X + base : Y + base, nbytes);
-  const __amdgpu_buffer_rsrc_t ro = pc_rsrc(Out + base, nbytes);
-  const __amdgpu_buffer_rsrc_t rv = pc_rsrc(V, nbytes);
-
-  for (int t = threadIdx.x; t < 2 * LR * LW; t += 64 * NWV) (&tile[0][0])[t] = T(0);
-  for (int e = threadIdx.x; e < LR * zm; e += 64 * NWV) {
-    const int t = e / zm, z = zlo + (e - t * zm);
-    const int j = j0 - R + t;
-    mtab[e] = (j >= 0 && j < ny && z >= 0 && z < nz) ? g.meta[j + ny * z] : make_int2(0, 0);
-  }
-  __syncthreads();
-
-  auto mrow = [&](int t, int z) -> int2 {
-    const int2 m = mtab[t * zm + (z - zlo)];
-    return make_int2(__builtin_amdgcn_readfirstlane(m.x), __builtin_amdgcn_readfirstlane(m.y));
-  };
-  const int i0 = 2 * lane;
-  const int last2 = (int)g.npts - 2;           // the host checks npts >= 2
-  // flat start of the pair (m.x + i0) clamped to [0, npts-2]
-  auto pair_start = [&](int2 m) -> int { return min(max(m.x + i0, 0), last2); };
-  // byte offset of the pair: out of range unless a point is in the chord
-  auto off_pair = [&](int2 m) -> int {
-    const int lo = m.y & 0xffff, len = (m.y >> 16) - lo;
-    const bool any = (unsigned)(i0 - lo) < (unsigned)len || (unsigned)(i0 + 1 - lo) < (unsigned)len;
-    return any ? pair_start(m) * ES : OOB;
-  };
-  // the pair loaded from pair_start(m), shifted back to x = i0, i0+1, with the
-  // points outside the chord set to zero
-  auto fix_pair = [&](int2 m, pc_f2 a) -> pc_f2 {
-    const int start = m.x + i0, st = pair_start(m);
-    const int lo = m.y & 0xffff, len = (m.y >> 16) - lo;
-    T x0 = start > st ? a.y : (start < st ? T(0) : a.x);
-    T x1 = start < st ? a.x : (start > st ? T(0) : a.y);
-    pc_f2 r;
-    r.x = (unsigned)(i0 - lo) < (unsigned)len ? x0 : T(0);
-    r.y = (unsigned)(i0 + 1 - lo) < (unsigned)len ? x1 : T(0);
-    return r;
-  };
-
-  const int town = R + wv;
-  int th[HT];
-#pragma unroll
-  for (int u = 0; u < HT; ++u) {
-    const int k = wv + NWV * u;
-    th[u] = k < R ? k : k + TY;
-  }
-  auto has_halo = [&](int u) { return wv + NWV * u < NHI; };
-
-  pc_f2 q[QL];
-  pc_f2 xq[NS], vq[NS], hq[NS][HT];
-  // prefill planes zb-R .. zb-R+QL-1; the 2R planes zb-R .. zb+R-1 are used
-  // before the march masks anything, so they are masked here
-#pragma unroll
-  for (int d = 0; d < QL; ++d) q[d] = pc_bload2(ry, off_pair(mrow(town, zb - R + d)));
-#pragma unroll
-  for (int d = 0; d < 2 * R; ++d) q[d] = fix_pair(mrow(town, zb - R + d), q[d]);
-
-  auto issue_plane = [&](auto set, int z) {
-    constexpr int S = decltype(set)::value;
-    const int po = pair_start(mrow(town, z)) * ES;
-    vq[S] = pc_bload2(rv, po);
-    if constexpr (HASX) xq[S] = pc_bload2(rx, po);
-#pragma unroll
-    for (int u = 0; u < HT; ++u)
-      if (has_halo(u)) hq[S][u] = pc_bload2(ry, off_pair(mrow(th[u], z)));
-  };
-  pc_unroll_seq(std::make_integer_sequence<int, NS - 1>{}, [&](auto k) {
-    constexpr int K = decltype(k)::value;
-    issue_plane(std::integral_constant<int, K>{}, zb + K);
-  });
-
-  const T w0 = T(g.w[0]);
-  T wd[R + 1];
-#pragma unroll
-  for (int d = 1; d <= R; ++d) wd[d] = T(g.w[d]);
-
-  auto plane = [&](auto phase, int z) {
-    constexpr int P = decltype(phase)::value;
-    constexpr int S = P % NS;
-    constexpr int B = P & 1;
-    issue_plane(std::integral_constant<int, (P + NS - 1) % NS>{}, z + NS - 1);
-    __builtin_amdgcn_sched_barrier(0);
-    // plane z+R enters the stencil: shift and zero its points outside the chord
-    q[(P + 2 * R) % QL] = fix_pair(mrow(town, z + R), q[(P + 2 * R) % QL]);
-    T* tb = tile[B];
-    {
-      const pc_f2 c = q[(P + R) % QL];
-      tb[town * LW + R + i0] = c.x;
-      tb[town * LW + R + i0 + 1] = c.y;
-    }
-#pragma unroll
-    for (int u = 0; u < HT; ++u) {
-      if (has_halo(u)) {
-        const pc_f2 h = fix_pair(mrow(th[u], z), hq[S][u]);
-        tb[th[u] * LW + R + i0] = h.x;
-        tb[th[u] * LW + R + i0 + 1] = h.y;
-      }
-    }
-    lds_barrier();
-    const int2 mo = mrow(town, z);
-    const T* trow = tb + town * LW + R + i0;
-    T xs[2 * R + 2];                           // own row at x = i0-R .. i0+R+1
-#pragma unroll
-    for (int d = 0; d < 2 * R + 2; ++d) xs[d] = trow[d - R];
-    const pc_f2 yc = q[(P + R) % QL];
-    pc_f2 acc = w0 * yc;
-#pragma unroll
-    for (int d = 1; d <= R; ++d) {
-      // the summation order of stencil_lean: x-, x+, y-, y+, z-, z+
-      const pc_f2 zm = q[(P + R - d) % QL], zp = q[(P + R + d) % QL];
-      pc_f2 nb;
-      nb.x = xs[R - d] + xs[R + d] + trow[-d * LW] + trow[d * LW] + zm.x + zp.x;
-      nb.y = xs[R + 1 - d] + xs[R + 1 + d] + trow[-d * LW + 1] + trow[d * LW + 1] + zm.y + zp.y;
-      acc += wd[d] * nb;
-    }
-    pc_f2 o = acc + (ca * fix_pair(mo, vq[S]) + cb) * yc;
-    if constexpr (HASX) o += cc * fix_pair(mo, xq[S]);
-    {
-      const int lo = mo.y & 0xffff, len = (mo.y >> 16) - lo;
-      const bool inz = z < ze;
-      const bool in0 = inz && (unsigned)(i0 - lo) < (unsigned)len;
-      const bool in1 = inz && (unsigned)(i0 + 1 - lo) < (unsigned)len;
-      const int o2 = (in0 && in1) ? (mo.x + i0) * ES : OOB;
-      const int o1 = (in0 != in1) ? (mo.x + i0 + (in0 ? 0 : 1)) * ES : OOB;
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(pc_u2, o), ro, o2, 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, in0 ? o.x : o.y), ro, o1, 0, 0);
-    }
-    q[P] = pc_bload2(ry, off_pair(mrow(town, z - R + QL)));
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  for (int z0 = zb; z0 < ze; z0 += QL) {
-    pc_unroll_seq(std::make_integer_sequence<int, QL>{}, [&](auto ph) {
-      constexpr int P = decltype(ph)::value;
-      plane(ph, z0 + P);
-    });
-  }
-}
-
-#ifndef PC_STENCIL_PAIR
-#define PC_STENCIL_PAIR 1
-#endif
-
-template <int R>
-int launch_pair(const GridDev* gd, const float* Y, const float* X, float* Out, const float* V, int nvec, long long ld,
-                double scale, double ca, double cb, double cc, hipStream_t st) {
-  constexpr int TY = PC_LEAN_TY;
-  constexpr int QL = pc_lean_ql(R);
-  constexpr int WPG = TY;
-  StArgs a;
-  a.nx = gd->nx; a.ny = gd->ny; a.nz = gd->nz; a.npts = gd->npts;
-  a.lo = gd->lo; a.hi = gd->hi; a.off = gd->off; a.zrange = gd->zrange; a.meta = gd->meta;
-  a.ld = ld;
-  a.nslab = (gd->ny + TY - 1) / TY;
-  a.nvec = nvec;
-  pc_zchunks(a, gd->nz, WPG);
-  a.nblocks = a.nslab * a.nzc * nvec;
-  a.nb8 = (a.nblocks + 7) / 8;
-  for (int d = 0; d < 8; ++d) a.w[d] = 0.0;
-  a.w[0] = 3.0 * gd->w[0] * scale;
-  for (int d = 1; d <= R; ++d) a.w[d] = gd->w[d] * scale;
-  const dim3 grid(8 * a.nb8), block(64 * TY);
-  const size_t mbytes = sizeof(int2) * (size_t)(TY + 2 * R) * (size_t)(gd->nz + 2 * QL);
-  if (X)
-    hipLaunchKernelGGL((stencil_pair<R, TY, true>), grid, block, mbytes, st, a, Y, X, Out, V, float(ca), float(cb),
-                       float(cc));
-  else
-    hipLaunchKernelGGL((stencil_pair<R, TY, false>), grid, block, mbytes, st, a, Y, X, Out, V, float(ca), float(cb),
-                       float(cc));
-  PC_LAUNCH_CHECK();
-  return pc::PC_OK;
-}
-
-template <typename T, int R, int SX, int TYW, int NV, int NB = 2, int NW = 4>
-constexpr int zmarch_lds_bytes() {
-  return NB * NV * (NW * TYW + 2 * R) * (64 * SX + 2 * R) * (int)sizeof(T);
-}
-
-template <typename T, int R, int SX, int TYW, int NV, int NB = 2, int PD = 1, int NW = 4>
-int launch_cfg(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, int nvec, long long ld, double scale,
-               double ca, double cb, double cc, double* dot_part, hipStream_t st) {
-  constexpr int TY = NW * TYW;
-  StArgs a;
-  a.nx = gd->nx; a.ny = gd->ny; a.nz = gd->nz; a.npts = gd->npts;
-  a.lo = gd->lo; a.hi = gd->hi; a.off = gd->off; a.zrange = gd->zrange; a.meta = gd->meta;
-  a.ld = ld;
-  a.nslab = (gd->ny + TY - 1) / TY;
-  a.nvec = nvec;
-  a.nzc = 1;
-  a.zc = gd->nz;
-  a.nblocks = a.nslab * ((nvec + NV - 1) / NV);
-  a.nb8 = (a.nblocks + 7) / 8;
-  for (int d = 0; d < 8; ++d) a.w[d] = 0.0;
-  a.w[0] = 3.0 * gd->w[0] * scale;
-  for (int d = 1; d <= R; ++d) a.w[d] = gd->w[d] * scale;
   const dim3 grid(8 * a.nb8), block(64 * NW);
-  if (dot_part) {
-    if constexpr (NV == 1) {
-      if (X)
-        hipLaunchKernelGGL((stencil_zmarch<T, R, SX, TYW, NV, NB, true, true, PD, NW>), grid, block, 0, st, a, Y, X,
-                           Out, V, T(ca), T(cb), T(cc), dot_part);
-      else
-        hipLaunchKernelGGL((stencil_zmarch<T, R, SX, TYW, NV, NB, false, true, PD, NW>), grid, block, 0, st, a, Y, X,
-                           Out, V, T(ca), T(cb), T(cc), dot_part);
-    } else {
-      pc::set_error("stencil: partial sums need one vector per workgroup");
-      return pc::PC_ERR_ARG;
-    }
-  } else if (X) {
-    hipLaunchKernelGGL((stencil_zmarch<T, R, SX, TYW, NV, NB, true, false, PD, NW>), grid, block, 0, st, a, Y, X, Out,
-                       V, T(ca), T(cb), T(cc), dot_part);
-  } else {
-    hipLaunchKernelGGL((stencil_zmarch<T, R, SX, TYW, NV, NB, false, false, PD, NW>), grid, block, 0, st, a, Y, X, Out,
-                       V, T(ca), T(cb), T(cc), dot_part);
-  }
+  if (X)
+    hipLaunchKernelGGL((stencil_zmarch<T, R, SX, 1, 1, 2, true, true, 1, NW>), grid, block, 0, st, a, Y, X, Out, V,
+                       T(ca), T(cb), T(cc), dot_part);
+  else
+    hipLaunchKernelGGL((stencil_zmarch<T, R, SX, 1, 1, 2, false, true, 1, NW>), grid, block, 0, st, a, Y, X, Out, V,
+                       T(ca), T(cb), T(cc), dot_part);
   PC_LAUNCH_CHECK();
   return pc::PC_OK;
-}
-
-#ifndef PC_STENCIL_NW
-#define PC_STENCIL_NW 8
-#endif
-#ifndef PC_STENCIL_NV
-#define PC_STENCIL_NV 1
-#endif
-
-// One y-row per wavefront (TYW = 1), PC_STENCIL_NW = 8 wavefronts (y-rows) and
-// PC_STENCIL_NV = 1 vector per workgroup where the LDS tiles fit in 56 KB, else
-// 4 wavefronts.  Measured on Si87H76 (one recurrence step, 275 vectors):
-//   4 rows: FP32 0.95 ms with 2 vectors, 0.96 ms with 1, 1.04 ms with 4;
-//           FP64 1.72 ms with 2, 1.79 ms with 1;
-//   8 rows: FP32 0.91 ms with 2 vectors (92 VGPRs, 5 waves per SIMD), 0.84 ms
-//           with 1 (60 VGPRs, 8 waves per SIMD); FP64 1.65 ms with 1;
-//   16 rows, 1 vector: FP32 0.84 ms, FP64 1.66 ms.
-// A prefetch depth of two planes (PD = 2) was slower (1.22 ms FP32, 4 vectors):
-// the registers it takes cost more occupancy than the extra plane gains.
-template <typename T, int R, int SX>
-int launch_r_sx(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, int nvec, long long ld, double scale,
-                double ca, double cb, double cc, double* dot_part, hipStream_t st) {
-  constexpr int kLds = 56 * 1024;
-  constexpr int NW = PC_STENCIL_NW;
-  if (dot_part)   // per-vector partial sums need one vector per workgroup
-    return launch_cfg<T, R, SX, 1, 1, 2, 1, 4>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
-#if PC_STENCIL_PAIR
-  // Measured on MI355X (one FP32 recurrence step, lean vs paired, identical
-  // results): Si87H76 sphere nx 106, 275 vectors, radius 4: 801 vs 881 us;
-  // radius 3: 716 vs 880 us; C10H8 sphere nx 92, 49 vectors: 133 vs 178 us;
-  // sphere nx 75, radius 1: 46 vs 72 us; 128^3 sphere, 256 vectors, radius 6:
-  // 1539 vs 1430 us.  The paired kernel needs 89 VGPRs at radius 4 (5 waves
-  // per SIMD against 8), which costs more than the wider accesses gain,
-  // except at radius 6, where the lean kernel's queue is long too.
-  if constexpr (SX == 2 && sizeof(T) == 4 && R >= 6)
-    if (gd->npts >= 2)
-      return launch_pair<R>(gd, reinterpret_cast<const float*>(Y), reinterpret_cast<const float*>(X),
-                          reinterpret_cast<float*>(Out), reinterpret_cast<const float*>(V), nvec, ld, scale, ca, cb,
-                          cc, st);
-#endif
-  if constexpr (SX <= 2 && R == 4) {
-    bool use_cc = g_stencil_cc == 1;
-    if (g_stencil_cc == 2 && sizeof(T) == 4 && nvec < 128) {
-      constexpr int CPW = SX > 2 ? SX / 2 : 1;
-      const long long lean_waves = (long long)((gd->ny + PC_LEAN_TY - 1) / PC_LEAN_TY) * nvec * (PC_LEAN_TY * SX / CPW);
-      use_cc = lean_waves >= PC_LEAN_ZCHUNK_WAVES;
-    }
-    if (use_cc && gd->cc_wmax > 0) return launch_cc<T, R>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, st);
-  }
-#ifndef PC_STENCIL_NO_LEAN
-  if constexpr (SX <= 2) return launch_lean<T, R, SX>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, st);
-#endif
-  if constexpr (PC_STENCIL_NV >= 2 && zmarch_lds_bytes<T, R, SX, 1, 2, 2, NW>() <= kLds)
-    return launch_cfg<T, R, SX, 1, 2, 2, 1, NW>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
-  else if constexpr (zmarch_lds_bytes<T, R, SX, 1, 1, 2, NW>() <= kLds)
-    return launch_cfg<T, R, SX, 1, 1, 2, 1, NW>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
-  else
-    return launch_cfg<T, R, SX, 1, 1, 2, 1, 4>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
 }
 
 template <typename T, int R>
 int launch_r(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, int nvec, long long ld, double scale,
              double ca, double cb, double cc, double* dot_part, hipStream_t st) {
-  if (gd->nx <= 64) return launch_r_sx<T, R, 1>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
-  if (gd->nx <= 128) return launch_r_sx<T, R, 2>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
-  return launch_r_sx<T, R, 4>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
+  if (!dot_part) return launch_win<T, R>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, st);
+  if (gd->nx <= 64) return launch_dot<T, R, 1>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
+  if (gd->nx <= 128) return launch_dot<T, R, 2>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
+  return launch_dot<T, R, 4>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
 }
 
 template <typename T>
@@ -1262,7 +702,7 @@ int launch_direct_r(const GridDev* gd, const T* Y, const T* X, T* Out, const T* 
   StArgs a;
   a.nx = gd->nx; a.ny = gd->ny; a.nz = gd->nz; a.npts = gd->npts;
   a.lo = gd->lo; a.hi = gd->hi; a.off = gd->off; a.zrange = gd->zrange; a.meta = gd->meta;
-  a.ld = ld; a.nslab = 0; a.nvec = nvec; a.nblocks = 0; a.nb8 = 0; a.nzc = 1; a.zc = gd->nz;
+  a.ld = ld; a.nslab = 0; a.nvec = nvec; a.nblocks = 0; a.nb8 = 0;
   for (int d = 0; d < 8; ++d) a.w[d] = 0.0;
   a.w[0] = 3.0 * gd->w[0] * scale;
   for (int d = 1; d <= R; ++d) a.w[d] = gd->w[d] * scale;
@@ -1459,45 +899,48 @@ int pc_grid_create(int nx, int ny, int nz, const int* row_lo, const int* row_hi,
   for (int r = 0; r < nrow; ++r) meta[r] = make_int2(off[r] - lo[r], lo[r] | (hi[r] << 16));
   GridDev* g = new GridDev();
   g->nx = nx; g->ny = ny; g->nz = nz; g->npts = cnt; g->radius = radius;
-  g->cc_tab = nullptr;
-  g->cc_wmax = 0;
-  // stencil_cc column lists: per slab of kCcTY rows, each own row's and halo
-  // row's x-range over the planes of the slab's march (an interval on a convex
-  // domain), as (tile row << 16 | x)
-  std::vector<int> cc;
-  int ccw = 0;
-  if (nx <= 128) {
-    const int TY = kCcTY, nslab = (ny + TY - 1) / TY, LR = TY + 2 * radius;
-    std::vector<std::vector<int>> own(nslab), hal(nslab);
-    for (int sl = 0; sl < nslab; ++sl) {
-      int zb = nz, ze = 0;
-      for (int t = 0; t < TY; ++t) {
-        const int j = sl * TY + t;
-        if (j < ny) { zb = std::min(zb, zr[2 * j]); ze = std::max(ze, zr[2 * j + 1]); }
-      }
-      for (int t = 0; t < LR; ++t) {
-        const int j = sl * TY - radius + t;
-        if (j < 0 || j >= ny || zb >= ze) continue;
-        int xl = nx, xh = 0;
-        for (int k = zb; k < ze; ++k) {
-          const int r = j + ny * k;
-          if (hi[r] > lo[r]) { xl = std::min(xl, lo[r]); xh = std::max(xh, hi[r]); }
+  // stencil_win: per slab of rows the columns they touch, as one window of up to
+  // 64 or as windows of equal lane counts (an inner edge has radius halo lanes,
+  // an outer one none), with the planes they touch
+  std::vector<int4> win;
+  const int ty = win_ty(radius);
+  for (int j0 = 0; j0 < ny; j0 += ty) {
+    int xl = nx, xh = 0;
+    const int j1 = std::min(ny, j0 + ty);
+    for (int j = j0; j < j1; ++j)
+      for (int k = zr[2 * j]; k < zr[2 * j + 1]; ++k)
+        if (hi[j + ny * k] > lo[j + ny * k]) {
+          xl = std::min(xl, lo[j + ny * k]);
+          xh = std::max(xh, hi[j + ny * k]);
         }
-        const bool is_own = t >= radius && t < radius + TY;
-        for (int x = xl; x < xh; ++x) (is_own ? own[sl] : hal[sl]).push_back((t << 16) | x);
-      }
-      ccw = std::max(ccw, (int)std::max((own[sl].size() + 63) / 64, (hal[sl].size() + 63) / 64));
-    }
-    if (ccw >= 1 && ccw <= 16) {
-      cc.assign((size_t)nslab * 2 * ccw * 64, -1);
-      for (int sl = 0; sl < nslab; ++sl) {
-        std::copy(own[sl].begin(), own[sl].end(), cc.begin() + (size_t)sl * 2 * ccw * 64);
-        std::copy(hal[sl].begin(), hal[sl].end(), cc.begin() + (size_t)sl * 2 * ccw * 64 + ccw * 64);
-      }
-    } else {
-      ccw = 0;
+    if (xl >= xh) continue;
+    int n = 1;
+    while (xh - xl + 2 * radius * (n - 1) > 64 * n) ++n;
+    const int lanes = xh - xl + 2 * radius * (n - 1);
+    auto cut = [&](int i) { return i == 0 ? xl : i == n ? xh : xl + lanes * i / n - radius * (2 * i - 1); };
+    for (int i = 0; i < n; ++i) {
+      const int x0 = cut(i), x1 = cut(i + 1);
+      int zb = nz, ze = 0;
+      for (int j = j0; j < j1; ++j)
+        for (int k = zr[2 * j]; k < zr[2 * j + 1]; ++k)
+          if (std::max(lo[j + ny * k], x0) < std::min(hi[j + ny * k], x1)) {
+            zb = std::min(zb, k);
+            ze = std::max(ze, k + 1);
+          }
+      if (zb < ze) win.push_back(make_int4(j0, x0 | ((x1 - x0) << 16) | ((i ? radius : 0) << 28), zb, ze));
     }
   }
+  g->win = nullptr;
+  g->nwin = (int)win.size();
+  g->pmeta = nullptr;
+  g->nyp = ny + 2 * kWinPadY;
+  g->nzp = nz + radius + kWinPadZ;
+  std::vector<int2> pmeta((size_t)g->nyp * g->nzp, make_int2(0, 0));
+  for (int k = 0; k < nz; ++k)
+    for (int j = 0; j < ny; ++j) {
+      const int r = j + ny * k;
+      pmeta[(size_t)(k + radius) * g->nyp + j + kWinPadY] = make_int2(off[r], lo[r] | ((hi[r] - lo[r]) << 16));
+    }
   for (int d = 0; d < 8; ++d) g->w[d] = d <= radius ? weights[d] : 0.0;
   hipError_t e = hipSuccess;
   e = hipMalloc(&g->lo, nrow * sizeof(int));
@@ -1515,11 +958,10 @@ int pc_grid_create(int nx, int ny, int nz, const int* row_lo, const int* row_hi,
   if (e == hipSuccess) e = hipMemcpy(g->hi, hi.data(), nrow * sizeof(int), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(g->off, off.data(), nrow * sizeof(int), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(g->zrange, zr.data(), 2 * ny * sizeof(int), hipMemcpyHostToDevice);
-  if (e == hipSuccess && ccw > 0) {
-    e = hipMalloc(&g->cc_tab, cc.size() * sizeof(int));
-    if (e == hipSuccess) e = hipMemcpy(g->cc_tab, cc.data(), cc.size() * sizeof(int), hipMemcpyHostToDevice);
-    if (e == hipSuccess) g->cc_wmax = ccw;
-  }
+  if (e == hipSuccess) e = hipMalloc(&g->win, std::max<size_t>(1, win.size()) * sizeof(int4));
+  if (e == hipSuccess) e = hipMemcpy(g->win, win.data(), win.size() * sizeof(int4), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMalloc(&g->pmeta, pmeta.size() * sizeof(int2));
+  if (e == hipSuccess) e = hipMemcpy(g->pmeta, pmeta.data(), pmeta.size() * sizeof(int2), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     pc::set_error(std::string("pc_grid_create: ") + hipGetErrorString(e));
     return pc::PC_ERR_HIP;
@@ -1534,17 +976,15 @@ int pc_grid_destroy(void* grid) {
   if (!g) return pc::PC_OK;
   (void)hipFree(g->lo); (void)hipFree(g->hi); (void)hipFree(g->off); (void)hipFree(g->zrange);
   (void)hipFree(g->meta); (void)hipFree(g->prow);
-  if (g->cc_tab) (void)hipFree(g->cc_tab);
+  (void)hipFree(g->win); (void)hipFree(g->pmeta);
   delete g;
   return pc::PC_OK;
 }
 
-// Stencil kernel for radius-4 grids of at most 128 points per row
-// (process-wide): 0 = stencil_lean, 1 = stencil_cc, 2 = stencil_cc where it
-// measured faster (the default; see g_stencil_cc).
+// Kept for its callers: one kernel serves every block now, so the value has no effect.
 int pc_stencil_set_variant(int variant) {
   PC_CHECK_ARG(variant >= 0 && variant <= 2, "variant must be 0, 1 or 2");
-  g_stencil_cc = variant;
+  (void)variant;
   return pc::PC_OK;
 }
 
