@@ -1,5 +1,7 @@
 // Shared helpers for the PARSEC hot-path HIP library (gfx950 / CDNA4).
 #pragma once
+#include <type_traits>
+#include <utility>
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <cstdio>
@@ -70,6 +72,12 @@ __device__ __forceinline__ double pc_wave_sum(double v) {
   PC_ROW_ROR(8) PC_ROW_ROR(4) PC_ROW_ROR(2) PC_ROW_ROR(1)
 #undef PC_ROW_ROR
   return v;
+}
+
+// f(integral_constant I) for I = 0, 1, ...
+template <int... I, class F>
+__device__ __forceinline__ void pc_unroll_seq(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
 }
 
 // Block-wide FP64 sum of one value per thread (blockDim.x multiple of 64,

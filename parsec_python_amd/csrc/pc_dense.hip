@@ -47,8 +47,8 @@ struct DenseCtx {
   double* P;        // method 2: padded copy of G, 64*ceil(kmax/64) x (kmax+1)
   double* resid;    // syevj: off-diagonal norm at exit
   int* sweeps;      // syevj: sweeps used
-  int* sync;             // sytrd_lower_mwg: flags and abort word
-  double* pub;           // sytrd_lower_mwg: published p and column, [4][320]
+  int* sync;             // sytrd_lower_mwg: abort word
+  unsigned long long* pub;  // sytrd_lower_mwg: published p and column of each step
   bool mwg_ok;           // false after a multi-workgroup reduction gave up waiting
   int mwg_aborts;        // reductions repeated with the one-workgroup kernel
   int trd_spin;          // polls of one wait before sytrd_lower_mwg gives up
@@ -424,11 +424,6 @@ constexpr int kTrdMax = 512;                    // largest n
 constexpr int kTrdThreads = 512;
 constexpr int kTrdWaves = kTrdThreads / 64;
 
-__device__ __forceinline__ double wave_allsum(double x) {
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-  return x;   // the same in every lane (butterfly)
-}
-
 template <int NCH>
 __global__ __launch_bounds__(kTrdThreads) void sytrd_lower_1wg(const double* __restrict__ G, int ldg, int n,
                                                                double* __restrict__ P, double* __restrict__ d,
@@ -470,7 +465,7 @@ __global__ __launch_bounds__(kTrdThreads) void sytrd_lower_1wg(const double* __r
       const int r = lane + 64 * q;
       sq += (r >= j + 2 && r < n) ? col[q] * col[q] : 0.0;
     }
-    const double xnorm2 = wave_allsum(sq);
+    const double xnorm2 = pc_wave_sum(sq);
     double beta = alpha, t = 0.0, scal = 0.0;
     if (xnorm2 > 0.0) {
       const double nrm = sqrt(alpha * alpha + xnorm2);
@@ -575,7 +570,7 @@ __global__ __launch_bounds__(kTrdThreads) void sytrd_lower_1wg(const double* __r
         col[q] = act ? colsh[rr] : 0.0;
         dp += wq[q] * vq[q];
       }
-      const double alpha2 = -0.5 * tau_cur * wave_allsum(dp);
+      const double alpha2 = -0.5 * tau_cur * pc_wave_sum(dp);
 #pragma unroll
       for (int q = 0; q < NCH; ++q) {
         const int rr = lane + 64 * q;
@@ -597,235 +592,233 @@ __global__ __launch_bounds__(kTrdThreads) void sytrd_lower_1wg(const double* __r
   if (n == 1 && tid == 0) d[0] = P[0];
 }
 
-// ---- multi-workgroup Householder tridiagonalization (same output as above)
+// ---- many-wavefront Householder tridiagonalization (same output as above)
 //
-// kTrdW workgroups of 256 threads; column c of the matrix lives in the LDS of
-// workgroup c % kTrdW for the whole reduction, so the trailing updates read and
-// write LDS instead of L2.  Step i:
-//   wave 0 of every workgroup (redundantly): w_{i-1} from the published
-//     p_{i-1}, then column i (published by its owner, updated through step
-//     i-2) brought up to date with (v_{i-1}, w_{i-1}) and reflector i built
-//     from it -- the same arithmetic in every workgroup, so no broadcast;
-//   all waves: each owned column c >= i+1 gets the pending rank-2 update of
-//     step i-1 and p_i(c) = column . v_i; p_i(c) and column i+1 are published;
-//   a barrier over the workgroups: each writes its step number to its own
-//     flag after a release fence, and polls the others' flags.
-// Published values, flags and the abort word are agent-scope atomics, so the
-// exchange does not depend on where the workgroups run.  A wait that exceeds
-// kTrdSpin polls (settable per context, for tests) sets the abort word and
-// every workgroup returns; the host then repeats the reduction with the
-// one-workgroup kernel.  All kTrdW workgroups must be resident at once: each
-// takes one CU's worth of LDS at most, far below the device's CU count, and the
-// kernel is the only work on its stream.  Measured at k = 275: 1.27 ms with
-// 32 workgroups, 1.36 ms with 16, 3.26 ms for the one-workgroup kernel.
-#ifndef PC_TRD_W
-#define PC_TRD_W 32
-#endif
-constexpr int kTrdW = PC_TRD_W;           // workgroups (at most 64: one poll lane each)
-constexpr int kTrdMwgMax = 320;           // largest n (LDS: ceil(320 / kTrdW) columns of 320 rows)
+// kTrdW workgroups of one wavefront; wavefront w holds the columns w, w + 64,
+// w + 128, ... in registers for the whole reduction (lane l: rows l + 64 q), so
+// element c of a distributed vector that column c = w + 64 m needs is lane w of
+// its register m.  Step i, by every wavefront on its own:
+//   w_{i-1} from the published p_{i-1}; column i (published by its owner,
+//     updated through step i-2) brought up to date with (v_{i-1}, w_{i-1}) and
+//     reflector i built from it -- the same arithmetic everywhere, no broadcast;
+//   each own column c >= i+1: the pending rank-2 update of step i-1, then
+//     p_i(c) = column . v_i; column i+1 and the p_i(c) are published.
+// The exchange is the data: every step has published words of its own, preset to
+// kTrdUnset (trd_preset), and a reader polls the words themselves, so a value
+// costs one store and one successful load, with no flags, fences or barriers.
+// Published words and the abort word are agent-scope atomics, so the exchange
+// does not depend on where the wavefronts run.  A wait that exceeds kTrdSpin
+// polls (settable per context, for tests) sets the abort word and every
+// wavefront returns; the host then repeats the reduction with the one-workgroup
+// kernel.  The wavefronts must be resident at once: 64 of one each, on 256 CUs,
+// and the kernel is the only work on its stream.  A wavefront leaves when its
+// last column is done; the last one (which never owns more columns than the
+// others) stays and writes the reflectors.
+// What bounds it: the serial chain of a step (a store seen by another XCD's
+// load, two wave sums, a root and a quotient, the dots), 2.1 us each.  At k =
+// 275 590 us; 1245 us with 32 workgroups of four wavefronts, columns in LDS, a
+// release fence, a flag per workgroup and an acquire fence (4.5 us per step),
+// the same bits; 3.26 ms with the one-workgroup kernel.
+constexpr int kTrdW = 64;
+constexpr int kTrdMwgMax = 320;           // largest n: 5 columns of 5 registers per lane
 constexpr int kTrdMwgMin = 128;           // smaller n use the one-workgroup kernel
 constexpr int kTrdSpin = 1 << 21;         // polls before a wait is declared failed
-constexpr int kTrdFlagStride = 32;        // ints between two workgroups' flags
-constexpr int kTrdSyncInts = kTrdFlagStride * (kTrdW + 1);   // flags, then the abort word
-constexpr int kTrdLoc = (kTrdMwgMax + kTrdW - 1) / kTrdW;
+constexpr unsigned long long kTrdUnset = 0xfffc5a7e3d91b26fULL;   // a NaN no arithmetic makes
+constexpr long long kTrdPub = 2LL * kTrdMwgMax * kTrdMwgMax;      // words: p_i and column i+1 of each step
 
-__device__ __forceinline__ void pub_store(double* p, double x) {
-  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), (unsigned long long)__double_as_longlong(x),
-                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void pub_store(unsigned long long* p, double x) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+  __hip_atomic_store(p, b == kTrdUnset ? b ^ 1 : b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ double pub_load(const double* p) {
-  return __longlong_as_double((long long)__hip_atomic_load(reinterpret_cast<const unsigned long long*>(p),
-                                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+__device__ __forceinline__ unsigned long long pub_load(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(256) void trd_preset(unsigned long long* pub, int words, int* abort_word) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t < words) pub[t] = kTrdUnset;
+  if (t == 0) *abort_word = 0;
 }
 
 template <int NCH>
-__global__ __launch_bounds__(256) void sytrd_lower_mwg(const double* __restrict__ G, int ldg, int n,
-                                                       double* __restrict__ P, double* __restrict__ d,
-                                                       double* __restrict__ e, double* __restrict__ tau,
-                                                       int* sync, double* pub, int* info_abort,
-                                                       int spin_limit) {
+__global__ __launch_bounds__(64) void sytrd_lower_mwg(const double* __restrict__ G, int ldg, int n,
+                                                      double* __restrict__ P, double* __restrict__ d,
+                                                      double* __restrict__ e, double* __restrict__ tau,
+                                                      int* abort_word, unsigned long long* pub, int* info_abort,
+                                                      int spin_limit) {
   constexpr int LDP = 64 * NCH;
-  __shared__ double loc[kTrdLoc * LDP];                 // owned columns, rows 0..LDP
-  __shared__ double vp[LDP + 1], wp[LDP + 1], vc[LDP + 1], colsh[LDP];
-  __shared__ double tau_sh;
-  __shared__ int abort_sh;
-  const int wg = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int nloc = (n - wg + kTrdW - 1) / kTrdW;        // columns wg, wg + W, ... < n
-  int* flags = sync;
-  int* abort_word = sync + kTrdFlagStride * kTrdW;
-  double* pbuf = pub;                                   // [2][LDP]: p_i
-  double* cbuf = pub + 2 * LDP;                         // [2][LDP]: column i+1
-  for (int t = tid; t < kTrdLoc * LDP; t += 256) {
-    const int lc = t / LDP, r = t - lc * LDP;
-    const int c = wg + kTrdW * lc;
-    loc[t] = (lc < nloc && r < n) ? G[(long long)c * ldg + r] : 0.0;
+  const int w = blockIdx.x, lane = threadIdx.x;
+  const bool writer = w == kTrdW - 1;
+  double a[NCH][NCH];          // a[m][q]: row lane + 64 q of column w + 64 m
+  double vq[NCH], x[NCH];      // v_{i-1} and column i
+#pragma unroll
+  for (int m = 0; m < NCH; ++m)
+#pragma unroll
+    for (int q = 0; q < NCH; ++q) {
+      const int c = w + 64 * m, r = lane + 64 * q;
+      a[m][q] = c < n && r < n ? G[(long long)c * ldg + r] : 0.0;
+    }
+#pragma unroll
+  for (int q = 0; q < NCH; ++q) {
+    vq[q] = 0.0;
+    x[q] = lane + 64 * q < n ? G[lane + 64 * q] : 0.0;
   }
-  for (int r = tid; r <= LDP; r += 256) {
-    vp[r] = 0.0;
-    wp[r] = 0.0;
-    vc[r] = 0.0;
-  }
-  if (tid == 0) abort_sh = 0;
-  __syncthreads();
-  for (int i = 0; i + 1 < n; ++i) {
-    // ---- wave 0: w_{i-1}, column i, reflector i
-    if (wv == 0) {
-      double x[NCH];
-      if (i > 0) {
-        const double* pb = pbuf + ((i - 1) & 1) * LDP;
-        const double* cb = cbuf + ((i - 1) & 1) * LDP;   // column i, published at step i-1
-        double pq[NCH], vq[NCH], dp = 0.0;
+  double t_prev = 0.0;
+
+  // the same rounding for column i and for the column that its owner keeps
+  auto rank2 = [](double v, double wc, double ww, double vc) { return __builtin_fma(v, wc, ww * vc); };
+  // p_{i-1} and column i, rows i .. n-1, in registers Q ..; false: gave up
+  auto receive = [&](auto Qc, int i, double (&pq)[NCH]) -> bool {
+    constexpr int Q = decltype(Qc)::value;
+    const unsigned long long* pb = pub + (long long)(i - 1) * 2 * LDP;
+    for (int spins = 0;;) {
+      unsigned long long bp[NCH], bc[NCH];
 #pragma unroll
-        for (int q = 0; q < NCH; ++q) {
-          const int r = lane + 64 * q;
-          pq[q] = (r >= i && r < n) ? pub_load(pb + r) : 0.0;
-          x[q] = r < n ? pub_load(cb + r) : 0.0;
-        }
-        const double t_prev = tau_sh;
-#pragma unroll
-        for (int q = 0; q < NCH; ++q) {
-          const int r = lane + 64 * q;
-          vq[q] = vc[r];
-          pq[q] *= t_prev;
-          dp += pq[q] * vq[q];
-        }
-        const double alpha2 = -0.5 * t_prev * wave_allsum(dp);
-#pragma unroll
-        for (int q = 0; q < NCH; ++q) {
-          const int r = lane + 64 * q;
-          const double wr = pq[q] + alpha2 * vq[q];
-          wp[r] = wr;
-          vp[r] = vq[q];
-        }
-        __builtin_amdgcn_wave_barrier();
-        const double wi = wp[i], vi = vp[i];
-#pragma unroll
-        for (int q = 0; q < NCH; ++q) {
-          const int r = lane + 64 * q;
-          x[q] -= vp[r] * wi + wp[r] * vi;
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < NCH; ++q) {
-          const int r = lane + 64 * q;
-          x[q] = r < n ? G[r] : 0.0;
-        }
+      for (int q = Q; q < NCH; ++q) {
+        bp[q] = pub_load(pb + lane + 64 * q);
+        bc[q] = pub_load(pb + LDP + lane + 64 * q);
       }
+      const int ab = __hip_atomic_load(abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      bool ok = true;
 #pragma unroll
-      for (int q = 0; q < NCH; ++q) colsh[lane + 64 * q] = x[q];
-      __builtin_amdgcn_wave_barrier();
-      const double dj = colsh[i], alpha = colsh[i + 1];
-      double sq = 0.0;
-#pragma unroll
-      for (int q = 0; q < NCH; ++q) {
+      for (int q = Q; q < NCH; ++q) {
         const int r = lane + 64 * q;
-        sq += (r >= i + 2 && r < n) ? x[q] * x[q] : 0.0;
+        const bool need = r >= i && r < n;
+        ok = ok && (!need || (bp[q] != kTrdUnset && bc[q] != kTrdUnset));
+        pq[q] = need ? __longlong_as_double((long long)bp[q]) : 0.0;
+        x[q] = need ? __longlong_as_double((long long)bc[q]) : 0.0;
       }
-      const double xnorm2 = wave_allsum(sq);
-      double beta = alpha, t = 0.0, scal = 0.0;
-      if (xnorm2 > 0.0) {
-        const double nrm = sqrt(alpha * alpha + xnorm2);
-        beta = alpha >= 0.0 ? -nrm : nrm;
-        t = (beta - alpha) / beta;
-        scal = 1.0 / (alpha - beta);
+      if (__builtin_amdgcn_readfirstlane(ab) != 0) return false;
+      if (__all(ok)) return true;
+      if (++spins >= spin_limit) {
+        if (lane == 0) __hip_atomic_store(abort_word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
       }
+    }
+  };
+  // w_{i-1} (in pq) and column i brought up to date
+  auto advance = [&](auto Qc, int l, double (&pq)[NCH]) {
+    constexpr int Q = decltype(Qc)::value;
+    double dp = 0.0;
+#pragma unroll
+    for (int q = Q; q < NCH; ++q) {
+      pq[q] *= t_prev;
+      dp += pq[q] * vq[q];
+    }
+    const double alpha2 = -0.5 * t_prev * pc_wave_sum(dp);
+#pragma unroll
+    for (int q = Q; q < NCH; ++q) pq[q] += alpha2 * vq[q];
+    const double wi = cb_readlane(pq[Q], l), vi = cb_readlane(vq[Q], l);
+#pragma unroll
+    for (int q = Q; q < NCH; ++q) x[q] -= rank2(vq[q], wi, pq[q], vi);
+  };
+  // step i = 64 Q + l; false: gave up
+  auto step = [&](auto Qc, int l) -> bool {
+    constexpr int Q = decltype(Qc)::value;
+    const int i = 64 * Q + l;
+    double wq[NCH];
+    if (i > 0) {
+      if (!receive(Qc, i, wq)) return false;
+      advance(Qc, l, wq);
+    } else {
+#pragma unroll
+      for (int q = 0; q < NCH; ++q) wq[q] = 0.0;
+    }
+    const double dj = cb_readlane(x[Q], l);
+    const double alpha = l < 63 ? cb_readlane(x[Q], l + 1) : cb_readlane(x[Q + 1 < NCH ? Q + 1 : Q], 0);
+    double sq = 0.0;
+#pragma unroll
+    for (int q = Q; q < NCH; ++q) {
+      const int r = lane + 64 * q;
+      sq += (r >= i + 2 && r < n) ? x[q] * x[q] : 0.0;
+    }
+    const double xnorm2 = pc_wave_sum(sq);
+    double beta = alpha, t = 0.0, scal = 0.0;
+    if (xnorm2 > 0.0) {
+      const double nrm = sqrt(alpha * alpha + xnorm2);
+      beta = alpha >= 0.0 ? -nrm : nrm;
+      t = (beta - alpha) / beta;
+      scal = 1.0 / (alpha - beta);
+    }
+    double vn[NCH];
+#pragma unroll
+    for (int q = Q; q < NCH; ++q) {
+      const int r = lane + 64 * q;
+      vn[q] = (r <= i || r >= n) ? 0.0 : (r == i + 1 ? 1.0 : x[q] * scal);
+    }
+    unsigned long long* pb = pub + (long long)i * 2 * LDP;
+    double acc[NCH];
+#pragma unroll
+    for (int m = Q; m < NCH; ++m) {
+      const int c = w + 64 * m;
+      acc[m] = 0.0;
+      if (c < i + 1 || c >= n) continue;
+      const double vpc = cb_readlane(vq[m], w), wpc = cb_readlane(wq[m], w);
+#pragma unroll
+      for (int q = Q; q < NCH; ++q) a[m][q] -= rank2(vq[q], wpc, wq[q], vpc);
+      if (c == i + 1) {
+#pragma unroll
+        for (int q = Q; q < NCH; ++q) pub_store(pb + LDP + lane + 64 * q, a[m][q]);
+      }
+#pragma unroll
+      for (int q = Q; q < NCH; ++q) acc[m] += a[m][q] * vn[q];
+    }
+    // lane m holds p_i(w + 64 m)
+    double pm = 0.0;
+#pragma unroll
+    for (int m = Q; m < NCH; ++m) {
+      const double s = pc_wave_sum(acc[m]);
+      pm = lane == m ? s : pm;
+    }
+    const int cm = w + 64 * lane;
+    if (lane < NCH && cm >= i + 1 && cm < n) pub_store(pb + cm, pm);
+    if (writer) {
       double* __restrict__ pj = P + (long long)i * LDP;
 #pragma unroll
-      for (int q = 0; q < NCH; ++q) {
+      for (int q = Q; q < NCH; ++q) {
         const int r = lane + 64 * q;
-        const double out = r == i ? dj : (r == i + 1 ? beta : x[q] * scal);
-        vc[r] = (r <= i || r >= n) ? 0.0 : (r == i + 1 ? 1.0 : out);
-        if (wg == 0 && r >= i && r < n) pj[r] = out;
+        if (r >= i && r < n) pj[r] = r == i ? dj : (r == i + 1 ? beta : vn[q]);
       }
-      if (wg == 0 && lane == 0) {
+      if (lane == 0) {
         d[i] = dj;
         e[i] = beta;
         tau[i] = t;
       }
-      if (lane == 0) tau_sh = t;
     }
-    __syncthreads();
-    // ---- all waves: pending update of step i-1 on the owned columns c >= i+1, p_i(c)
-    double* pb = pbuf + (i & 1) * LDP;
-    double* cb = cbuf + (i & 1) * LDP;
-    for (int lc = wv; lc < nloc; lc += 4) {
-      const int c = wg + kTrdW * lc;
-      if (c < i + 1) continue;
-      double* col = loc + lc * LDP;
-      const double vpc = vp[c], wpc = wp[c];
-      double acc = 0.0;
 #pragma unroll
-      for (int q = 0; q < NCH; ++q) {
-        const int r = lane + 64 * q;
-        const double y = col[r] - (vp[r] * wpc + wp[r] * vpc);
-        col[r] = y;
-        acc += y * vc[r];
-        if (c == i + 1) pub_store(cb + r, y);
-      }
-      acc = wave_allsum(acc);
-      if (lane == 0) pub_store(pb + c, acc);
-    }
-    // ---- barrier over the workgroups
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __syncthreads();
-    if (wv == 0) {
-      if (lane == 0) __hip_atomic_store(flags + kTrdFlagStride * wg, i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      int spins = 0;
-      bool ok = false;
-      while (true) {
-        const int f = lane < kTrdW ? __hip_atomic_load(flags + kTrdFlagStride * lane, __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_AGENT) : (i + 1);
-        const int ab = __builtin_amdgcn_readfirstlane(
-            __hip_atomic_load(abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        const bool all = __all(f >= i + 1);
-        if (ab != 0) break;
-        if (all) {
-          ok = true;
-          break;
+    for (int q = Q; q < NCH; ++q) vq[q] = vn[q];
+    t_prev = t;
+    return true;
+  };
+
+  const int last = w + 64 * ((n - 1 - w) / 64);   // this wavefront's last column (w < n)
+  bool done = w >= n, ok = true;
+  auto block = [&](auto Qc) {
+    constexpr int Q = decltype(Qc)::value;
+    for (int l = 0; l < 64 && !done; ++l) {
+      const int i = 64 * Q + l;
+      if (i == n - 1 || (!writer && i >= last)) {   // i = last: nothing of this wavefront's is left
+        done = true;
+        if (writer) {                               // the last diagonal entry: column n-1 through step n-2
+          double wq[NCH];
+          if (i > 0) {
+            ok = receive(Qc, i, wq);
+            if (ok) advance(Qc, l, wq);
+          }
+          const double dn = cb_readlane(x[Q], l);
+          if (ok && lane == 0) {
+            P[(long long)i * LDP + i] = dn;
+            d[i] = dn;
+          }
         }
-        if (++spins >= spin_limit) {
-          if (lane == 0) __hip_atomic_store(abort_word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      if (lane == 0) abort_sh = ok ? 0 : 1;
-    }
-    __syncthreads();
-    if (abort_sh) {
-      if (wg == 0 && tid == 0) *info_abort = 1;
-      return;
-    }
-  }
-  // last diagonal entry: column n-1 through step n-2 (wave 0 of workgroup 0)
-  if (wg == 0 && wv == 0) {
-    const int i = n - 1;
-    const double* pb = pbuf + ((i - 1) & 1) * LDP;
-    const double* cb = cbuf + ((i - 1) & 1) * LDP;
-    const double t_prev = tau_sh;
-    double pq[NCH], vq[NCH], dp = 0.0;
-#pragma unroll
-    for (int q = 0; q < NCH; ++q) {
-      const int r = lane + 64 * q;
-      pq[q] = (r >= i && r < n) ? t_prev * pub_load(pb + r) : 0.0;
-      vq[q] = vc[r];
-      dp += pq[q] * vq[q];
-    }
-    const double alpha2 = -0.5 * t_prev * wave_allsum(dp);
-    // only row n-1 is needed: x(n-1) - 2 v(n-1) w(n-1), with v(n-1) = 1
-    double dn = 0.0;
-#pragma unroll
-    for (int q = 0; q < NCH; ++q) {
-      const int r = lane + 64 * q;
-      if (r == i) {
-        const double wr = pq[q] + alpha2 * vq[q];
-        dn = pub_load(cb + r) - 2.0 * vq[q] * wr;
-        P[(long long)i * LDP + i] = dn;
-        d[i] = dn;
+      } else if (!step(Qc, l)) {
+        ok = false;
+        done = true;
       }
     }
-  }
+  };
+  pc_unroll_seq(std::make_integer_sequence<int, NCH>{}, block);
+  if (!ok && lane == 0) *info_abort = 1;
 }
 
 // ---- eigenpairs of the symmetric tridiagonal matrix (d, e) -----------------
@@ -1435,8 +1428,8 @@ int pc_dense_create(void* stream, int kmax, void** out_ctx) {
   if (kmax <= kTrdMax)
     PC_HIP(hipMalloc(&c->P, (size_t)(64 * ((kmax + 63) / 64)) * (kmax + 1) * sizeof(double)));
   PC_HIP(hipHostMalloc(&c->host_out, (size_t)(kmax + 4) * sizeof(double), hipHostMallocDefault));
-  PC_HIP(hipMalloc(&c->sync, kTrdSyncInts * sizeof(int)));
-  PC_HIP(hipMalloc(&c->pub, 4 * kTrdMwgMax * sizeof(double)));
+  PC_HIP(hipMalloc(&c->sync, sizeof(int)));
+  PC_HIP(hipMalloc(&c->pub, kTrdPub * sizeof(unsigned long long)));
   c->tri_mode = 2;
   c->blk_fallbacks = 0;
   c->orm_mode = 1;
@@ -1614,11 +1607,13 @@ int pc_dense_rr(void* ctx, int k, double* S, int lds, double* Gy, int ldg, doubl
       const int nch = (k + 63) / 64;
       mwg = (c->method == 2 || c->method == 4) && c->mwg_ok && k >= kTrdMwgMin && k <= kTrdMwgMax;
       if (mwg) {
-        PC_HIP(hipMemsetAsync(c->sync, 0, kTrdSyncInts * sizeof(int), c->stream));
+        const int words = 2 * (k - 1) * 64 * nch;   // each step's p and column
+        hipLaunchKernelGGL(trd_preset, dim3((words + 255) / 256), dim3(256), 0, c->stream, c->pub, words, c->sync);
+        PC_LAUNCH_CHECK();
         switch (nch) {
 #define PC_TRDM(N)                                                                                            \
   case N:                                                                                                     \
-    hipLaunchKernelGGL(sytrd_lower_mwg<N>, dim3(kTrdW), dim3(256), 0, c->stream, Gy, ldg, k, c->P, c->out,   \
+    hipLaunchKernelGGL(sytrd_lower_mwg<N>, dim3(kTrdW), dim3(64), 0, c->stream, Gy, ldg, k, c->P, c->out,   \
                        c->E, c->tau, c->sync, c->pub, c->info + 3, c->trd_spin);                              \
     break;
           PC_TRDM(2) PC_TRDM(3) PC_TRDM(4) PC_TRDM(5)

@@ -393,11 +393,6 @@ __device__ __forceinline__ void pc_bstore(__amdgpu_buffer_rsrc_t r, int off, T v
   }
 }
 
-template <int... I, class F>
-__device__ __forceinline__ void pc_unroll_seq(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-
 // rows (wavefronts) per workgroup: one halo row per wavefront from radius 4 on
 constexpr int win_ty(int R) { return R <= 4 ? 8 : 2 * R; }
 constexpr int kWinNS = 2;    // register sets of X, V and halo values in flight
