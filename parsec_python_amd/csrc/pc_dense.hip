@@ -402,6 +402,8 @@ __global__ __launch_bounds__(256) void chol_blk_inverse(const double* __restrict
 
 // ---- one-workgroup Householder tridiagonalization (LAPACK dsytrd layout, lower)
 //
+// Serves 128 < n <= 512 where the many-wavefront kernel below does not (n > 320,
+// another method chosen, or after it gave up waiting).
 // For i = 0..n-2 the reflector H(i) = I - tau_i v_i v_i^T (v_i(i+1) = 1,
 // v_i(i+2:) stored in P(i+2:, i)) annihilates P(i+2:, i) of the trailing
 // matrix; d = diagonal, e = subdiagonal of the tridiagonal Q^T G Q with
@@ -590,6 +592,143 @@ __global__ __launch_bounds__(kTrdThreads) void sytrd_lower_1wg(const double* __r
     __syncthreads();
   }
   if (n == 1 && tid == 0) d[0] = P[0];
+}
+
+// ---- the same reduction with the matrix in registers (n <= 128)
+//
+// One workgroup of 8 wavefronts; wavefront o holds the columns o + 8 u in
+// registers (lane l: rows l + 64 q), so the pass over the trailing columns reads
+// nothing from memory and a column's scalars v(c), w(c) come by readlane from a
+// register known at compile time.  Every wavefront does the serial part (w_i,
+// column i+1, reflector i+1) for itself from the partial sums of p and the column
+// in LDS, in two sets used in turn: one barrier per step.  The partial sums take
+// the order of sytrd_lower_1wg (columns i+1+t, i+1+t+8, ... one after the other,
+// then t = 0..7), and the products its FMA form: the same bits.
+// Bound by the serial chain of a step (8 partial sums, two wave sums, a root and
+// a quotient), 1.4 us each: 66 us at n = 49 (173 us through L2), the dense step at
+// n = 23, 80 and 127 232 -> 180, 772 -> 448 and 1073 -> 651 us.
+constexpr int kTrdRegMax = 128;
+
+template <int NCH>
+__global__ __launch_bounds__(512) void sytrd_lower_reg(const double* __restrict__ G, int ldg, int n,
+                                                       double* __restrict__ P, double* __restrict__ d,
+                                                       double* __restrict__ e, double* __restrict__ tau) {
+  constexpr int LDP = 64 * NCH, NU = 8 * NCH;
+  __shared__ double red[2][8][LDP], colsh[2][LDP];
+  const int lane = threadIdx.x & 63;
+  const int o = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double a[NU][NCH], col[NCH], v[NCH], w[NCH], vn[NCH];
+#pragma unroll
+  for (int u = 0; u < NU; ++u)
+#pragma unroll
+    for (int q = 0; q < NCH; ++q) {
+      const int c = o + 8 * u, r = lane + 64 * q;
+      a[u][q] = c < n && r < n ? G[(long long)c * ldg + r] : 0.0;
+    }
+#pragma unroll
+  for (int q = 0; q < NCH; ++q) {
+    col[q] = lane + 64 * q < n ? G[lane + 64 * q] : 0.0;
+    v[q] = w[q] = vn[q] = 0.0;
+  }
+  double t_cur = 0.0;
+  bool done = false;
+  auto step = [&](auto Qc, int l) {
+    constexpr int Q = decltype(Qc)::value;
+    const int j = 64 * Q + l;
+    if (j > 0) {   // w_{j-1}, column j
+      const int s = (j - 1) & 1;
+      double dp = 0.0;
+#pragma unroll
+      for (int q = Q; q < NCH; ++q) {
+        const int r = lane + 64 * q;
+        const bool act = r >= j && r < n;
+        double p = 0.0;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) p += red[s][t][r];
+        const double c = colsh[s][r];
+        v[q] = act ? vn[q] : 0.0;
+        w[q] = act ? t_cur * p : 0.0;
+        col[q] = act ? c : 0.0;
+        dp = __builtin_fma(w[q], v[q], dp);
+      }
+      const double alpha2 = -0.5 * t_cur * pc_wave_sum(dp);
+#pragma unroll
+      for (int q = Q; q < NCH; ++q) w[q] = __builtin_fma(alpha2, v[q], w[q]);
+      const double w1 = cb_readlane(w[Q], l);
+#pragma unroll
+      for (int q = Q; q < NCH; ++q) col[q] -= __builtin_fma(v[q], w1, w[q]);
+    }
+    const double dj = cb_readlane(col[Q], l);
+    if (j == n - 1) {
+      if (o == 7 && lane == 0) {
+        P[(long long)j * LDP + j] = dj;
+        d[j] = dj;
+      }
+      done = true;
+      return;
+    }
+    const double alpha = l < 63 ? cb_readlane(col[Q], l + 1) : cb_readlane(col[Q + 1 < NCH ? Q + 1 : Q], 0);
+    double sq = 0.0;
+#pragma unroll
+    for (int q = Q; q < NCH; ++q) {
+      const int r = lane + 64 * q;
+      sq += (r >= j + 2 && r < n) ? col[q] * col[q] : 0.0;
+    }
+    const double xnorm2 = pc_wave_sum(sq);
+    double beta = alpha, t = 0.0, scal = 0.0;
+    if (xnorm2 > 0.0) {
+      const double nrm = sqrt(__builtin_fma(alpha, alpha, xnorm2));
+      beta = alpha >= 0.0 ? -nrm : nrm;
+      t = (beta - alpha) / beta;
+      scal = 1.0 / (alpha - beta);
+    }
+#pragma unroll
+    for (int q = Q; q < NCH; ++q) {
+      const int r = lane + 64 * q;
+      vn[q] = (r <= j || r >= n) ? 0.0 : (r == j + 1 ? 1.0 : col[q] * scal);
+    }
+    if (o == 7) {
+      double* __restrict__ pj = P + (long long)j * LDP;
+#pragma unroll
+      for (int q = Q; q < NCH; ++q) {
+        const int r = lane + 64 * q;
+        if (r >= j && r < n) pj[r] = r == j ? dj : (r == j + 1 ? beta : vn[q]);
+      }
+      if (lane == 0) {
+        d[j] = dj;
+        e[j] = beta;
+        tau[j] = t;
+      }
+    }
+    t_cur = t;
+    // the pending update on the own columns c >= j+1, and their part of p_j
+    double pacc[NCH];
+#pragma unroll
+    for (int q = Q; q < NCH; ++q) pacc[q] = 0.0;
+#pragma unroll
+    for (int u = 8 * Q; u < NU; ++u) {
+      const int c = o + 8 * u;
+      if (c < j + 1 || c >= n) continue;
+      const int cl = o + 8 * (u & 7);
+      const double pv = cb_readlane(v[u >> 3], cl), pw = cb_readlane(w[u >> 3], cl), vc = cb_readlane(vn[u >> 3], cl);
+#pragma unroll
+      for (int q = Q; q < NCH; ++q) {
+        const double y = a[u][q] - __builtin_fma(w[q], pv, v[q] * pw);
+        a[u][q] = y;
+        pacc[q] = __builtin_fma(y, vc, pacc[q]);
+        if (c == j + 1) colsh[j & 1][lane + 64 * q] = y;
+      }
+    }
+#pragma unroll
+    for (int q = Q; q < NCH; ++q) red[j & 1][(o - j - 1) & 7][lane + 64 * q] = pacc[q];
+    // an LDS-only barrier: the stores of P stay in flight
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+  pc_unroll_seq(std::make_integer_sequence<int, NCH>{}, [&](auto Qc) {
+    for (int l = 0; l < 64 && !done; ++l) step(Qc, l);
+  });
 }
 
 // ---- many-wavefront Householder tridiagonalization (same output as above)
@@ -1620,6 +1759,11 @@ int pc_dense_rr(void* ctx, int k, double* S, int lds, double* Gy, int ldg, doubl
 #undef PC_TRDM
           default: break;
         }
+      } else if (k <= kTrdRegMax) {
+        if (nch == 1)
+          hipLaunchKernelGGL(sytrd_lower_reg<1>, dim3(1), dim3(512), 0, c->stream, Gy, ldg, k, c->P, c->out, c->E, c->tau);
+        else
+          hipLaunchKernelGGL(sytrd_lower_reg<2>, dim3(1), dim3(512), 0, c->stream, Gy, ldg, k, c->P, c->out, c->E, c->tau);
       } else {
         switch (nch) {
 #define PC_TRD(N)                                                                                                  \
@@ -1627,7 +1771,7 @@ int pc_dense_rr(void* ctx, int k, double* S, int lds, double* Gy, int ldg, doubl
     hipLaunchKernelGGL(sytrd_lower_1wg<N>, dim3(1), dim3(kTrdThreads), 0, c->stream, Gy, ldg, k, c->P, c->out,  \
                        c->E, c->tau);                                                                              \
     break;
-          PC_TRD(1) PC_TRD(2) PC_TRD(3) PC_TRD(4) PC_TRD(5) PC_TRD(6) PC_TRD(7) PC_TRD(8)
+          PC_TRD(3) PC_TRD(4) PC_TRD(5) PC_TRD(6) PC_TRD(7) PC_TRD(8)
 #undef PC_TRD
         }
       }
