@@ -197,45 +197,100 @@ __device__ __forceinline__ double cb_readlane(double v, int l) {
   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
 }
 
-// Cholesky factor and inverse of the symmetric 32 x 32 block in W (LDS), by
-// wavefront 0: lane t holds column t % 32 in registers and reads row c of R
-// from the lanes that hold it.  On success W holds R (upper, zero below) and
-// Di = R^-1 (upper, zero below).  Returns the 1-based column of the first
-// pivot that is not positive (or not finite), 0 on success.
-__device__ __forceinline__ int cb_chol32(double* W, double* Di) {
-  const int t = threadIdx.x & 31;
-  double w[kCb];
-#pragma unroll
-  for (int r = 0; r < kCb; ++r) w[r] = W[t * kCbLW + r];
-#pragma unroll
-  for (int c = 0; c < kCb; ++c) {
-    const double d = cb_readlane(w[c], c);
-    if (!(d > 0.0) || !(d < __builtin_inf())) return c + 1;
-    const double sq = __builtin_sqrt(d);
-    const double is = 1.0 / sq;
-    w[c] = t == c ? sq : w[c] * is;
-    // rows a > c of column t: W(a, t) -= R(c, a) R(c, t) (below the diagonal: unused)
-#pragma unroll
-    for (int a = c + 1; a < kCb; ++a) w[a] -= cb_readlane(w[c], a) * w[c];
-  }
-#pragma unroll
-  for (int r = 0; r < kCb; ++r) W[t * kCbLW + r] = r <= t ? w[r] : 0.0;
+__device__ __forceinline__ void cb_wave_sync() {   // this wavefront's LDS writes before its next reads
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  // column t of R^-1 by back substitution, R's columns read from LDS
-  double x[kCb];
+}
+
+// One 16 x 16 tile (tm, tn) of the block M in LDS, by one wavefront: rows r with
+// lo <= r < hi get M(r, t) -= sum_k a(r, k) b(k, t) over k = 0..7 in order (the
+// MFMA is the chain of FMAs in ascending k).
+template <class FA, class FB>
+__device__ __forceinline__ void cb_tile_update(double* M, int tm, int tn, int lo, int hi, FA&& fa, FB&& fb) {
+  const int lane = threadIdx.x & 63, lm = lane & 15, lk = lane >> 4;
+  const int ar = 16 * tm + lm, bt = 16 * tn + lm;
+  v4d acc;
 #pragma unroll
-  for (int r = 0; r < kCb; ++r) x[r] = r == t ? 1.0 : 0.0;
+  for (int r = 0; r < 4; ++r) acc[r] = M[bt * kCbLW + 16 * tm + 4 * r + lk];
 #pragma unroll
-  for (int c = kCb - 1; c >= 0; --c) {
-    x[c] = x[c] / W[c * kCbLW + c];
-#pragma unroll
-    for (int i = 0; i < c; ++i) x[i] -= W[c * kCbLW + i] * x[c];
+  for (int s = 0; s < 2; ++s) {
+    const double av = fa(ar, 4 * s + lk), bv = fb(4 * s + lk, bt);
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ar >= lo && ar < hi ? -av : 0.0, bv, acc, 0, 0, 0);
   }
 #pragma unroll
-  for (int r = 0; r < kCb; ++r) Di[t * kCbLW + r] = x[r];
-  return 0;
+  for (int r = 0; r < 4; ++r) M[bt * kCbLW + 16 * tm + 4 * r + lk] = acc[r];
+}
+
+// Cholesky factor and inverse of the symmetric 32 x 32 block in W (LDS), by one
+// wavefront.  W then holds R (upper, zero below) and Di = R^-1 (upper, zero
+// below).  Returns the 1-based column of the first pivot that is not positive (or
+// not finite; what W and Di hold is then meaningless), 0 on success.  Four rounds
+// of 8 rows, lane t holding column t % 32 of them in registers; the other rows
+// take a round's 8 terms by MFMA, in the order of the columns.  What is left is
+// the chain of a root (102 cycles), a quotient (78) and two dependent FMAs per
+// column.  One block of 32 alone: 13.5 us (27 us with every term on the vector
+// unit, 40 KB of unrolled code).
+__device__ __forceinline__ int cb_chol32(double* W, double* Di) {
+  constexpr int NC = 8;
+  const int t = threadIdx.x & 31;
+  int bad = 0;
+#pragma unroll 1
+  for (int c0 = 0; c0 < kCb; c0 += NC) {
+    double w[NC];
+#pragma unroll
+    for (int r = 0; r < NC; ++r) w[r] = W[t * kCbLW + c0 + r];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const double d = cb_readlane(w[c], c0 + c);
+      bad = bad == 0 && !(d > 0.0 && d < __builtin_inf()) ? c0 + c + 1 : bad;
+      const double sq = __builtin_sqrt(d);
+      const double is = 1.0 / sq;
+      w[c] = t == c0 + c ? sq : w[c] * is;
+      // rows a > c of column t: W(a, t) -= R(c, a) R(c, t) (below the diagonal: unused)
+#pragma unroll
+      for (int a = c + 1; a < NC; ++a) w[a] -= cb_readlane(w[c], c0 + a) * w[c];
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) W[t * kCbLW + c0 + c] = c0 + c <= t ? w[c] : 0.0;
+    cb_wave_sync();
+    auto ra = [&](int a, int k) { return W[a * kCbLW + c0 + k]; };   // R(c0 + k, a)
+    auto rt = [&](int k, int u) { return W[u * kCbLW + c0 + k]; };
+    if (c0 == 0) {
+      cb_tile_update(W, 0, 0, NC, kCb, ra, rt);
+      cb_tile_update(W, 0, 1, NC, kCb, ra, rt);
+    }
+    if (c0 + NC < kCb) cb_tile_update(W, 1, 1, c0 + NC, kCb, ra, rt);
+    cb_wave_sync();
+  }
+  // column t of R^-1 by back substitution, rows from the last to the first
+#pragma unroll
+  for (int r = 0; r < kCb; ++r) Di[t * kCbLW + r] = r == t ? 1.0 : 0.0;
+  cb_wave_sync();
+#pragma unroll 1
+  for (int c0 = kCb - NC; c0 >= 0; c0 -= NC) {
+    double x[NC];
+#pragma unroll
+    for (int r = 0; r < NC; ++r) x[r] = Di[t * kCbLW + c0 + r];
+#pragma unroll
+    for (int c = NC - 1; c >= 0; --c) {
+      const double* col = W + (c0 + c) * kCbLW + c0;
+      x[c] = x[c] / col[c];
+#pragma unroll
+      for (int i = 0; i < c; ++i) x[i] -= col[i] * x[c];
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) Di[t * kCbLW + c0 + c] = x[c];
+    cb_wave_sync();
+    // rows above, columns of R^-1 that are not zero yet
+    auto wc = [&](int i, int k) { return W[(c0 + NC - 1 - k) * kCbLW + i]; };   // R(i, c0 + 7 - k)
+    auto xc = [&](int k, int u) { return Di[u * kCbLW + c0 + NC - 1 - k]; };
+    if (c0 > 0) cb_tile_update(Di, 0, 1, 0, c0, wc, xc);
+    if (c0 > 16) cb_tile_update(Di, 1, 1, 0, c0, wc, xc);
+    else if (c0 == NC) cb_tile_update(Di, 0, 0, 0, c0, wc, xc);
+    cb_wave_sync();
+  }
+  return bad;
 }
 
 // acc += op(A) B over K = 32 for a whole 32 x 32 block by one wavefront: four
@@ -274,91 +329,119 @@ __global__ void chol_blk_init(const double* __restrict__ S, int lds, int k, doub
   R[(long long)c * KP + r] = (r < k && c < k) ? S[(long long)c * lds + r] : (r == c ? 1.0 : 0.0);
 }
 
-// One workgroup of 256 threads, right-looking by block columns: R (ld 32 nb)
-// holds the upper blocks of S padded with the identity (chol_blk_init); for each block
-// column j the diagonal block is factored and inverted by wavefront 0
-// (cb_chol32), then the wavefronts share out the panel blocks
-// R_jc = R_jj^-T A_jc (c > j) and afterwards the trailing blocks
-// A_ab -= R_ja^T R_jb (j < a <= b), one whole 32 x 32 block per wavefront at a
-// time: three dependent phases per block column.  Dinv (nb blocks,
-// column-major 32 x 32): the inverses of R's diagonal blocks; info[0]: as
-// potrf's (0, or the 1-based column of the first pivot that is not positive).
-__global__ __launch_bounds__(256) void chol_blk_factor(const double* __restrict__ S, int lds, int k, double* R,
-                                                       double* Dinv, int* info) {
-  __shared__ double W[kCb * kCbLW], Di[kCb * kCbLW];
-  __shared__ int fail;
+// One workgroup of 8 wavefronts, right-looking by block columns: R (ld 32 nb)
+// holds the upper blocks of S padded with the identity (chol_blk_init).  Block
+// column j: the wavefronts share out the panel blocks R_jc = R_jj^-T A_jc (c > j),
+// kept in LDS for the trailing blocks A_ab -= R_ja^T R_jb (j < a <= b), one whole
+// 32 x 32 block per wavefront at a time.  Wavefront 0 takes A_{j+1,j+1} first and
+// factors and inverts it (cb_chol32) while the others do the rest, which it then
+// joins.  Dinv (nb blocks, column-major 32 x 32): the inverses of R's diagonal
+// blocks; info[0]: as potrf's (0, or the 1-based column of the first pivot that
+// is not positive).  LDS: W, Di and nb - 1 panel blocks.
+// Bound by the chain of nb diagonal blocks (32 roots and 64 quotients, each
+// waiting for the one before).  k = 23, 49, 127, 275: 13.5, 27, 58, 181 us; on 4
+// wavefronts with the panel read back through L2, all of them waiting for the
+// diagonal block, 22, 51, 150 and 404 us.  The same bits.
+constexpr int kCholWaves = 8;
+constexpr int chol_lds(int nb) { return (nb + 1) * kCb * kCbLW * (int)sizeof(double); }
+
+__global__ __launch_bounds__(64 * kCholWaves) void chol_blk_factor(int k, double* R, double* Dinv, int* info) {
+  extern __shared__ double chol_sh[];
+  double* W = chol_sh;
+  double* Di = W + kCb * kCbLW;
+  double* panel = Di + kCb * kCbLW;   // block c - j - 1: R_jc
+  __shared__ int fail, next;
   const int nb = (k + kCb - 1) / kCb, KP = kCb * nb;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // (the factor's loops branch on it)
   const int lm = lane & 15, lk = lane >> 4;
+  const int kThreads = 64 * kCholWaves;
+  for (int e = threadIdx.x; e < kCb * kCb; e += kThreads) {
+    const int a = e & (kCb - 1), b = e / kCb;
+    W[b * kCbLW + a] = R[(long long)b * KP + a];
+  }
   if (threadIdx.x == 0) {
     fail = 0;
     info[0] = 0;
   }
   __syncthreads();
-  for (int j = 0; j < nb; ++j) {
-    double* rjj = R + cb_blk(j, j, KP);
-    for (int e = threadIdx.x; e < kCb * kCb; e += 256) {
-      const int a = e & (kCb - 1), b = e / kCb;
-      W[b * kCbLW + a] = rjj[(long long)b * KP + a];
-    }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-      const int f = cb_chol32(W, Di);
-      if (threadIdx.x == 0 && f != 0) {
-        fail = 1;
-        info[0] = kCb * j + f;
-      }
-    }
-    __syncthreads();
-    if (fail) return;
-    {
+  for (int j = -1; j < nb && fail == 0; ++j) {
+    if (j >= 0) {
+      double* rjj = R + cb_blk(j, j, KP);
       double* dj = Dinv + (long long)j * kCb * kCb;
-      for (int e = threadIdx.x; e < kCb * kCb; e += 256) {
+      for (int e = threadIdx.x; e < kCb * kCb; e += kThreads) {
         const int a = e & (kCb - 1), b = e / kCb;
         rjj[(long long)b * KP + a] = W[b * kCbLW + a];
         dj[e] = Di[b * kCbLW + a];
       }
+      // panel: R_jc = Dinv_j^T A_jc, one block per wavefront at a time
+      for (int c = j + 1 + wv; c < nb; c += kCholWaves) {
+        v4d acc[2][2] = {{{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}}, {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}}};
+        double* rjc = R + cb_blk(j, c, KP);
+        double* pc = panel + (c - j - 1) * kCb * kCbLW;
+        cb_mma_block<true>(acc, Di, kCbLW, rjc, KP, 1.0);
+        // every lane's loads of A_jc are done before any lane overwrites it
+        __builtin_amdgcn_s_waitcnt(0);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int tm = 0; tm < 2; ++tm)
+#pragma unroll
+          for (int tn = 0; tn < 2; ++tn)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int row = 16 * tm + 4 * r + lk, col = 16 * tn + lm;
+              rjc[(long long)col * KP + row] = acc[tm][tn][r];
+              pc[col * kCbLW + row] = acc[tm][tn][r];
+            }
+      }
     }
-    // panel: R_jc = Dinv_j^T A_jc, one block per wavefront at a time (Dinv_j from LDS)
-    for (int c = j + 1 + wv; c < nb; c += 4) {
-      v4d acc[2][2] = {{{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}}, {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}}};
-      double* rjc = R + cb_blk(j, c, KP);
-      cb_mma_block<true>(acc, Di, kCbLW, rjc, KP, 1.0);
-      // every lane's loads of A_jc are done before any lane overwrites it
-      __builtin_amdgcn_s_waitcnt(0);
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int tm = 0; tm < 2; ++tm)
-#pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            rjc[(long long)(16 * tn + lm) * KP + 16 * tm + 4 * r + lk] = acc[tm][tn][r];
-    }
+    if (threadIdx.x == 0) next = 1;
     __syncthreads();
-    // trailing blocks: A_ab -= R_ja^T R_jb for j < a <= b, one block per wavefront at a time
-    const int nt = nb - 1 - j;
-    for (int q = wv; q < nt * (nt + 1) / 2; q += 4) {
-      // q -> (a, b), a <= b, row by row of the upper triangle of the trailing blocks
-      int a = 0, rem = q;
-      while (rem >= nt - a) { rem -= nt - a; ++a; }
-      const int b = a + rem;
-      const int ga = j + 1 + a, gb = j + 1 + b;
-      double* aab = R + cb_blk(ga, gb, KP);
-      v4d acc[2][2];
+    // trailing blocks: A_ab -= R_ja^T R_jb for j < a <= b; q counts the upper
+    // triangle of the trailing blocks row by row, q = 0 is wavefront 0's (at the
+    // start, where nothing trails, the first diagonal block as it is)
+    const int nt = nb - 1 - j, nq = j < 0 ? 1 : nt * (nt + 1) / 2;
+    int q = 0;
+    auto take = [&]() {
+      int t = 0;
+      if (lane == 0) t = atomicAdd(&next, 1);
+      q = __builtin_amdgcn_readfirstlane(t);
+    };
+    if (wv != 0) take();
+    while (q < nq) {
+      if (j >= 0) {
+        int a = 0, rem = q;
+        while (rem >= nt - a) { rem -= nt - a; ++a; }
+        const int b = a + rem;
+        double* aab = R + cb_blk(j + 1 + a, j + 1 + b, KP);
+        v4d acc[2][2];
 #pragma unroll
-      for (int tm = 0; tm < 2; ++tm)
+        for (int tm = 0; tm < 2; ++tm)
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
+          for (int tn = 0; tn < 2; ++tn)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[tm][tn][r] = aab[(long long)(16 * tn + lm) * KP + 16 * tm + 4 * r + lk];
-      cb_mma_block<true>(acc, R + cb_blk(j, ga, KP), KP, R + cb_blk(j, gb, KP), KP, -1.0);
+            for (int r = 0; r < 4; ++r) acc[tm][tn][r] = aab[(long long)(16 * tn + lm) * KP + 16 * tm + 4 * r + lk];
+        cb_mma_block<true>(acc, panel + a * kCb * kCbLW, kCbLW, panel + b * kCb * kCbLW, kCbLW, -1.0);
 #pragma unroll
-      for (int tm = 0; tm < 2; ++tm)
+        for (int tm = 0; tm < 2; ++tm)
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
+          for (int tn = 0; tn < 2; ++tn)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) aab[(long long)(16 * tn + lm) * KP + 16 * tm + 4 * r + lk] = acc[tm][tn][r];
+            for (int r = 0; r < 4; ++r) {
+              const int row = 16 * tm + 4 * r + lk, col = 16 * tn + lm;
+              if (q == 0) W[col * kCbLW + row] = acc[tm][tn][r];
+              else aab[(long long)col * KP + row] = acc[tm][tn][r];
+            }
+      }
+      if (q == 0) {
+        cb_wave_sync();
+        const int f = cb_chol32(W, Di);
+        if (lane == 0 && f != 0) {
+          fail = 1;
+          info[0] = kCb * (j + 1) + f;
+        }
+      }
+      take();
     }
     __syncthreads();
   }
@@ -1584,6 +1667,8 @@ int pc_dense_create(void* stream, int kmax, void** out_ctx) {
   c->chol_lds = 0;
   {
     const int kb = std::min(kmax, kCholMaxK), nbb = (kb + kCb - 1) / kCb, kp = kCb * nbb;
+    PC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&chol_blk_factor),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, chol_lds(kCbMaxNb)));
     PC_HIP(hipMalloc(&c->cR, (size_t)kp * kp * sizeof(double)));
     PC_HIP(hipMalloc(&c->cRi, (size_t)kp * kp * sizeof(double)));
     PC_HIP(hipMalloc(&c->cD, (size_t)nbb * kCb * kCb * sizeof(double)));
@@ -1706,7 +1791,8 @@ int pc_dense_rr(void* ctx, int k, double* S, int lds, double* Gy, int ldg, doubl
       hipLaunchKernelGGL(chol_blk_init, dim3((kCb * nbk * kCb * nbk + 255) / 256), dim3(256), 0, c->stream, S, lds,
                          k, c->cR);
       PC_LAUNCH_CHECK();
-      hipLaunchKernelGGL(chol_blk_factor, dim3(1), dim3(256), 0, c->stream, S, lds, k, c->cR, c->cD, c->info);
+      hipLaunchKernelGGL(chol_blk_factor, dim3(1), dim3(64 * kCholWaves), chol_lds(nbk), c->stream, k, c->cR, c->cD,
+                         c->info);
       PC_LAUNCH_CHECK();
       hipLaunchKernelGGL(chol_blk_inverse, dim3(nbk), dim3(256), 0, c->stream, c->cR, c->cD, k, c->cRi);
       PC_LAUNCH_CHECK();
@@ -1906,7 +1992,8 @@ static int side_end(DenseCtx* c, int k, const double* S, int lds) {
     hipLaunchKernelGGL(chol_blk_init, dim3((kCb * nbk * kCb * nbk + 255) / 256), dim3(256), 0, c->side, S, lds, k,
                        c->cR);
     PC_LAUNCH_CHECK();
-    hipLaunchKernelGGL(chol_blk_factor, dim3(1), dim3(256), 0, c->side, S, lds, k, c->cR, c->cD, c->cinfo);
+    hipLaunchKernelGGL(chol_blk_factor, dim3(1), dim3(64 * kCholWaves), chol_lds(nbk), c->side, k, c->cR, c->cD,
+                       c->cinfo);
     PC_LAUNCH_CHECK();
     hipLaunchKernelGGL(chol_blk_inverse, dim3(nbk), dim3(256), 0, c->side, c->cR, c->cD, k, c->cRi);
     PC_LAUNCH_CHECK();
