@@ -349,47 +349,52 @@ __global__ __launch_bounds__(64 * NW) void stencil_zmarch(StArgs g, const T* __r
 //   * the z-queue is a ring of QL registers per lane, indexed by the plane's
 //     phase; the plane loop is unrolled QL times so the ring turns by renaming
 //     instead of register moves (slot (z - zb + R) mod QL holds plane z);
-//   * every global access is a raw buffer access on the row's own chord (base and
-//     size from scalar registers): a lane outside the chord, before or after it,
-//     has an out-of-range offset, so its load returns 0 and its store is dropped;
-//     one vector subtraction per access, no masks and no branches;
-//   * a row's {offset, extent} of 64 planes sits in a lane each and is read with
-//     v_readlane; the table is padded with empty rows, so nothing is clamped;
+//   * every global access is a raw buffer access on the row's own chord (its begin
+//     as the scalar offset, its end as num_records: a lane is in range if its
+//     offset is less than their difference): a lane outside the chord, before or
+//     after it, has an out-of-range offset, so its load returns 0 and its store is
+//     dropped; one vector subtraction per access, no masks and no branches;
+//   * a row's begin, end and first column of 64 planes, in bytes, sit in a lane
+//     each and are read with v_readlane; the table is padded with empty rows, so
+//     nothing is clamped;
 //   * X, V and the halo rows of plane z+1 go out before plane z is computed, the
 //     queue front of plane z-R+QL right after plane z's last use of slot z-R.
-// What bounds it: per row and plane 37 vector, 38 scalar and 11 LDS instructions
-// at radius 4 against 5 loads and stores, with one barrier; on large blocks the
-// three passes over memory take 60 % of the time.  Occupancy is the registers':
-// two vectors per workgroup, three register sets or forced occupancy (spills)
+// What bounds it: per row and plane 40 vector, 15 scalar and 11 LDS instructions
+// at radius 4 against 5 loads and stores, with one barrier; no unit is busy more
+// than half of the time, on large blocks the three passes over memory take 60 %
+// (the reads miss L2 once: 1.44 GB for 1.33 GB of Y and X).  Occupancy is the
+// registers': two vectors per workgroup, three register sets or forced occupancy
 // were slower, and so were 4, 6 and 16 rows at radius 4 (the halo is 2R rows per
 // slab, the barrier is over all its wavefronts) and non-temporal X or stores.
+// Row ranges by readlane and buffer ranges instead of scalar arithmetic on a base
+// per row (38 scalar instructions): FP32 98 -> 85 us on C10H8.
 // One recurrence step; before: one slab and two 64-column chunks of a row in one
 // workgroup, masks and tables in vector registers, the windows full or half empty:
 //   605,808 points, radius 4 (Si87H76 sphere), 275 vectors:
-//                                   FP32 721 -> 700 us, FP64 1508 -> 1260 us
-//   C10H8 sphere, radius 4:         FP32 111 -> 98 us,  FP64 260 -> 186 us
-//   52^3 cube, radius 4, 23:        FP32 17.2 -> 16.8,  FP64 30.2 -> 24.8 us
-//   radius 6 (FD12), 103 columns:   256 vectors FP32 1310 -> 1212 us,
-//                                   64 vectors FP64 640 -> 587 us
-//   70^3 cube, 40 vectors:          radius 3 FP32 48.9 -> 47.6, radius 2 FP64 87.5 -> 81.5 us
+//                                   FP32 721 -> 680 us, FP64 1508 -> 1250 us
+//   C10H8 sphere, radius 4, 49:     FP32 111 -> 80 us,  FP64 260 -> 175 us
+//   52^3 cube, radius 4, 23:        FP32 17.2 -> 14.9,  FP64 30.2 -> 24.4 us
+//   radius 6 (FD12), 103 columns:   256 vectors FP32 1310 -> 1165 us,
+//                                   64 vectors FP64 640 -> 551 us
+//   70^3 cube, 40 vectors:          radius 3 FP32 48.9 -> 46.6, radius 2 FP64 87.5 -> 76.5 us
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t pc_rsrc(const void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
 template <typename T>
-__device__ __forceinline__ T pc_bload(__amdgpu_buffer_rsrc_t r, int off) {
+__device__ __forceinline__ T pc_bload(__amdgpu_buffer_rsrc_t r, int off, int soff) {
   if constexpr (sizeof(T) == 4) {
-    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, off, soff, 0));
   } else {
-    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
   }
 }
 template <typename T>
-__device__ __forceinline__ void pc_bstore(__amdgpu_buffer_rsrc_t r, int off, T v) {
+__device__ __forceinline__ void pc_bstore(__amdgpu_buffer_rsrc_t r, int off, int soff, T v) {
   if constexpr (sizeof(T) == 4) {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off, soff, 0);
   } else {
     using V2 = decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0, 0, 0));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V2, v), r, off, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V2, v), r, off, soff, 0);
   }
 }
 
@@ -454,21 +459,25 @@ __global__ __launch_bounds__(64 * win_ty(R)) void stencil_win(WinArgs g, const T
     th[u] = k < 2 * R ? (k < R ? k : k + TY) : LR;
     jh[u] = k < 2 * R ? win.x - R + th[u] + kWinPadY : 0;                  // (row 0 of the table is empty)
   }
+  struct Row { int off, end, lo; };   // in bytes
+  auto row_load = [&](int i) -> Row {
+    const int2 m = g.meta[i];
+    return {m.x * ES, (m.x + (m.y >> 16)) * ES, (m.y & 0xffff) * ES};
+  };
   int wb;
-  int2 wo, wh[HT];
+  Row wo, wh[HT];
   auto windows = [&](int z) {
     wb = z;
     const int row = min(z + R + lane, g.nzp - 1) * g.nyp;
-    wo = g.meta[row + jo];
+    wo = row_load(row + jo);
 #pragma unroll
-    for (int u = 0; u < HT; ++u) wh[u] = g.meta[row + jh[u]];
+    for (int u = 0; u < HT; ++u) wh[u] = row_load(row + jh[u]);
   };
-  struct Row { int off, lo, len; };
-  auto row_of = [&](int2 m, int z) -> Row {
-    const int a = __builtin_amdgcn_readlane(m.x, z - wb), b = __builtin_amdgcn_readlane(m.y, z - wb);
-    return {a, b & 0xffff, b >> 16};
+  auto row_of = [&](Row w, int z) -> Row {
+    return {__builtin_amdgcn_readlane(w.off, z - wb), __builtin_amdgcn_readlane(w.end, z - wb),
+            __builtin_amdgcn_readlane(w.lo, z - wb)};
   };
-  auto yload = [&](Row r) -> T { return pc_bload<T>(pc_rsrc(yv + r.off, (unsigned)(r.len * ES)), lx - r.lo * ES); };
+  auto yload = [&](Row r) -> T { return pc_bload<T>(pc_rsrc(yv, r.end), lx - r.lo, r.off); };
 
   T q[QL];
   T xq[NS], vq[NS], hq[NS][HT];
@@ -481,9 +490,9 @@ __global__ __launch_bounds__(64 * win_ty(R)) void stencil_win(WinArgs g, const T
     constexpr int S = decltype(set)::value;
     const Row r = row_of(wo, z);
     ro[S] = r;
-    const int off = lo_ - r.lo * ES;
-    vq[S] = pc_bload<T>(pc_rsrc(V + r.off, (unsigned)(r.len * ES)), off);
-    if constexpr (HASX) xq[S] = pc_bload<T>(pc_rsrc(xv + r.off, (unsigned)(r.len * ES)), off);
+    const int off = lo_ - r.lo;
+    vq[S] = pc_bload<T>(pc_rsrc(V, r.end), off, r.off);
+    if constexpr (HASX) xq[S] = pc_bload<T>(pc_rsrc(xv, r.end), off, r.off);
 #pragma unroll
     for (int u = 0; u < HT; ++u) hq[S][u] = yload(row_of(wh[u], z));
   };
@@ -524,7 +533,7 @@ __global__ __launch_bounds__(64 * win_ty(R)) void stencil_win(WinArgs g, const T
     T o = acc + (ca * vq[S] + cb) * yc;
     if constexpr (HASX) o += cc * xq[S];
     const Row r = ro[S];
-    pc_bstore<T>(pc_rsrc(ov + r.off, z < ze ? (unsigned)(r.len * ES) : 0u), lo_ - r.lo * ES, o);
+    pc_bstore<T>(pc_rsrc(ov, z < ze ? r.end : r.off), lo_ - r.lo, r.off, o);
     // slot P (plane z-R) is free: plane z-R+QL, the queue front of plane z-2R+QL
     q[P] = yload(row_of(wo, z - R + QL));
     __builtin_amdgcn_sched_barrier(0);
@@ -539,10 +548,12 @@ __global__ __launch_bounds__(64 * win_ty(R)) void stencil_win(WinArgs g, const T
 }
 
 // z-chunks: with few vectors the windows x vectors do not fill the chip (256
-// CUs x 32 wavefronts), so each window's z-range is split until the wavefronts
-// would fill it once, keeping at least 8 planes per chunk (a chunk re-reads 2R
-// queue planes of its neighbour).
-constexpr long long kWinWaves = 8192;
+// CUs x 32 wavefronts), so each window's z-range is split until there are twice as
+// many wavefronts as that, so that a last round is not nearly empty, keeping at
+// least 8 planes per chunk (a chunk re-reads 2R queue planes of its neighbour).
+// C10H8, 49 vectors (8256 wavefronts unsplit): one chunk FP32 85, FP64 186 us, two
+// 80 and 175, five 91 and 195.
+constexpr long long kWinWaves = 16384;
 inline void win_zchunks(WinArgs& a, int nz, int nvec, int waves_per_wg) {
   const long long base = (long long)a.nwin * nvec * waves_per_wg;
   int nzc = 1;
@@ -925,6 +936,8 @@ int pc_grid_create(int nx, int ny, int nz, const int* row_lo, const int* row_hi,
       if (zb < ze) win.push_back(make_int4(j0, x0 | ((x1 - x0) << 16) | ((i ? radius : 0) << 28), zb, ze));
     }
   }
+  // the longest first: what runs last is short
+  std::stable_sort(win.begin(), win.end(), [](const int4& x, const int4& y) { return x.w - x.z > y.w - y.z; });
   g->win = nullptr;
   g->nwin = (int)win.size();
   g->pmeta = nullptr;
