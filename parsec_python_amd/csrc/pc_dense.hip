@@ -149,52 +149,16 @@ struct CbLane {
 
 __device__ __forceinline__ long long cb_blk(int i, int j, int ld) { return (long long)(kCb * j) * ld + kCb * i; }
 
-// acc += op(A) B over K = 32 (A, B column-major blocks; op(A) = A^T when TA)
-template <bool TA>
-__device__ __forceinline__ v4d cb_mma(v4d acc, const double* A, int lda, const double* B, int ldb, const CbLane& q) {
-  const int m = 16 * q.wm + q.lm, n = 16 * q.wn + q.lm;
-  double a[8], b[8];
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    const int kk = 4 * s + q.lk;
-    a[s] = TA ? A[m * lda + kk] : A[kk * lda + m];
-    b[s] = B[n * ldb + kk];
-  }
-#pragma unroll
-  for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], acc, 0, 0, 0);
-  return acc;
-}
-
-// acc += sum_{u < nt} op(A[u]) B[u]; the operands of four terms are loaded
-// before their MFMAs, so four block reads are in flight at once
-template <bool TA>
-__device__ __forceinline__ v4d cb_mma_sum(v4d acc, const double* const* A, int lda, const double* const* B, int ldb,
-                                          int nt, const CbLane& q) {
-  const int m = 16 * q.wm + q.lm, n = 16 * q.wn + q.lm;
-  for (int u0 = 0; u0 < nt; u0 += 4) {
-    double a[4][8], b[4][8];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const bool in = u0 + u < nt;
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        const int kk = 4 * s + q.lk;
-        a[u][s] = in ? (TA ? A[u0 + u][m * lda + kk] : A[u0 + u][kk * lda + m]) : 0.0;
-        b[u][s] = in ? B[u0 + u][n * ldb + kk] : 0.0;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][s], b[u][s], acc, 0, 0, 0);
-  }
-  return acc;
-}
-
 __device__ __forceinline__ double cb_readlane(double v, int l) {
   const long long b = __builtin_bit_cast(long long, v);
   const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+
+__device__ __forceinline__ void cb_lds_barrier() {   // a barrier that waits for LDS only: loads and stores stay in flight
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 __device__ __forceinline__ void cb_wave_sync() {   // this wavefront's LDS writes before its next reads
@@ -449,37 +413,75 @@ __global__ __launch_bounds__(64 * kCholWaves) void chol_blk_factor(int k, double
 
 // Workgroup j (nb of them) writes block column j of Ri = R^-1 (ld 32 nb):
 // X_jj = Dinv_j, X_ij = -Dinv_i sum_{l=i+1..j} R_il X_lj for i = j-1 .. 0,
-// zero below the diagonal blocks.
+// zero below the diagonal blocks.  Each wavefront makes a quarter of every block.
+// Bound by the chain of the last column's nb - 1 blocks, each a chain of MFMAs:
+// the X_lj stay in LDS, and the blocks of R and Dinv that the next row needs are
+// loaded into registers while this row's second product runs.  k = 23, 49,
+// 127, 275: 2.4, 4.4, 10, 34 us; with every operand from memory when its turn came
+// 3.8, 5.8, 16, 61 us.  The same bits.
+constexpr int chol_inv_lds(int nb) { return (nb + 1) * kCb * kCbLW * (int)sizeof(double); }
+
 __global__ __launch_bounds__(256) void chol_blk_inverse(const double* __restrict__ R, const double* __restrict__ Dinv,
                                                         int k, double* Ri) {
-  __shared__ double Y[kCb * kCbLW];
-  __shared__ const double* pa[kCbMaxNb];
-  __shared__ const double* pb[kCbMaxNb];
+  extern __shared__ double chol_sh[];
+  double* Y = chol_sh;
+  double* X = Y + kCb * kCbLW;   // X_lj at X + l kCb kCbLW
+  constexpr int NL = kCbMaxNb - 1;
   const int nb = (k + kCb - 1) / kCb, KP = kCb * nb;
   const int j = blockIdx.x;
   const CbLane q;
+  const int m = 16 * q.wm + q.lm, n = 16 * q.wn + q.lm;
+  double a[NL][8], da[8];
+  // R_il for l = i+1 .. j (the last one again past j) and Dinv_i
+  auto load_row = [&](int i) {
+#pragma unroll
+    for (int u = 0; u < NL; ++u) {
+      if (u >= nb - 1) continue;
+      const double* A = R + cb_blk(i, min(i + 1 + u, j), KP);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) a[u][s] = A[(long long)(4 * s + q.lk) * KP + m];
+    }
+    const double* D = Dinv + (long long)i * kCb * kCb;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) da[s] = D[(4 * s + q.lk) * kCb + m];
+  };
+  load_row(max(j - 1, 0));
   for (int e = threadIdx.x; e < kCb * kCb; e += 256) {
-    const int a = e & (kCb - 1), b = e / kCb;
-    Ri[cb_blk(j, j, KP) + (long long)b * KP + a] = Dinv[(long long)j * kCb * kCb + e];
-    for (int i = j + 1; i < nb; ++i) Ri[cb_blk(i, j, KP) + (long long)b * KP + a] = 0.0;
+    const int r = e & (kCb - 1), c = e / kCb;
+    const double x = Dinv[(long long)j * kCb * kCb + e];
+    Ri[cb_blk(j, j, KP) + (long long)c * KP + r] = x;
+    X[(j * kCb + c) * kCbLW + r] = x;
+    for (int i = j + 1; i < nb; ++i) Ri[cb_blk(i, j, KP) + (long long)c * KP + r] = 0.0;
   }
   for (int i = j - 1; i >= 0; --i) {
-    if (threadIdx.x < j - i) {
-      const int l = i + 1 + threadIdx.x;
-      pa[threadIdx.x] = R + cb_blk(i, l, KP);
-      pb[threadIdx.x] = Ri + cb_blk(l, j, KP);
-    }
-    __syncthreads();   // also: the blocks X_lj written before are visible
+    cb_lds_barrier();   // X_lj for l > i
     v4d acc = {0.0, 0.0, 0.0, 0.0};
-    acc = cb_mma_sum<false>(acc, pa, KP, pb, KP, j - i, q);
+#pragma unroll
+    for (int u = 0; u < NL; ++u) {
+      if (i + 1 + u > j) continue;
+      const double* B = X + ((i + 1 + u) * kCb + n) * kCbLW;
+      double b[8];
+#pragma unroll
+      for (int s = 0; s < 8; ++s) b[s] = B[4 * s + q.lk];
+#pragma unroll
+      for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][s], b[s], acc, 0, 0, 0);
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) Y[q.col() * kCbLW + q.row(r)] = acc[r];
-    __syncthreads();
-    v4d o = {0.0, 0.0, 0.0, 0.0};
-    o = cb_mma<false>(o, Dinv + (long long)i * kCb * kCb, kCb, Y, kCbLW, q);
+    double d[8];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) Ri[cb_blk(i, j, KP) + (long long)q.col() * KP + q.row(r)] = -o[r];
-    __syncthreads();
+    for (int s = 0; s < 8; ++s) d[s] = da[s];
+    load_row(max(i - 1, 0));
+    cb_lds_barrier();
+    v4d o = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      o = __builtin_amdgcn_mfma_f64_16x16x4f64(d[s], Y[n * kCbLW + 4 * s + q.lk], o, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      Ri[cb_blk(i, j, KP) + (long long)q.col() * KP + q.row(r)] = -o[r];
+      X[(i * kCb + q.col()) * kCbLW + q.row(r)] = -o[r];
+    }
   }
 }
 
@@ -804,10 +806,7 @@ __global__ __launch_bounds__(512) void sytrd_lower_reg(const double* __restrict_
     }
 #pragma unroll
     for (int q = Q; q < NCH; ++q) red[j & 1][(o - j - 1) & 7][lane + 64 * q] = pacc[q];
-    // an LDS-only barrier: the stores of P stay in flight
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    cb_lds_barrier();   // (the stores of P stay in flight)
   };
   pc_unroll_seq(std::make_integer_sequence<int, NCH>{}, [&](auto Qc) {
     for (int l = 0; l < 64 && !done; ++l) step(Qc, l);
@@ -1051,8 +1050,9 @@ __global__ __launch_bounds__(64) void sytrd_lower_mwg(const double* __restrict__
 //                below 64 equally spaced shifts of the current interval and the
 //                interval shrinks 65-fold, until it is 2 eps |lambda| +
 //                1e-2 eps ||T|| wide (about 10 rounds; two interleaved chains
-//                of 128 shifts per round measured slower: the step is bound
-//                by FP64 issue, not latency);
+//                of 128 shifts per round measured slower, and so did 4 or 8
+//                wavefronts per eigenvalue (136 -> 218 us at k = 275): the
+//                step is bound by FP64 issue, not latency);
 //   tri_invit:   inverse iteration, one thread per eigenvalue: LU with partial
 //                pivoting of T - sigma I, three solves from a fixed start
 //                vector, each normalised; equal shifts are separated by
@@ -1667,6 +1667,8 @@ int pc_dense_create(void* stream, int kmax, void** out_ctx) {
   c->chol_lds = 0;
   {
     const int kb = std::min(kmax, kCholMaxK), nbb = (kb + kCb - 1) / kCb, kp = kCb * nbb;
+    PC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&chol_blk_inverse),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, chol_inv_lds(kCbMaxNb)));
     PC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&chol_blk_factor),
                                hipFuncAttributeMaxDynamicSharedMemorySize, chol_lds(kCbMaxNb)));
     PC_HIP(hipMalloc(&c->cR, (size_t)kp * kp * sizeof(double)));
@@ -1794,7 +1796,7 @@ int pc_dense_rr(void* ctx, int k, double* S, int lds, double* Gy, int ldg, doubl
       hipLaunchKernelGGL(chol_blk_factor, dim3(1), dim3(64 * kCholWaves), chol_lds(nbk), c->stream, k, c->cR, c->cD,
                          c->info);
       PC_LAUNCH_CHECK();
-      hipLaunchKernelGGL(chol_blk_inverse, dim3(nbk), dim3(256), 0, c->stream, c->cR, c->cD, k, c->cRi);
+      hipLaunchKernelGGL(chol_blk_inverse, dim3(nbk), dim3(256), chol_inv_lds(nbk), c->stream, c->cR, c->cD, k, c->cRi);
       PC_LAUNCH_CHECK();
     }
     const double zero = 0.0;
@@ -1995,7 +1997,7 @@ static int side_end(DenseCtx* c, int k, const double* S, int lds) {
     hipLaunchKernelGGL(chol_blk_factor, dim3(1), dim3(64 * kCholWaves), chol_lds(nbk), c->side, k, c->cR, c->cD,
                        c->cinfo);
     PC_LAUNCH_CHECK();
-    hipLaunchKernelGGL(chol_blk_inverse, dim3(nbk), dim3(256), 0, c->side, c->cR, c->cD, k, c->cRi);
+    hipLaunchKernelGGL(chol_blk_inverse, dim3(nbk), dim3(256), chol_inv_lds(nbk), c->side, c->cR, c->cD, k, c->cRi);
     PC_LAUNCH_CHECK();
     c->chol_made = true;
   }

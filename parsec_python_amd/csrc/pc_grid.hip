@@ -359,7 +359,7 @@ __global__ __launch_bounds__(64 * NW) void stencil_zmarch(StArgs g, const T* __r
 //     nothing is clamped;
 //   * X, V and the halo rows of plane z+1 go out before plane z is computed, the
 //     queue front of plane z-R+QL right after plane z's last use of slot z-R.
-// What bounds it: per row and plane 40 vector, 15 scalar and 11 LDS instructions
+// What bounds it: per row and plane 40 vector, 11 scalar and 10 LDS instructions
 // at radius 4 against 5 loads and stores, with one barrier; no unit is busy more
 // than half of the time, on large blocks the three passes over memory take 60 %
 // (the reads miss L2 once: 1.44 GB for 1.33 GB of Y and X).  Occupancy is the
