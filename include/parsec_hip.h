@@ -111,7 +111,7 @@ int pc_dense_syevd(void* ctx, int k, double* A, int lda, double* w_host);
  * tridiagonal eigensolver of this library (multisection bisection, inverse
  * iteration, Gram-Schmidt and Rayleigh-Ritz within clusters of close
  * eigenvalues; rocSOLVER stedc for a cluster of more than 32) + Q Z
- * (pc_dense_set_backtransform) (default; 32 workgroups exchanging through agent-scope atomics for
+ * (pc_dense_set_backtransform) (default; 64 wavefronts exchanging through agent-scope atomics for
  * 128 <= k <= 320, one workgroup up to 512, larger k uses syevd), 3 = as 2
  * with the one-workgroup reduction always, 4 = as 2 with stedc always */
 int pc_dense_set_method(void* ctx, int method);

@@ -2042,7 +2042,7 @@ int pc_dense_gram_chol_async(void* ctx, int fp32, const void* Y, long long ldy, 
 // Eigensolver of the projected k x k problem: 0 = divide and conquer
 // (rocSOLVER syevd), 1 = cyclic Jacobi (rocSOLVER syevj, tolerance = machine
 // precision, at most 100 sweeps), 2 = Householder tridiagonalization in one
-// launch (32 workgroups for 128 <= k <= 320, one workgroup otherwise; k > 512
+// launch (64 wavefronts for 128 <= k <= 320, one workgroup otherwise; k > 512
 // uses syevd) + the tri_* tridiagonal eigensolver (rocSOLVER stedc if a
 // cluster of close eigenvalues exceeds kTriMaxM) + ormtr, 3 = as 2 with one
 // workgroup always, 4 = as 2 with stedc always.

@@ -42,7 +42,7 @@ struct GridDev {
   int radius;
   double w[8];   // 1D -d2/dx2 weights, centre first (unscaled)
   int4* win;     // stencil_win: windows {first row, first column | columns << 16 | left halo lanes << 28, zb, ze}
-  int nwin;
+  int nwin, winz;  // their number and mean number of planes
   int2* pmeta;   // its padded row table {offset, lo | length << 16}, nyp x nzp
   int nyp, nzp;
 };
@@ -361,8 +361,9 @@ __global__ __launch_bounds__(64 * NW) void stencil_zmarch(StArgs g, const T* __r
 //     queue front of plane z-R+QL right after plane z's last use of slot z-R.
 // What bounds it: per row and plane 40 vector, 11 scalar and 10 LDS instructions
 // at radius 4 against 5 loads and stores, with one barrier; no unit is busy more
-// than half of the time, on large blocks the three passes over memory take 60 %
-// (the reads miss L2 once: 1.44 GB for 1.33 GB of Y and X).  Occupancy is the
+// than half of the time.  Large blocks on a sphere are bound by the fabric: 3.7 GB
+// per step for 2.0 GB of Y, X and Out at 605,808 x 275 FP32 (V per vector, and halo
+// rows of slabs that march out of phase).  Occupancy is the
 // registers': two vectors per workgroup, three register sets or forced occupancy
 // were slower, and so were 4, 6 and 16 rows at radius 4 (the halo is 2R rows per
 // slab, the barrier is over all its wavefronts) and non-temporal X or stores.
@@ -373,10 +374,10 @@ __global__ __launch_bounds__(64 * NW) void stencil_zmarch(StArgs g, const T* __r
 //   605,808 points, radius 4 (Si87H76 sphere), 275 vectors:
 //                                   FP32 721 -> 680 us, FP64 1508 -> 1250 us
 //   C10H8 sphere, radius 4, 49:     FP32 111 -> 80 us,  FP64 260 -> 175 us
-//   52^3 cube, radius 4, 23:        FP32 17.2 -> 14.9,  FP64 30.2 -> 24.4 us
+//   52^3 cube, radius 4, 23:        FP32 17.2 -> 15.0,  FP64 30.2 -> 22.0 us
 //   radius 6 (FD12), 103 columns:   256 vectors FP32 1310 -> 1165 us,
 //                                   64 vectors FP64 640 -> 551 us
-//   70^3 cube, 40 vectors:          radius 3 FP32 48.9 -> 46.6, radius 2 FP64 87.5 -> 76.5 us
+//   70^3 cube, 40 vectors:          radius 3 FP32 49 -> 48, radius 2 FP64 87.5 -> 80.5 us
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t pc_rsrc(const void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
@@ -547,18 +548,29 @@ __global__ __launch_bounds__(64 * win_ty(R)) void stencil_win(WinArgs g, const T
   }
 }
 
-// z-chunks: with few vectors the windows x vectors do not fill the chip (256
-// CUs x 32 wavefronts), so each window's z-range is split until there are twice as
-// many wavefronts as that, so that a last round is not nearly empty, keeping at
-// least 8 planes per chunk (a chunk re-reads 2R queue planes of its neighbour).
-// C10H8, 49 vectors (8256 wavefronts unsplit): one chunk FP32 85, FP64 186 us, two
-// 80 and 175, five 91 and 195.
-constexpr long long kWinWaves = 16384;
-inline void win_zchunks(WinArgs& a, int nz, int nvec, int waves_per_wg) {
-  const long long base = (long long)a.nwin * nvec * waves_per_wg;
-  int nzc = 1;
-  if (base < kWinWaves) nzc = (int)std::min<long long>((kWinWaves + base - 1) / base, std::max(1, nz / 8));
-  a.zc = (nz + nzc - 1) / nzc;
+// z-chunks: a window's z-range is split where that fills the chip's rounds better.
+// A round is the workgroups that run at once (4 per CU in FP32, 2 in FP64 where
+// the registers or the bandwidth allow no more, half of that with the 12
+// wavefronts of radius 6); a chunk costs its planes and about 2R + 8 more for its
+// start (the queue's planes, the first loads), so the number of chunks with the
+// fewest rounds x (planes + start) is taken, at least 8 planes per chunk.  Against
+// filling 16,384 wavefronts whatever the rounds: 58^3 cube, 79 vectors, FP64 102 ->
+// 81 us; 62^3, radius 6, 20 vectors, FP64 59 -> 29; 52^3, 23 vectors, FP64 24.5 ->
+// 22.2; against one chunk: C10H8, 49 vectors, FP32 85 -> 81, FP64 186 -> 175 us.
+template <typename T, int R>
+void win_zchunks(WinArgs& a, int nz, int planes, int nvec) {
+  constexpr long long kRound = 256 * (sizeof(T) == 4 ? 4 : 2) / (R > 4 ? 2 : 1);
+  const long long wgs = (long long)a.nwin * nvec;
+  int best = 1;
+  double least = 0.0;
+  for (int n = 1; n <= std::max(1, nz / 8); ++n) {
+    const double cost = (double)((wgs * n + kRound - 1) / kRound) * ((double)planes / n + 2 * R + 8);
+    if (n == 1 || cost < least) {
+      best = n;
+      least = cost;
+    }
+  }
+  a.zc = (nz + best - 1) / best;
   a.nzc = (nz + a.zc - 1) / a.zc;
 }
 
@@ -571,7 +583,7 @@ int launch_win(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, in
   if (a.nwin == 0) return pc::PC_OK;   // no points
   a.meta = gd->pmeta; a.nyp = gd->nyp; a.nzp = gd->nzp;
   a.ld = ld;
-  win_zchunks(a, gd->nz, nvec, win_ty(R));
+  win_zchunks<T, R>(a, gd->nz, gd->winz, nvec);
   const long long nb = (long long)a.nwin * a.nzc * nvec;
   PC_CHECK_ARG(nb < (1LL << 30), "too many workgroups");
   a.nblocks = (int)nb;
@@ -940,6 +952,9 @@ int pc_grid_create(int nx, int ny, int nz, const int* row_lo, const int* row_hi,
   std::stable_sort(win.begin(), win.end(), [](const int4& x, const int4& y) { return x.w - x.z > y.w - y.z; });
   g->win = nullptr;
   g->nwin = (int)win.size();
+  long long planes = 0;
+  for (const int4& w : win) planes += w.w - w.z;
+  g->winz = win.empty() ? 0 : (int)(planes / (long long)win.size());
   g->pmeta = nullptr;
   g->nyp = ny + 2 * kWinPadY;
   g->nzp = nz + radius + kWinPadZ;
