@@ -86,7 +86,7 @@ def _log(msg):
 def measured_traffic(name):
     """HBM bytes per launch of the recurrence stencil from the committed
     counter summary (FETCH_SIZE + WRITE_SIZE, copy-calibrated), or None."""
-    path = os.path.join(ROOT, "profiles", f"stencil_lean_{name}_traffic.json")
+    path = os.path.join(ROOT, "profiles", f"stencil_{name}_traffic.json")
     if not os.path.exists(path):
         return None
     with open(path) as f:
@@ -422,7 +422,7 @@ def main():
                           "mixed_vs_converged_fp64_ha_per_atom": None if e_ref is None else abs(e_mixed - e_ref),
                           "fp64_stop_vs_converged_fp64_ha_per_atom": None if e_ref is None else abs(e_fp64 - e_ref)},
         "energy_ry": {"mixed": res.energies["total_ry"], "fp64": res64.energies["total_ry"]},
-        "roofline": {"kernel": "stencil_lean<float> (fused FD stencil + V + Chebyshev step)", "bound": "hbm",
+        "roofline": {"kernel": "stencil_win<float> (fused FD stencil + V + Chebyshev step)", "bound": "hbm",
                      "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "launches": int(len(durs)), "avg_launch_us": round(1e3 * float(durs.mean()), 2) if len(durs) else None,
