@@ -67,7 +67,7 @@ __global__ __launch_bounds__(64 * kGW) void proj_gather(ProjDev P, const T* __re
     T y[kGE][kGV];
 #pragma unroll
     for (int k = 0; k < kGE; ++k) {
-      const int e = min(eb + 64 * kGW * k, e1 - 1);   // past the end: the last entry, times 0
+      const int e = min(eb + 64 * kGW * k, e1 - 1);   // past the end: the last entry, its product replaced by 0 * 0
       pt[k] = P.ent_pt[e];
 #pragma unroll
       for (int m = 0; m < 3; ++m) w[k][m] = P.ent_u[3 * (long long)e + m];
@@ -80,9 +80,11 @@ __global__ __launch_bounds__(64 * kGW) void proj_gather(ProjDev P, const T* __re
     for (int k = 0; k < kGE; ++k) {
       const bool in = eb + 64 * kGW * k < e1;
 #pragma unroll
-      for (int u = 0; u < kGV; ++u)
+      for (int u = 0; u < kGV; ++u) {
+        const double yu = in ? y[k][u] : T(0);   // (0 times an infinite value would be a NaN)
 #pragma unroll
-        for (int m = 0; m < 3; ++m) s[u][m] += (in ? w[k][m] : 0.0) * (double)y[k][u];
+        for (int m = 0; m < 3; ++m) s[u][m] += (in ? w[k][m] : 0.0) * yu;
+      }
     }
   }
 #pragma unroll

@@ -1,0 +1,38 @@
+"""Infinities stay where the sums put them: lanes that a kernel fills up beyond
+its sum (the last round of a projector's support, taps past the 27th, voxels of a
+box beyond the volume) must not turn an infinity next to them into a NaN."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+INF = float("inf")
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("size", [1, 63, 65, 300])
+def test_projector_gather_infinite_value(gpu, size, dtype):
+    """The support's last point holds an infinity: C is that infinity, by the signs of u."""
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    print(f"projector infinity size={size} {dtype}", flush=True)
+    npts, nvec = 512, 5
+    aptr = np.array([0, size, 2 * size], np.int32)
+    pts = np.concatenate([np.arange(size), 100 + np.arange(size)]).astype(np.int32)
+    uv = np.tile([1.0, -2.0, 0.5], (2 * size, 1))
+    sc = np.ones(2)
+    handle = C.c_void_p()
+    pi, pd = C.POINTER(C.c_int), C.POINTER(C.c_double)
+    _lib.call("pc_proj_create", 2, aptr.ctypes.data_as(pi), pts.ctypes.data_as(pi), uv.ctypes.data_as(pd),
+              sc.ctypes.data_as(pd), npts, C.byref(handle))
+    Y = torch.ones((nvec, npts), dtype=torch.float64 if dtype == "f64" else torch.float32, device="cuda")
+    Y[2, 99 + size] = INF          # the second atom's last point, vector 2
+    cb = torch.empty((2, nvec, 3), dtype=torch.float64, device="cuda")
+    _lib.call(f"pc_proj_gather_{dtype}", handle, ptr(Y), npts, nvec, ptr(cb), stream())
+    ref = np.tile(size * np.array([1.0, -2.0, 0.5]), (2, nvec, 1))
+    ref[1, 2] = [INF, -INF, INF]
+    assert np.array_equal(cb.cpu().numpy(), ref)
+    _lib.call("pc_proj_destroy", handle)
