@@ -310,6 +310,8 @@ __global__ __launch_bounds__(256) void conv_tile1(Vol vol, Boxes bx, const unsig
     off[e] = (tt / 9 * HY + tt / 3 % 3) * HX + tt % 3;
     av[e] = (t < 27 && co < cout) ? Wt[(long long)co * 27 + t] : 0;
   }
+  // of the second product's taps 16 + 4 lk .. + 3, those below 27
+  const unsigned tm[2] = {lk < 3 ? ~0u : 0u, lk < 2 ? ~0u : (lk == 2 ? 0xffffu : 0u)};
   const u32x2 a0 = {av[0] | av[1] << 16, av[2] | av[3] << 16}, a1 = {av[4] | av[5] << 16, av[6] | av[7] << 16};
   __syncthreads();
 #pragma unroll
@@ -319,6 +321,8 @@ __global__ __launch_bounds__(256) void conv_tile1(Vol vol, Boxes bx, const unsig
     u32x4 b;
 #pragma unroll
     for (int e = 0; e < 4; ++e) b[e] = xs[p + off[2 * e]] | (unsigned)xs[p + off[2 * e + 1]] << 16;
+    b[2] &= tm[0];   // (a tap past 26 repeats tap 0, and 0 times an infinite value would be a NaN)
+    b[3] &= tm[1];
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(bf16x4, a0),
                                                     __builtin_bit_cast(bf16x4, u32x2{b[0], b[1]}), acc, 0, 0, 0);

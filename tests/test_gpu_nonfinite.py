@@ -36,3 +36,22 @@ def test_projector_gather_infinite_value(gpu, size, dtype):
     ref[1, 2] = [INF, -INF, INF]
     assert np.array_equal(cb.cpu().numpy(), ref)
     _lib.call("pc_proj_destroy", handle)
+
+
+@pytest.mark.parametrize("dims", [(5, 6, 7), (64, 32, 64)])
+def test_one_channel_conv_infinite_voxel(gpu, dims):
+    """One input channel: the infinity reaches its 27 neighbours as an infinity."""
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    print(f"conv infinity dims={dims}", flush=True)
+    d, h, w = dims
+    X = torch.ones((d, h, w), dtype=torch.bfloat16, device="cuda")
+    z, y, x = 2, 3, 4
+    X[z, y, x] = INF
+    W = torch.ones((16, 27), dtype=torch.bfloat16, device="cuda")
+    Y = torch.zeros((d, h, w, 16), device="cuda")
+    _lib.call("pc_unet_conv3d_fwd", ptr(X), 1, 1, ptr(W), None, 16, d, h, w, 2, 0.1, ptr(Y), 16, stream())
+    ones = torch.nn.functional.conv3d(torch.ones(1, 1, d, h, w), torch.ones(1, 1, 3, 3, 3), padding=1)[0, 0].cuda()
+    ones[z - 1:z + 2, y - 1:y + 2, x - 1:x + 2] = INF
+    assert torch.equal(Y, ones[..., None].expand(d, h, w, 16))
