@@ -438,6 +438,8 @@ __global__ __launch_bounds__(384) void conv_wgrad(Vol vol, Boxes bx, const unsig
       if ((int)threadIdx.x + 384 * u < ZU) put(tz[u], mz[u], zs, CZ, TX, ZG, threadIdx.x + 384 * u);
     __syncthreads();
     if (box + nsplit < nbox) fetch_box(box + nsplit);   // in flight during the products
+    const int x0 = box % bx.nx * TX, y0 = box / bx.nx % bx.ny * TY, z0 = box / (bx.nx * bx.ny) * TZ;
+    const bool edge = x0 + TX > vol.W || y0 + TY > vol.H || z0 + TZ > vol.D;
 #pragma unroll 2
     for (int g = kh; g < NG; g += 2) {
       const int row = g * RPK + (TX == 16 ? lk >> 1 : lk);        // this lane's row of the box
@@ -446,6 +448,9 @@ __global__ __launch_bounds__(384) void conv_wgrad(Vol vol, Boxes bx, const unsig
       const u32x2* za = reinterpret_cast<const u32x2*>(&zs[ln * CZ + row * TX + xh]);
       const u32x2 z0v = za[0], z1v = za[1];
       const u32x4 a = {z0v[0], z0v[1], z1v[0], z1v[1]};
+      // this lane's voxels in the volume: X's side of the others is zeroed as dZ's
+      // is (0 times an infinite value would be a NaN)
+      const int nv = y0 + y < vol.H && z0 + z < vol.D ? vol.W - x0 - xh : 0;
 #pragma unroll
       for (int dy = 0; dy < 3; ++dy) {
         const unsigned short* xr = &xs[ln * CX + ((z + dz) * HY + y + dy) * RS + 4 + xh];
@@ -454,9 +459,19 @@ __global__ __launch_bounds__(384) void conv_wgrad(Vol vol, Boxes bx, const unsig
         const unsigned s0 = __builtin_amdgcn_alignbit(wa[0], wm, 16), s1 = __builtin_amdgcn_alignbit(wa[1], wa[0], 16);
         const unsigned s2 = __builtin_amdgcn_alignbit(wb[0], wa[1], 16), s3 = __builtin_amdgcn_alignbit(wb[1], wb[0], 16);
         const unsigned s4 = __builtin_amdgcn_alignbit(wp, wb[1], 16);
-        acc[3 * dy] = mfma32(a, u32x4{s0, s1, s2, s3}, acc[3 * dy]);
-        acc[3 * dy + 1] = mfma32(a, u32x4{wa[0], wa[1], wb[0], wb[1]}, acc[3 * dy + 1]);
-        acc[3 * dy + 2] = mfma32(a, u32x4{s1, s2, s3, s4}, acc[3 * dy + 2]);
+        u32x4 b0 = {s0, s1, s2, s3}, b1 = {wa[0], wa[1], wb[0], wb[1]}, b2 = {s1, s2, s3, s4};
+        if (edge) {
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const unsigned in = nv >= 2 * w + 2 ? ~0u : nv == 2 * w + 1 ? 0xffffu : 0u;
+            b0[w] &= in;
+            b1[w] &= in;
+            b2[w] &= in;
+          }
+        }
+        acc[3 * dy] = mfma32(a, b0, acc[3 * dy]);
+        acc[3 * dy + 1] = mfma32(a, b1, acc[3 * dy + 1]);
+        acc[3 * dy + 2] = mfma32(a, b2, acc[3 * dy + 2]);
       }
     }
   }

@@ -55,3 +55,29 @@ def test_one_channel_conv_infinite_voxel(gpu, dims):
     ones = torch.nn.functional.conv3d(torch.ones(1, 1, d, h, w), torch.ones(1, 1, 3, 3, 3), padding=1)[0, 0].cuda()
     ones[z - 1:z + 2, y - 1:y + 2, x - 1:x + 2] = INF
     assert torch.equal(Y, ones[..., None].expand(d, h, w, 16))
+
+
+@pytest.mark.parametrize("cin,cout", [(16, 16), (16, 1), (1, 16)])
+@pytest.mark.parametrize("dims", [(5, 6, 7), (4, 8, 17), (9, 8, 16), (4, 9, 24)])
+def test_conv_weight_gradient_infinite_corner(gpu, cin, cout, dims):
+    """An infinity in the volume's last voxel reaches only the taps that pair it
+    with a voxel of the volume (also where the boxes go beyond the volume)."""
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    print(f"wgrad infinity cin={cin} cout={cout} dims={dims}", flush=True)
+    d, h, w = dims
+    X = torch.ones((d, h, w, cin), dtype=torch.bfloat16, device="cuda")
+    X[-1, -1, -1, 0] = INF
+    Z = torch.ones((d, h, w, cout), dtype=torch.bfloat16, device="cuda")
+    n = C.c_size_t()
+    _lib.call("pc_unet_wgrad_workspace", cout, cin, C.byref(n))
+    work = torch.empty(n.value, dtype=torch.uint8, device="cuda")
+    dw = torch.empty((cout, 3, 3, 3, cin), device="cuda")
+    _lib.call("pc_unet_conv3d_wgrad", ptr(Z), cout, cout, ptr(X), cin, cin, d, h, w, ptr(dw), ptr(work), n.value,
+              stream())
+    # tap (a, b, c) pairs voxel v with v + (a - 1, b - 1, c - 1): the last voxel is in it unless a component is -1
+    count = [np.array([s - 1.0, s, s - 1.0]) for s in dims]
+    ref = np.einsum("a,b,c->abc", *count)[..., None].repeat(cin, -1)
+    ref[1:, 1:, 1:, 0] = INF
+    assert np.array_equal(dw.cpu().numpy(), np.broadcast_to(ref, dw.shape))
