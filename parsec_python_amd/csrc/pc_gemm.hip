@@ -733,8 +733,9 @@ struct GramPlan {
 // column 1.5 and 3 times as often); so 275 columns take 96-wide
 // tiles, 256 take 64-wide ones and a symmetric product of up to 96 32-wide ones.  Chunks: about as many workgroups as the
 // chip holds at once, all with the same work (one round, no short last one),
-// and at least 256 points each; sp = points per stage.
-GramPlan plan_gram(long long n, int kx, int ky, int sym, int sp) {
+// at least 256 points each and no more than the workspace holds; sp = points
+// per stage.  nchunk = 0: not even one per tile fits.
+GramPlan plan_gram(long long n, int kx, int ky, int sym, int sp, size_t bytes) {
   GramPlan p{};
   double best = 0.0;
   for (int nt = 3; nt >= 1; --nt) {
@@ -748,16 +749,19 @@ GramPlan plan_gram(long long n, int kx, int ky, int sym, int sp) {
   }
   const int resident = p.nt == 3 ? 512 : p.nt == 2 ? 1024 : 2048;
   const int rest = n % sp != 0;   // the points past the last whole stage are a chunk of their own
+  const long long nw = n - n % sp;
+  const long long room = (long long)(bytes / sizeof(double)) / (p.ntile * p.tile_size()) - rest;
+  if (room < (nw > 0 ? 1 : 0)) return p;
   const long long target = std::max<long long>(1, resident / p.ntile - rest);
   const long long maxch = std::max<long long>(1, (n + 255) / 256);
-  const long long nw = n - n % sp;
-  p.nchunk = (int)std::min(target, maxch);
+  p.nchunk = (int)std::min({target, maxch, std::max<long long>(1, room)});
   p.chunk = std::max<long long>(32, ((nw + p.nchunk - 1) / p.nchunk + 31) / 32 * 32);
   p.nchunk = (int)((nw + p.chunk - 1) / p.chunk) + rest;
   return p;
 }
 
-// The form for unaligned columns keeps 64-wide tiles.
+// The form for any alignment keeps 64-wide tiles; its workspace is the smallest
+// that either form takes.
 GramPlan plan_gram_unaligned(long long n, int kx, int ky, int sym) {
   GramPlan p{};
   p.nt = 2;
@@ -782,12 +786,16 @@ int gram_impl(const T* X, long long ldx, const T* Y, long long ldy, long long n,
   constexpr int E = 16 / (int)sizeof(T);
   const bool vec = (ldx % E == 0) && (ldy % E == 0) && (reinterpret_cast<uintptr_t>(X) % 16 == 0) &&
                    (reinterpret_cast<uintptr_t>(Y) % 16 == 0);
-  const GramPlan p = vec ? plan_gram(n, kx, ky, sym, kGramStage / (int)sizeof(T)) : plan_gram_unaligned(n, kx, ky, sym);
-  PC_CHECK_ARG(work_bytes >= gram_work_bytes(p), "workspace too small");
+  const GramPlan any = plan_gram_unaligned(n, kx, ky, sym);
+  PC_CHECK_ARG(work_bytes >= gram_work_bytes(any), "workspace too small");
+  GramPlan p{};
+  if (vec) p = plan_gram(n, kx, ky, sym, kGramStage / (int)sizeof(T), work_bytes);
+  const bool tiled = p.nchunk > 0;
+  if (!tiled) p = any;
   hipStream_t st = static_cast<hipStream_t>(stream);
   double* part = static_cast<double*>(work);
   const int nb = p.ntile * p.nchunk, nb8 = (nb + 7) / 8;
-  if (vec) {
+  if (tiled) {
 #define PC_GRAM(NT)                                                                                              \
   hipLaunchKernelGGL((gram_tile<T, NT>), dim3(8 * nb8), dim3(256), 0, st, X, ldx, Y, ldy, n, kx, ky, p.ti_n, p.tj_n, \
                      p.ntile, sym, nb, nb8, p.chunk, part)
@@ -891,7 +899,8 @@ extern "C" {
 
 int pc_gram_workspace(long long n, int kx, int ky, int sym, size_t* out_bytes) {
   PC_CHECK_ARG(out_bytes, "null pointer");
-  *out_bytes = std::max({gram_work_bytes(plan_gram(n, kx, ky, sym, 16)), gram_work_bytes(plan_gram(n, kx, ky, sym, 32)),
+  *out_bytes = std::max({gram_work_bytes(plan_gram(n, kx, ky, sym, 16, SIZE_MAX)),
+                         gram_work_bytes(plan_gram(n, kx, ky, sym, 32, SIZE_MAX)),
                          gram_work_bytes(plan_gram_unaligned(n, kx, ky, sym))});
   return pc::PC_OK;
 }
