@@ -410,7 +410,10 @@ __global__ __launch_bounds__(256) void rotate_kernel(const T* __restrict__ X, lo
 // TF/s (1067 us with Q guarded per value, 115 instead of 31 vector instructions
 // beside a slab's 144 MFMAs), FP64 1669 us (2987 us with 64 columns per
 // workgroup and Q from memory).
-template <typename T, int NCH>
+// LONG: 64-bit addresses per lane, for columns whose slab of X exceeds 32-bit
+// byte offsets (they take 4 to 8 registers more, which costs FP64 a wavefront
+// per SIMD at 96 columns).
+template <typename T, int NCH, bool LONG>
 __global__ __launch_bounds__(256, 2) void rotate_wide(const T* __restrict__ X, long long ldx,
                                                       const T* __restrict__ Qt, T* __restrict__ Z, long long ldz,
                                                       long long n, int kx, int ky, int ncb, int nblocks, int nb8) {
@@ -460,15 +463,23 @@ __global__ __launch_bounds__(256, 2) void rotate_wide(const T* __restrict__ X, l
 #pragma unroll
       for (int t = 0; t < QPT; ++t) qs[bf][qk * LQ + qc + TR * t] = qr[t];
     };
-    // X of step st of the slab at kb (32-bit offsets from the slab's first vector)
+    // X of step st of the slab at kb
+    const T* const xlane = X + (long long)lk * ldx + pl;
+    const T* const xlast = X + (long long)(kx - 1) * ldx + pl;
     auto xfetch = [&](int kb, int st) {
-      const char* base = reinterpret_cast<const char*>(X + (long long)kb * ldx);
-      const unsigned off = ((unsigned)min(4 * st + lk, kx - 1 - kb) * (unsigned)ldx + (unsigned)pl) * (unsigned)sizeof(T);
+      const char* src;
+      if constexpr (LONG) {
+        const T* s = xlane + (long long)(kb + 4 * st) * ldx;
+        src = reinterpret_cast<const char*>(kb + 4 * st + lk < kx ? s : xlast);
+      } else {   // 32-bit offsets from the slab's first vector
+        const unsigned row = min(4 * st + lk, kx - 1 - kb);
+        src = reinterpret_cast<const char*>(X + (long long)kb * ldx) + (row * (unsigned)ldx + (unsigned)pl) * (unsigned)sizeof(T);
+      }
       if constexpr (EDGE) {
 #pragma unroll
-        for (int j = 0; j < E; ++j) x[st][j] = pl + j < n ? *reinterpret_cast<const T*>(base + off + sizeof(T) * j) : T(0);
+        for (int j = 0; j < E; ++j) x[st][j] = pl + j < n ? *reinterpret_cast<const T*>(src + sizeof(T) * j) : T(0);
       } else {
-        const VT t = *reinterpret_cast<const VT*>(base + off);
+        const VT t = *reinterpret_cast<const VT*>(src);
 #pragma unroll
         for (int j = 0; j < E; ++j) x[st][j] = t[j];
       }
@@ -836,8 +847,7 @@ int rotate_impl(const T* X, long long ldx, const double* Q, int ldq, T* Z, long 
   };
   constexpr int E = 16 / (int)sizeof(T);
   const bool vec = (ldx % E == 0) && (ldz % E == 0) && (reinterpret_cast<uintptr_t>(X) % 16 == 0) &&
-                   (reinterpret_cast<uintptr_t>(Z) % 16 == 0) &&
-                   ldx < (1LL << 24);   // 16 vectors in 32-bit byte offsets
+                   (reinterpret_cast<uintptr_t>(Z) % 16 == 0);
   if constexpr (sizeof(T) == 4) {
     const int nch = (ky + 31) / 32;
     if (vec && nch <= 9 && g_rotate_bf3 && work_bytes >= bf3_work_bytes(kx, ky)) {
@@ -870,11 +880,13 @@ int rotate_impl(const T* X, long long ldx, const double* Q, int ldq, T* Z, long 
     PC_CHECK_ARG(npt * ncb < (1LL << 30), "too many workgroups");
     const int nb = (int)(npt * ncb);
     const int nb8 = (nb + 7) / 8;
+    // a slab's X in 32-bit byte offsets: to 2^26 points per column and more in FP32, 2^25 in FP64
+    const bool wide_offsets = ((std::min(kx, 16) - 1) * ldx + n) * (long long)sizeof(T) >= (1LL << 32);
     switch (nch) {
-#define PC_ROT(N)                                                                                                   \
-  case N:                                                                                                           \
-    hipLaunchKernelGGL((rotate_wide<T, N>), dim3(8 * nb8), dim3(256), 0, st, X, ldx, qt, Z, ldz, n, kx, ky, ncb, nb, \
-                       nb8);                                                                                        \
+#define PC_ROT(N)                                                                                               \
+  case N:                                                                                                       \
+    hipLaunchKernelGGL((wide_offsets ? rotate_wide<T, N, true> : rotate_wide<T, N, false>), dim3(8 * nb8),      \
+                       dim3(256), 0, st, X, ldx, qt, Z, ldz, n, kx, ky, ncb, nb, nb8);                          \
     break;
       PC_ROT(1) PC_ROT(2) PC_ROT(3) PC_ROT(4) PC_ROT(5) PC_ROT(6) PC_ROT(7) PC_ROT(8) PC_ROT(9)
 #undef PC_ROT

@@ -1,4 +1,5 @@
-"""Gram products in the smallest workspaces that they take."""
+"""Gram and rotation at the limits of their arguments: the smallest workspaces
+that the Gram product takes, and columns beyond 2^24 points."""
 import numpy as np
 import pytest
 
@@ -41,3 +42,89 @@ def test_gram_smallest_workspace(gpu, n, kx, ky, sym, dtype):
     tol = (n + 2) * 2.0 ** -53 if dtype == "f64" else 17 * 2.0 ** -24 + n * 2.0 ** -53
     assert np.all(np.abs(S.cpu().numpy() - y @ x.T) <= 2 * tol * (np.abs(y) @ np.abs(x).T))
     assert bool((work[nbytes // 8:] == 7.0).all())
+
+
+def _rotate(X, n, Q, dtype, ldz, Z=None):
+    """Z = X Q through pc_rotate_*; X: (kx, ldx), Q: (ky, kx) with row j = column j."""
+    import ctypes as C
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    ky, kx = Q.shape
+    nbytes = C.c_size_t()
+    _lib.call("pc_rotate_workspace", kx, ky, int(dtype == "f32"), C.byref(nbytes))
+    work = torch.empty(nbytes.value, dtype=torch.uint8, device="cuda")
+    if Z is None:
+        Z = torch.full((ky, ldz), 7.0, dtype=X.dtype, device="cuda")
+    _lib.call(f"pc_rotate_{dtype}", ptr(X), X.shape[1], ptr(Q), kx, ptr(Z), ldz, n, kx, ky, ptr(work), nbytes.value,
+              stream())
+    return Z
+
+
+# columns just beyond 2^24 points; columns whose 16 exceed 32-bit byte offsets
+@pytest.mark.parametrize("dtype,n,ldx,kx,ky", [("f32", 2 ** 24 + 21, 2 ** 24 + 32, 3, 2), ("f64", 2 ** 24 + 21, 2 ** 24 + 32, 3, 2),
+                                               ("f32", 1003, 72_000_000, 17, 20), ("f64", 1003, 36_000_000, 17, 20)])
+def test_rotate_long_columns(gpu, dtype, n, ldx, kx, ky):
+    """Tolerance: kx products added in order, ((kx + 2) u), Q rounded once in FP32."""
+    import torch
+    print(f"long columns {dtype} n={n} ldx={ldx} kx={kx} ky={ky}", flush=True)
+    tdt, u = (torch.float64, 2.0 ** -53) if dtype == "f64" else (torch.float32, 2.0 ** -24)
+    g = torch.Generator(device="cuda").manual_seed(kx)
+    X = torch.empty((kx, ldx), dtype=tdt, device="cuda")
+    X[:, :n] = torch.randn((kx, n), generator=g, dtype=tdt, device="cuda")
+    X[:, n:n + 64] = float("nan")
+    Q = torch.randn((ky, kx), generator=g, dtype=torch.float64, device="cuda")
+    Z = _rotate(X, n, Q, dtype, (n + 15) // 16 * 16)
+    for j in range(ky):
+        ref = (Q[j, :, None] * X[:, :n].double()).sum(0)
+        mag = (Q[j, :, None] * X[:, :n].double()).abs().sum(0)
+        assert bool(((Z[j, :n].double() - ref).abs() <= 2 * (kx + 2) * u * mag).all())
+    assert bool((Z[:, n:] == 7.0).all())
+
+
+def test_rotate_long_columns_split_bf16(gpu):
+    """The optional split form serves long columns too: the bits of the same block in short ones."""
+    import torch
+    from parsec_python_amd import _lib
+    n, kx, ky = 1003, 17, 20
+    print("long columns, split form", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    short = torch.randn((kx, 1008), generator=g, device="cuda")
+    long = torch.empty((kx, 2 ** 24 + 32), device="cuda")
+    long[:, :n] = short[:, :n]
+    Q = torch.randn((ky, kx), generator=g, dtype=torch.float64, device="cuda")
+    plain = _rotate(short, n, Q, "f32", 1008)
+    try:
+        _lib.call("pc_rotate_set_split_bf16", 1)
+        a, b = _rotate(short, n, Q, "f32", 1008), _rotate(long, n, Q, "f32", 1008)
+    finally:
+        _lib.call("pc_rotate_set_split_bf16", 0)
+    assert not torch.equal(a, plain)
+    assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+def test_rotate_long_columns_keep_their_speed(gpu, dtype):
+    """Columns on either side of 2^24 points take the same kernel (96 columns of
+    400,000 points: 93 us in FP32 and 165 in FP64, 150 and 350 with the general one)."""
+    import torch
+    print(f"long columns' time {dtype}", flush=True)
+    n, k = 400_000, 96
+    tdt = torch.float64 if dtype == "f64" else torch.float32
+    Q = torch.ones((k, k), dtype=torch.float64, device="cuda")
+    blocks = [torch.zeros((k, 2 ** 24 + d), dtype=tdt, device="cuda") for d in (-1040, 1040)]
+    times = [[], []]
+    for _ in range(9):
+        for i, X in enumerate(blocks):
+            torch.cuda.synchronize()
+            e0, e1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            Z = _rotate(X, n, Q, dtype, n)
+            e0.record()
+            for _ in range(4):
+                _rotate(X, n, Q, dtype, n, Z)
+            e1.record()
+            torch.cuda.synchronize()
+            times[i].append(e0.elapsed_time(e1))
+    short, long = (sorted(t)[4] for t in times)
+    print(f"{250 * short:.1f} and {250 * long:.1f} us", flush=True)
+    assert long <= 1.25 * short
