@@ -24,6 +24,11 @@ enum Status : int {
 
 constexpr int kWave = 64;
 
+// Workgroups per launch, at most: a grid dimension holds fewer than 2^32
+// work-items, and a launch of more wraps round without an error.  Entry points
+// whose workgroups may be more launch in parts.
+constexpr long long kMaxGrid = 1LL << 21;
+
 }  // namespace pc
 
 #define PC_CHECK_ARG(cond, msg)                                   \

@@ -876,22 +876,24 @@ int rotate_impl(const T* X, long long ldx, const double* Q, int ldq, T* Z, long 
     // column blocks of at most 288, of equal width
     const int ncb = (ky + 287) / 288;
     const int nch = ((ky + ncb - 1) / ncb + 31) / 32;
-    const long long npt = (n + 32 * E - 1) / (32 * E);
-    PC_CHECK_ARG(npt * ncb < (1LL << 30), "too many workgroups");
-    const int nb = (int)(npt * ncb);
-    const int nb8 = (nb + 7) / 8;
     // a slab's X in 32-bit byte offsets: to 2^26 points per column and more in FP32, 2^25 in FP64
     const bool wide_offsets = ((std::min(kx, 16) - 1) * ldx + n) * (long long)sizeof(T) >= (1LL << 32);
-    switch (nch) {
+    const long long step = pc::kMaxGrid / ncb * (32 * E);   // points per launch
+    for (long long p0 = 0; p0 < n; p0 += step) {
+      const long long np = std::min(step, n - p0);
+      const int nb = (int)((np + 32 * E - 1) / (32 * E) * ncb);
+      const int nb8 = (nb + 7) / 8;
+      switch (nch) {
 #define PC_ROT(N)                                                                                               \
   case N:                                                                                                       \
     hipLaunchKernelGGL((wide_offsets ? rotate_wide<T, N, true> : rotate_wide<T, N, false>), dim3(8 * nb8),      \
-                       dim3(256), 0, st, X, ldx, qt, Z, ldz, n, kx, ky, ncb, nb, nb8);                          \
+                       dim3(256), 0, st, X + p0, ldx, qt, Z + p0, ldz, np, kx, ky, ncb, nb, nb8);               \
     break;
-      PC_ROT(1) PC_ROT(2) PC_ROT(3) PC_ROT(4) PC_ROT(5) PC_ROT(6) PC_ROT(7) PC_ROT(8) PC_ROT(9)
+        PC_ROT(1) PC_ROT(2) PC_ROT(3) PC_ROT(4) PC_ROT(5) PC_ROT(6) PC_ROT(7) PC_ROT(8) PC_ROT(9)
 #undef PC_ROT
+      }
+      PC_LAUNCH_CHECK();
     }
-    PC_LAUNCH_CHECK();
     return pc::PC_OK;
   }
   if (convert_q() != pc::PC_OK) return pc::PC_ERR_HIP;

@@ -1,0 +1,37 @@
+"""Calls whose workgroups are more than one launch dimension of 2^32 work-items
+holds, or whose volume has 2^31 voxels and more: small results of large operands,
+exact by construction (whole numbers and single products)."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def room(gpu):
+    """room(bytes): skips where the card has less than that free, and frees the cache afterwards."""
+    import torch
+
+    def need(nbytes):
+        torch.cuda.empty_cache()
+        if torch.cuda.mem_get_info()[0] < nbytes * 1.1:
+            pytest.skip("not enough free device memory")
+    yield need
+    torch.cuda.empty_cache()
+
+
+def test_rotation_of_one_very_long_column(gpu, room):
+    """FP64, 2^30 + 70 points: 2^24 workgroups of 64 points and more."""
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    n = 2 ** 30 + 70
+    print(f"rotation of {n} points", flush=True)
+    ld = (n + 15) // 16 * 16
+    room(3 * ld * 8)
+    X = torch.arange(ld, dtype=torch.float64, device="cuda")
+    Z = torch.full((ld,), -1.0, dtype=torch.float64, device="cuda")
+    Q = torch.full((1,), 3.0, dtype=torch.float64, device="cuda")
+    work = torch.empty(1, dtype=torch.float64, device="cuda")
+    _lib.call("pc_rotate_f64", ptr(X), ld, ptr(Q), 1, ptr(Z), ld, n, 1, 1, ptr(work), 8, stream())
+    assert bool((Z[n:] == -1.0).all())
+    assert torch.equal(Z[:n], X[:n].mul_(3.0))
