@@ -146,11 +146,17 @@ int gather_impl(void* proj, const T* Y, long long ld, int nvec, double* C, void*
   const ProjDev* P = static_cast<const ProjDev*>(proj);
   PC_CHECK_ARG(P && Y && C, "null pointer");
   if (P->natoms == 0 || nvec == 0) return pc::PC_OK;
-  const long long nb = (long long)P->natoms * ((nvec + kGV - 1) / kGV);
-  PC_CHECK_ARG(nb < (1LL << 30), "too many workgroups");
-  const dim3 grid((unsigned)((nb + 7) / 8 * 8));
-  hipLaunchKernelGGL(proj_gather<T>, grid, dim3(64 * kGW), 0, static_cast<hipStream_t>(stream), *P, Y, ld, nvec, C);
-  PC_LAUNCH_CHECK();
+  const long long groups = (nvec + kGV - 1) / kGV;
+  const int step = (int)std::max<long long>(1, pc::kMaxGrid / groups);   // atoms per launch
+  for (int a0 = 0; a0 < P->natoms; a0 += step) {
+    ProjDev part = *P;
+    part.atom_ptr += a0;
+    part.natoms = std::min(step, P->natoms - a0);
+    const dim3 grid((unsigned)((part.natoms * groups + 7) / 8 * 8));
+    hipLaunchKernelGGL(proj_gather<T>, grid, dim3(64 * kGW), 0, static_cast<hipStream_t>(stream), part, Y, ld, nvec,
+                       C + (long long)a0 * nvec * 3);
+    PC_LAUNCH_CHECK();
+  }
   return pc::PC_OK;
 }
 

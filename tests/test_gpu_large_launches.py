@@ -1,6 +1,9 @@
 """Calls whose workgroups are more than one launch dimension of 2^32 work-items
 holds, or whose volume has 2^31 voxels and more: small results of large operands,
 exact by construction (whole numbers and single products)."""
+import ctypes as C
+
+import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -17,6 +20,31 @@ def room(gpu):
             pytest.skip("not enough free device memory")
     yield need
     torch.cuda.empty_cache()
+
+
+def test_gather_of_many_atoms_and_vectors(gpu, room):
+    """4,099 atoms of one point each, 16,385 vectors: 2^24 workgroups and more."""
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    na, nvec, npts = 4099, 16385, 64
+    print(f"gather of {na} atoms and {nvec} vectors", flush=True)
+    room(na * nvec * 3 * 8 * 2)
+    aptr, pts = np.arange(na + 1, dtype=np.int32), (np.arange(na) % npts).astype(np.int32)
+    uv = np.stack([np.arange(na) % 7 + 1.0, np.arange(na) % 5 - 2.0, np.arange(na) % 3 + 0.5], 1)
+    sc = np.ones(na)
+    handle = C.c_void_p()
+    pi, pd = C.POINTER(C.c_int), C.POINTER(C.c_double)
+    _lib.call("pc_proj_create", na, aptr.ctypes.data_as(pi), pts.ctypes.data_as(pi), uv.ctypes.data_as(pd),
+              sc.ctypes.data_as(pd), npts, C.byref(handle))
+    Y = torch.arange(nvec * npts, device="cuda").remainder(1009).float().view(nvec, npts)
+    cb = torch.full((na, nvec, 3), float("nan"), dtype=torch.float64, device="cuda")
+    _lib.call("pc_proj_gather_f32", handle, ptr(Y), npts, nvec, ptr(cb), stream())
+    u = torch.tensor(uv, device="cuda")
+    y = Y.double().T[torch.tensor(pts, device="cuda").long()]          # (na, nvec)
+    for m in range(3):
+        assert torch.equal(cb[:, :, m], u[:, m, None] * y)
+    _lib.call("pc_proj_destroy", handle)
 
 
 def test_rotation_of_one_very_long_column(gpu, room):
