@@ -586,19 +586,23 @@ int launch_win(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, in
   a.meta = gd->pmeta; a.nyp = gd->nyp; a.nzp = gd->nzp;
   a.ld = ld;
   win_zchunks<T, R>(a, gd->nz, gd->winz, nvec);
-  const long long nb = (long long)a.nwin * a.nzc * nvec;
-  PC_CHECK_ARG(nb < (1LL << 30), "too many workgroups");
-  a.nblocks = (int)nb;
-  a.nb8 = (a.nblocks + 7) / 8;
   for (int d = 0; d < 8; ++d) a.w[d] = 0.0;
   a.w[0] = 3.0 * gd->w[0] * scale;
   for (int d = 1; d <= R; ++d) a.w[d] = gd->w[d] * scale;
-  const dim3 grid(8 * a.nb8), block(64 * win_ty(R));
-  if (X)
-    hipLaunchKernelGGL((stencil_win<T, R, true>), grid, block, 0, st, a, Y, X, Out, V, T(ca), T(cb), T(cc));
-  else
-    hipLaunchKernelGGL((stencil_win<T, R, false>), grid, block, 0, st, a, Y, X, Out, V, T(ca), T(cb), T(cc));
-  PC_LAUNCH_CHECK();
+  const int per = a.nwin * a.nzc, step = (int)std::max<long long>(1, pc::kMaxGrid / per);   // vectors per launch
+  for (int v0 = 0; v0 < nvec; v0 += step) {
+    const long long at = (long long)v0 * ld;
+    a.nblocks = per * std::min(step, nvec - v0);
+    a.nb8 = (a.nblocks + 7) / 8;
+    const dim3 grid(8 * a.nb8), block(64 * win_ty(R));
+    if (X)
+      hipLaunchKernelGGL((stencil_win<T, R, true>), grid, block, 0, st, a, Y + at, X + at, Out + at, V, T(ca), T(cb),
+                         T(cc));
+    else
+      hipLaunchKernelGGL((stencil_win<T, R, false>), grid, block, 0, st, a, Y + at, X, Out + at, V, T(ca), T(cb),
+                         T(cc));
+    PC_LAUNCH_CHECK();
+  }
   return pc::PC_OK;
 }
 

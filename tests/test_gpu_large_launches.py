@@ -63,3 +63,29 @@ def test_rotation_of_one_very_long_column(gpu, room):
     _lib.call("pc_rotate_f64", ptr(X), ld, ptr(Q), 1, ptr(Z), ld, n, 1, 1, ptr(work), 8, stream())
     assert bool((Z[n:] == -1.0).all())
     assert torch.equal(Z[:n], X[:n].mul_(3.0))
+
+
+def test_stencil_of_many_vectors(gpu, room):
+    """2^3 points, radius 6, 6,000,001 vectors: more than 2^32 work-items in workgroups of 768."""
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    from parsec_python_amd.grid import DeviceGrid, make_grid
+    nvec, ld = 6_000_001, 8
+    print(f"stencil of {nvec} vectors", flush=True)
+    room(4 * nvec * ld * 4)
+    dg = DeviceGrid(make_grid(2, 0.5, 1.0, "cube"), 6)
+    Y = torch.arange(nvec * ld, device="cuda").remainder(1013).float().view(nvec, ld)
+    X = torch.arange(nvec * ld, device="cuda").remainder(17).float().view(nvec, ld)
+    V = torch.ones(8, device="cuda")
+    out = torch.full((nvec, ld), float("nan"), device="cuda")
+
+    def step(v0, n, o):
+        _lib.call("pc_stencil_f32", dg.handle, ptr(Y[v0:]), ptr(X[v0:]), ptr(o), ptr(V), n, ld, 0.5, 1.0, -0.25, 2.0,
+                  None, stream())
+    step(0, nvec, out)
+    part = torch.empty_like(out)
+    for v0 in range(0, nvec, 1_000_000):
+        step(v0, min(1_000_000, nvec - v0), part[v0:])
+    assert torch.equal(out, part)
+    dg.close()
