@@ -763,18 +763,20 @@ int pc_unet_conv3d_fwd(const void* X, int ldx, int cin, const void* W, const flo
   const bool w8 = size == 512   ? padded(8, 8, 8) < padded(16, 8, 4)
                   : size == 256 ? padded(8, 8, 4) < padded(16, 4, 4)
                                 : padded(8, 4, 4) < padded(16, 4, 2);
-#define PC_CONV(NCB, TX, TY, TZ)                                                                                     \
+  // the channel blocks that one launch holds at a time
+#define PC_CONV_PARTS(KERNEL, TX, TY, TZ)                                                                            \
   do {                                                                                                               \
-    const Boxes bx = make_boxes(vol, TX, TY, TZ, ct);                                                                \
-    hipLaunchKernelGGL((conv_tile<NCB, TX, TY, TZ>), dim3(8 * bx.nb8), dim3(256), 0, st, vol, bx, X16, ldx, W16, bias, \
-                       cout, mode, slope, Y, ldy, yvec);                                                             \
+    const int step = (int)std::max(1LL, std::min<long long>(ct, pc::kMaxGrid / box_count(vol, TX, TY, TZ)));         \
+    for (int c = 0; c < ct; c += step) {                                                                             \
+      const Boxes bx = make_boxes(vol, TX, TY, TZ, std::min(step, ct - c));                                          \
+      void* y = mode == 1 ? (void*)(static_cast<unsigned short*>(Y) + 16 * c) : (void*)(static_cast<float*>(Y) + 16 * c); \
+      hipLaunchKernelGGL((KERNEL), dim3(8 * bx.nb8), dim3(256), 0, st, vol, bx, X16, ldx, W16 + 16LL * c * 27 * cin, \
+                         bias ? bias + 16 * c : nullptr, cout - 16 * c, mode, slope, y, ldy, yvec);                  \
+      PC_LAUNCH_CHECK();                                                                                             \
+    }                                                                                                                \
   } while (0)
-#define PC_CONV1(TX, TY, TZ)                                                                                         \
-  do {                                                                                                               \
-    const Boxes bx = make_boxes(vol, TX, TY, TZ, ct);                                                                \
-    hipLaunchKernelGGL((conv_tile1<TX, TY, TZ>), dim3(8 * bx.nb8), dim3(256), 0, st, vol, bx, X16, ldx, W16, bias,   \
-                       cout, mode, slope, Y, ldy, yvec);                                                             \
-  } while (0)
+#define PC_CONV(NCB, TX, TY, TZ) PC_CONV_PARTS((conv_tile<NCB, TX, TY, TZ>), TX, TY, TZ)
+#define PC_CONV1(TX, TY, TZ) PC_CONV_PARTS((conv_tile1<TX, TY, TZ>), TX, TY, TZ)
 #define PC_CONV128(NCB)                \
   do {                                 \
     if (w8) PC_CONV(NCB, 8, 4, 4);     \
@@ -824,6 +826,7 @@ int pc_unet_conv3d_fwd(const void* X, int ldx, int cin, const void* W, const flo
   }
 #undef PC_CONV
 #undef PC_CONV1
+#undef PC_CONV_PARTS
 #undef PC_CONV128
 #undef PC_CONV256
   PC_LAUNCH_CHECK();

@@ -89,3 +89,29 @@ def test_stencil_of_many_vectors(gpu, room):
         step(v0, min(1_000_000, nvec - v0), part[v0:])
     assert torch.equal(out, part)
     dg.close()
+
+
+def test_conv_of_many_output_channels(gpu, room):
+    """128 x 128 x 64 voxels, 64 -> 2^15 + 16 channels: 2^24 workgroups and more;
+    equal to the same weights' channels in calls of their own."""
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    d, h, w, cin, cout = 128, 128, 64, 64, 2 ** 15 + 16
+    print(f"conv of {cout} output channels", flush=True)
+    V = d * h * w
+    room(V * cout * 2)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    X = torch.randn((V, cin), generator=g, device="cuda").to(torch.bfloat16)
+    W = torch.randn((cout, 27, cin), generator=g, device="cuda").to(torch.bfloat16)
+    b = torch.randn(cout, generator=g, device="cuda")
+    Y = torch.empty((V, cout), dtype=torch.bfloat16, device="cuda")
+
+    def conv(c0, n, out):
+        _lib.call("pc_unet_conv3d_fwd", ptr(X), cin, cin, ptr(W[c0:]), ptr(b[c0:]), n, d, h, w, 1, 0.1, ptr(out), n,
+                  stream())
+    conv(0, cout, Y)
+    part = torch.empty((V, 64), dtype=torch.bfloat16, device="cuda")
+    for c0 in (0, 8160, 16352, 24544, cout - 64):
+        conv(c0, 64, part)
+        assert torch.equal(Y[:, c0:c0 + 64], part), c0
