@@ -859,7 +859,6 @@ int pc_unet_conv3d_wgrad(const void* dZ, int ldz, int cout, const void* X, int l
   PC_CHECK_ARG(work_bytes >= kWgradSplitMin * n * sizeof(float), "workspace too small");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const Vol vol = make_vol(D, H, Wd);
-  PC_CHECK_ARG(vol.V < (1LL << 31), "volume too large");
   auto dZ16 = static_cast<const unsigned short*>(dZ);
   auto X16 = static_cast<const unsigned short*>(X);
   float* part = static_cast<float*>(work);

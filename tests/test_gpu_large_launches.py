@@ -115,3 +115,30 @@ def test_conv_of_many_output_channels(gpu, room):
     for c0 in (0, 8160, 16352, 24544, cout - 64):
         conv(c0, 64, part)
         assert torch.equal(Y[:, c0:c0 + 64], part), c0
+
+
+def test_weight_gradient_of_a_large_volume(gpu, room):
+    """2048 x 1024 x 1024 voxels, one channel on either side."""
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    dims = (2048, 1024, 1024)
+    print(f"weight gradient of {dims} voxels", flush=True)
+    room(2 * 2 * 2 ** 31)
+    X, Z = (torch.zeros(dims, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    ref = np.zeros((3, 3, 3))
+    for q, (z, y, x) in enumerate([(0, 0, 0), (1023, 512, 3), (1024, 0, 0), (2047, 1023, 1023)]):
+        Z[z, y, x] = q + 2.0
+        for a in range(3):
+            for b in range(3):
+                for c in range(3):
+                    p = (z + a - 1, y + b - 1, x + c - 1)
+                    if all(0 <= p[i] < dims[i] for i in range(3)):
+                        X[p] = 9.0 * a + 3.0 * b + c + 1.0
+                        ref[a, b, c] += (q + 2.0) * (9.0 * a + 3.0 * b + c + 1.0)
+    n = C.c_size_t()
+    _lib.call("pc_unet_wgrad_workspace", 1, 1, C.byref(n))
+    work = torch.empty(n.value, dtype=torch.uint8, device="cuda")
+    dw = torch.empty((3, 3, 3), device="cuda")
+    _lib.call("pc_unet_conv3d_wgrad", ptr(Z), 1, 1, ptr(X), 1, 1, *dims, ptr(dw), ptr(work), n.value, stream())
+    assert np.array_equal(dw.cpu().numpy(), ref)
