@@ -903,9 +903,10 @@ int pc_unet_act_bwd(const float* dA, int lda, const void* a, int lda_a, int C, i
   const long long V = (long long)D * H * Wd;
   PC_CHECK_ARG(work_bytes >= (size_t)((V + kActChunkMax - 1) / kActChunkMax) * C * sizeof(float), "workspace too small");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // the smallest chunk of at least kActChunk voxels whose partial sums fit
+  // the smallest chunk of at least kActChunk voxels whose partial sums fit and whose workgroups one launch holds
   long long chunk = kActChunk;
-  while ((size_t)((V + chunk - 1) / chunk) * C * sizeof(float) > work_bytes) chunk *= 2;
+  while ((size_t)((V + chunk - 1) / chunk) * C * sizeof(float) > work_bytes || (V + chunk - 1) / chunk > pc::kMaxGrid)
+    chunk *= 2;
   const int nb = (int)((V + chunk - 1) / chunk);
   float* part = static_cast<float*>(work);
   auto a16 = static_cast<const unsigned short*>(a);

@@ -142,3 +142,26 @@ def test_weight_gradient_of_a_large_volume(gpu, room):
     dw = torch.empty((3, 3, 3), device="cuda")
     _lib.call("pc_unet_conv3d_wgrad", ptr(Z), 1, 1, ptr(X), 1, 1, *dims, ptr(dw), ptr(work), n.value, stream())
     assert np.array_equal(dw.cpu().numpy(), ref)
+
+
+def test_activation_backward_of_a_large_volume(gpu, room):
+    """2048^3 voxels of one channel: 2^24 chunks of 512."""
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    n = 2048
+    print("activation backward of 2048^3 voxels", flush=True)
+    room(6 * n ** 3)
+    dA = torch.zeros(n ** 3, device="cuda")
+    dZ = torch.full((n ** 3,), 7.0, dtype=torch.bfloat16, device="cuda")
+    at = torch.tensor([0, 511, 2 ** 32 - 1, 2 ** 32, n ** 3 - 1], device="cuda")
+    dA[at] = torch.tensor([1.0, -2.0, 4.0, 8.0, 16.0], device="cuda")
+    nb = C.c_size_t()
+    _lib.call("pc_unet_act_bwd_workspace", 1, n ** 3, C.byref(nb))
+    work = torch.empty(nb.value, dtype=torch.uint8, device="cuda")
+    db = torch.empty(1, device="cuda")
+    _lib.call("pc_unet_act_bwd", ptr(dA), 1, None, 1, 1, n, n, n, 0.1, ptr(dZ), 1, ptr(db), ptr(work), nb.value,
+              stream())
+    assert db.item() == 27.0
+    assert dZ[at].tolist() == [1.0, -2.0, 4.0, 8.0, 16.0]
+    assert int(torch.count_nonzero(dZ)) == 5
