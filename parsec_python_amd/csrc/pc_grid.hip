@@ -45,6 +45,7 @@ struct GridDev {
   double w[8];   // 1D -d2/dx2 weights, centre first (unscaled)
   int4* win;     // stencil_win: windows {first row, first column | columns << 16 | left halo lanes << 28, zb, ze}
   int nwin, winz;  // their number and mean number of planes
+  int winsx;       // wavefronts of 64 columns per row of a window
   int2* pmeta;   // its padded row table {offset, lo | length << 16}, nyp x nzp
   int nyp, nzp;
 };
@@ -343,10 +344,11 @@ __global__ __launch_bounds__(64 * NW) void stencil_zmarch(StArgs g, const T* __r
 
 
 // ---- the windowed z-march (one vector per workgroup, no partial sums) ---------
-// A workgroup owns one vector and one window of a slab of win_ty(R) y-rows, one
-// wavefront of 64 columns per row.  A window is all the columns that the slab's
-// rows touch, where these are at most 64 (the columns beyond are zero); else a
-// part of them, with R columns of each neighbouring window among its 64 lanes.
+// A workgroup owns one vector and one window of a slab of win_ty(R, SX) y-rows, one
+// wavefront of 64 columns (SX = 1) or two (SX = 2) per row.  A window is all the
+// columns that the slab's rows touch, where these are at most 64 SX (the columns
+// beyond are zero); else a part of them, with R columns of each neighbouring window
+// among its lanes.
 // The host lists the windows with the planes they touch.  The march along z:
 //   * the z-queue is a ring of QL registers per lane, indexed by the plane's
 //     phase; the plane loop is unrolled QL times so the ring turns by renaming
@@ -380,6 +382,10 @@ __global__ __launch_bounds__(64 * NW) void stencil_zmarch(StArgs g, const T* __r
 //   radius 6 (FD12), 103 columns:   256 vectors FP32 1310 -> 1165 us,
 //                                   64 vectors FP64 640 -> 551 us
 //   70^3 cube, 40 vectors:          radius 3 FP32 49 -> 48, radius 2 FP64 87.5 -> 80.5 us
+//   52^3 cube, 150 vectors:         radius 1 FP32 52 -> 48, radius 2 FP64 138 -> 126 us
+//                                   (55 and 147 us with 8 rows per workgroup)
+//   128^3 cube, 23 vectors (SX 2):  radius 4 FP32 144 -> 156, FP64 291 -> 280 us (174
+//                                   and 341 us as three windows), radius 6 FP64 338 -> 298
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t pc_rsrc(const void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
@@ -402,12 +408,14 @@ __device__ __forceinline__ void pc_bstore(__amdgpu_buffer_rsrc_t r, int off, int
 }
 
 // rows (wavefronts) per workgroup: one halo row per wavefront from radius 4 on
-constexpr int win_ty(int R) { return R <= 4 ? 8 : 2 * R; }
-constexpr int kWinNS = 2;    // register sets of X, V and halo values in flight
+// (radius 1 and 2: half of that, their plane is short against its barrier); two
+// wavefronts per row (SX = 2): 16 wavefronts at most
+constexpr int win_ty(int R, int SX) { return SX == 2 ? (R == 1 ? 4 : 8) : R <= 2 ? 4 : R <= 4 ? 8 : 2 * R; }
+constexpr int win_ns(int R) { return R == 1 ? 3 : 2; }    // register sets of X, V and halo values in flight
 // queue length: 2R+1 planes plus 3 fronts in flight, rounded up to a multiple of
-// 2 kWinNS (tile parity and register sets repeat within the block)
-constexpr int win_ql(int R) { return (2 * R + 1 + 3 + 2 * kWinNS - 1) / (2 * kWinNS) * (2 * kWinNS); }
-constexpr int kWinPadY = 24;  // empty rows around the padded row table (>= win_ty(R) + R) ...
+// 2 win_ns (tile parity and register sets repeat within the block)
+constexpr int win_ql(int R) { return (2 * R + 1 + 3 + 2 * win_ns(R) - 1) / (2 * win_ns(R)) * (2 * win_ns(R)); }
+constexpr int kWinPadY = 24;  // empty rows around the padded row table (>= win_ty(R, SX) + R) ...
 constexpr int kWinPadZ = 64;  // ... and planes above (>= 2 win_ql(R)); R planes below
 
 struct WinArgs {
@@ -420,14 +428,17 @@ struct WinArgs {
   double w[8];         // scaled weights; w[0] already includes the factor 3
 };
 
-template <typename T, int R, bool HASX>
-__global__ __launch_bounds__(64 * win_ty(R)) void stencil_win(WinArgs g, const T* Y, const T* X, T* Out, const T* V, T ca,
-                                                          T cb, T cc) {
-  constexpr int TY = win_ty(R), NS = kWinNS, QL = win_ql(R);
+// (two workgroups of 16 wavefronts per CU in FP32: 64 registers at radius 4, which has 65 otherwise)
+constexpr int win_occ(int bytes, int R, int SX) { return SX == 2 && bytes == 4 && R <= 4 ? 8 : 1; }
+
+template <typename T, int R, bool HASX, int SX>
+__global__ __launch_bounds__(64 * SX * win_ty(R, SX), win_occ(sizeof(T), R, SX))
+void stencil_win(WinArgs g, const T* Y, const T* X, T* Out, const T* V, T ca, T cb, T cc) {
+  constexpr int TY = win_ty(R, SX), NS = win_ns(R), QL = win_ql(R);
   constexpr int LR = TY + 2 * R;
   constexpr int HT = (2 * R + TY - 1) / TY;   // halo rows per wavefront
   constexpr int ES = (int)sizeof(T);
-  constexpr int LW = 64 + 2 * R;         // R zero columns either side
+  constexpr int LW = 64 * SX + 2 * R;    // R zero columns either side
   // row LR takes what wavefronts without a halo row write
   __shared__ T tile[2][(LR + 1) * LW];
   const int L = (blockIdx.x & 7) * g.nb8 + (blockIdx.x >> 3);
@@ -439,18 +450,20 @@ __global__ __launch_bounds__(64 * win_ty(R)) void stencil_win(WinArgs g, const T
   const int zb = win.z + zci * g.zc, ze = min(win.w, zb + g.zc);
   if (zb >= ze) return;
   const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wv = SX == 2 ? wave >> 1 : wave;                      // row of the slab
+  const int col = SX == 2 ? lane + 64 * (wave & 1) : lane;        // column of the window
   const long long base = (long long)v * g.ld;
   const T* __restrict__ yv = Y + base;
   const T* xv = HASX ? X + base : Y + base;
   T* ov = Out + base;
   // win.y: first column | columns << 16 | halo lanes << 28
   const int halo = win.y >> 28, width = win.y >> 16 & 0xfff;
-  const int lx = ((win.y & 0xffff) - halo + lane) * ES;                         // loads of Y
-  const int lo_ = lane >= halo && lane < halo + width ? lx : 0x40000000;        // X, V and the store: the window's columns
-  for (int e = threadIdx.x; e < 2 * (LR + 1) * 2 * R; e += 64 * TY) {
+  const int lx = ((win.y & 0xffff) - halo + col) * ES;                         // loads of Y
+  const int lo_ = col >= halo && col < halo + width ? lx : 0x40000000;          // X, V and the store: the window's columns
+  for (int e = threadIdx.x; e < 2 * (LR + 1) * 2 * R; e += 64 * SX * TY) {
     const int row = e / (2 * R), c = e % (2 * R);
-    (&tile[0][0])[row * LW + (c < R ? c : 64 + c)] = T(0);
+    (&tile[0][0])[row * LW + (c < R ? c : 64 * SX + c)] = T(0);
   }
 
   // row metadata: lane l holds plane wb + l
@@ -518,11 +531,11 @@ __global__ __launch_bounds__(64 * win_ty(R)) void stencil_win(WinArgs g, const T
     issue_plane(std::integral_constant<int, (P + NS - 1) % NS>{}, z + NS - 1);
     __builtin_amdgcn_sched_barrier(0);
     T* tb = &tile[B][R];
-    tb[(wv + R) * LW + lane] = q[(P + R) % QL];
+    tb[(wv + R) * LW + col] = q[(P + R) % QL];
 #pragma unroll
-    for (int u = 0; u < HT; ++u) tb[th[u] * LW + lane] = hq[S][u];
+    for (int u = 0; u < HT; ++u) tb[th[u] * LW + col] = hq[S][u];
     lds_barrier();
-    const T* trow = tb + (wv + R) * LW + lane;
+    const T* trow = tb + (wv + R) * LW + col;
     const T yc = q[(P + R) % QL];
     T acc = w0 * yc;
 #pragma unroll
@@ -551,17 +564,17 @@ __global__ __launch_bounds__(64 * win_ty(R)) void stencil_win(WinArgs g, const T
 }
 
 // z-chunks: a window's z-range is split where that fills the chip's rounds better.
-// A round is the workgroups that run at once (4 per CU in FP32, 2 in FP64 where
-// the registers or the bandwidth allow no more, half of that with the 12
-// wavefronts of radius 6); a chunk costs its planes and about 2R + 8 more for its
+// A round is the workgroups that run at once (32 wavefronts per CU in FP32, 16 in
+// FP64 where the registers or the bandwidth allow no more; the 12 wavefronts of
+// radius 6 count as 16); a chunk costs its planes and about 2R + 8 more for its
 // start (the queue's planes, the first loads), so the number of chunks with the
 // fewest rounds x (planes + start) is taken, at least 8 planes per chunk.  Against
 // filling 16,384 wavefronts whatever the rounds: 58^3 cube, 79 vectors, FP64 102 ->
 // 81 us; 62^3, radius 6, 20 vectors, FP64 59 -> 29; 52^3, 23 vectors, FP64 24.5 ->
 // 22.2; against one chunk: C10H8, 49 vectors, FP32 85 -> 81, FP64 186 -> 175 us.
-template <typename T, int R>
+template <typename T, int R, int SX>
 void win_zchunks(WinArgs& a, int nz, int planes, int nvec) {
-  constexpr long long kRound = 256 * (sizeof(T) == 4 ? 4 : 2) / (R > 4 ? 2 : 1);
+  constexpr long long kRound = 256 * (sizeof(T) == 4 ? 32 : 16) / (SX * (R > 4 ? 16 / SX : win_ty(R, SX)));
   const long long wgs = (long long)a.nwin * nvec;
   int best = 1;
   double least = 0.0;
@@ -576,7 +589,7 @@ void win_zchunks(WinArgs& a, int nz, int planes, int nvec) {
   a.nzc = (nz + a.zc - 1) / a.zc;
 }
 
-template <typename T, int R>
+template <typename T, int R, int SX>
 int launch_win(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, int nvec, long long ld, double scale,
                double ca, double cb, double cc, hipStream_t st) {
   WinArgs a;
@@ -585,7 +598,7 @@ int launch_win(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, in
   if (a.nwin == 0) return pc::PC_OK;   // no points
   a.meta = gd->pmeta; a.nyp = gd->nyp; a.nzp = gd->nzp;
   a.ld = ld;
-  win_zchunks<T, R>(a, gd->nz, gd->winz, nvec);
+  win_zchunks<T, R, SX>(a, gd->nz, gd->winz, nvec);
   for (int d = 0; d < 8; ++d) a.w[d] = 0.0;
   a.w[0] = 3.0 * gd->w[0] * scale;
   for (int d = 1; d <= R; ++d) a.w[d] = gd->w[d] * scale;
@@ -594,12 +607,12 @@ int launch_win(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, in
     const long long at = (long long)v0 * ld;
     a.nblocks = per * std::min(step, nvec - v0);
     a.nb8 = (a.nblocks + 7) / 8;
-    const dim3 grid(8 * a.nb8), block(64 * win_ty(R));
+    const dim3 grid(8 * a.nb8), block(64 * SX * win_ty(R, SX));
     if (X)
-      hipLaunchKernelGGL((stencil_win<T, R, true>), grid, block, 0, st, a, Y + at, X + at, Out + at, V, T(ca), T(cb),
+      hipLaunchKernelGGL((stencil_win<T, R, true, SX>), grid, block, 0, st, a, Y + at, X + at, Out + at, V, T(ca), T(cb),
                          T(cc));
     else
-      hipLaunchKernelGGL((stencil_win<T, R, false>), grid, block, 0, st, a, Y + at, X, Out + at, V, T(ca), T(cb),
+      hipLaunchKernelGGL((stencil_win<T, R, false, SX>), grid, block, 0, st, a, Y + at, X, Out + at, V, T(ca), T(cb),
                          T(cc));
     PC_LAUNCH_CHECK();
   }
@@ -636,7 +649,8 @@ int launch_dot(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, in
 template <typename T, int R>
 int launch_r(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, int nvec, long long ld, double scale,
              double ca, double cb, double cc, double* dot_part, hipStream_t st) {
-  if (!dot_part) return launch_win<T, R>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, st);
+  if (!dot_part && gd->winsx == 2) return launch_win<T, R, 2>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, st);
+  if (!dot_part) return launch_win<T, R, 1>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, st);
   if (gd->nx <= 64) return launch_dot<T, R, 1>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
   if (gd->nx <= 128) return launch_dot<T, R, 2>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
   return launch_dot<T, R, 4>(gd, Y, X, Out, V, nvec, ld, scale, ca, cb, cc, dot_part, st);
@@ -924,34 +938,55 @@ int pc_grid_create(int nx, int ny, int nz, const int* row_lo, const int* row_hi,
   GridDev* g = new GridDev();
   g->nx = nx; g->ny = ny; g->nz = nz; g->npts = cnt; g->radius = radius;
   // stencil_win: per slab of rows the columns they touch, as one window of up to
-  // 64 or as windows of equal lane counts (an inner edge has radius halo lanes,
-  // an outer one none), with the planes they touch
-  std::vector<int4> win;
-  const int ty = win_ty(radius);
-  for (int j0 = 0; j0 < ny; j0 += ty) {
-    int xl = nx, xh = 0;
-    const int j1 = std::min(ny, j0 + ty);
-    for (int j = j0; j < j1; ++j)
-      for (int k = zr[2 * j]; k < zr[2 * j + 1]; ++k)
-        if (hi[j + ny * k] > lo[j + ny * k]) {
-          xl = std::min(xl, lo[j + ny * k]);
-          xh = std::max(xh, hi[j + ny * k]);
-        }
-    if (xl >= xh) continue;
-    int n = 1;
-    while (xh - xl + 2 * radius * (n - 1) > 64 * n) ++n;
-    const int lanes = xh - xl + 2 * radius * (n - 1);
-    auto cut = [&](int i) { return i == 0 ? xl : i == n ? xh : xl + lanes * i / n - radius * (2 * i - 1); };
-    for (int i = 0; i < n; ++i) {
-      const int x0 = cut(i), x1 = cut(i + 1);
-      int zb = nz, ze = 0;
+  // 64 sx or as windows of equal lane counts (an inner edge has radius halo lanes,
+  // an outer one none), with the planes they touch; lanes: those of all planes
+  auto windows = [&](int sx, std::vector<int4>& win) {
+    long long lanes_all = 0;
+    const int ty = win_ty(radius, sx), lw = 64 * sx;
+    for (int j0 = 0; j0 < ny; j0 += ty) {
+      int xl = nx, xh = 0;
+      const int j1 = std::min(ny, j0 + ty);
       for (int j = j0; j < j1; ++j)
         for (int k = zr[2 * j]; k < zr[2 * j + 1]; ++k)
-          if (std::max(lo[j + ny * k], x0) < std::min(hi[j + ny * k], x1)) {
-            zb = std::min(zb, k);
-            ze = std::max(ze, k + 1);
+          if (hi[j + ny * k] > lo[j + ny * k]) {
+            xl = std::min(xl, lo[j + ny * k]);
+            xh = std::max(xh, hi[j + ny * k]);
           }
-      if (zb < ze) win.push_back(make_int4(j0, x0 | ((x1 - x0) << 16) | ((i ? radius : 0) << 28), zb, ze));
+      if (xl >= xh) continue;
+      int n = 1;
+      while (xh - xl + 2 * radius * (n - 1) > lw * n) ++n;
+      const int lanes = xh - xl + 2 * radius * (n - 1);
+      auto cut = [&](int i) { return i == 0 ? xl : i == n ? xh : xl + lanes * i / n - radius * (2 * i - 1); };
+      for (int i = 0; i < n; ++i) {
+        const int x0 = cut(i), x1 = cut(i + 1);
+        int zb = nz, ze = 0;
+        for (int j = j0; j < j1; ++j)
+          for (int k = zr[2 * j]; k < zr[2 * j + 1]; ++k)
+            if (std::max(lo[j + ny * k], x0) < std::min(hi[j + ny * k], x1)) {
+              zb = std::min(zb, k);
+              ze = std::max(ze, k + 1);
+            }
+        if (zb >= ze) continue;
+        win.push_back(make_int4(j0, x0 | ((x1 - x0) << 16) | ((i ? radius : 0) << 28), zb, ze));
+        lanes_all += (long long)(ze - zb) * lw * ty;
+      }
+    }
+    return lanes_all;
+  };
+  std::vector<int4> win, win2;
+  g->winsx = 1;
+  const long long lanes1 = windows(1, win);
+  // Two wavefronts per row share one tile, so a row of up to 128 columns has no
+  // inner edges: taken where that saves a fifth of the lanes (121 to 128 full
+  // columns at radius 4, which are three windows otherwise: 128^3, 23 vectors,
+  // FP64 341 -> 280 us, radius 6 361 -> 298), at radius 1 where it costs none
+  // (126^3, 49 vectors FP32 289 -> 263).  With two windows either way one wavefront
+  // per row is the faster (100^3 FP32 radius 4 11 %, spheres 20 to 40 %).
+  if (nx > 64 && nx <= 128) {
+    const long long lanes2 = windows(2, win2);
+    if (radius == 1 ? lanes2 <= lanes1 : 5 * lanes2 <= 4 * lanes1) {
+      g->winsx = 2;
+      win.swap(win2);
     }
   }
   // the longest first: what runs last is short
