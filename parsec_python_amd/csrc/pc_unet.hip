@@ -353,7 +353,8 @@ __global__ void conv_wflip(const unsigned short* __restrict__ W, int cout, int c
 // share their reads (funnel shifts).  dW_part[s][co][t][ci].  Bound by LDS reads
 // and the transposing staging; 64^3 volume, 48 x 16 channels: 47 us (611 us
 // with 2-byte gathers from global memory per tap).
-template <int TX, int TY, int TZ, bool ZVEC, bool XVEC>   // 16-byte aligned channels, a multiple of 16
+// RAGGED: boxes may reach beyond the volume.
+template <int TX, int TY, int TZ, bool ZVEC, bool XVEC, bool RAGGED>   // VEC: 16-byte aligned channels, a multiple of 16
 __global__ __launch_bounds__(384) void conv_wgrad(Vol vol, Boxes bx, const unsigned short* __restrict__ dZ, int ldz,
                                                   int cout, const unsigned short* __restrict__ X, int ldx, int cin,
                                                   int nsplit, float* __restrict__ part) {
@@ -364,6 +365,8 @@ __global__ __launch_bounds__(384) void conv_wgrad(Vol vol, Boxes bx, const unsig
   constexpr int CZ = (TZ * TY * TX + 107) / 128 * 128 + 20;
   constexpr int RPK = 32 / TX;                    // rows per group of 32 voxels
   constexpr int NG = TX * TY * TZ / 32;           // groups per box
+  constexpr int ZERO = HZ * HY * RS + 4;          // zeros in the first channel's padding
+  static_assert(ZERO + 12 <= CX && ZERO % 4 == 0, "no room for the zeros");
   __shared__ __align__(16) unsigned short xs[16 * CX], zs[16 * CZ];
   const int co0 = blockIdx.x * 16, ci0 = blockIdx.y * 16;
   const int s = blockIdx.z;
@@ -427,6 +430,7 @@ __global__ __launch_bounds__(384) void conv_wgrad(Vol vol, Boxes bx, const unsig
       fetch(std::integral_constant<bool, ZVEC>{}, dZ, ldz, cout, co0, threadIdx.x + 384 * u, ZU, ZG, TY, 0, x0, y0, z0,
             tz[u], mz[u]);
   };
+  if (RAGGED && threadIdx.x < 16) xs[ZERO - 4 + threadIdx.x] = 0;
   fetch_box(s);
   for (int box = s; box < nbox; box += nsplit) {
     __syncthreads();
@@ -438,40 +442,38 @@ __global__ __launch_bounds__(384) void conv_wgrad(Vol vol, Boxes bx, const unsig
       if ((int)threadIdx.x + 384 * u < ZU) put(tz[u], mz[u], zs, CZ, TX, ZG, threadIdx.x + 384 * u);
     __syncthreads();
     if (box + nsplit < nbox) fetch_box(box + nsplit);   // in flight during the products
+    // A voxel just beyond the volume has gradient zero, but its tap towards the
+    // volume reads an activation, and 0 times an infinite one would be a NaN: planes
+    // beyond the volume are left out, rows beyond it read zeros in the first y-tap,
+    // and such a voxel of a row is zeroed in the first x-tap.
     const int x0 = box % bx.nx * TX, y0 = box / bx.nx % bx.ny * TY, z0 = box / (bx.nx * bx.ny) * TZ;
-    const bool edge = x0 + TX > vol.W || y0 + TY > vol.H || z0 + TZ > vol.D;
+    const int ng = RAGGED ? min(NG, (vol.D - z0) * (TY / RPK)) : NG;
+    u32x4 first = {~0u, ~0u, ~0u, ~0u};
+    if constexpr (RAGGED) {
+      const int j = vol.W - x0 - (TX == 16 ? 8 * (lk & 1) : 0);   // that voxel among this lane's 8
+#pragma unroll
+      for (int w = 0; w < 4; ++w) first[w] = j == 2 * w ? 0xffff0000u : j == 2 * w + 1 ? 0xffffu : ~0u;
+    }
 #pragma unroll 2
-    for (int g = kh; g < NG; g += 2) {
+    for (int g = kh; g < ng; g += 2) {
       const int row = g * RPK + (TX == 16 ? lk >> 1 : lk);        // this lane's row of the box
       const int xh = TX == 16 ? 8 * (lk & 1) : 0;
       const int y = row % TY, z = row / TY;
       const u32x2* za = reinterpret_cast<const u32x2*>(&zs[ln * CZ + row * TX + xh]);
       const u32x2 z0v = za[0], z1v = za[1];
       const u32x4 a = {z0v[0], z0v[1], z1v[0], z1v[1]};
-      // this lane's voxels in the volume: X's side of the others is zeroed as dZ's
-      // is (0 times an infinite value would be a NaN)
-      const int nv = y0 + y < vol.H && z0 + z < vol.D ? vol.W - x0 - xh : 0;
 #pragma unroll
       for (int dy = 0; dy < 3; ++dy) {
         const unsigned short* xr = &xs[ln * CX + ((z + dz) * HY + y + dy) * RS + 4 + xh];
+        if (RAGGED && dy == 0) xr = y0 + y >= vol.H ? &xs[ZERO] : xr;
         const unsigned wm = *reinterpret_cast<const unsigned*>(xr - 2), wp = *reinterpret_cast<const unsigned*>(xr + 8);
         const u32x2 wa = *reinterpret_cast<const u32x2*>(xr), wb = *reinterpret_cast<const u32x2*>(xr + 4);
         const unsigned s0 = __builtin_amdgcn_alignbit(wa[0], wm, 16), s1 = __builtin_amdgcn_alignbit(wa[1], wa[0], 16);
         const unsigned s2 = __builtin_amdgcn_alignbit(wb[0], wa[1], 16), s3 = __builtin_amdgcn_alignbit(wb[1], wb[0], 16);
         const unsigned s4 = __builtin_amdgcn_alignbit(wp, wb[1], 16);
-        u32x4 b0 = {s0, s1, s2, s3}, b1 = {wa[0], wa[1], wb[0], wb[1]}, b2 = {s1, s2, s3, s4};
-        if (edge) {
-#pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            const unsigned in = nv >= 2 * w + 2 ? ~0u : nv == 2 * w + 1 ? 0xffffu : 0u;
-            b0[w] &= in;
-            b1[w] &= in;
-            b2[w] &= in;
-          }
-        }
-        acc[3 * dy] = mfma32(a, b0, acc[3 * dy]);
-        acc[3 * dy + 1] = mfma32(a, b1, acc[3 * dy + 1]);
-        acc[3 * dy + 2] = mfma32(a, b2, acc[3 * dy + 2]);
+        acc[3 * dy] = mfma32(a, u32x4{s0, s1, s2, s3} & first, acc[3 * dy]);
+        acc[3 * dy + 1] = mfma32(a, u32x4{wa[0], wa[1], wb[0], wb[1]}, acc[3 * dy + 1]);
+        acc[3 * dy + 2] = mfma32(a, u32x4{s1, s2, s3, s4}, acc[3 * dy + 2]);
       }
     }
   }
@@ -869,18 +871,24 @@ int pc_unet_conv3d_wgrad(const void* dZ, int ldz, int cout, const void* X, int l
   const int room = (int)std::min<long long>(kWgradSplit, (long long)(work_bytes / sizeof(float)) / n);
   const int nsplit = std::min(room, bx.nblocks);
   dim3 grid((cout + 15) / 16, (cin + 15) / 16, nsplit);
-#define PC_WGRAD(TX, ZV, XV)                                                                                     \
-  hipLaunchKernelGGL((conv_wgrad<TX, 8, 4, ZV, XV>), grid, dim3(384), 0, st, vol, bx, dZ16, ldz, cout, X16, ldx, \
+  const bool ragged = Wd % (w8 ? 8 : 16) != 0 || H % 8 != 0 || D % 4 != 0;
+#define PC_WGRAD(TX, ZV, XV, RG)                                                                                     \
+  hipLaunchKernelGGL((conv_wgrad<TX, 8, 4, ZV, XV, RG>), grid, dim3(384), 0, st, vol, bx, dZ16, ldz, cout, X16, ldx, \
                      cin, nsplit, part)
-#define PC_WGRAD_V(TX)                                 \
+#define PC_WGRAD_V(TX, RG)                             \
   do {                                                 \
-    if (zvec && xvec) PC_WGRAD(TX, true, true);        \
-    else if (zvec) PC_WGRAD(TX, true, false);          \
-    else if (xvec) PC_WGRAD(TX, false, true);          \
-    else PC_WGRAD(TX, false, false);                   \
+    if (zvec && xvec) PC_WGRAD(TX, true, true, RG);    \
+    else if (zvec) PC_WGRAD(TX, true, false, RG);      \
+    else if (xvec) PC_WGRAD(TX, false, true, RG);      \
+    else PC_WGRAD(TX, false, false, RG);               \
   } while (0)
-  if (w8) PC_WGRAD_V(8);
-  else PC_WGRAD_V(16);
+  if (w8) {
+    if (ragged) PC_WGRAD_V(8, true);
+    else PC_WGRAD_V(8, false);
+  } else {
+    if (ragged) PC_WGRAD_V(16, true);
+    else PC_WGRAD_V(16, false);
+  }
 #undef PC_WGRAD
 #undef PC_WGRAD_V
   PC_LAUNCH_CHECK();
