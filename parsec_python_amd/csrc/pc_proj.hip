@@ -32,75 +32,86 @@ struct ProjDev {
   double* se_u;    // [3*nent] scale[atom] * u of the t-th entry in point order
 };
 
-// C[a][v][m] = sum_e u_m[e] * Y[v][pt[e]] (FP64 accumulation).  Workgroup = one
-// atom x 4 vectors: the entry tables are read once for the 4.  Its wavefronts take
-// the atom's entries in rounds of 64 (wavefront w the rounds w, w + 4, ...), kGE
-// rounds loaded together, and their sums are added in order.
+// C[a][v][m] = sum_e u_m[e] * Y[v][pt[e]] (FP64 accumulation).  GW wavefronts take
+// one atom and 4 vectors, so the entry tables are read once for the 4: the atom's
+// entries in rounds of 64 (wavefront w the rounds w, w + GW, ...), up to kGE rounds
+// loaded together, their sums added in order.  A workgroup holds kGW / GW atoms.
 // Small blocks are bound by the chain of dependent loads (the atom's range, its
 // points, their values), large ones by the 128-byte lines that a support's short
 // rows touch (5.6 points of 32 in FP32).  One wavefront per atom and 4
 // vectors, round after round, atoms spread over the XCDs -> now: 3 atoms x 23
 // vectors FP64 9.6 -> 4.4 us, 18 x 49 FP32 10.3 -> 5.0, 163 x 275 FP32 78 -> 61
-// (83 without the XCD order, 65 with 8 vectors).
-constexpr int kGV = 4;   // vectors per workgroup in the gather
-constexpr int kGE = 3;   // rounds in flight: an atom's support is some 250 to 750 points
-constexpr int kGW = 4;   // wavefronts
-template <typename T>
+// (83 without the XCD order, 65 with 8 vectors), 1,500 atoms of 20 points x 275
+// FP32 157 -> 75 (222 with four wavefronts, each loading three rounds at any size).
+constexpr int kGV = 4;   // vectors per wavefront in the gather
+constexpr int kGE = 3;   // rounds in flight
+constexpr int kGW = 4;   // wavefronts per workgroup
+template <typename T, int GW>   // GW wavefronts per atom
 __global__ __launch_bounds__(64 * kGW) void proj_gather(ProjDev P, const T* __restrict__ Y, long long ld, int nvec,
                                                         double* __restrict__ C) {
+  constexpr int NA = kGW / GW;   // atoms per workgroup
   __shared__ double part[kGW][kGV * 3];
   // the atoms of one vector group follow each other on one XCD: atoms share lines
-  const int nb = P.natoms * ((nvec + kGV - 1) / kGV), L = (blockIdx.x & 7) * ((nb + 7) / 8) + (blockIdx.x >> 3);
+  const int na = (P.natoms + NA - 1) / NA;
+  const int nb = na * ((nvec + kGV - 1) / kGV), L = (blockIdx.x & 7) * ((nb + 7) / 8) + (blockIdx.x >> 3);
   if (L >= nb) return;
-  const int a = L % P.natoms, v0 = L / P.natoms * kGV;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wv = wave % GW, v0 = L / na * kGV, a0 = L % na * NA, a = a0 + wave / GW;
   double s[kGV][3];
 #pragma unroll
   for (int u = 0; u < kGV; ++u) s[u][0] = s[u][1] = s[u][2] = 0.0;
-  const int e0 = P.atom_ptr[a], e1 = P.atom_ptr[a + 1];
+  const int e0 = a < P.natoms ? P.atom_ptr[a] : 0, e1 = a < P.natoms ? P.atom_ptr[a + 1] : 0;
   const T* yv[kGV];
 #pragma unroll
   for (int u = 0; u < kGV; ++u) yv[u] = Y + (long long)min(v0 + u, nvec - 1) * ld;
-  for (int eb = e0 + 64 * wv + lane; eb - lane < e1; eb += 64 * kGW * kGE) {
-    int pt[kGE];
-    double w[kGE][3];
-    T y[kGE][kGV];
+  // N rounds from entry eb on, of which only the last may be short: lanes past its
+  // end take the last entry, with zeros (0 times an infinite value would be a NaN)
+  auto rounds = [&](auto n, int eb) {
+    constexpr int N = decltype(n)::value;
+    int pt[N];
+    double w[N][3];
+    T y[N][kGV];
+    const bool in = eb + 64 * GW * (N - 1) + lane < e1;
 #pragma unroll
-    for (int k = 0; k < kGE; ++k) {
-      const int e = min(eb + 64 * kGW * k, e1 - 1);   // past the end: the last entry, its product replaced by 0 * 0
-      pt[k] = P.ent_pt[e];
+    for (int k = 0; k < N; ++k) {
+      const int e = eb + 64 * GW * k + lane, ec = k == N - 1 ? min(e, e1 - 1) : e;
+      pt[k] = P.ent_pt[ec];
 #pragma unroll
-      for (int m = 0; m < 3; ++m) w[k][m] = P.ent_u[3 * (long long)e + m];
+      for (int m = 0; m < 3; ++m) w[k][m] = P.ent_u[3 * (long long)ec + m];
     }
 #pragma unroll
-    for (int k = 0; k < kGE; ++k)
+    for (int k = 0; k < N; ++k)
 #pragma unroll
       for (int u = 0; u < kGV; ++u) y[k][u] = yv[u][pt[k]];
+    __builtin_amdgcn_sched_barrier(0);   // every load first
 #pragma unroll
-    for (int k = 0; k < kGE; ++k) {
-      const bool in = eb + 64 * kGW * k < e1;
+    for (int k = 0; k < N; ++k)
 #pragma unroll
       for (int u = 0; u < kGV; ++u) {
-        const double yu = in ? y[k][u] : T(0);   // (0 times an infinite value would be a NaN)
+        const double yu = k == N - 1 && !in ? T(0) : y[k][u];
 #pragma unroll
-        for (int m = 0; m < 3; ++m) s[u][m] += (in ? w[k][m] : 0.0) * yu;
+        for (int m = 0; m < 3; ++m) s[u][m] += (k == N - 1 && !in ? 0.0 : w[k][m]) * yu;
       }
-    }
+  };
+  for (int eb = e0 + 64 * wv; eb < e1; eb += 64 * GW * kGE) {
+    if (eb + 64 * GW * 2 < e1) rounds(std::integral_constant<int, 3>{}, eb);
+    else if (eb + 64 * GW < e1) rounds(std::integral_constant<int, 2>{}, eb);
+    else rounds(std::integral_constant<int, 1>{}, eb);
   }
 #pragma unroll
   for (int u = 0; u < kGV; ++u)
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
       const double t = pc_wave_sum(s[u][m]);
-      if (lane == 0) part[wv][3 * u + m] = t;
+      if (lane == 0) part[wave][3 * u + m] = t;
     }
   __syncthreads();
-  const int t = threadIdx.x;
-  if (t < kGV * 3 && v0 + t / 3 < nvec) {
-    double c = part[0][t];
+  const int t = threadIdx.x % (kGV * 3), q = threadIdx.x / (kGV * 3);
+  if (q < NA && a0 + q < P.natoms && v0 + t / 3 < nvec) {
+    double c = part[q * GW][t];
 #pragma unroll
-    for (int k = 1; k < kGW; ++k) c += part[k][t];
-    C[((long long)a * nvec + v0) * 3 + t] = c;
+    for (int k = 1; k < GW; ++k) c += part[q * GW + k][t];
+    C[((long long)(a0 + q) * nvec + v0) * 3 + t] = c;
   }
 }
 
@@ -147,17 +158,28 @@ int gather_impl(void* proj, const T* Y, long long ld, int nvec, double* C, void*
   PC_CHECK_ARG(P && Y && C, "null pointer");
   if (P->natoms == 0 || nvec == 0) return pc::PC_OK;
   const long long groups = (nvec + kGV - 1) / kGV;
-  const int step = (int)std::max<long long>(1, pc::kMaxGrid / groups);   // atoms per launch
-  for (int a0 = 0; a0 < P->natoms; a0 += step) {
-    ProjDev part = *P;
-    part.atom_ptr += a0;
-    part.natoms = std::min(step, P->natoms - a0);
-    const dim3 grid((unsigned)((part.natoms * groups + 7) / 8 * 8));
-    hipLaunchKernelGGL(proj_gather<T>, grid, dim3(64 * kGW), 0, static_cast<hipStream_t>(stream), part, Y, ld, nvec,
-                       C + (long long)a0 * nvec * 3);
-    PC_LAUNCH_CHECK();
-  }
-  return pc::PC_OK;
+  auto launch = [&](auto gw) -> int {
+    constexpr int GW = decltype(gw)::value, NA = kGW / GW;
+    const int step = (int)std::max<long long>(1, pc::kMaxGrid / groups) * NA;   // atoms per launch
+    for (int a0 = 0; a0 < P->natoms; a0 += step) {
+      ProjDev part = *P;
+      part.atom_ptr += a0;
+      part.natoms = std::min(step, P->natoms - a0);
+      const dim3 grid((unsigned)(((part.natoms + NA - 1) / NA * groups + 7) / 8 * 8));
+      hipLaunchKernelGGL((proj_gather<T, GW>), grid, dim3(64 * kGW), 0, static_cast<hipStream_t>(stream), part, Y, ld,
+                         nvec, C + (long long)a0 * nvec * 3);
+      PC_LAUNCH_CHECK();
+    }
+    return pc::PC_OK;
+  };
+  // As many wavefronts per atom as its support has rounds of 64, by the mean: more
+  // only add sums and barriers, fewer wait for one round after the other.  FP32, 275
+  // vectors, with 1, 2 and 4: 1,500 atoms of 20 points 75, 123, 223 us; 500 of 203
+  // points 99, 97, 106; 163 of 478 points 75, 69, 65; of 905 points 126, 115, 107.
+  const int mean = P->nent / P->natoms;
+  return mean <= 64    ? launch(std::integral_constant<int, 1>{})
+         : mean <= 256 ? launch(std::integral_constant<int, 2>{})
+                       : launch(std::integral_constant<int, kGW>{});
 }
 
 template <typename T>
