@@ -93,10 +93,10 @@ __device__ __forceinline__ void conv_store(f32x4 acc, long long v, int co0, int 
 constexpr int kNT = 2;   // 16-voxel tiles per wavefront
 constexpr int kWaves = 4;
 
-// Any number of input channels (a multiple of 16): each wavefront owns 16*MT
-// output channels x 32 voxels, its operands gathered straight from the
-// channel-last tensors.
-template <int MT>
+// Any number of input channels (a multiple of 16, or 1): each wavefront owns 16*MT
+// output channels x 32 voxels in flat order, its operands gathered straight from
+// the channel-last tensors.
+template <int MT, bool CIN1>
 __global__ __launch_bounds__(256) void conv_fwd(Vol vol, const unsigned short* __restrict__ X, int ldx, int cin,
                                                 const unsigned short* __restrict__ Wt, const float* __restrict__ bias,
                                                 int cout, int mode, float slope, void* Y, int ldy) {
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(256) void conv_fwd(Vol vol, const unsigned short* _
 #pragma unroll
     for (int n = 0; n < kNT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  {
+  if constexpr (!CIN1) {
     const int ncb = cin >> 4;
     for (int t = 0; t < 27; ++t) {
       int dz, dy, dx;
@@ -152,6 +152,36 @@ __global__ __launch_bounds__(256) void conv_fwd(Vol vol, const unsigned short* _
 #pragma unroll
           for (int n = 0; n < kNT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[n], acc[m][n], 0, 0, 0);
         }
+      }
+    }
+  } else {
+    // one input channel: K = the 27 taps (two k-steps of 16, taps 27..31 zero)
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x4 b[kNT];
+      short av[MT][4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = ks * 16 + 4 * lk + j;
+        int dz = 0, dy = 0, dx = 0;
+        if (t < 27) tap_offsets(t, dz, dy, dx);
+#pragma unroll
+        for (int n = 0; n < kNT; ++n) {
+          const int z = vz[n] + dz, y = vy[n] + dy, x = vx[n] + dx;
+          const bool ok = t < 27 && vin[n] && z >= 0 && z < vol.D && y >= 0 && y < vol.H && x >= 0 && x < vol.W;
+          b[n][j] = ok ? (short)X[((long long)(z * vol.H + y) * vol.W + x) * ldx] : (short)0;
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          const int co = co_base + 16 * m + ln;
+          av[m][j] = (t < 27 && co < cout) ? (short)Wt[(long long)co * 27 + t] : (short)0;
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const bf16x4 a = {av[m][0], av[m][1], av[m][2], av[m][3]};
+#pragma unroll
+        for (int n = 0; n < kNT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[n], acc[m][n], 0, 0, 0);
       }
     }
   }
@@ -499,6 +529,69 @@ __global__ __launch_bounds__(384) void conv_wgrad(Vol vol, Boxes bx, const unsig
   }
 }
 
+// The same over voxels in flat order, for volumes that boxes cover badly: workgroup
+// (tap t, 16 output channels, 16 NTC input channels, voxel split s), its operands
+// gathered from global memory.
+template <int NTC>
+__global__ __launch_bounds__(256) void conv_wgrad_flat(Vol vol, const unsigned short* __restrict__ dZ, int ldz,
+                                                       int cout, const unsigned short* __restrict__ X, int ldx, int cin,
+                                                       long long vchunk, float* __restrict__ part) {
+  __shared__ float red[kWaves][16 * 16 * NTC];
+  const int lane = threadIdx.x & 63;
+  const int wv = threadIdx.x >> 6;
+  const int ln = lane & 15, lk = lane >> 4;
+  const int t = blockIdx.x % 27;
+  const int cob = blockIdx.x / 27;
+  const int cib = blockIdx.y;
+  const int s = blockIdx.z;
+  int dz, dy, dx;
+  tap_offsets(t, dz, dy, dx);
+  const int co = cob * 16 + ln;
+  const long long v0 = (long long)s * vchunk;
+  const long long v1 = min(v0 + vchunk, vol.V);
+  f32x4 acc[NTC];
+#pragma unroll
+  for (int n = 0; n < NTC; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // each wavefront takes every 4th group of 16 voxels
+  for (long long vb = v0 + 16 * wv; vb < v1; vb += 16 * kWaves) {
+    bf16x4 a;
+    bf16x4 b[NTC];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const long long v = vb + 4 * lk + j;
+      const bool vok = v < v1;
+      a[j] = (vok && co < cout) ? (short)dZ[v * ldz + co] : (short)0;
+      long long src = -1;
+      if (vok) {
+        const int x = (int)(v % vol.W) + dx;
+        const int y = (int)((v / vol.W) % vol.H) + dy;
+        const int z = (int)(v / ((long long)vol.W * vol.H)) + dz;
+        if (z >= 0 && z < vol.D && y >= 0 && y < vol.H && x >= 0 && x < vol.W)
+          src = ((long long)(z * vol.H + y) * vol.W + x) * ldx;
+      }
+#pragma unroll
+      for (int n = 0; n < NTC; ++n) {
+        const int ci = cib * 16 * NTC + 16 * n + ln;
+        b[n][j] = (src >= 0 && ci < cin) ? (short)X[src + ci] : (short)0;
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < NTC; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[n], acc[n], 0, 0, 0);
+  }
+  // D[m = co row 4*lk + r][n = ci col ln]
+#pragma unroll
+  for (int n = 0; n < NTC; ++n)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wv][(4 * lk + r) * (16 * NTC) + 16 * n + ln] = acc[n][r];
+  __syncthreads();
+  for (int e = threadIdx.x; e < 16 * 16 * NTC; e += 256) {
+    const float sum = red[0][e] + red[1][e] + red[2][e] + red[3][e];
+    const int m = e / (16 * NTC), c = e % (16 * NTC);
+    const int com = cob * 16 + m, cim = cib * 16 * NTC + c;
+    if (com < cout && cim < cin) part[(((long long)s * cout + com) * 27 + t) * cin + cim] = sum;
+  }
+}
+
 // dW[i] = sum_s part[s][i]: 32 elements per workgroup, 8 threads each taking
 // every 8th split in order, their sums added in order
 __global__ __launch_bounds__(256) void reduce_splits(const float* __restrict__ part, int nsplit, long long n,
@@ -754,10 +847,10 @@ int pc_unet_conv3d_fwd(const void* X, int ldx, int cin, const void* W, const flo
   const bool yvec = ldy % 4 == 0 && aligned(Y, mode == 1 ? 8 : 16);
   const bool xvec = ldx % 8 == 0 && aligned(X, 16);
   // Boxes of 512 voxels for one group of 16 input channels, 256 for two or
-  // three and 128 for up to seven (LDS: two workgroups per CU), 16 or 8 wide
+  // three and 128 for up to seven (LDS: two workgroups per CU, one for seven groups
+  // and for six in 16-wide boxes), 16 or 8 wide
   // (whichever pads the volume less); 128 also where larger ones would not give
-  // every CU a workgroup.  More input channels, or columns without 16-byte
-  // alignment: conv_fwd.
+  // every CU a workgroup.
   const int ncb = cin / 16;
   auto padded = [&](int tx, int ty, int tz) { return box_count(vol, tx, ty, tz) * tx * ty * tz; };
   const bool fill512 = padded(16, 8, 4) / 512 * ct >= 256, fill256 = padded(16, 4, 4) / 256 * ct >= 256;
@@ -765,6 +858,16 @@ int pc_unet_conv3d_fwd(const void* X, int ldx, int cin, const void* W, const flo
   const bool w8 = size == 512   ? padded(8, 8, 8) < padded(16, 8, 4)
                   : size == 256 ? padded(8, 8, 4) < padded(16, 4, 4)
                                 : padded(8, 4, 4) < padded(16, 4, 2);
+  // conv_fwd: more input channels, columns without 16-byte alignment, and volumes
+  // that the boxes pad by so much that gathering every operand is the shorter
+  // (once the chip is full, at 2^18 padded voxels x channel blocks; a 300,000 x 1 x 1
+  // volume, 64 -> 64 channels: 14.5 ms in boxes, 0.53 gathered; 300 x 2 x 300, padded
+  // twice: 112 -> 48 channels 0.75 and 0.38, 48 -> 64 0.18 and 0.27).
+  const long long pad = size == 512   ? std::min(padded(8, 8, 8), padded(16, 8, 4))
+                        : size == 256 ? std::min(padded(8, 8, 4), padded(16, 4, 4))
+                                      : std::min(padded(8, 4, 4), padded(16, 4, 2));
+  const double most = cin == 1 ? 12.0 : ncb == 1 ? 4.2 : ncb <= 3 ? 2.2 : ncb <= 5 ? 1.8 : 1.3;
+  const bool gather = pad * ct >= (1 << 18) && (double)pad > most * (double)vol.V;
   // the channel blocks that one launch holds at a time
 #define PC_CONV_PARTS(KERNEL, TX, TY, TZ)                                                                            \
   do {                                                                                                               \
@@ -789,7 +892,13 @@ int pc_unet_conv3d_fwd(const void* X, int ldx, int cin, const void* W, const flo
     if (w8) PC_CONV(NCB, 8, 8, 4);     \
     else PC_CONV(NCB, 16, 4, 4);       \
   } while (0)
-  if (cin == 1) {
+  if (gather || (cin > 1 && (ncb > 7 || !xvec))) {
+    const long long vox_per_block = 16LL * kNT * kWaves;
+    dim3 grid((unsigned)((vol.V + vox_per_block - 1) / vox_per_block), (unsigned)((cout + 63) / 64));
+    auto general = ct == 1 ? conv_fwd<1, false> : ct == 2 ? conv_fwd<2, false> : ct == 3 ? conv_fwd<3, false> : conv_fwd<4, false>;
+    if (cin == 1) general = ct == 1 ? conv_fwd<1, true> : ct == 2 ? conv_fwd<2, true> : ct == 3 ? conv_fwd<3, true> : conv_fwd<4, true>;
+    hipLaunchKernelGGL(general, grid, dim3(256), 0, st, vol, X16, ldx, cin, W16, bias, cout, mode, slope, Y, ldy);
+  } else if (cin == 1) {
     if (size == 512) {
       if (w8) PC_CONV1(8, 8, 8);
       else PC_CONV1(16, 8, 4);
@@ -797,11 +906,6 @@ int pc_unet_conv3d_fwd(const void* X, int ldx, int cin, const void* W, const flo
       if (w8) PC_CONV1(8, 4, 4);
       else PC_CONV1(16, 4, 2);
     }
-  } else if (ncb > 7 || !xvec) {
-    const long long vox_per_block = 16LL * kNT * kWaves;
-    dim3 grid((unsigned)((vol.V + vox_per_block - 1) / vox_per_block), (unsigned)((cout + 63) / 64));
-    auto general = ct == 1 ? conv_fwd<1> : ct == 2 ? conv_fwd<2> : ct == 3 ? conv_fwd<3> : conv_fwd<4>;
-    hipLaunchKernelGGL(general, grid, dim3(256), 0, st, vol, X16, ldx, cin, W16, bias, cout, mode, slope, Y, ldy);
   } else {
     switch (ncb) {
       case 1:
@@ -867,8 +971,23 @@ int pc_unet_conv3d_wgrad(const void* dZ, int ldz, int cout, const void* X, int l
   const bool zvec = ldz % 8 == 0 && cout % 16 == 0 && aligned(dZ, 16);
   const bool xvec = ldx % 8 == 0 && cin % 16 == 0 && aligned(X, 16);
   const bool w8 = box_count(vol, 8, 8, 4) * 8 < box_count(vol, 16, 8, 4) * 16;   // padded rows
-  const Boxes bx = w8 ? make_boxes(vol, 8, 8, 4, 1) : make_boxes(vol, 16, 8, 4, 1);
   const int room = (int)std::min<long long>(kWgradSplit, (long long)(work_bytes / sizeof(float)) / n);
+  // Volumes that the boxes pad twelvefold and more (lines of voxels): over the
+  // voxels in flat order.  1 x 1 x 300,000, 48 -> 16 channels: 1.9 ms in boxes,
+  // 0.6 flat; 2 x 2 x 40,000, padded eightfold: 0.27 and 0.36.
+  if ((w8 ? box_count(vol, 8, 8, 4) * 256 : box_count(vol, 16, 8, 4) * 512) >= 12 * vol.V && vol.V >= 512) {
+    const int splits = (int)std::min<long long>(std::min(room, kWgradSplitMin), (vol.V + 255) / 256);
+    const long long vchunk = (vol.V + splits - 1) / splits;
+    const int ntc = cin >= 32 ? 2 : 1;
+    hipLaunchKernelGGL((ntc == 2 ? conv_wgrad_flat<2> : conv_wgrad_flat<1>),
+                       dim3(27 * ((cout + 15) / 16), (cin + 16 * ntc - 1) / (16 * ntc), splits), dim3(256), 0, st, vol,
+                       dZ16, ldz, cout, X16, ldx, cin, vchunk, part);
+    PC_LAUNCH_CHECK();
+    hipLaunchKernelGGL(reduce_splits, dim3(nblk(n, 32)), dim3(256), 0, st, part, splits, n, dW);
+    PC_LAUNCH_CHECK();
+    return pc::PC_OK;
+  }
+  const Boxes bx = w8 ? make_boxes(vol, 8, 8, 4, 1) : make_boxes(vol, 16, 8, 4, 1);
   const int nsplit = std::min(room, bx.nblocks);
   dim3 grid((cout + 15) / 16, (cin + 15) / 16, nsplit);
   const bool ragged = Wd % (w8 ? 8 : 16) != 0 || H % 8 != 0 || D % 4 != 0;
