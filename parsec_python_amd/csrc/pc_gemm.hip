@@ -313,16 +313,20 @@ __global__ __launch_bounds__(256, 2) void gram_tile(const T* __restrict__ X, lon
 // the chunks g, g + 8, ... in order and the 8 sums are added in order
 // (deterministic).  With one thread per element the chunks of a single-tile
 // Gram matrix were one serial chain (23 us at 385 chunks).
+// With at most 8 chunks (ONE) one thread per element adds them in order: the same
+// sums from an eighth of the threads.
+template <bool ONE>
 __global__ __launch_bounds__(256) void gram_reduce(const double* __restrict__ part, int W, int ntile, int nchunk,
                                                    int ti_n, int tj_n, int kx, int ky, double* __restrict__ S,
                                                    long long lds, int sym) {
   __shared__ double red[8][32];
-  const int per = W * W / 32;
+  constexpr int E = ONE ? 256 : 32;   // elements per workgroup
+  const int per = W * W / E;
   const int tile = blockIdx.x / per;
   int ti, tj;
   tile_coords(tile, ti_n, tj_n, sym, ti, tj);
-  const int el = threadIdx.x & 31, g = threadIdx.x >> 5;
-  const int e = (blockIdx.x - tile * per) * 32 + el;
+  const int el = threadIdx.x & (E - 1), g = threadIdx.x / E;
+  const int e = (blockIdx.x - tile * per) * E + el;
   const int jj = e / W, ii = e - jj * W;
   const int i = ti * W + ii, j = tj * W + jj;
   const bool in = i < kx && j < ky;
@@ -331,14 +335,18 @@ __global__ __launch_bounds__(256) void gram_reduce(const double* __restrict__ pa
     const double* p = part + (long long)tile * W * W + e;
     const long long st = (long long)ntile * W * W;
 #pragma unroll 8
-    for (int c = g; c < nchunk; c += 8) s += p[c * st];
+    for (int c = g; c < nchunk; c += ONE ? 1 : 8) s += p[c * st];
   }
-  red[g][el] = s;
-  __syncthreads();
+  if constexpr (!ONE) {
+    red[g][el] = s;
+    __syncthreads();
+  }
   if (g == 0 && in) {
-    double t = red[0][el];
+    double t = s;
+    if constexpr (!ONE) {
 #pragma unroll
-    for (int q = 1; q < 8; ++q) t += red[q][el];
+      for (int q = 1; q < 8; ++q) t += red[q][el];
+    }
     S[(long long)j * lds + i] = t;
     if (sym && ti != tj) S[(long long)i * lds + j] = t;
   }
@@ -758,13 +766,22 @@ GramPlan plan_gram(long long n, int kx, int ky, int sym, int sp, size_t bytes) {
       p.nt = nt; p.ti_n = ti; p.tj_n = tj; p.ntile = ntile;
     }
   }
+  // short columns: narrower tiles until a quarter of the CUs have a workgroup (128
+  // points, 275 columns, FP32: 15.1 -> 7.5 us with the reduction's ONE form, 10.4
+  // with 64-wide tiles and neither; with every CU 10,000 points, 96 columns lose 10 %)
+  const long long maxch = std::max<long long>(1, (n + 255) / 256);
+  while (p.nt > 1 && p.ntile * maxch < 64) {
+    const int w = 32 * --p.nt;
+    p.ti_n = (kx + w - 1) / w;
+    p.tj_n = (ky + w - 1) / w;
+    p.ntile = sym ? p.ti_n * (p.ti_n + 1) / 2 : p.ti_n * p.tj_n;
+  }
   const int resident = p.nt == 3 ? 512 : p.nt == 2 ? 1024 : 2048;
   const int rest = n % sp != 0;   // the points past the last whole stage are a chunk of their own
   const long long nw = n - n % sp;
   const long long room = (long long)(bytes / sizeof(double)) / (p.ntile * p.tile_size()) - rest;
   if (room < (nw > 0 ? 1 : 0)) return p;
   const long long target = std::max<long long>(1, resident / p.ntile - rest);
-  const long long maxch = std::max<long long>(1, (n + 255) / 256);
   p.nchunk = (int)std::min({target, maxch, std::max<long long>(1, room)});
   p.chunk = std::max<long long>(32, ((nw + p.nchunk - 1) / p.nchunk + 31) / 32 * 32);
   p.nchunk = (int)((nw + p.chunk - 1) / p.chunk) + rest;
@@ -820,8 +837,12 @@ int gram_impl(const T* X, long long ldx, const T* Y, long long ldy, long long n,
   }
   PC_LAUNCH_CHECK();
   const int w = 32 * p.nt;
-  hipLaunchKernelGGL(gram_reduce, dim3(p.ntile * (w * w / 32)), dim3(256), 0, st, part, w, p.ntile, p.nchunk, p.ti_n,
-                     p.tj_n, kx, ky, S, lds, sym);
+  if (p.nchunk <= 8)
+    hipLaunchKernelGGL(gram_reduce<true>, dim3(p.ntile * (w * w / 256)), dim3(256), 0, st, part, w, p.ntile, p.nchunk,
+                       p.ti_n, p.tj_n, kx, ky, S, lds, sym);
+  else
+    hipLaunchKernelGGL(gram_reduce<false>, dim3(p.ntile * (w * w / 32)), dim3(256), 0, st, part, w, p.ntile, p.nchunk,
+                       p.ti_n, p.tj_n, kx, ky, S, lds, sym);
   PC_LAUNCH_CHECK();
   return pc::PC_OK;
 }
@@ -873,9 +894,15 @@ int rotate_impl(const T* X, long long ldx, const double* Q, int ldq, T* Z, long 
   }
   if (vec) {
     if (convert_q() != pc::PC_OK) return pc::PC_ERR_HIP;
-    // column blocks of at most 288, of equal width
-    const int ncb = (ky + 287) / 288;
-    const int nch = ((ky + ncb - 1) / ncb + 31) / 32;
+    // column blocks of at most 288, of equal width; for short columns narrower ones,
+    // until 96 CUs have a workgroup (520 columns, FP32, 1,000 points: 105 -> 48 us,
+    // 67 with 64 columns per workgroup in the general form; with every CU 10,000
+    // points, 275 columns, FP64 61 -> 87)
+    const long long tiles = (n + 32 * E - 1) / (32 * E);
+    const int nblk = (ky + 287) / 288;
+    int nch = ((ky + nblk - 1) / nblk + 31) / 32;
+    while (nch > 2 && tiles * ((ky + 32 * nch - 1) / (32 * nch)) < 96) --nch;
+    const int ncb = (ky + 32 * nch - 1) / (32 * nch);
     // a slab's X in 32-bit byte offsets: to 2^26 points per column and more in FP32, 2^25 in FP64
     const bool wide_offsets = ((std::min(kx, 16) - 1) * ldx + n) * (long long)sizeof(T) >= (1LL << 32);
     const long long step = pc::kMaxGrid / ncb * (32 * E);   // points per launch

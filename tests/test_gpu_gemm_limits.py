@@ -128,3 +128,37 @@ def test_rotate_long_columns_keep_their_speed(gpu, dtype):
     short, long = (sorted(t)[4] for t in times)
     print(f"{250 * short:.1f} and {250 * long:.1f} us", flush=True)
     assert long <= 1.25 * short
+
+
+@pytest.mark.parametrize("n,k", [(16, 33), (100, 100), (128, 275), (255, 289), (257, 520), (1000, 300), (2001, 577)])
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_short_columns(gpu, n, k, dtype):
+    """Narrower Gram tiles and rotation blocks, few chunks: against FP64 (tolerances as above)."""
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    import ctypes as C
+    print(f"short columns n={n} k={k} {dtype}", flush=True)
+    tdt, u = (torch.float64, 2.0 ** -53) if dtype == "f64" else (torch.float32, 2.0 ** -24)
+    ld = (n + 15) // 16 * 16
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    X = torch.full((k, ld), float("nan"), dtype=tdt, device="cuda")
+    Y = torch.full((k + 3, ld), float("nan"), dtype=tdt, device="cuda")
+    X[:, :n] = torch.randn((k, n), generator=g, dtype=tdt, device="cuda")
+    Y[:, :n] = torch.randn((k + 3, n), generator=g, dtype=tdt, device="cuda")
+    x, y = X[:, :n].double().cpu().numpy(), Y[:, :n].double().cpu().numpy()
+    tol = (n + 2) * 2.0 ** -53 if dtype == "f64" else 17 * 2.0 ** -24 + n * 2.0 ** -53
+    for ky, other, sym in ((k, X, 1), (k + 3, Y, 0)):
+        nb = C.c_size_t()
+        _lib.call("pc_gram_workspace", n, k, ky, sym, C.byref(nb))
+        work = torch.full((nb.value // 8 + 64,), 7.0, dtype=torch.float64, device="cuda")
+        S = torch.full((ky, k), float("nan"), dtype=torch.float64, device="cuda")
+        _lib.call(f"pc_gram_{dtype}", ptr(X), ld, ptr(other), ld, n, k, ky, ptr(S), k, sym, ptr(work), nb.value, stream())
+        b = x if sym else y
+        assert np.all(np.abs(S.cpu().numpy() - b @ x.T) <= 2 * tol * (np.abs(b) @ np.abs(x).T))
+        assert bool((work[nb.value // 8:] == 7.0).all())
+    Q = torch.randn((k + 3, k), generator=g, dtype=torch.float64, device="cuda")
+    Z = _rotate(X, n, Q, dtype, ld)
+    q = Q.cpu().numpy()
+    assert np.all(np.abs(Z[:, :n].double().cpu().numpy() - q @ x) <= 2 * (k + 2) * u * (np.abs(q) @ np.abs(x)))
+    assert bool((Z[:, n:] == 7.0).all())
