@@ -776,7 +776,7 @@ struct SinglePass {
 };
 
 template <int R, int SX>
-__global__ __launch_bounds__(pcz::threads(SX), SX == 2 ? 4 : 2) void stencil_single(pcz::ZMap zm, SinglePass p) {
+__global__ __launch_bounds__(pcz::threads(SX), SX == 2 && R <= 4 ? 4 : 2) void stencil_single(pcz::ZMap zm, SinglePass p) {
   __shared__ double tile[pcz::Tile<R, SX>::SIZE];
   const int L = pcz::block_of(zm);
   if (L >= zm.nwg) return;

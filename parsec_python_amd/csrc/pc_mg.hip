@@ -102,12 +102,12 @@ __device__ __forceinline__ double dom_at(const Fine& g, const double* __restrict
 // x-chunk, where twice as many workgroups fill more of the chip.  Chunks of planes from
 // multiples of zc, so that every 2 x 2 x 2 cell lies in one workgroup and the
 // restriction needs no launch of its own.  Wider rows: the march.
-constexpr int mg_rows(int sx) { return sx == 2 ? 8 : pcz::kZW; }
+constexpr int mg_rows(int sx, int R) { return sx == 2 && R <= 4 ? 8 : pcz::kZW; }
 template <int R, int SX, int VALUES, class P>   // VALUES loaded per point
 __device__ __forceinline__ bool mg_pass(const ZMap& zm, int L, double* tile, P& p, double& s) {
   // 128 registers per thread: two values per point of radius 4 do not fit beside the formed field
-  constexpr bool early = SX == 2 && VALUES * (2 * R + pcz::kZP) > 20;
-  return pcz::zpass<R, SX, mg_rows(SX), false, SX <= 2, early>(zm, L, tile, p, s);
+  constexpr bool early = SX == 2 && R <= 4 && VALUES * (2 * R + pcz::kZP) > 20;
+  return pcz::zpass<R, SX, mg_rows(SX, R), false, SX <= 2, early>(zm, L, tile, p, s);
 }
 
 // r = rhs - A x; partials of r.r (once per solve)
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(kB) void mg_init(Fine g, const double* __restrict__
 // t0 = r - c0 A r: the residual after one damped-Jacobi step from zero
 // (rows of more than 128 points), or restricted at once: b_1 = the average of
 // each cell's children.
-template <int SX>
+template <int R, int SX>
 struct Res0Pass {
   struct Raw { double r; };
   typedef pcz::NoExt Ext;
@@ -162,7 +162,7 @@ struct Res0Pass {
   }
   // the plane, x and y pairs of each cell: registers, neighbouring lanes, LDS
   __device__ __forceinline__ void post(const double* t, int i, int j, int z, int zend, int row) const {
-    constexpr int W = 32 * SX, H = mg_rows(SX) / 2;
+    constexpr int W = 32 * SX, H = mg_rows(SX, R) / 2;
     double c[pcz::kZP / 2];
 #pragma unroll
     for (int q = 0; q < pcz::kZP / 2; ++q) {
@@ -181,9 +181,9 @@ struct Res0Pass {
   }
 };
 template <int R, int SX>
-__global__ __launch_bounds__(pcz::threads(SX, mg_rows(SX))) void mg_res0(ZMap zm, Res0Pass<SX> p) {
-  __shared__ double tile[pcz::Tile<R, SX, mg_rows(SX)>::SIZE];
-  __shared__ double buf[SX <= 2 ? pcz::kZP / 2 * (mg_rows(SX) / 2) * 32 * SX : 1];
+__global__ __launch_bounds__(pcz::threads(SX, mg_rows(SX, R)), mg_rows(SX, R) == 8 ? 4 : 2) void mg_res0(ZMap zm, Res0Pass<R, SX> p) {
+  __shared__ double tile[pcz::Tile<R, SX, mg_rows(SX, R)>::SIZE];
+  __shared__ double buf[SX <= 2 ? pcz::kZP / 2 * (mg_rows(SX, R) / 2) * 32 * SX : 1];
   const int L = pcz::block_of(zm);
   if (L >= zm.nwg) return;
   p.buf = buf;
@@ -232,8 +232,8 @@ struct Up0Pass {
   }
 };
 template <int R, int SX>
-__global__ __launch_bounds__(pcz::threads(SX, mg_rows(SX))) void mg_up0(ZMap zm, Up0Pass p, double* __restrict__ prz) {
-  __shared__ double tile[pcz::Tile<R, SX, mg_rows(SX)>::SIZE];
+__global__ __launch_bounds__(pcz::threads(SX, mg_rows(SX, R)), mg_rows(SX, R) == 8 ? 4 : 2) void mg_up0(ZMap zm, Up0Pass p, double* __restrict__ prz) {
+  __shared__ double tile[pcz::Tile<R, SX, mg_rows(SX, R)>::SIZE];
   __shared__ double red[16];
   const int L = pcz::block_of(zm);
   if (L >= zm.nwg) return;
@@ -300,8 +300,8 @@ struct ApplyPass {
   }
 };
 template <int R, int SX>
-__global__ __launch_bounds__(pcz::threads(SX, mg_rows(SX))) void mg_apply(ZMap zm, ApplyPass p, double* __restrict__ ppq) {
-  __shared__ double tile[pcz::Tile<R, SX, mg_rows(SX)>::SIZE];
+__global__ __launch_bounds__(pcz::threads(SX, mg_rows(SX, R)), mg_rows(SX, R) == 8 ? 4 : 2) void mg_apply(ZMap zm, ApplyPass p, double* __restrict__ ppq) {
+  __shared__ double tile[pcz::Tile<R, SX, mg_rows(SX, R)>::SIZE];
   __shared__ double red[16], red2[16], red3[16];
   const int L = pcz::block_of(zm);
   if (L >= zm.nwg) return;
@@ -592,10 +592,10 @@ size_t work_bytes_for(long long n) {
 template <int R, int SX>
 struct FineLaunch {
   static dim3 grid(const MGCtx* c) { return dim3(8 * c->zm.nwg8); }
-  static dim3 block() { return dim3(pcz::threads(SX, mg_rows(SX))); }
+  static dim3 block() { return dim3(pcz::threads(SX, mg_rows(SX, R))); }
   static void res0(const MGCtx* c, hipStream_t st, const double* r, const double* sc) {
     const Cube& c1 = c->lev[1];
-    const Res0Pass<SX> p{c->g.c0, r, c->t0, c1.b, c1.nx, c1.ny, c1.nz, sc, nullptr};
+    const Res0Pass<R, SX> p{c->g.c0, r, c->t0, c1.b, c1.nx, c1.ny, c1.nz, sc, nullptr};
     hipLaunchKernelGGL((mg_res0<R, SX>), grid(c), block(), 0, st, c->zm, p);
     if (SX > 2)
       hipLaunchKernelGGL(mg_restrict0, dim3((unsigned)((c1.cells + kB - 1) / kB)), dim3(kB), 0, st, c->g, c->t0, c1, sc);
@@ -676,7 +676,7 @@ int pc_mg_create(void* grid, double h, void** out_mg) {
   g.nb = (int)((g.n + g.chunk - 1) / g.chunk);
   g.nb8 = (g.nb + 7) / 8;
   int rz = 0;
-  if (pcz::zmap_init(grid, g.w, c->zm, &rz, mg_rows(g.nx <= 64 ? 1 : (g.nx <= 128 ? 2 : 4)), 2)) {
+  if (pcz::zmap_init(grid, g.w, c->zm, &rz, mg_rows(g.nx <= 64 ? 1 : (g.nx <= 128 ? 2 : 4), c->radius), 2)) {
     delete c;
     PC_CHECK_ARG(false, "nx > 256");
   }

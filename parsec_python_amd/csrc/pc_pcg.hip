@@ -178,7 +178,7 @@ struct ApplyPass {
 };
 
 template <int R, int SX, int MODE>
-__global__ __launch_bounds__(pcz::threads(SX), SX == 2 ? 4 : 2) void cg_apply_z(ZMap g, ApplyPass<MODE> p, double* __restrict__ part_pq) {
+__global__ __launch_bounds__(pcz::threads(SX), SX == 2 && R <= 4 ? 4 : 2) void cg_apply_z(ZMap g, ApplyPass<MODE> p, double* __restrict__ part_pq) {
   __shared__ double tile[pcz::Tile<R, SX, pcz::kZW, true>::SIZE];
   __shared__ double red[8], red2[8];
   const int L = pcz::block_of(g);
