@@ -16,8 +16,9 @@
 // Chebyshev filters (src/Eigensolvers/ch_filter.py:66-80, first_filt.py:94-101).
 // x may alias out (each point reads x before writing out at the same place).
 //
-// Kernel shape (CDNA4): a workgroup owns one vector, a slab of y-rows and a window
-// of up to 64 columns, and marches along z.  Each thread keeps its point's 2R+1
+// Kernel shape (CDNA4; stencil_win, and stencil_zmarch where partial sums are asked
+// for): a workgroup owns one vector, a slab of y-rows and a window of up to 64 or 128
+// columns (its whole rows), and marches along z.  Each thread keeps its point's 2R+1
 // z-values in registers; the current plane of the slab plus R halo rows
 // above/below sits in LDS for the x/y differences.  Workgroup ids are remapped so
 // the windows of one vector run on the same XCD (its L2 then serves the halos).
@@ -84,51 +85,35 @@ __device__ __forceinline__ T meta_val(const T* __restrict__ y, int2 m, int i) {
   return (i >= lo && i < hi) ? y[m.x + i] : T(0);
 }
 
-// Software-pipelined z-march: while plane z is computed from LDS and the
-// register queues, the loads for the next PD planes (queue entry z+R+1.., halo
-// rows, V and x) are already in flight (PD register stages, the z loop unrolled
-// by PD).  A workgroup handles NV vectors at once: the row metadata, the V
-// values and the control flow are shared by them.  Two LDS tiles alternate,
+// The step with per-workgroup sums of out * y: a workgroup owns one vector and 4
+// y-rows, one wavefront of SX 64-column parts per row, and marches z.  While plane
+// z is computed from LDS and the register queues, the loads for the next plane
+// (queue entry z+R+1, halo rows, V and x) are in flight.  Two LDS tiles alternate,
 // so one barrier per plane suffices.
-template <typename T, int R, int SX, int TYW, int NV, int NB, bool HASX, bool DOT, int PD = 1, int NW = 4>
-__global__ __launch_bounds__(64 * NW) void stencil_zmarch(StArgs g, const T* __restrict__ Y, const T* X,
-                                                          T* Out, const T* __restrict__ V, T ca, T cb, T cc,
-                                                          double* __restrict__ dot_part) {
-  constexpr int TY = NW * TYW;
-  constexpr int NXP = 64 * SX;
-  constexpr int LW = NXP + 2 * R;   // LDS row stride (R zero columns each side)
-  constexpr int LR = TY + 2 * R;    // LDS rows
-  constexpr int HT = (2 * R + NW - 1) / NW;  // halo rows per wave
-  static_assert(PD == 1 || PD == 2, "prefetch depth 1 or 2");
-  static_assert(PD == 1 || NB == 2, "two planes in flight need two LDS tiles");
-  __shared__ T tile[NB][NV][LR * LW];
-  __shared__ double red[NW];
+template <typename T, int R, int SX, bool HASX>
+__global__ __launch_bounds__(256) void stencil_zmarch(StArgs g, const T* __restrict__ Y, const T* X, T* Out,
+                                                      const T* __restrict__ V, T ca, T cb, T cc,
+                                                      double* __restrict__ dot_part) {
+  constexpr int TY = 4;
+  constexpr int LW = 64 * SX + 2 * R;          // LDS row stride (R zero columns each side)
+  constexpr int LR = TY + 2 * R;               // LDS rows
+  constexpr int HT = (2 * R + TY - 1) / TY;    // halo rows per wave
+  __shared__ T tile[2][LR * LW];
+  __shared__ double red[TY];
 
   const int bid = blockIdx.x;
   const int L = (bid & 7) * g.nb8 + (bid >> 3);
   if (L >= g.nblocks) return;
-  const int vg = L / g.nslab;
-  const int slab = L - vg * g.nslab;
-  const int j0 = slab * TY;
+  const int v = L / g.nslab;
+  const int j0 = (L - v * g.nslab) * TY;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ny = g.ny, nz = g.nz;
   const int2* __restrict__ meta = g.meta;
-
-  const T* yv[NV];
-  const T* xv[NV];
-  T* ov[NV];
-  bool act[NV];
-#pragma unroll
-  for (int u = 0; u < NV; ++u) {
-    const int v = vg * NV + u;
-    act[u] = v < g.nvec;
-    const long long base = (long long)(act[u] ? v : vg * NV) * g.ld;
-    yv[u] = Y + base;
-    xv[u] = X ? X + base : nullptr;
-    ov[u] = Out + base;
-  }
-  constexpr bool hasx = HASX;
+  const long long base = (long long)v * g.ld;
+  const T* yv = Y + base;
+  const T* xv = HASX ? X + base : nullptr;
+  T* ov = Out + base;
 
   int zb = nz, ze = 0;
   for (int t = 0; t < TY; ++t) {
@@ -138,15 +123,11 @@ __global__ __launch_bounds__(64 * NW) void stencil_zmarch(StArgs g, const T* __r
       ze = max(ze, g.zrange[2 * j + 1]);
     }
   }
-  double dot = 0.0;
   if (zb >= ze) {
-    if constexpr (DOT) {
-      const double s = pc_block_sum(0.0, red);
-      if (threadIdx.x == 0) dot_part[L] = s;
-    }
+    if (threadIdx.x == 0) dot_part[L] = 0.0;
     return;
   }
-  for (int t = threadIdx.x; t < NB * NV * LR * LW; t += 64 * NW) (&tile[0][0][0])[t] = T(0);
+  for (int t = threadIdx.x; t < 2 * LR * LW; t += 256) (&tile[0][0])[t] = T(0);
   __syncthreads();
 
   auto rowmeta = [&](int j, int z) -> int2 {
@@ -168,180 +149,97 @@ __global__ __launch_bounds__(64 * NW) void stencil_zmarch(StArgs g, const T* __r
     const int l = z - w.wb;
     return make_int2(__builtin_amdgcn_readlane(w.v.x, l), __builtin_amdgcn_readlane(w.v.y, l));
   };
-  Win wown[TYW], whalo[HT];
+  // tile row of this wavefront's t-th halo row (LR and more: none)
+  auto halo = [&](int t) { return wv + TY * t < R ? wv + TY * t : wv + TY * t + TY; };
+  Win wown, whalo[HT];
+  win_load(wown, j0 + wv, zb - R);
 #pragma unroll
-  for (int r = 0; r < TYW; ++r) win_load(wown[r], j0 + wv + NW * r, zb - R);
-#pragma unroll
-  for (int t = 0; t < HT; ++t) {
-    const int hr = wv + NW * t;
-    const int tr = hr < R ? hr : hr + TY;
-    win_load(whalo[t], j0 - R + tr, zb);
-  }
+  for (int t = 0; t < HT; ++t) win_load(whalo[t], j0 - R + halo(t), zb);
 
-  T q[NV][TYW][SX][2 * R + 1];
-  T xq[NV][TYW][SX];
-  T vq[TYW][SX];
-  T hc[NV][HT][SX] = {};
-  int2 mcur[TYW];
-  // prefetch stages
-  T nq[PD][NV][TYW][SX], nxv[PD][NV][TYW][SX];
-  T nv[PD][TYW][SX];
-  T hn[PD][NV][HT][SX] = {};
-  int2 mnext[PD][TYW];
-
-  // prefill planes zb-R .. zb+R-1
+  T q[SX][2 * R + 1], xq[SX], vq[SX], hc[HT][SX] = {};
+  T nq[SX], nxv[SX], nv[SX], hn[HT][SX] = {};   // the next plane's
+  int2 mcur, mnext;
+  // planes zb-R .. zb+R-1
 #pragma unroll
-  for (int r = 0; r < TYW; ++r) {
-    const int j = j0 + wv + NW * r;
+  for (int s = 0; s < SX; ++s) q[s][0] = T(0);
 #pragma unroll
-    for (int u = 0; u < NV; ++u)
+  for (int dz = 1; dz <= 2 * R; ++dz) {
+    const int2 m = win_at(wown, zb - R - 1 + dz);
 #pragma unroll
-      for (int s = 0; s < SX; ++s) q[u][r][s][0] = T(0);
-#pragma unroll
-    for (int dz = 1; dz <= 2 * R; ++dz) {
-      const int2 m = win_at(wown[r], zb - R - 1 + dz);
-#pragma unroll
-      for (int u = 0; u < NV; ++u)
-#pragma unroll
-        for (int s = 0; s < SX; ++s) q[u][r][s][dz] = meta_val(yv[u], m, lane + 64 * s);
-    }
+    for (int s = 0; s < SX; ++s) q[s][dz] = meta_val(yv, m, lane + 64 * s);
   }
-  // issue everything plane z needs into stage S
-  auto prefetch = [&](auto stage, int z) {
-    constexpr int S = decltype(stage)::value;
+  auto prefetch = [&](int z) {
+    if (z + R >= wown.wb + 64) win_load(wown, j0 + wv, z);
+    const int2 mq = win_at(wown, z + R);
+    mnext = win_at(wown, z);
+    const int lo = mnext.y & 0xffff, hi = mnext.y >> 16;
 #pragma unroll
-    for (int r = 0; r < TYW; ++r) {
-      if (z + R >= wown[r].wb + 64) win_load(wown[r], j0 + wv + NW * r, z);
-      const int2 mq = win_at(wown[r], z + R);
-      const int2 mo = win_at(wown[r], z);
-      mnext[S][r] = mo;
-      const int lo = mo.y & 0xffff, hi = mo.y >> 16;
-#pragma unroll
-      for (int s = 0; s < SX; ++s) {
-        const int i = lane + 64 * s;
-        const bool in = i >= lo && i < hi;
-        nv[S][r][s] = in ? V[mo.x + i] : T(0);
-#pragma unroll
-        for (int u = 0; u < NV; ++u) {
-          nq[S][u][r][s] = meta_val(yv[u], mq, i);
-          nxv[S][u][r][s] = (in && hasx) ? xv[u][mo.x + i] : T(0);
-        }
-      }
+    for (int s = 0; s < SX; ++s) {
+      const int i = lane + 64 * s;
+      const bool in = i >= lo && i < hi;
+      nv[s] = in ? V[mnext.x + i] : T(0);
+      nq[s] = meta_val(yv, mq, i);
+      nxv[s] = (HASX && in) ? xv[mnext.x + i] : T(0);
     }
 #pragma unroll
     for (int t = 0; t < HT; ++t) {
-      const int hr = wv + NW * t;
-      if (hr < 2 * R) {
-        const int tr = hr < R ? hr : hr + TY;
-        if (z >= whalo[t].wb + 64) win_load(whalo[t], j0 - R + tr, z);
-        const int2 mh = win_at(whalo[t], z);
+      if (halo(t) >= LR) continue;
+      if (z >= whalo[t].wb + 64) win_load(whalo[t], j0 - R + halo(t), z);
+      const int2 mh = win_at(whalo[t], z);
 #pragma unroll
-        for (int u = 0; u < NV; ++u)
-#pragma unroll
-          for (int s = 0; s < SX; ++s) hn[S][u][t][s] = meta_val(yv[u], mh, lane + 64 * s);
-      }
+      for (int s = 0; s < SX; ++s) hn[t][s] = meta_val(yv, mh, lane + 64 * s);
     }
   };
-  // plane z from stage S: commit, refill the stage with plane z+PD, compute
-  auto plane = [&](auto stage, int z) {
-    constexpr int S = decltype(stage)::value;
-    const int b = NB == 2 ? ((z - zb) & 1) : 0;
+  double dot = 0.0;
+  prefetch(zb);
+  for (int z = zb; z < ze; ++z) {
+    T* tb = tile[(z - zb) & 1];
+    mcur = mnext;
 #pragma unroll
-    for (int r = 0; r < TYW; ++r) {
-      mcur[r] = mnext[S][r];
+    for (int s = 0; s < SX; ++s) {
+      vq[s] = nv[s];
 #pragma unroll
-      for (int s = 0; s < SX; ++s) {
-        vq[r][s] = nv[S][r][s];
+      for (int d = 0; d < 2 * R; ++d) q[s][d] = q[s][d + 1];
+      q[s][2 * R] = nq[s];
+      xq[s] = nxv[s];
 #pragma unroll
-        for (int u = 0; u < NV; ++u) {
-#pragma unroll
-          for (int d = 0; d < 2 * R; ++d) q[u][r][s][d] = q[u][r][s][d + 1];
-          q[u][r][s][2 * R] = nq[S][u][r][s];
-          xq[u][r][s] = nxv[S][u][r][s];
-        }
-      }
+      for (int t = 0; t < HT; ++t) hc[t][s] = hn[t][s];
     }
+    if (z + 1 < ze) prefetch(z + 1);
 #pragma unroll
-    for (int u = 0; u < NV; ++u)
+    for (int s = 0; s < SX; ++s) tb[(wv + R) * LW + R + lane + 64 * s] = q[s][R];
 #pragma unroll
-      for (int t = 0; t < HT; ++t)
+    for (int t = 0; t < HT; ++t) {
+      if (halo(t) >= LR) continue;
 #pragma unroll
-        for (int s = 0; s < SX; ++s) hc[u][t][s] = hn[S][u][t][s];
-    // issue the loads for plane z + PD
-    if (z + PD < ze) prefetch(stage, z + PD);
-    // plane z into LDS
-#pragma unroll
-    for (int u = 0; u < NV; ++u) {
-      T* tb = tile[b][u];
-#pragma unroll
-      for (int r = 0; r < TYW; ++r) {
-        const int tr = wv + NW * r + R;
-#pragma unroll
-        for (int s = 0; s < SX; ++s) tb[tr * LW + R + lane + 64 * s] = q[u][r][s][R];
-      }
-#pragma unroll
-      for (int t = 0; t < HT; ++t) {
-        const int hr = wv + NW * t;
-        if (hr < 2 * R) {
-          const int tr = hr < R ? hr : hr + TY;
-#pragma unroll
-          for (int s = 0; s < SX; ++s) tb[tr * LW + R + lane + 64 * s] = hc[u][t][s];
-        }
-      }
+      for (int s = 0; s < SX; ++s) tb[halo(t) * LW + R + lane + 64 * s] = hc[t][s];
     }
     lds_barrier();
-    // outputs of plane z
+    const int lo = mcur.y & 0xffff, hi = mcur.y >> 16;
 #pragma unroll
-    for (int r = 0; r < TYW; ++r) {
-      const int2 mo = mcur[r];
-      const int lo = mo.y & 0xffff, hi = mo.y >> 16;
-      const int tr = wv + NW * r + R;
+    for (int s = 0; s < SX; ++s) {
+      const int i = lane + 64 * s;
+      // computed on every lane (values outside the domain are zeros), stored inside it
+      const T va = ca * vq[s] + cb;
+      const T yc = q[s][R];
+      T acc = T(g.w[0]) * yc;
+      const T* trow = tb + (wv + R) * LW + R + i;
 #pragma unroll
-      for (int s = 0; s < SX; ++s) {
-        const int i = lane + 64 * s;
-        // computed on every lane (values outside the domain are zeros), stored inside it
-        const bool in = i >= lo && i < hi;
-        const T va = ca * vq[r][s] + cb;
-#pragma unroll
-        for (int u = 0; u < NV; ++u) {
-          const T yc = q[u][r][s][R];
-          T acc = T(g.w[0]) * yc;
-          const T* trow = tile[b][u] + tr * LW + R + i;
-#pragma unroll
-          for (int d = 1; d <= R; ++d) {
-            const T nb = trow[-d] + trow[d] + trow[-d * LW] + trow[d * LW] + q[u][r][s][R - d] +
-                         q[u][r][s][R + d];
-            acc += T(g.w[d]) * nb;
-          }
-          T o = acc + va * yc;
-          if constexpr (HASX) o += cc * xq[u][r][s];
-          if (in && act[u]) {
-            ov[u][mo.x + i] = o;
-            if constexpr (DOT) dot += (double)o * (double)yc;
-          }
-        }
+      for (int d = 1; d <= R; ++d) {
+        const T nb = trow[-d] + trow[d] + trow[-d * LW] + trow[d * LW] + q[s][R - d] + q[s][R + d];
+        acc += T(g.w[d]) * nb;
+      }
+      T o = acc + va * yc;
+      if constexpr (HASX) o += cc * xq[s];
+      if (i >= lo && i < hi) {
+        ov[mcur.x + i] = o;
+        dot += (double)o * (double)yc;
       }
     }
-    if (NB == 1) lds_barrier();   // one tile: the next plane overwrites it
-  };
-  using S0 = std::integral_constant<int, 0>;
-  using S1 = std::integral_constant<int, PD - 1>;
-  prefetch(S0{}, zb);
-  if constexpr (PD == 2) {
-    if (zb + 1 < ze) prefetch(S1{}, zb + 1);
-    for (int z = zb; z < ze; z += 2) {
-      plane(S0{}, z);
-      if (z + 1 < ze) plane(S1{}, z + 1);
-    }
-  } else {
-    for (int z = zb; z < ze; ++z) plane(S0{}, z);
   }
-  if constexpr (DOT) {
-    const double s = pc_block_sum(dot, red);
-    if (threadIdx.x == 0) dot_part[L] = s;
-  }
+  const double s = pc_block_sum(dot, red);
+  if (threadIdx.x == 0) dot_part[L] = s;
 }
-
 
 // ---- the windowed z-march (one vector per workgroup, no partial sums) ---------
 // A workgroup owns one vector and one window of a slab of win_ty(R, SX) y-rows, one
@@ -623,24 +521,23 @@ int launch_win(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, in
 template <typename T, int R, int SX>
 int launch_dot(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, int nvec, long long ld, double scale,
                double ca, double cb, double cc, double* dot_part, hipStream_t st) {
-  constexpr int NW = 4;
   StArgs a;
   a.nx = gd->nx; a.ny = gd->ny; a.nz = gd->nz; a.npts = gd->npts;
   a.lo = gd->lo; a.hi = gd->hi; a.off = gd->off; a.zrange = gd->zrange; a.meta = gd->meta;
   a.ld = ld;
-  a.nslab = (gd->ny + NW - 1) / NW;
+  a.nslab = (gd->ny + 3) / 4;
   a.nvec = nvec;
   a.nblocks = a.nslab * nvec;
   a.nb8 = (a.nblocks + 7) / 8;
   for (int d = 0; d < 8; ++d) a.w[d] = 0.0;
   a.w[0] = 3.0 * gd->w[0] * scale;
   for (int d = 1; d <= R; ++d) a.w[d] = gd->w[d] * scale;
-  const dim3 grid(8 * a.nb8), block(64 * NW);
+  const dim3 grid(8 * a.nb8), block(256);
   if (X)
-    hipLaunchKernelGGL((stencil_zmarch<T, R, SX, 1, 1, 2, true, true, 1, NW>), grid, block, 0, st, a, Y, X, Out, V,
+    hipLaunchKernelGGL((stencil_zmarch<T, R, SX, true>), grid, block, 0, st, a, Y, X, Out, V,
                        T(ca), T(cb), T(cc), dot_part);
   else
-    hipLaunchKernelGGL((stencil_zmarch<T, R, SX, 1, 1, 2, false, true, 1, NW>), grid, block, 0, st, a, Y, X, Out, V,
+    hipLaunchKernelGGL((stencil_zmarch<T, R, SX, false>), grid, block, 0, st, a, Y, X, Out, V,
                        T(ca), T(cb), T(cc), dot_part);
   PC_LAUNCH_CHECK();
   return pc::PC_OK;
