@@ -837,6 +837,7 @@ int pc_grid_create(int nx, int ny, int nz, const int* row_lo, const int* row_hi,
   // stencil_win: per slab of rows the columns they touch, as one window of up to
   // 64 sx or as windows of equal lane counts (an inner edge has radius halo lanes,
   // an outer one none), with the planes they touch; lanes: those of all planes
+  int most = 0;   // windows of one slab
   auto windows = [&](int sx, std::vector<int4>& win) {
     long long lanes_all = 0;
     const int ty = win_ty(radius, sx), lw = 64 * sx;
@@ -852,6 +853,7 @@ int pc_grid_create(int nx, int ny, int nz, const int* row_lo, const int* row_hi,
       if (xl >= xh) continue;
       int n = 1;
       while (xh - xl + 2 * radius * (n - 1) > lw * n) ++n;
+      most = std::max(most, n);
       const int lanes = xh - xl + 2 * radius * (n - 1);
       auto cut = [&](int i) { return i == 0 ? xl : i == n ? xh : xl + lanes * i / n - radius * (2 * i - 1); };
       for (int i = 0; i < n; ++i) {
@@ -879,7 +881,7 @@ int pc_grid_create(int nx, int ny, int nz, const int* row_lo, const int* row_hi,
   // FP64 341 -> 280 us, radius 6 361 -> 298), at radius 1 where it costs none
   // (126^3, 49 vectors FP32 289 -> 263).  With two windows either way one wavefront
   // per row is the faster (100^3 FP32 radius 4 11 %, spheres 20 to 40 %).
-  if (nx > 64 && nx <= 128) {
+  if (nx > 64 && nx <= 128 && most >= (radius == 1 ? 2 : 3)) {
     const long long lanes2 = windows(2, win2);
     if (radius == 1 ? lanes2 <= lanes1 : 5 * lanes2 <= 4 * lanes1) {
       g->winsx = 2;
