@@ -153,9 +153,8 @@ __global__ __launch_bounds__(256) void gram_kernel(const T* __restrict__ X, long
 // loads are in flight while the MFMAs run, one barrier per stage.  Columns past
 // the edge are loaded from the last column (their products only reach outputs
 // that gram_reduce skips), so the stage loop has no branches; only the last
-// chunk's last stage checks its points.  A symmetric tile on the diagonal of
-// X^T X reads one operand.  FP32: 16 points accumulate in the MFMA from zero
-// and are added to the FP64 accumulators while the next 16 run.
+// chunk's last stage checks its points.  FP32: 16 points accumulate in the MFMA
+// from zero and are added to the FP64 accumulators while the next 16 run.
 // Bound by the MFMA rate once the operand strips stay on chip: consecutive
 // workgroups of one XCD take the tiles of one chunk, so its L2 serves the
 // columns to all of them (with the tiles dealt over the XCDs every L2 fetched

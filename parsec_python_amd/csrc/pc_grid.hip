@@ -277,7 +277,7 @@ __global__ __launch_bounds__(256) void stencil_zmarch(StArgs g, const T* __restr
 //                                   FP32 721 -> 680 us, FP64 1508 -> 1250 us
 //   C10H8 sphere, radius 4, 49:     FP32 111 -> 80 us,  FP64 260 -> 175 us
 //   52^3 cube, radius 4, 23:        FP32 17.2 -> 15.0,  FP64 30.2 -> 22.0 us
-//   radius 6 (FD12), 103 columns:   256 vectors FP32 1310 -> 1165 us,
+//   128^3 sphere r = 60, radius 6:  256 vectors FP32 1310 -> 1165 us,
 //                                   64 vectors FP64 640 -> 551 us
 //   70^3 cube, 40 vectors:          radius 3 FP32 49 -> 48, radius 2 FP64 87.5 -> 80.5 us
 //   52^3 cube, 150 vectors:         radius 1 FP32 52 -> 48, radius 2 FP64 138 -> 126 us

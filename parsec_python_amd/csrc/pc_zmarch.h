@@ -52,9 +52,10 @@ struct ZMap {
 };
 
 // Fills the map for `grid` with weights w[0..7] (w[0] already the 3D centre
-// weight) and slabs of zw rows.  zc = 6 planes per chunk (measured on a 106^3
-// sphere: 38 us per CG iteration at 6 planes, 41 us at 2), raised in steps of
-// zstep until the workgroups fit kMaxWG.
+// weight) and slabs of zw rows.  zc = 6 planes per chunk (106^3 sphere, one plane
+// of loads in flight: 38 us per CG iteration at 6 planes, 41 us at 2; 25 us with
+// all of 6 planes in flight), raised in steps of zstep until the workgroups fit
+// kMaxWG.
 inline int zmap_init(void* grid, const double* w, ZMap& zm, int* radius, int zw = kZW, int zstep = 1) {
   int ny, nz;
   const int* prow;
