@@ -32,6 +32,15 @@
 
 namespace {
 
+// One way to cut the windows into z-chunks: planes per chunk, chunks of the longest
+// window; over all windows the chunks that have planes and their planes in whole
+// blocks; the longest chunk.
+struct WinSplit {
+  int zc, nzc, wgs;
+  long long planes;
+  int longest;
+};
+
 struct GridDev {
   int nx, ny, nz;
   long long npts;
@@ -45,7 +54,8 @@ struct GridDev {
   int radius;
   double w[8];   // 1D -d2/dx2 weights, centre first (unscaled)
   int4* win;     // stencil_win: windows {first row, first column | columns << 16 | left halo lanes << 28, zb, ze}
-  int nwin, winz;  // their number and mean number of planes
+  int nwin;        // their number
+  std::vector<WinSplit> splits;   // ways to cut them, the longest chunks first
   int winsx;       // wavefronts of 64 columns per row of a window
   int2* pmeta;   // its padded row table {offset, lo | length << 16}, nyp x nzp
   int nyp, nzp;
@@ -461,30 +471,33 @@ void stencil_win(WinArgs g, const T* Y, const T* X, T* Out, const T* V, T ca, T 
   }
 }
 
-// z-chunks: a window's z-range is split where that fills the chip's rounds better.
-// A round is the workgroups that run at once (32 wavefronts per CU in FP32, 16 in
-// FP64 where the registers or the bandwidth allow no more; the 12 wavefronts of
-// radius 6 count as 16); a chunk costs its planes and about 2R + 8 more for its
-// start (the queue's planes, the first loads), so the number of chunks with the
-// fewest rounds x (planes + start) is taken, at least 8 planes per chunk.  Against
-// filling 16,384 wavefronts whatever the rounds: 58^3 cube, 79 vectors, FP64 102 ->
-// 81 us; 62^3, radius 6, 20 vectors, FP64 59 -> 29; 52^3, 23 vectors, FP64 24.5 ->
-// 22.2; against one chunk: C10H8, 49 vectors, FP32 85 -> 81, FP64 186 -> 175 us.
+// z-chunks: a window's z-range is split where that fills the chip better.  The march
+// runs whole blocks of win_ql planes, so chunks are multiples of that.  A CU holds
+// kSlots workgroups (32 wavefronts in FP32, 16 in FP64 where the registers or the
+// bandwidth allow no more; the 12 wavefronts of radius 6 count as 16).  A round of r
+// workgroups per CU costs r + kSlots / 4 for each plane, and 2 planes for its start;
+// its planes are the mean chunk's, nearer to the longest's the fewer rounds there
+// are.  The cheapest cut is taken: 0.8 % slower in the mean than the fastest one over
+// 1,417 cubes and spheres of 18 to 128 points, 1 to 200 vectors, both types.  Against
+// rounds of the whole chip, counted by planes without the blocks: 64^3, 23 vectors,
+// radius 4 FP32 27.4 -> 21 us; 41^3 sphere, 49 vectors, radius 3 FP32 22.5 -> 17,
+// FP64 37 -> 27; 5 % in the mean.
 template <typename T, int R, int SX>
-void win_zchunks(WinArgs& a, int nz, int planes, int nvec) {
-  constexpr long long kRound = 256 * (sizeof(T) == 4 ? 32 : 16) / (SX * (R > 4 ? 16 / SX : win_ty(R, SX)));
-  const long long wgs = (long long)a.nwin * nvec;
-  int best = 1;
+void win_zchunks(WinArgs& a, const std::vector<WinSplit>& splits, int nvec) {
+  constexpr int kSlots = (sizeof(T) == 4 ? 32 : 16) / (SX * (R > 4 ? 16 / SX : win_ty(R, SX)));
   double least = 0.0;
-  for (int n = 1; n <= std::max(1, nz / 8); ++n) {
-    const double cost = (double)((wgs * n + kRound - 1) / kRound) * ((double)planes / n + 2 * R + 8);
-    if (n == 1 || cost < least) {
-      best = n;
+  a.nzc = 0;
+  for (const WinSplit& s : splits) {
+    const long long per_cu = ((long long)s.wgs * nvec + 255) / 256, rest = per_cu % kSlots;
+    const double mean = (double)s.planes / s.wgs, rounds = (double)((per_cu + kSlots - 1) / kSlots);
+    const double len = 2.0 + mean + ((double)s.longest - mean) / rounds;
+    const double cost = len * (1.25 * (double)(per_cu - rest) + (rest ? (double)rest + 0.25 * kSlots : 0.0));
+    if (a.nzc == 0 || cost < least) {
       least = cost;
+      a.zc = s.zc;
+      a.nzc = s.nzc;
     }
   }
-  a.zc = (nz + best - 1) / best;
-  a.nzc = (nz + a.zc - 1) / a.zc;
 }
 
 template <typename T, int R, int SX>
@@ -496,7 +509,7 @@ int launch_win(const GridDev* gd, const T* Y, const T* X, T* Out, const T* V, in
   if (a.nwin == 0) return pc::PC_OK;   // no points
   a.meta = gd->pmeta; a.nyp = gd->nyp; a.nzp = gd->nzp;
   a.ld = ld;
-  win_zchunks<T, R, SX>(a, gd->nz, gd->winz, nvec);
+  win_zchunks<T, R, SX>(a, gd->splits, nvec);
   for (int d = 0; d < 8; ++d) a.w[d] = 0.0;
   a.w[0] = 3.0 * gd->w[0] * scale;
   for (int d = 1; d <= R; ++d) a.w[d] = gd->w[d] * scale;
@@ -891,9 +904,19 @@ int pc_grid_create(int nx, int ny, int nz, const int* row_lo, const int* row_hi,
   // the longest first: what runs last is short
   std::stable_sort(win.begin(), win.end(), [](const int4& x, const int4& y) { return x.w - x.z > y.w - y.z; });
   g->nwin = (int)win.size();
-  long long planes = 0;
-  for (const int4& w : win) planes += w.w - w.z;
-  g->winz = win.empty() ? 0 : (int)(planes / (long long)win.size());
+  const int ql = win_ql(radius), blocks = win.empty() ? 0 : (win[0].w - win[0].z + ql - 1) / ql;
+  for (int n = 1, last = 0; n <= std::min(blocks, 256); ++n) {   // n chunks of about equal numbers b of blocks
+    const int b = (blocks + n - 1) / n;
+    if (b == last) continue;
+    last = b;
+    WinSplit s{b * ql, (blocks + b - 1) / b, 0, 0, b * ql};
+    for (const int4& w : win) {
+      const int n = (w.w - w.z + ql - 1) / ql;
+      s.wgs += (n + b - 1) / b;
+      s.planes += (long long)n * ql;
+    }
+    g->splits.push_back(s);
+  }
   g->nyp = ny + 2 * kWinPadY;
   g->nzp = nz + radius + kWinPadZ;
   std::vector<int2> pmeta((size_t)g->nyp * g->nzp, make_int2(0, 0));
