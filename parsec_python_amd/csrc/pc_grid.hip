@@ -891,12 +891,16 @@ int pc_grid_create(int nx, int ny, int nz, const int* row_lo, const int* row_hi,
   // Two wavefronts per row share one tile, so a row of up to 128 columns has no
   // inner edges: taken where that saves a fifth of the lanes (121 to 128 full
   // columns at radius 4, which are three windows otherwise: 128^3, 23 vectors,
-  // FP64 341 -> 280 us, radius 6 361 -> 298), at radius 1 where it costs none
-  // (126^3, 49 vectors FP32 289 -> 263).  With two windows either way one wavefront
-  // per row is the faster (100^3 FP32 radius 4 11 %, spheres 20 to 40 %).
-  if (nx > 64 && nx <= 128 && most >= (radius == 1 ? 2 : 3)) {
+  // FP64 341 -> 280 us, radius 6 361 -> 298), and where it costs none at radius 1
+  // (126^3, 49 vectors FP32 289 -> 263) and up to radius 4 on rows that are full to
+  // seven eighths (120^3, 23 vectors FP32 radius 2 130 -> 107, 3 130 -> 114, 4 129 ->
+  // 117 us; 112 columns gain nothing at radius 3 and 4).  Elsewhere, with two windows
+  // either way, one wavefront per row is the faster (100^3 radius 4 3 to 15 %,
+  // spheres 5 to 40 %).
+  const bool full = radius <= 4 && 8 * cnt > 7 * 128LL * ny * nz;
+  if (nx > 64 && nx <= 128 && most >= (radius == 1 || full ? 2 : 3)) {
     const long long lanes2 = windows(2, win2);
-    if (radius == 1 ? lanes2 <= lanes1 : 5 * lanes2 <= 4 * lanes1) {
+    if (radius == 1 || full ? lanes2 <= lanes1 : 5 * lanes2 <= 4 * lanes1) {
       g->winsx = 2;
       win.swap(win2);
     }

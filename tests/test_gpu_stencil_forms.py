@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
 # nx, ny, nz, radius
 SHAPES = [(64, 5, 9, 4), (65, 7, 70, 2), (128, 9, 11, 4), (128, 21, 5, 6), (128, 6, 70, 1), (121, 17, 6, 4),
           (120, 17, 6, 4), (117, 9, 8, 6), (116, 9, 8, 6), (127, 11, 7, 1), (126, 10, 7, 2), (123, 8, 9, 3),
-          (129, 6, 5, 4), (200, 3, 6, 6)]
+          (129, 6, 5, 4), (200, 3, 6, 6), (113, 8, 9, 2), (116, 16, 5, 3), (112, 9, 6, 3)]
 
 
 @pytest.mark.parametrize("dtype", ["f64", "f32"])
@@ -114,5 +114,41 @@ def test_stencil_time_per_point_of_wide_cubes(gpu, dtype, nvec):
     narrow, wide = (sorted(t)[4] for t in times)
     print(f"{1e6 * narrow:.3f} and {1e6 * wide:.3f} ns", flush=True)
     assert wide <= 1.1 * narrow
+    for _step, _npts, dg in steps:
+        dg.close()
+
+
+def test_stencil_time_per_point_of_full_rows(gpu):
+    """Radius 2, 23 vectors, FP32: rows of 120 columns cost no more per point than
+    rows of 126 (as two windows of 60 with inner edges 1.2 times)."""
+    import torch
+    from parsec_python_amd import _lib
+    from parsec_python_amd.device import ptr, stream
+    from parsec_python_amd.grid import DeviceGrid, make_grid
+    from parsec_python_amd.hamiltonian import leading_dim
+    steps, times = [], [[], []]
+    for nx in (120, 126):
+        print(f"stencil time {nx}^3", flush=True)
+        g = make_grid(nx, 0.4, 0.2 * (nx - 1), "cube")
+        dg, ld = DeviceGrid(g, 2), leading_dim(g.npts)
+        Y, X = (torch.zeros((23, ld), device="cuda") for _ in range(2))
+        V = torch.zeros(g.npts, device="cuda")
+
+        def step(dg=dg, ld=ld, Y=Y, X=X, V=V):
+            _lib.call("pc_stencil_f32", dg.handle, ptr(Y), ptr(X), ptr(X), ptr(V), 23, ld, 0.5, 1.0, 0.0, 0.5, None, stream())
+        steps.append((step, g.npts, dg))
+    for _ in range(9):
+        for i, (step, npts, _dg) in enumerate(steps):
+            e0, e1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            step()
+            e0.record()
+            for _ in range(4):
+                step()
+            e1.record()
+            torch.cuda.synchronize()
+            times[i].append(e0.elapsed_time(e1) / npts)
+    full, wide = (sorted(t)[4] for t in times)
+    print(f"{1e6 * full:.3f} and {1e6 * wide:.3f} ns", flush=True)
+    assert full <= 1.1 * wide
     for _step, _npts, dg in steps:
         dg.close()
