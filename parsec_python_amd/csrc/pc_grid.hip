@@ -292,7 +292,7 @@ __global__ __launch_bounds__(256) void stencil_zmarch(StArgs g, const T* __restr
 //   70^3 cube, 40 vectors:          radius 3 FP32 49 -> 48, radius 2 FP64 87.5 -> 80.5 us
 //   52^3 cube, 150 vectors:         radius 1 FP32 52 -> 48, radius 2 FP64 138 -> 126 us
 //                                   (55 and 147 us with 8 rows per workgroup)
-//   128^3 cube, 23 vectors (SX 2):  radius 4 FP32 144 -> 156, FP64 291 -> 280 us (174
+//   128^3 cube, 23 vectors (SX 2):  radius 4 FP32 147 -> 141, FP64 292 -> 274 us (174
 //                                   and 341 us as three windows), radius 6 FP64 338 -> 298
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t pc_rsrc(const void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
